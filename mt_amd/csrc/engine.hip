@@ -342,8 +342,8 @@ int mte_destroy(mte_engine *e) {
     if (e->flags_host) (void)hipHostFree(e->flags_host);
     for (auto &kv : e->graphs) (void)hipGraphExecDestroy(kv.second);
     for (void *p : e->allocations) (void)hipFree(p);
-    for (void *p : {(void *)e->mlp.x, (void *)e->mlp.t, (void *)e->mlp.hid, (void *)e->mlp.y, (void *)e->mlp.g4,
-                    (void *)e->mlp.ga, (void *)e->mlp.gb, (void *)e->mlp.partial})
+    for (void *p : {(void *)e->mlp.x, (void *)e->mlp.t, (void *)e->mlp.y, (void *)e->mlp.gpart, (void *)e->mlp.lpart,
+                    (void *)e->mlp.loss})
         if (p) (void)hipFree(p);
     if (e->noise) (void)hipFree(e->noise);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1168,40 +1168,43 @@ static int need_mlp(mte_engine *e) {
     return MTE_OK;
 }
 
-static int mlp_reserve(mte_engine *e, int n) {
+// Device rows for the samples of a call.
+static int mlp_reserve(mte_engine *e, int64_t n) {
     MlpBuffers &M = e->mlp;
     if (n <= M.cap) return MTE_OK;
-    for (void *p : {(void *)M.x, (void *)M.t, (void *)M.hid, (void *)M.y, (void *)M.g4, (void *)M.ga, (void *)M.gb,
-                    (void *)M.partial})
-        if (p) {
-            (void)hipStreamSynchronize(e->stream);
-            (void)hipFree(p);
-        }
+    (void)hipStreamSynchronize(e->stream);
+    for (float **p : {&M.x, &M.t, &M.y}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
     M.cap = 0;
     const size_t nn = (size_t)n;
     if (hipMalloc(&M.x, sizeof(float) * nn * MLP_IN) != hipSuccess ||
         hipMalloc(&M.t, sizeof(float) * nn * MLP_OUT) != hipSuccess ||
-        hipMalloc(&M.hid, sizeof(float) * 3 * nn * MLP_H) != hipSuccess ||
-        hipMalloc(&M.y, sizeof(float) * nn * MLP_OUT) != hipSuccess ||
-        hipMalloc(&M.g4, sizeof(float) * nn * MLP_OUT) != hipSuccess ||
-        hipMalloc(&M.ga, sizeof(float) * nn * MLP_H) != hipSuccess ||
-        hipMalloc(&M.gb, sizeof(float) * nn * MLP_H) != hipSuccess ||
-        hipMalloc(&M.partial, sizeof(double) * ((nn * MLP_OUT + 255) / 256 + 1)) != hipSuccess)
+        hipMalloc(&M.y, sizeof(float) * nn * MLP_OUT) != hipSuccess)
         return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
     M.cap = n;
     return MTE_OK;
 }
 
-static double mlp_loss(mte_engine *e, int n) {
-    const int nblk = (n * MLP_OUT + 255) / 256;
-    std::vector<double> part(nblk);
-    if (hipMemcpyAsync(part.data(), e->mlp.partial, sizeof(double) * nblk, hipMemcpyDeviceToHost, e->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(e->stream) != hipSuccess)
-        return -1.0;
-    double s = 0;
-    for (double v : part) s += v;
-    return s / ((double)n * MLP_OUT);
+// Partial gradients of as many workgroups as training launches at most, and
+// the losses of `iters` iterations.
+static int mlp_reserve_train(mte_engine *e, int iters) {
+    MlpBuffers &M = e->mlp;
+    const size_t nwg = (size_t)mlp_train_groups(e, INT32_MAX);
+    if ((!M.gpart && hipMalloc(&M.gpart, sizeof(float) * nwg * MLP_NPARAM) != hipSuccess) ||
+        (!M.lpart && hipMalloc(&M.lpart, sizeof(double) * nwg) != hipSuccess))
+        return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
+    if (iters > M.loss_cap) {
+        (void)hipStreamSynchronize(e->stream);
+        if (M.loss) (void)hipFree(M.loss);
+        M.loss = nullptr;
+        M.loss_cap = 0;
+        if (hipMalloc(&M.loss, sizeof(double) * (size_t)iters) != hipSuccess)
+            return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
+        M.loss_cap = iters;
+    }
+    return MTE_OK;
 }
 
 int mte_mlp_set_weights(mte_engine *e, const float *w, int64_t n) {
@@ -1246,7 +1249,7 @@ int mte_mlp_forward(mte_engine *e, const float *features, int64_t n, float *out)
     if (rc) return rc;
     if (!features || !out || n <= 0) return fail(e, MTE_ERR_ARG, "mte_mlp_forward: bad arguments");
     HIPCHK(hipSetDevice(e->device));
-    rc = mlp_reserve(e, (int)n);
+    rc = mlp_reserve(e, n);
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(e->mlp.x, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(launch_mlp_forward(e, e->mlp.x, (int)n, e->mlp.y));
@@ -1278,13 +1281,14 @@ int mte_mlp_loss_grad(mte_engine *e, const float *features, const float *labels,
     if (rc) return rc;
     if (!features || !labels || n <= 0) return fail(e, MTE_ERR_ARG, "mte_mlp_loss_grad: bad arguments");
     HIPCHK(hipSetDevice(e->device));
-    rc = mlp_reserve(e, (int)n);
-    if (rc) return rc;
+    if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, 1))) return rc;
     HIPCHK(hipMemcpyAsync(e->mlp.x, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->mlp.t, labels, sizeof(float) * MLP_OUT * n, hipMemcpyHostToDevice, e->stream));
-    HIPCHK(launch_mlp_grad(e, e->mlp.x, e->mlp.t, (int)n));
+    HIPCHK(launch_mlp_grad(e, e->mlp.x, e->mlp.t, (int)n, e->mlp.loss, 0.f, 0));
     if (grad) HIPCHK(hipMemcpyAsync(grad, e->mlp.grad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, e->stream));
-    const double l = mlp_loss(e, (int)n);
+    double l = 0.0;
+    HIPCHK(hipMemcpyAsync(&l, e->mlp.loss, sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipStreamSynchronize(e->stream));
     if (loss) *loss = l;
     return MTE_OK;
 }
@@ -1297,34 +1301,23 @@ int mte_mlp_train(mte_engine *e, const float *features, const float *labels, int
         return fail(e, MTE_ERR_ARG, "mte_mlp_train: bad arguments");
     if (!e->mlp.ready) return fail(e, MTE_ERR_STATE, "mte_mlp_train: set initial weights first");
     HIPCHK(hipSetDevice(e->device));
-    // the whole training set stays on the device; batches are consecutive slices
-    float *X = nullptr, *Y = nullptr;
-    HIPCHK(hipMalloc(&X, sizeof(float) * MLP_IN * n));
-    if (hipMalloc(&Y, sizeof(float) * MLP_OUT * n) != hipSuccess) {
-        (void)hipFree(X);
-        return fail(e, MTE_ERR_HIP, "mte_mlp_train: allocation failed");
+    // the whole training set goes to the device; batches are consecutive
+    // slices, and the losses come back together at the end
+    if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, iters))) return rc;
+    float *X = e->mlp.x, *Y = e->mlp.t;
+    HIPCHK(hipMemcpyAsync(X, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
+    HIPCHK(hipMemcpyAsync(Y, labels, sizeof(float) * MLP_OUT * n, hipMemcpyHostToDevice, e->stream));
+    int64_t pos = 0;
+    for (int it = 0; it < iters; it++) {
+        if (pos + batch > n) pos = 0;
+        HIPCHK(launch_mlp_grad(e, X + pos * MLP_IN, Y + pos * MLP_OUT, batch, e->mlp.loss + it, lr, ++e->mlp.adam_t));
+        pos += batch;
     }
-    rc = mlp_reserve(e, batch);
-    int out = rc;
-    if (!rc) {
-        if (hipMemcpyAsync(X, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream) != hipSuccess ||
-            hipMemcpyAsync(Y, labels, sizeof(float) * MLP_OUT * n, hipMemcpyHostToDevice, e->stream) != hipSuccess)
-            out = fail(e, MTE_ERR_HIP, "mte_mlp_train: upload failed");
-        int64_t pos = 0;
-        for (int it = 0; it < iters && !out; it++) {
-            if (pos + batch > n) pos = 0;
-            hipError_t s = launch_mlp_grad(e, X + pos * MLP_IN, Y + pos * MLP_OUT, batch);
-            if (s == hipSuccess) s = launch_mlp_adam(e, lr, ++e->mlp.adam_t);
-            if (s != hipSuccess) out = fail(e, MTE_ERR_HIP, std::string("mte_mlp_train: ") + hipGetErrorString(s));
-            if (losses && !out) losses[it] = mlp_loss(e, batch);
-            pos += batch;
-        }
-        if (!out && launch_mlp_pack(e) != hipSuccess) out = fail(e, MTE_ERR_HIP, "mte_mlp_train: weight image failed");
-        (void)hipStreamSynchronize(e->stream);
-    }
-    (void)hipFree(X);
-    (void)hipFree(Y);
-    return out;
+    HIPCHK(launch_mlp_pack(e));
+    if (losses && iters > 0)
+        HIPCHK(hipMemcpyAsync(losses, e->mlp.loss, sizeof(double) * iters, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipStreamSynchronize(e->stream));
+    return MTE_OK;
 }
 
 int mte_set_hi_mode(mte_engine *e, int32_t mode, int32_t check_every, float tolerance) {

@@ -99,10 +99,14 @@ struct MlpBuffers {
     double *err = nullptr;                    // per trajectory: squared error, squared label norm
     double *err_part = nullptr;               // their partial sums, MLP_ERR_PARTS per trajectory
     int *nbad = nullptr;                      // beads whose prediction failed the Cholesky check
-    // training work space for up to `cap` samples
-    int cap = 0;
-    float *x = nullptr, *t = nullptr, *hid = nullptr, *y = nullptr, *g4 = nullptr, *ga = nullptr, *gb = nullptr;
-    double *partial = nullptr;
+    // samples of a call (features, labels, outputs) for up to `cap` rows
+    int64_t cap = 0;
+    float *x = nullptr, *t = nullptr, *y = nullptr;
+    // training: partial gradients and squared errors of the workgroups, and
+    // the losses of up to `loss_cap` iterations
+    float *gpart = nullptr;
+    double *lpart = nullptr, *loss = nullptr;
+    int loss_cap = 0;
     int adam_t = 0;
     bool ready = false;                       // weights uploaded or trained
 };
@@ -212,8 +216,8 @@ hipError_t launch_mlp_forward(mte_engine *e, const float *feat, int n, float *ou
 hipError_t noalloc_scratch_init(int device, float **ptr);
 hipError_t launch_mlp_step(mte_engine *e, const float *noise_step, float *yout);
 hipError_t launch_mlp_error(mte_engine *e, const float *y, const float *t);
-hipError_t launch_mlp_grad(mte_engine *e, const float *feat, const float *targ, int n);
-hipError_t launch_mlp_adam(mte_engine *e, float lr, int t);
+int mlp_train_groups(const mte_engine *e, int n);
+hipError_t launch_mlp_grad(mte_engine *e, const float *feat, const float *targ, int n, double *loss, float lr, int t);
 hipError_t launch_mlp_round(mte_engine *e);
 hipError_t launch_mlp_pack(mte_engine *e);
 size_t mlp_image_bytes();

@@ -15,8 +15,9 @@
 // (cs >= 12 nm); inference fused with the integrator on the matrix cores
 // (v_mfma_f32_16x16x32_bf16: bf16 weights, activations carried as bf16
 // hi + lo pairs, FP32 accumulation; the weight fragments sit in LDS and the
-// activations stay in registers from layer to layer); training (forward with
-// stored activations, backward, Adam) in FP32 on the vector ALUs.
+// activations stay in registers from layer to layer); training (forward,
+// backward and weight gradients of a sample tile in one kernel, then the
+// reduction over tiles with the Adam step) in FP32 on the matrix cores.
 #include "engine_internal.h"
 
 #include <mutex>
@@ -24,7 +25,6 @@
 namespace mte {
 
 constexpr int MLP_BLOCK = MLP_SEARCH_BLOCK;
-constexpr int ROW = MLP_H + 1;   // LDS row pitch (odd: no bank conflicts between lanes)
 constexpr float MLP_RC = 12.f, MLP_RIN = 8.f;
 // flat parameter offsets
 constexpr int OW1 = 0, OB1 = OW1 + MLP_IN * MLP_H, OW2 = OB1 + MLP_H, OB2 = OW2 + MLP_H * MLP_H, OW3 = OB2 + MLP_H,
@@ -298,53 +298,6 @@ __global__ void __launch_bounds__(MLP_BLOCK)
 }
 
 // ------------------------------------------------------------------ network
-// One dense layer for this lane's sample: row (LDS, K inputs) -> row (M
-// outputs), weights W[k * M + m] and bias, tanh when `act`.  Outputs are
-// produced in chunks of 64 accumulators.
-template <int K, int M>
-__device__ __forceinline__ void dense_row(float *row, const float *__restrict__ W, const float *__restrict__ bias,
-                                          bool act, float *out_regs) {
-    constexpr int CH = M < 64 ? M : 64;
-    float res[M];
-#pragma unroll
-    for (int m0 = 0; m0 < M; m0 += CH) {
-        float acc[CH];
-#pragma unroll
-        for (int m = 0; m < CH; m++) acc[m] = bias[m0 + m];
-        for (int k = 0; k < K; k++) {
-            const float a = row[k];
-            const float *w = W + k * M + m0;
-#pragma unroll
-            for (int m = 0; m < CH; m++) acc[m] = fmaf(a, w[m], acc[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < CH; m++) res[m0 + m] = act ? tanhf(acc[m]) : acc[m];
-    }
-    if (out_regs) {
-#pragma unroll
-        for (int m = 0; m < M; m++) out_regs[m] = res[m];
-    } else {
-#pragma unroll
-        for (int m = 0; m < M; m++) row[m] = res[m];
-    }
-}
-
-// Full network on the lane's LDS row (features in, 9 outputs to y).
-// keep != nullptr stores the three hidden activations (training).
-__device__ __forceinline__ void mlp_eval(float *row, const float *__restrict__ w, float y[MLP_OUT], float *keep,
-                                         size_t stride) {
-    dense_row<MLP_IN, MLP_H>(row, w + OW1, w + OB1, true, nullptr);
-    if (keep)
-        for (int m = 0; m < MLP_H; m++) keep[m] = row[m];
-    dense_row<MLP_H, MLP_H>(row, w + OW2, w + OB2, true, nullptr);
-    if (keep)
-        for (int m = 0; m < MLP_H; m++) keep[stride + m] = row[m];
-    dense_row<MLP_H, MLP_H>(row, w + OW3, w + OB3, true, nullptr);
-    if (keep)
-        for (int m = 0; m < MLP_H; m++) keep[2 * stride + m] = row[m];
-    dense_row<MLP_H, MLP_OUT>(row, w + OW4, w + OB4, false, y);
-}
-
 // Cholesky factor of the symmetric 3x3 S (row-major); false when a pivot
 // falls below 1e-3 (not positive definite enough to use).
 __device__ __forceinline__ bool chol3(const float S[9], float Lc[6]) {
@@ -800,70 +753,295 @@ __global__ void __launch_bounds__(64) k_mlp_error_sum(int ntraj, const double *p
 }
 
 // ----------------------------------------------------------------- training
-__global__ void __launch_bounds__(MLP_BLOCK)
-    k_mlp_train_fwd(const float *__restrict__ w, const float *feat, int n, float *hid, float *y) {
-    __shared__ float rows[MLP_BLOCK * ROW];
-    const int s = blockIdx.x * MLP_BLOCK + threadIdx.x;
-    if (s >= n) return;
-    float *row = rows + threadIdx.x * ROW;
-    for (int k = 0; k < MLP_IN; k++) row[k] = feat[(size_t)s * MLP_IN + k];
-    float out[MLP_OUT];
-    // hidden layers stored sample-major: hid[(layer * n + s) * H + m]
-    mlp_eval(row, w, out, hid + (size_t)s * MLP_H, (size_t)n * MLP_H);
-    for (int q = 0; q < MLP_OUT; q++) y[(size_t)s * MLP_OUT + q] = out[q];
+// Forward, backward and every weight gradient of a sample tile in one kernel,
+// in FP32 on the matrix cores (v_mfma_f32_16x16x4_f32: FP32 operands and
+// accumulation).  A workgroup of 8 waves takes tiles of 32 samples (one per
+// CU and pass at the usual 8192-sample batch) and keeps their activations in
+// LDS; wave w owns neurons 16 w .. 16 w + 15 of each hidden layer.
+//   forward   D^T = W^T X^T: neurons are the 16 rows, samples the columns.
+//             K step r of block q reads inputs 16 q + 4 g + r (g = lane / 16),
+//             so four steps take one float4 of a sample's row, and the rows a
+//             lane receives (4 g + r of its wave's neurons) are the operand
+//             the output layer needs: its K is split over the waves without
+//             an exchange, the partial outputs added in wave order.
+//   backward  the same with W's rows; dL/d(pre-activation) overwrites the
+//             layer's activations (each wave only its own columns, which no
+//             other wave reads once that layer's weight gradient is taken).
+//   dW        in^T g over the tile's samples; K step st of a 16-sample block
+//             takes samples 4 g + st, which with row pitches of 4 mod 64
+//             words reads LDS without bank conflicts.  The sums stay in
+//             registers over a workgroup's tiles (23 16x16 tiles per wave).
+// Each workgroup writes one partial gradient; k_mlp_reduce adds the partials
+// in a fixed order (no atomics: training repeats bit for bit) and takes the
+// Adam step.
+// Bound at 8192 samples: 504 matrix instructions of 32 cycles per wave, two
+// waves per SIMD: 13 us of 2.27 GFLOP at the FP32 matrix rate, beside the
+// L2 latency of the weights at each layer and 48 MB of partials.
+// Measured per iteration of 8192 samples: 40 us here and 12 us in the
+// reduction; with one thread per sample, per weight and per activation, nine
+// launches, atomics and a read-back of the loss, 1290 us.  777 samples (25
+// workgroups): 34 + 4 us, before 480 us.
+constexpr int TR_TILE = 32, TR_WAVES = MLP_H / 16, TR_THREADS = 64 * TR_WAVES;
+constexpr int TR_PX = MLP_IN + 4, TR_PH = MLP_H + 4, TR_PY = 20;   // LDS row pitches
+constexpr int TR_OX = 0, TR_OH1 = TR_OX + TR_TILE * TR_PX, TR_OH2 = TR_OH1 + TR_TILE * TR_PH,
+              TR_OH3 = TR_OH2 + TR_TILE * TR_PH, TR_OG = TR_OH3 + TR_TILE * TR_PH, TR_OY = TR_OG + TR_TILE * TR_PY,
+              TR_END = TR_OY + TR_WAVES * TR_TILE * TR_PY;   // floats
+constexpr size_t TR_LDS = sizeof(float) * TR_END;
+static_assert(TR_PX % 64 == 36 && TR_PH % 64 == 4 && TR_TILE == 32 && TR_THREADS == 16 * TR_TILE, "training tile");
+
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+__device__ __forceinline__ void st4(float *p, f32x4 v) { *reinterpret_cast<f32x4 *>(p) = v; }
+
+// Keeps the compiler from requesting the operands of all following steps at
+// once (the 104 registers of sums leave no room for them).
+__device__ __forceinline__ void tr_fence() { __asm__ volatile("" ::: "memory"); }
+
+// This lane's share of a layer's weights for its wave's 16 rows: column
+// 16 w + i of W (forward) or row 16 w + i (backward), K of the reduction.
+// `of`: the lane's offset, made opaque once per tile so that the loads take
+// a scalar base and it instead of addresses kept in registers over the loop.
+template <int K>
+__device__ __forceinline__ void tr_wfwd(const float *__restrict__ W, uint32_t of, float (&a)[K / 4]) {
+#pragma unroll
+    for (int q = 0; q < K / 16; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) a[4 * q + r] = (W + (16 * q + r) * MLP_H)[of];
+}
+__device__ __forceinline__ void tr_wbwd(const float *__restrict__ W, uint32_t of, float (&a)[MLP_H / 4]) {
+#pragma unroll
+    for (int q = 0; q < MLP_H / 16; q++) {
+        const f32x4 v = ld4(W + 16 * q + of);
+#pragma unroll
+        for (int r = 0; r < 4; r++) a[4 * q + r] = v[r];
+    }
 }
 
-// dL/dy = 2 (y - t) / (n * 9); per-block squared-error partials.
-__global__ void __launch_bounds__(256)
-    k_mlp_out_grad(const float *y, const float *t, int n, float *g, double *partial) {
-    __shared__ double red[256];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    double e = 0;
-    if (i < n * MLP_OUT) {
-        const float d = y[i] - t[i];
-        g[i] = 2.f * d / (float)(n * MLP_OUT);
-        e = (double)d * d;
+// acc[sc] += the wave's 16 rows over K inputs held in LDS rows of `pitch`.
+template <int K>
+__device__ __forceinline__ void tr_rows(const float (&a)[K / 4], const float *in, int pitch, int g, int i,
+                                        f32x4 (&acc)[2]) {
+#pragma unroll
+    for (int q = 0; q < K / 16; q++) {
+        const f32x4 b0 = ld4(in + i * pitch + 16 * q + 4 * g), b1 = ld4(in + (16 + i) * pitch + 16 * q + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            acc[0] = mfma_f32(a[4 * q + r], b0[r], acc[0]);
+            acc[1] = mfma_f32(a[4 * q + r], b1[r], acc[1]);
+        }
     }
-    red[threadIdx.x] = e;
+}
+
+// Hidden layer: h = tanh(bias + W^T in), kept in registers and written to out.
+template <int K>
+__device__ __forceinline__ void tr_hidden(const float (&a)[K / 4], const float *__restrict__ bias, const float *in,
+                                          int pitch, float *out, int w, int g, int i, f32x4 (&h)[2]) {
+    f32x4 acc[2];
+#pragma unroll
+    for (int r = 0; r < 4; r++) acc[0][r] = acc[1][r] = bias[16 * w + 4 * g + r];
+    tr_rows<K>(a, in, pitch, g, i, acc);
+#pragma unroll
+    for (int sc = 0; sc < 2; sc++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[sc][r] = tanhf(acc[sc][r]);
+        st4(out + (16 * sc + i) * TR_PH + 16 * w + 4 * g, h[sc]);
+    }
+}
+
+// One operand of a weight gradient: column 16 c + i of the tile's rows, the
+// eight K steps of its 32 samples.
+__device__ __forceinline__ void tr_column(const float *m, int pitch, int c, int g, int i, float (&v)[8]) {
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int st = 0; st < 4; st++) v[4 * b + st] = m[(16 * b + 4 * g + st) * pitch + 16 * c + i];
+}
+__device__ __forceinline__ f32x4 tr_outer(const float (&a)[8], const float (&b)[8], f32x4 c) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) c = mfma_f32(a[k], b[k], c);
+    return c;
+}
+
+// Layer W (its inputs' activations h in `in`, its output gradients in `gout`):
+// dW of the wave's 16 input rows, then the gradient at the inputs over the
+// wave's columns of `in`.
+__device__ __forceinline__ void tr_back(const float (&a)[MLP_H / 4], const float *gout, float *in, int w, int g, int i,
+                                        f32x4 (&dw)[MT_H], f32x4 &db) {
+    float col[8];
+    tr_column(in, TR_PH, w, g, i, col);
+#pragma unroll
+    for (int mt = 0; mt < MT_H; mt++) {
+        float b[8];
+        tr_column(gout, TR_PH, mt, g, i, b);
+        dw[mt] = tr_outer(col, b, dw[mt]);
+        tr_fence();
+    }
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    tr_rows<MLP_H>(a, gout, TR_PH, g, i, acc);
+#pragma unroll
+    for (int sc = 0; sc < 2; sc++) {
+        float *own = in + (16 * sc + i) * TR_PH + 16 * w + 4 * g;
+        const f32x4 h = ld4(own);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[sc][r] *= 1.f - h[r] * h[r];
+        st4(own, acc[sc]);
+    }
+    db += acc[0] + acc[1];
+}
+
+__global__ void __launch_bounds__(TR_THREADS)
+    k_mlp_train(const float *__restrict__ w, const float *__restrict__ feat, const float *__restrict__ targ, int n,
+                float *__restrict__ gpart, double *__restrict__ lpart) {
+    extern __shared__ float tr_lds[];
+    float *X = tr_lds + TR_OX, *H1 = tr_lds + TR_OH1, *H2 = tr_lds + TR_OH2, *H3 = tr_lds + TR_OH3,
+          *G = tr_lds + TR_OG, *Y = tr_lds + TR_OY;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, i = lane & 15;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 dw1[MLP_IN / 16], dw2[MT_H], dw3[MT_H], dw4 = zero, db1 = zero, db2 = zero, db3 = zero;
+#pragma unroll
+    for (int k = 0; k < MLP_IN / 16; k++) dw1[k] = zero;
+#pragma unroll
+    for (int k = 0; k < MT_H; k++) dw2[k] = dw3[k] = zero;
+    float db4 = 0.f;
+    double loss = 0.0;
+    const float scale = 2.f / ((float)n * (float)MLP_OUT);
+    const int ntiles = (n + TR_TILE - 1) / TR_TILE;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int s0 = tile * TR_TILE;
+        uint32_t of = 4 * g * MLP_H + 16 * wv + i, ob = (16 * wv + i) * MLP_H + 4 * g;
+        __asm__ volatile("" : "+v"(of), "+v"(ob));
+        float a1[MLP_IN / 4], a2[MLP_H / 4];
+        tr_wfwd<MLP_IN>(w + OW1, of, a1);
+        for (int k = tid; k < TR_TILE * MLP_IN / 4; k += TR_THREADS) {
+            const int s = k / (MLP_IN / 4), c = k % (MLP_IN / 4);
+            st4(X + s * TR_PX + 4 * c, s0 + s < n ? ld4(feat + (size_t)(s0 + s) * MLP_IN + 4 * c) : zero);
+        }
+        __syncthreads();
+        f32x4 h[2], h3[2];
+        tr_wfwd<MLP_H>(w + OW2, of, a2);
+        tr_hidden<MLP_IN>(a1, w + OB1, X, TR_PX, H1, wv, g, i, h);
+        __syncthreads();
+        float a3[MLP_H / 4];
+        tr_wfwd<MLP_H>(w + OW3, of, a3);
+        tr_hidden<MLP_H>(a2, w + OB2, H1, TR_PH, H2, wv, g, i, h);
+        __syncthreads();
+        // output layer weights in both directions, and layer 3's rows for the way back
+        float o4[4], b4[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            o4[r] = i < MLP_OUT ? w[OW4 + (16 * wv + 4 * g + r) * MLP_OUT + i] : 0.f;
+            b4[r] = 4 * g + r < MLP_OUT ? w[OW4 + (16 * wv + i) * MLP_OUT + 4 * g + r] : 0.f;
+        }
+        float r3[MLP_H / 4];
+        tr_wbwd(w + OW3, ob, r3);
+        tr_hidden<MLP_H>(a3, w + OB3, H2, TR_PH, H3, wv, g, i, h3);
+        // output layer: this wave's 16 inputs, which its lanes hold
+#pragma unroll
+        for (int sc = 0; sc < 2; sc++) {
+            f32x4 y = zero;
+#pragma unroll
+            for (int r = 0; r < 4; r++) y = mfma_f32(o4[r], h3[sc][r], y);
+            st4(Y + (wv * TR_TILE + 16 * sc + i) * TR_PY + 4 * g, y);
+        }
+        __syncthreads();
+        {   // one thread per (sample, output of 16): dL/dy and the squared error
+            const int s = tid / 16, o = tid % 16;
+            float gy = 0.f;
+            if (o < MLP_OUT && s0 + s < n) {
+                float y = w[OB4 + o];
+#pragma unroll
+                for (int v = 0; v < TR_WAVES; v++) y += Y[(v * TR_TILE + s) * TR_PY + o];
+                const float d = y - targ[(size_t)(s0 + s) * MLP_OUT + o];
+                gy = scale * d;
+                loss += (double)d * d;
+            }
+            G[s * TR_PY + o] = gy;
+            db4 += gy;
+        }
+        __syncthreads();
+        float r2[MLP_H / 4];
+        tr_wbwd(w + OW2, ob, r2);
+        {
+            float hc[8], gc[8];
+            tr_column(H3, TR_PH, wv, g, i, hc);
+            tr_column(G, TR_PY, 0, g, i, gc);
+            dw4 = tr_outer(hc, gc, dw4);
+            f32x4 acc[2] = {zero, zero};
+#pragma unroll
+            for (int sc = 0; sc < 2; sc++) {
+                const f32x4 gy = ld4(G + (16 * sc + i) * TR_PY + 4 * g);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[sc] = mfma_f32(b4[r], gy[r], acc[sc]);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[sc][r] *= 1.f - h3[sc][r] * h3[sc][r];
+                st4(H3 + (16 * sc + i) * TR_PH + 16 * wv + 4 * g, acc[sc]);
+            }
+            db3 += acc[0] + acc[1];
+        }
+        __syncthreads();
+        tr_back(r3, H3, H2, wv, g, i, dw3, db2);
+        __syncthreads();
+        tr_back(r2, H2, H1, wv, g, i, dw2, db1);
+        {   // layer 1: the wave's own gradient columns against every input
+            float gc[8];
+            tr_column(H1, TR_PH, wv, g, i, gc);
+#pragma unroll
+            for (int kt = 0; kt < MLP_IN / 16; kt++) {
+                float xc[8];
+                tr_column(X, TR_PX, kt, g, i, xc);
+                dw1[kt] = tr_outer(xc, gc, dw1[kt]);
+                tr_fence();
+            }
+        }
+        __syncthreads();   // the tile's rows are free
+    }
+    float *gp = gpart + (size_t)blockIdx.x * MLP_NPARAM;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int k = 16 * wv + 4 * g + r;
+#pragma unroll
+        for (int kt = 0; kt < MLP_IN / 16; kt++) gp[OW1 + (16 * kt + 4 * g + r) * MLP_H + 16 * wv + i] = dw1[kt][r];
+#pragma unroll
+        for (int mt = 0; mt < MT_H; mt++) {
+            gp[OW2 + k * MLP_H + 16 * mt + i] = dw2[mt][r];
+            gp[OW3 + k * MLP_H + 16 * mt + i] = dw3[mt][r];
+        }
+        if (i < MLP_OUT) gp[OW4 + k * MLP_OUT + i] = dw4[r];
+        // bias gradients: over the 16 sample columns of the wave
+        float b1 = db1[r], b2 = db2[r], b3 = db3[r];
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) {
+            b1 += __shfl_xor(b1, m);
+            b2 += __shfl_xor(b2, m);
+            b3 += __shfl_xor(b3, m);
+        }
+        if (i == 0) {
+            gp[OB1 + k] = b1;
+            gp[OB2 + k] = b2;
+            gp[OB3 + k] = b3;
+        }
+    }
+    // output bias and loss: over the workgroup's threads, in a fixed order
+    float *rb = tr_lds;
+    double *rl = reinterpret_cast<double *>(tr_lds + TR_THREADS);
+    rb[tid] = db4;
+    rl[tid] = loss;
     __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+    for (int k = TR_THREADS / 2; k >= 16; k >>= 1) {
+        if (tid < k) {
+            rb[tid] += rb[tid + k];
+            rl[tid] += rl[tid + k];
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// dW[k][m] = sum_s in[s][k] g[s][m]; row k == K holds db[m] = sum_s g[s][m].
-// blockIdx.y splits the samples into DW_SPLIT slices added atomically into
-// zeroed dW / db.
-constexpr int DW_SPLIT = 32;
-__global__ void __launch_bounds__(256)
-    k_mlp_dw(const float *in, const float *g, int n, int K, int M, float *dW, float *db) {
-    const int id = blockIdx.x * 256 + threadIdx.x;
-    if (id >= (K + 1) * M) return;
-    const int k = id / M, m = id % M;
-    const int per = (n + DW_SPLIT - 1) / DW_SPLIT;
-    const int s0 = blockIdx.y * per, s1 = min(n, s0 + per);
-    float acc = 0.f;
-    if (k < K) {
-        for (int s = s0; s < s1; s++) acc = fmaf(in[(size_t)s * K + k], g[(size_t)s * M + m], acc);
-        atomicAdd(&dW[k * M + m], acc);
-    } else {
-        for (int s = s0; s < s1; s++) acc += g[(size_t)s * M + m];
-        atomicAdd(&db[m], acc);
+    if (tid < MLP_OUT) gp[OB4 + tid] = rb[tid];
+    if (tid == 0) {
+        double s = 0.0;
+        for (int k = 0; k < 16; k++) s += rl[k];
+        lpart[blockIdx.x] = s;
     }
-}
-
-// gin[s][k] = (sum_m g[s][m] W[k][m]) (1 - h[s][k]^2)   (tanh derivative)
-__global__ void __launch_bounds__(256)
-    k_mlp_dx(const float *g, const float *__restrict__ W, const float *h, int n, int K, int M, float *gin) {
-    const int id = blockIdx.x * 256 + threadIdx.x;
-    if (id >= n * K) return;
-    const int s = id / K, k = id % K;
-    float acc = 0.f;
-    for (int m = 0; m < M; m++) acc = fmaf(g[(size_t)s * M + m], W[k * M + m], acc);
-    const float hv = h[(size_t)s * K + k];
-    gin[id] = acc * (1.f - hv * hv);
 }
 
 __device__ __forceinline__ float round_bf16(float v) {
@@ -872,26 +1050,60 @@ __device__ __forceinline__ float round_bf16(float v) {
     return __uint_as_float(u);
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master weights; refreshes the
-// bf16-rounded copy used by inference.
-__global__ void __launch_bounds__(256)
-    k_mlp_adam(float *w, const float *g, float *m1, float *m2, float *wi, int n, float lr, float b1, float b2,
-               float eps, float c1, float c2) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.f - b1) * gi;
-    const float v = b2 * m2[i] + (1.f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = v;
-    const float nw = w[i] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-    w[i] = nw;
-    wi[i] = round_bf16(nw);
-}
+// Adam step (Kingma & Ba 2015) of the FP32 master weights: moment decay
+// rates, step size and the two bias corrections of this step.
+struct AdamStep {
+    float *w, *m1, *m2, *wi;   // wi: the bf16-rounded copy used by inference
+    float lr, b1, b2, eps, c1, c2;
+};
 
-__global__ void __launch_bounds__(256) k_fill_f32(float *p, int n, float v) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
+// The gradient, the workgroups' partials added in a fixed order (four waves
+// take a quarter of them each, sixteen loads in flight per lane), the Adam
+// step where w is given, and the mean squared error.  Bound by reading the
+// partials (48 MB from 256 workgroups).
+constexpr int RED_PARAMS = 64, RED_WAVES = 4;
+__global__ void __launch_bounds__(RED_PARAMS * RED_WAVES)
+    k_mlp_reduce(const float *__restrict__ gpart, const double *__restrict__ lpart, int nwg, int n, float *grad,
+                 double *loss, AdamStep A) {
+    __shared__ float part[RED_WAVES][RED_PARAMS];
+    const int lane = threadIdx.x % RED_PARAMS, wv = threadIdx.x / RED_PARAMS;
+    const int p = blockIdx.x * RED_PARAMS + lane;
+    const int per = (nwg + RED_WAVES - 1) / RED_WAVES, k0 = wv * per, k1 = min(nwg, k0 + per);
+    float s = 0.f;
+    if (p < MLP_NPARAM) {
+        const float *q = gpart + (size_t)k0 * MLP_NPARAM + p;
+        int k = k0;
+        for (; k + 16 <= k1; k += 16, q += (size_t)16 * MLP_NPARAM) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = q[(size_t)u * MLP_NPARAM];
+#pragma unroll
+            for (int u = 0; u < 16; u++) s += v[u];
+        }
+        for (; k < k1; k++, q += MLP_NPARAM) s += *q;
+    }
+    part[wv][lane] = s;
+    __syncthreads();
+    if (wv == 0 && p < MLP_NPARAM) {
+        const float gi = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+        grad[p] = gi;
+        if (A.w) {
+            const float a = A.b1 * A.m1[p] + (1.f - A.b1) * gi;
+            const float v = A.b2 * A.m2[p] + (1.f - A.b2) * gi * gi;
+            A.m1[p] = a;
+            A.m2[p] = v;
+            const float nw = A.w[p] - A.lr * (a / A.c1) / (sqrtf(v / A.c2) + A.eps);
+            A.w[p] = nw;
+            A.wi[p] = round_bf16(nw);
+        }
+    }
+    if (blockIdx.x == 0 && wv == 1) {
+        double e = 0.0;
+        for (int k = lane; k < nwg; k += RED_PARAMS) e += lpart[k];
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) e += __shfl_xor(e, m);
+        if (lane == 0) *loss = e / ((double)n * MLP_OUT);
+    }
 }
 
 __global__ void __launch_bounds__(256) k_mlp_round(const float *w, float *wi, int n) {
@@ -965,40 +1177,28 @@ hipError_t launch_mlp_error(mte_engine *e, const float *y, const float *t) {
     return hipGetLastError();
 }
 
-// Forward + backward over n samples already on the device; gradient into
-// e->mlp.grad, squared-error partials into e->mlp.partial.
-hipError_t launch_mlp_grad(mte_engine *e, const float *feat, const float *targ, int n) {
-    MlpBuffers &M = e->mlp;
-    const size_t H = MLP_H;
-    float *h1 = M.hid, *h2 = M.hid + (size_t)n * H, *h3 = M.hid + 2 * (size_t)n * H;
-    hipLaunchKernelGGL(k_mlp_train_fwd, dim3(blocks(n, MLP_BLOCK)), dim3(MLP_BLOCK), 0, e->stream, M.w, feat, n,
-                       M.hid, M.y);
-    hipLaunchKernelGGL(k_mlp_out_grad, dim3(blocks(n * MLP_OUT, 256)), dim3(256), 0, e->stream, M.y, targ, n, M.g4,
-                       M.partial);
-    float *gw = M.grad;
-    hipLaunchKernelGGL(k_fill_f32, dim3(blocks(MLP_NPARAM, 256)), dim3(256), 0, e->stream, gw, MLP_NPARAM, 0.f);
-    hipLaunchKernelGGL(k_mlp_dw, dim3(blocks((MLP_H + 1) * MLP_OUT, 256), DW_SPLIT), dim3(256), 0, e->stream, h3,
-                       M.g4, n, MLP_H, MLP_OUT, gw + OW4, gw + OB4);
-    hipLaunchKernelGGL(k_mlp_dx, dim3(blocks(n * MLP_H, 256)), dim3(256), 0, e->stream, M.g4, M.w + OW4, h3, n,
-                       MLP_H, MLP_OUT, M.ga);
-    hipLaunchKernelGGL(k_mlp_dw, dim3(blocks((MLP_H + 1) * MLP_H, 256), DW_SPLIT), dim3(256), 0, e->stream, h2, M.ga,
-                       n, MLP_H, MLP_H, gw + OW3, gw + OB3);
-    hipLaunchKernelGGL(k_mlp_dx, dim3(blocks(n * MLP_H, 256)), dim3(256), 0, e->stream, M.ga, M.w + OW3, h2, n,
-                       MLP_H, MLP_H, M.gb);
-    hipLaunchKernelGGL(k_mlp_dw, dim3(blocks((MLP_H + 1) * MLP_H, 256), DW_SPLIT), dim3(256), 0, e->stream, h1, M.gb,
-                       n, MLP_H, MLP_H, gw + OW2, gw + OB2);
-    hipLaunchKernelGGL(k_mlp_dx, dim3(blocks(n * MLP_H, 256)), dim3(256), 0, e->stream, M.gb, M.w + OW2, h1, n,
-                       MLP_H, MLP_H, M.ga);
-    hipLaunchKernelGGL(k_mlp_dw, dim3(blocks((MLP_IN + 1) * MLP_H, 256), DW_SPLIT), dim3(256), 0, e->stream, feat,
-                       M.ga, n, MLP_IN, MLP_H, gw + OW1, gw + OB1);
-    return hipGetLastError();
+// Workgroups of k_mlp_train, and so partial gradients, at most.
+int mlp_train_groups(const mte_engine *e, int n) {
+    return (int)std::min<int64_t>(((int64_t)n + TR_TILE - 1) / TR_TILE, e->num_cus);
 }
 
-hipError_t launch_mlp_adam(mte_engine *e, float lr, int t) {
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
-    hipLaunchKernelGGL(k_mlp_adam, dim3(blocks(MLP_NPARAM, 256)), dim3(256), 0, e->stream, e->mlp.w, e->mlp.grad,
-                       e->mlp.m1, e->mlp.m2, e->mlp.wi, MLP_NPARAM, lr, b1, b2, 1e-8f, c1, c2);
+// Gradient of n samples already on the device into e->mlp.grad and their
+// mean squared error into *loss (device); with t > 0 also Adam step t.
+hipError_t launch_mlp_grad(mte_engine *e, const float *feat, const float *targ, int n, double *loss, float lr, int t) {
+    MlpBuffers &M = e->mlp;
+    const hipError_t s = hipFuncSetAttribute((const void *)k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)TR_LDS);
+    if (s != hipSuccess) return s;
+    const int nwg = mlp_train_groups(e, n);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(TR_THREADS), TR_LDS, e->stream, M.w, feat, targ, n, M.gpart,
+                       M.lpart);
+    AdamStep A{};
+    if (t > 0) {
+        const float b1 = 0.9f, b2 = 0.999f;
+        A = AdamStep{M.w, M.m1, M.m2, M.wi, lr, b1, b2, 1e-8f, 1.f - powf(b1, (float)t), 1.f - powf(b2, (float)t)};
+    }
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(MLP_NPARAM, RED_PARAMS)), dim3(RED_PARAMS * RED_WAVES), 0, e->stream,
+                       (const float *)M.gpart, (const double *)M.lpart, nwg, n, M.grad, loss, A);
     return hipGetLastError();
 }
 
