@@ -47,11 +47,12 @@ static void release(mte_engine *e, void *p) {
 
 // Work units (trajectory, 256-bead i group, j chunk) of the TEA pair kernel
 // and its per-chunk partial buffer, for j-chunks of `chunk` beads; for
-// MTE_TEA_SYMMETRIC and MTE_TEA_MFMA, units (trajectory, 64-bead chunk I,
-// chunk J >= I) (for MTE_TEA_SYMMETRIC, one or two I chunks below J), and
-// for MTE_TEA_MFMA the tile tables as well.
+// MTE_TEA_SYMMETRIC, units (trajectory, pair of 64-bead chunks I, run of
+// chunks J at or above it); for MTE_TEA_MFMA, units (trajectory, chunk I,
+// chunk J >= I) and the tile tables.
 hipError_t mte::tea_build_units(mte_engine *e, int chunk) {
     release(e, e->tea.units);
+    release(e, e->tea.pair_units);
     release(e, e->tea.nchunks);
     release(e, e->tea.partial);
     release(e, e->tea.tiles);
@@ -60,6 +61,7 @@ hipError_t mte::tea_build_units(mte_engine *e, int chunk) {
     release(e, e->tea.rec);
     release(e, e->tea.rbead);
     e->tea.units = nullptr;
+    e->tea.pair_units = nullptr;
     e->tea.nchunks = nullptr;
     e->tea.partial = nullptr;
     e->tea.tiles = nullptr;
@@ -71,16 +73,40 @@ hipError_t mte::tea_build_units(mte_engine *e, int chunk) {
     std::vector<int4> units;
     std::vector<int> nchunks(e->ntraj, 0);
     int maxc = 0;
+    e->tea.jrun = 1;
+    e->tea.split = 1;
+    if (chunk == MTE_TEA_SYMMETRIC) {
+        // Blocks of (I pair, J chunk), and how a unit takes them.  Few: each
+        // block is a unit of its own, shared by several waves: a block's 128
+        // pair steps by one wave, alone on its SIMD, take 20 us.  Eight waves
+        // below two blocks per SIMD (312 beads: 18.4 -> 5.8 us), four below
+        // seven (64 x 1040 beads, 5 per SIMD: 46 -> 44 us; at 10 per SIMD the
+        // split costs more than the tail, 75 against 82 us).  Many: up to
+        // TEA_JRUN_MAX J chunks per unit, which writes its i-side sums once
+        // for all of them, while at least twelve units per SIMD are left to
+        // balance.
+        int64_t blocks = 0;
+        for (int t = 0; t < e->ntraj; t++) {
+            const int64_t c = (e->off[t + 1] - e->off[t] + 63) / 64, p = (c + 1) / 2;
+            blocks += p * c - p * (p - 1);   // c - 2 k over the pairs k
+        }
+        const int64_t simds = 4 * (int64_t)e->num_cus;
+        if (blocks < 2 * simds) e->tea.split = 8;
+        else if (blocks < 7 * simds) e->tea.split = 4;
+        while (e->tea.jrun < TEA_JRUN_MAX && blocks / (2 * e->tea.jrun) >= 12 * simds) e->tea.jrun *= 2;
+    }
+    const int jrun = e->tea.jrun;
     for (int t = 0; t < e->ntraj; t++) {
         const int n = (int)(e->off[t + 1] - e->off[t]);
         int c = 0;
         if (chunk == MTE_TEA_SYMMETRIC) {
-            // (trajectory, I, J, number of I chunks): the diagonal chunk
-            // alone, the chunks below J two at a time (I and I + 64)
-            for (int j0 = 0; j0 < n; j0 += 64, c++) {
-                units.push_back(make_int4(t, j0, j0, 1));
-                for (int i0 = 0; i0 < j0; i0 += 128) units.push_back(make_int4(t, i0, j0, i0 + 64 < j0 ? 2 : 1));
-            }
+            // (trajectory, I pair, first J, J count) over runs of jrun chunks
+            c = (n + 63) / 64;
+            for (int p = 0; 2 * p < c; p++)
+                for (int r = 2 * p / jrun; r * jrun < c; r++) {
+                    const int j0 = std::max(2 * p, r * jrun), j1 = std::min(c, (r + 1) * jrun);
+                    units.push_back(make_int4(t, p, j0, j1 - j0));
+                }
         } else if (chunk == MTE_TEA_MFMA) {
             for (int i0 = 0; i0 < n; i0 += 64, c++)
                 for (int j0 = i0; j0 < n; j0 += 64) units.push_back(make_int4(t, i0, j0, c));
@@ -92,11 +118,14 @@ hipError_t mte::tea_build_units(mte_engine *e, int chunk) {
         maxc = std::max(maxc, c);
     }
     if (chunk == MTE_TEA_SYMMETRIC || chunk == MTE_TEA_MFMA) {
-        // longest first: off-diagonal blocks (64 steps of both sides), then
-        // diagonal blocks (one-sided, one step per bead of the chunk)
+        // longest first, by pair steps: 64 for two chunks, 32 (symmetric
+        // form) or one per bead of the chunk for a chunk against itself
         auto cost = [&](const int4 &u) {
             const int n = (int)(e->off[u.x + 1] - e->off[u.x]);
-            return u.y == u.z ? std::min(64, n - u.z) : (chunk == MTE_TEA_SYMMETRIC ? 128 * u.w : 128);
+            if (chunk == MTE_TEA_MFMA) return u.y == u.z ? std::min(64, n - u.z) : 128;
+            int steps = 0;
+            for (int j = u.z; j < u.z + u.w; j++) steps += j == 2 * u.y ? 32 : j == 2 * u.y + 1 ? 96 : 128;
+            return steps;
         };
         std::stable_sort(units.begin(), units.end(),
                          [&](const int4 &a, const int4 &b) { return cost(a) > cost(b); });
@@ -142,17 +171,35 @@ hipError_t mte::tea_build_units(mte_engine *e, int chunk) {
             return s;
     }
     hipError_t s;
-    if ((s = dalloc(e, &e->tea.units, units.size())) != hipSuccess) return s;
     if ((s = dalloc(e, &e->tea.nchunks, (size_t)e->ntraj)) != hipSuccess) return s;
-    if ((s = dalloc(e, &e->tea.partial, (size_t)maxc * e->nb)) != hipSuccess) return s;
-    if ((s = hipMemcpyAsync(e->tea.units, units.data(), sizeof(int4) * units.size(), hipMemcpyHostToDevice,
-                            e->stream)) != hipSuccess)
+    if (chunk == MTE_TEA_SYMMETRIC) {
+        // slots: the I pairs, then the J runs
+        e->tea.ioff = (maxc + 1) / 2;
+        float *part = nullptr;
+        if ((s = dalloc(e, &part, (size_t)3 * (e->tea.ioff + (maxc + jrun - 1) / jrun) * e->nb)) != hipSuccess) return s;
+        e->tea.partial = reinterpret_cast<float4 *>(part);
+    } else if ((s = dalloc(e, &e->tea.partial, (size_t)maxc * e->nb)) != hipSuccess) {
         return s;
+    }
+    std::vector<PairUnit> pu;
+    if (chunk == MTE_TEA_SYMMETRIC) {
+        for (const int4 &u : units)
+            pu.push_back(PairUnit{(int)e->off[u.x], (int)(e->off[u.x + 1] - e->off[u.x]), e->box_h[u.x], u.y, u.z,
+                                  u.w, {0, 0}});
+        if ((s = dalloc(e, &e->tea.pair_units, pu.size())) != hipSuccess) return s;
+        if ((s = hipMemcpyAsync(e->tea.pair_units, pu.data(), sizeof(PairUnit) * pu.size(), hipMemcpyHostToDevice,
+                                e->stream)) != hipSuccess)
+            return s;
+    } else {
+        if ((s = dalloc(e, &e->tea.units, units.size())) != hipSuccess) return s;
+        if ((s = hipMemcpyAsync(e->tea.units, units.data(), sizeof(int4) * units.size(), hipMemcpyHostToDevice,
+                                e->stream)) != hipSuccess)
+            return s;
+    }
     if ((s = hipMemcpyAsync(e->tea.nchunks, nchunks.data(), sizeof(int) * nchunks.size(), hipMemcpyHostToDevice,
                             e->stream)) != hipSuccess)
         return s;
     e->tea.nunits = (int)units.size();
-    e->tea.max_chunks = maxc;
     e->tea.unit_chunk = chunk;
     e->tune.tea_chunk = chunk;
     return hipStreamSynchronize(e->stream);
@@ -379,6 +426,12 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
     const int nb = (int)e->off[nt];
     e->nb = nb;
     e->ntraj = nt;
+    e->box_h.assign(nt, 0.f);
+    if (topo->box) std::copy(topo->box, topo->box + nt, e->box_h.begin());
+    for (int t = 0; t < nt; t++) {
+        if (!(e->box_h[t] >= 0.f)) { e->err = "mte_create: periodic box side must be >= 0"; return bail(MTE_ERR_ARG); }
+        if (e->box_h[t] > 0.f) e->periodic = true;
+    }
     e->tune.stream_block = 256;
     e->tune.tea_chunk = 0;   // set when TEA's work units are built
     e->tune.cell_stencil = 1;
@@ -473,7 +526,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
     ALLOC(e->seeds, (size_t)2 * nb) ALLOC(e->fxyz, nb) ALLOC(e->fang, nb) ALLOC(e->en_bead, (size_t)7 * nb)
     ALLOC(e->en_traj, (size_t)7 * nt)
     if (e->P.tea_on) {
-        ALLOC(e->tea.ci, nb) ALLOC(e->tea.eps, nb) ALLOC(e->tea.beta, nt) ALLOC(e->tea.stats, 2 * nt)
+        ALLOC(e->tea.ci, nb) ALLOC(e->tea.bc, nb) ALLOC(e->tea.eps, nb) ALLOC(e->tea.beta, nt) ALLOC(e->tea.stats, 2 * nt)
         ALLOC(e->tea.status, 1) ALLOC(e->tea.R, nb)
         if (tea_build_units(e, TEA_CHUNK_BEADS) != hipSuccess || tea_build_eps_units(e) != hipSuccess) {
             e->err = "mte_create: TEA work units";
@@ -495,12 +548,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
         if (topo->on_tubule) ont[b] = topo->on_tubule[b];
     }
     if (topo->wall_z) std::copy(topo->wall_z, topo->wall_z + nt, zs.begin());
-    std::vector<float> box(nt, 0.f);
-    if (topo->box) std::copy(topo->box, topo->box + nt, box.begin());
-    for (int t = 0; t < nt; t++) {
-        if (!(box[t] >= 0.f)) { e->err = "mte_create: periodic box side must be >= 0"; return bail(MTE_ERR_ARG); }
-        if (box[t] > 0.f) e->periodic = true;
-    }
+    const std::vector<float> &box = e->box_h;
     std::vector<uint32_t> seeds((size_t)8 * nb);
     generate_seeds(opt->rseed, seeds.size(), seeds.data());
 

@@ -18,19 +18,31 @@ struct TimingSlot {
     int64_t launches = 0;
 };
 
+// Work unit of the symmetric TEA pair kernel (k_tea_pairs_sym): a trajectory
+// (first bead, beads, box), a pair of its 64-bead chunks and a run of chunks
+// at or above it.
+struct alignas(16) PairUnit {
+    int base, n;
+    float box;
+    int pair, J0, nJ, pad[2];
+};
+
 struct TeaBuffers {
+    float4 *bc = nullptr;      // per bead: beta C of the last refresh
     float4 *ci = nullptr;      // per bead: row sums of squares of D_hat (x, y, z)
     float *eps = nullptr;      // per bead: sum of all D_hat entries
     float *beta = nullptr;     // per trajectory
     double *stats = nullptr;   // per trajectory: eps, beta (FP64)
     int *status = nullptr;     // first capricious failure (1 + traj) or 0
-    float4 *R = nullptr;       // per bead: scaled random force
+    float4 *R = nullptr;       // per bead: scaled random force (extra beads: zero)
     int4 *units = nullptr;     // pair work units: traj, i0, j0, chunk index
+    PairUnit *pair_units = nullptr;   // or those of MTE_TEA_SYMMETRIC
     int nunits = 0;
     int unit_chunk = 0;        // j-chunk length the units were built for (the pair kernel's CHUNK)
     int *nchunks = nullptr;    // per trajectory
-    int max_chunks = 0;
-    float4 *partial = nullptr; // max_chunks x nb pair partial sums
+    float4 *partial = nullptr; // pair partial sums: slots x nb (MTE_TEA_SYMMETRIC: 3 floats a bead and slot)
+    int jrun = 1, ioff = 0;    // MTE_TEA_SYMMETRIC: J chunks per unit at most, first i-side slot
+    int split = 1;             // and waves per unit
     // MTE_TEA_MFMA: 64-bead tiles of the spatial order (trajectory, first
     // position), and per tile the bf16 hi/lo moment tables [2][64 columns]
     // [64 beads], the centre and radius, and the bead records [4][64] and
@@ -55,6 +67,9 @@ struct TeaBuffers {
 // largest partial-sum buffer it may take.
 constexpr int EPS_GROUP = 1024;
 constexpr size_t EPS_PART_MAX_BYTES = size_t(6) << 30;
+
+// MTE_TEA_SYMMETRIC: J chunks that a unit takes at most.
+constexpr int TEA_JRUN_MAX = 8;
 
 // j-chunk length of the TEA pair kernel.
 constexpr int TEA_CHUNK_BEADS = 128;
@@ -149,6 +164,7 @@ struct mte_engine {
     int *rb_order = nullptr;   // per trajectory: local bead handled at each rebuild position (spatial order)
     int *res_order = nullptr;  // per trajectory: local bead at each resident lane slot (immobile beads last)
     std::vector<uint8_t> fixed_h;   // host copy of the fixed flags (the resident lane order)
+    std::vector<float> box_h;        // and of the periodic box sides
     int res_mobile_max = 0;          // most mobile beads in one trajectory (the resident plan)
     bool any_extra = false;          // some bead is flagged extra (TEA's epsilon weights are needed)
     int *mtl_counts = nullptr, *mtl_flags = nullptr;   // mte_mt_length: per trajectory, per bead

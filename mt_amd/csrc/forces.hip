@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(BS)
             r = normals4(s);
             D.seeds[b] = s;
         }
-        D.R[b] = make_float4(r.x * var, r.y * var, r.z * var, 0.f);
+        D.R[b] = T.extra[b] ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
     }
 }
 
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(FORCE_TILE)
             r = normals4(s);
             D.seeds[b] = s;
         }
-        D.R[b] = make_float4(r.x * var, r.y * var, r.z * var, 0.f);
+        D.R[b] = T.extra[b] ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
     }
 }
 

@@ -361,9 +361,11 @@ __global__ void __launch_bounds__(256)
     eps[b] = s[4];
 }
 
-// FP64 epsilon / beta per trajectory, one workgroup each.
+// FP64 epsilon / beta per trajectory, one workgroup each; then beta C of its
+// beads.
 __global__ void __launch_bounds__(256)
-    k_tea_beta(mte_params P, DevTopo T, const float *eps, float *beta, double *stats, int *status) {
+    k_tea_beta(mte_params P, DevTopo T, const float *eps, const float4 *ci, float *beta, float4 *bc, double *stats,
+               int *status) {
     __shared__ double red[256];
     __shared__ int cnt[256];
     const int t = blockIdx.x;
@@ -405,31 +407,334 @@ __global__ void __launch_bounds__(256)
         stats[2 * t] = e;
         stats[2 * t + 1] = (double)(float)bt;
         if (fail) atomicCAS(status, 0, 1 + t);
+        red[0] = bt;
     }
+    __syncthreads();
+    // beta C_i = beta / sqrt(1 + beta^2 ci) (eq. 19), which the steps until
+    // the next refresh read
+    const float bt = (float)red[0], w = bt * bt;
+    for (int i = threadIdx.x; i < n; i += 256) {
+        const float4 c = ci[base + i];
+        bc[base + i] = make_float4(bt * rsq_fast(1.f + w * c.x), bt * rsq_fast(1.f + w * c.y),
+                                   bt * rsq_fast(1.f + w * c.z), 0.f);
+    }
+}
+
+// Keeps a loop constant in a vector register: an FP32 operation with a scalar
+// operand issues at half rate (4 cycles per wave, measured, against 2).
+__device__ __forceinline__ float in_vgpr(float v) {
+    __asm__("" : "+v"(v));
+    return v;
+}
+
+// Pair sums with each (i, j) RPY block evaluated once for both beads.  Work
+// unit: (trajectory, I pair p: the 64-bead chunks 2p and 2p + 1, chunks J of a
+// range at or above 2p).  D_hat_ji = D_hat_ij, so a block serves
+//   i-side  D_hat_ij (F_j + beta C_i . R_j)  into acc of bead i,
+//   j-side  D_hat_ij (F_i + beta C_j . R_i)  into g, carried with j.
+// Lane l holds bead l of both I chunks and meets j = (l + s) mod 64 of J at
+// step s, so no two lanes meet the same j in a step; after each step g moves
+// one lane down (DPP wave_rol:1), so it sits in the lane that meets j next.
+//   J > 2p + 1  both I chunks, 64 steps, their j-side sums in one g;
+//   J = 2p + 1  chunk 2p against J, and J against itself;
+//   J = 2p      the chunk against itself: steps 1 .. 31 meet every pair of it
+//               but the opposite ones once, both sides; step 32 meets those
+//               from both ends and takes the i-side only.  No bead meets
+//               itself.
+// Partials (12 bytes per bead, planes of x, y, z): slot p of a j bead holds
+// its sum over I pair p, slot ioff + J0 / jrun of an i bead its sum over the
+// unit's J range, each written by exactly one unit (k_tea_finish adds them
+// in slot order).  Beads past the trajectory's end and extra beads carry
+// zero F and R, so their terms vanish.
+//
+// Lengths in the loop are nm on open boundaries.  In a periodic box they are
+// units of box / 2^32 and positions 32-bit integers, so a difference wraps
+// to the minimum image by itself: 3 subtractions and 3 conversions (18 issue
+// cycles) instead of subtract, scale, round, fused subtract (30).  A float
+// position far from the origin is the coarser of the two.
+// The coefficients are those beyond 2a; a wave with a pair inside 2a (margin
+// over the rounding of r / a) selects the near ones in a branch.
+//
+// SPLIT waves share a unit, each taking its part of the steps, and add their
+// sums in wave order (small batches, tea_build_units).
+// Bound: VALU issue, 45 operations per pair and 64 lanes: 98 issue cycles open
+// and 110 in a box (of them 8 for the reciprocal square root, 4 for the near
+// test, 6 for moving g); the constants sit in vector registers because an FP32
+// operation with a scalar operand takes 4 cycles and not 2.
+// Measured, against the same pairs with float minimum images, near and far
+// coefficients selected per pair, scalar constants, one J chunk per unit and
+// one slot per chunk: four periodic trajectories of 24k-37k beads 2.20 ->
+// 1.71 ms (89% of the issue rate at the 2.07 GHz that the chip holds here) and
+// the finish kernel 206 -> 57 us; 64 x 1040 beads 53.5 -> 44.3 us (a third of
+// it ramp and tail); one trajectory of 312 beads 18.4 -> 5.8 us.
+constexpr int SYM_CHUNK = 64;
+// What a pair's evaluation needs beside the beads.
+struct PairCoef {
+    float k1, k3, k5;       // cii = k1 w + k3 w^3, crr / r^2 = w^3 (k1 + k5 w^2), w = 1 / r in loop units
+    float near2, ia, r2min; // (2a)^2 with its margin, 1 / a, the clamp of coincident beads
+};
+struct PairBead {
+    float3 x, F, R, C;      // position (loop units), force, random force, beta C
+};
+// sc: nm per loop unit.
+__device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float sc) {
+    const float a = P.tea_a / sc, lim = 2.002f * a;
+    PairCoef K;
+    K.k1 = in_vgpr(0.75f * a);
+    K.k3 = in_vgpr(0.5f * a * a * a);
+    K.k5 = in_vgpr(-1.5f * a * a * a);
+    K.near2 = in_vgpr(lim * lim);
+    K.ia = sc * rcp_fast(P.tea_a);
+    K.r2min = 1e-12f / (sc * sc);
+    return K;
+}
+
+// One coordinate in loop units: x itself, or its place in the box as a
+// 32-bit integer (bit pattern), taken modulo the box in FP64.
+template <bool INT>
+__device__ __forceinline__ float pair_coord(float x, double ibox) {
+    if (!INT) return x;
+    double v = (double)x * ibox;
+    v -= rint(v);
+    // 1.5 2^52 leaves the rounded integer in the low mantissa word
+    return __int_as_float(__double2loint(fma(v, 4294967296.0, 6755399441055744.0)));
+}
+template <bool INT>
+__device__ __forceinline__ float pair_diff(float a, float b) {
+    return INT ? (float)(__float_as_int(a) - __float_as_int(b)) : a - b;
+}
+
+// Bead b (zeros where it is not valid); extra beads have zero F and R.
+template <bool INT>
+__device__ __forceinline__ PairBead pair_bead(const float4 *xyz, const float4 *fxyz, const float4 *R, const float4 *bc,
+                                              int b, bool valid, double ibox) {
+    PairBead v;
+    v.x = v.F = v.R = v.C = make_float3(0.f, 0.f, 0.f);
+    if (valid) {
+        const float3 x = f3(xyz[b]), F = f3(fxyz[b]);
+        v.x = make_float3(pair_coord<INT>(x.x, ibox), pair_coord<INT>(x.y, ibox), pair_coord<INT>(x.z, ibox));
+        // zero for a finite position; a lost one (inf, NaN), which an
+        // integer cannot hold, spreads through F as it would through r
+        const float lost = INT ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
+        v.F = make_float3(F.x + lost, F.y + lost, F.z + lost);
+        v.R = f3(R[b]);
+        v.C = f3(bc[b]);
+    }
+    return v;
+}
+
+// Bead I against the j of (A, B, Cq): i-side into acc, and j-side into g
+// (BOTH).
+template <bool INT, bool BOTH>
+__device__ __forceinline__ void pair_block(const PairCoef &K, const PairBead &I, float4 A, float4 B, float4 Cq,
+                                           float3 &acc, float3 &g) {
+    const float dx = pair_diff<INT>(A.x, I.x.x), dy = pair_diff<INT>(A.y, I.x.y), dz = pair_diff<INT>(A.z, I.x.z);
+    const float r2 = dx * dx + dy * dy + dz * dz;
+    const float w = rsq_fast(r2);
+    const float w2 = w * w;
+    float cii = w * fmaf(K.k3, w2, K.k1);
+    float cr = (w * w2) * fmaf(K.k5, w2, K.k1);
+    if (__any(r2 <= K.near2)) {
+        __asm__ volatile("");   // a branch: the near form is not evaluated otherwise
+        const float r2c = fmaxf(r2, K.r2min), wc = rsq_fast(r2c);
+        const float ra = r2c * wc * K.ia;
+        const bool nr = !(ra > 2.f);
+        cii = nr ? fmaf(-0.28125f, ra, 1.f) : cii;
+        cr = nr ? 0.09375f * ra * wc * wc : cr;
+    }
+    // i-side: F_j + beta C_i . R_j
+    const float vx = fmaf(I.C.x, B.z, A.w), vy = fmaf(I.C.y, B.w, B.x), vz = fmaf(I.C.z, Cq.x, B.y);
+    const float sv = cr * fmaf(dz, vz, fmaf(dy, vy, dx * vx));
+    acc.x = fmaf(sv, dx, fmaf(cii, vx, acc.x));
+    acc.y = fmaf(sv, dy, fmaf(cii, vy, acc.y));
+    acc.z = fmaf(sv, dz, fmaf(cii, vz, acc.z));
+    if (BOTH) {
+        // j-side: F_i + beta C_j . R_i (e e^T is even in e)
+        const float wx = fmaf(Cq.y, I.R.x, I.F.x), wy = fmaf(Cq.z, I.R.y, I.F.y), wz = fmaf(Cq.w, I.R.z, I.F.z);
+        const float sw = cr * fmaf(dz, wz, fmaf(dy, wy, dx * wx));
+        g.x = fmaf(sw, dx, fmaf(cii, wx, g.x));
+        g.y = fmaf(sw, dy, fmaf(cii, wy, g.y));
+        g.z = fmaf(sw, dz, fmaf(cii, wz, g.z));
+    }
+}
+
+__device__ __forceinline__ void rotate(float3 &g) {
+    g.x = wave_rol1(g.x);
+    g.y = wave_rol1(g.y);
+    g.z = wave_rol1(g.z);
+}
+
+template <bool INT, int SPLIT>
+__device__ __forceinline__ void pair_unit(const mte_params &P, const PairUnit &U, int nb, const float4 *xyz,
+                                          const float4 *fxyz, const float4 *R, const float4 *bc, int jrun, int ioff,
+                                          float *partial, float4 (*jd)[2 * SYM_CHUNK],
+                                          float (*red)[9][SPLIT == 1 ? 1 : SYM_CHUNK]) {
+    const int l = threadIdx.x % SYM_CHUNK, k = threadIdx.x / SYM_CHUNK;
+    const int base = U.base, n = U.n, pair = U.pair, J0 = U.J0, J1 = U.J0 + U.nJ;
+    const double ibox = INT ? 1.0 / (double)U.box : 0.0;
+    const PairCoef K = pair_coef(P, INT ? U.box * 0x1p-32f : 1.f);
+    const int c0 = 2 * pair, i0 = c0 * SYM_CHUNK + l;
+    PairBead I[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int li = i0 + h * SYM_CHUNK;
+        I[h] = pair_bead<INT>(xyz, fxyz, R, bc, base + li, li < n, ibox);
+    }
+    float3 acc[2] = {make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f)};
+    auto load_j = [&](int J) {
+        const int lj = J * SYM_CHUNK + l;
+        return pair_bead<INT>(xyz, fxyz, R, bc, base + lj, lj < n, ibox);
+    };
+    PairBead next{};
+    if (SPLIT == 1) next = load_j(J0);
+    for (int J = J0; J < J1; J++) {
+        // the chunk's beads, packed and written twice (q and q + 64) so that
+        // lane l reads slot l + s at step s with no wrap
+        if (SPLIT == 1 || k == 0) {
+            if (SPLIT > 1) next = load_j(J);
+            const float4 d0 = make_float4(next.x.x, next.x.y, next.x.z, next.F.x),
+                         d1 = make_float4(next.F.y, next.F.z, next.R.x, next.R.y),
+                         d2 = make_float4(next.R.z, next.C.x, next.C.y, next.C.z);
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                jd[0][l + q * SYM_CHUNK] = d0;
+                jd[1][l + q * SYM_CHUNK] = d1;
+                jd[2][l + q * SYM_CHUNK] = d2;
+            }
+        }
+        __syncthreads();
+        if (SPLIT == 1 && J + 1 < J1) next = load_j(J + 1);   // requested ahead of this chunk's steps
+        const float4 *j0 = &jd[0][l], *j1 = &jd[1][l], *j2 = &jd[2][l];
+        float3 g = make_float3(0.f, 0.f, 0.f);
+        // this wave's steps of a full sweep and of a chunk against itself
+        constexpr int W = SYM_CHUNK / SPLIT, D = SYM_CHUNK / 2 / SPLIT;
+        const int s0 = k * W, s1 = s0 + W;
+        if (J > c0 + 1) {
+#pragma unroll 1
+            for (int s = s0; s < s1; s++) {
+                const float4 A = j0[s], B = j1[s], Cq = j2[s];
+                pair_block<INT, true>(K, I[0], A, B, Cq, acc[0], g);
+                pair_block<INT, true>(K, I[1], A, B, Cq, acc[1], g);
+                rotate(g);
+            }
+        } else {
+            if (J > c0)
+#pragma unroll 1
+                for (int s = s0; s < s1; s++) {
+                    pair_block<INT, true>(K, I[0], j0[s], j1[s], j2[s], acc[0], g);
+                    rotate(g);
+                }
+            const int h = J - c0;
+            const PairBead &D0 = h ? I[1] : I[0];
+            float3 own = make_float3(0.f, 0.f, 0.f), gd = own;
+            const int t0 = 1 + k * D, t1 = t0 + D, t2 = min(t1, SYM_CHUNK / 2);
+#pragma unroll 1
+            for (int s = t0; s < t2; s++) {
+                pair_block<INT, true>(K, D0, j0[s], j1[s], j2[s], own, gd);
+                rotate(gd);
+            }
+            if (t2 < t1) pair_block<INT, false>(K, D0, j0[t2], j1[t2], j2[t2], own, gd);
+            // lane l holds the j-side sums of bead l + t2 of the chunk
+            const int src = (l - t2) & (SYM_CHUNK - 1);
+            own.x += __shfl(gd.x, src);
+            own.y += __shfl(gd.y, src);
+            own.z += __shfl(gd.z, src);
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+                if (q == h) {
+                    acc[q].x += own.x;
+                    acc[q].y += own.y;
+                    acc[q].z += own.z;
+                }
+        }
+        const int lj = J * SYM_CHUNK + l;
+        float *out = partial + (size_t)3 * pair * nb + base + lj;
+        if (SPLIT == 1) {
+            if (J > c0 && lj < n) {
+                out[0] = g.x;
+                out[nb] = g.y;
+                out[2 * (size_t)nb] = g.z;
+            }
+            __syncthreads();   // the chunk's slots are free
+        } else {
+            // lane l holds the sums of bead l + s1 of J
+            const int q = (l + s1) & (SYM_CHUNK - 1);
+            red[k][6][q] = g.x;
+            red[k][7][q] = g.y;
+            red[k][8][q] = g.z;
+            __syncthreads();
+            if (k < 3 && J > c0 && lj < n) {
+                float v = 0.f;
+#pragma unroll
+                for (int w = 0; w < SPLIT; w++) v += red[w][6 + k][l];
+                out[(size_t)k * nb] = v;
+            }
+            __syncthreads();
+        }
+    }
+    float *out = partial + (size_t)3 * (ioff + J0 / jrun) * nb + base + i0;
+    if (SPLIT == 1) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (i0 + h * SYM_CHUNK < n) {
+                out[h * SYM_CHUNK] = acc[h].x;
+                out[(size_t)nb + h * SYM_CHUNK] = acc[h].y;
+                out[2 * (size_t)nb + h * SYM_CHUNK] = acc[h].z;
+            }
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            red[k][3 * h][l] = acc[h].x;
+            red[k][3 * h + 1][l] = acc[h].y;
+            red[k][3 * h + 2][l] = acc[h].z;
+        }
+        __syncthreads();
+        for (int c = k; c < 6; c += SPLIT) {
+            const int h = c / 3, o = h * SYM_CHUNK;
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < SPLIT; w++) v += red[w][c][l];
+            if (i0 + o < n) out[(size_t)(c % 3) * nb + o] = v;
+        }
+    }
+}
+
+template <bool PERIODIC, int SPLIT>
+__global__ void __launch_bounds__(SYM_CHUNK *SPLIT, 5)
+    k_tea_pairs_sym(mte_params P, int nb, const float4 *xyz, const float4 *fxyz, const float4 *R, const float4 *bc,
+                    const PairUnit *units, int jrun, int ioff, float *partial) {
+    static_assert(SPLIT == 1 || SPLIT >= 3, "three waves add the j-side components");
+    __shared__ float4 jd[3][2 * SYM_CHUNK];
+    __shared__ float red[SPLIT][9][SPLIT == 1 ? 1 : SYM_CHUNK];
+    const PairUnit U = units[blockIdx.x];
+    if (PERIODIC && U.box > 0.f)
+        pair_unit<true, SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
+    else
+        pair_unit<false, SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
 }
 
 // Pair sums of one (trajectory, 256-bead i group, j chunk) work unit:
 //   partial_i = sum_{j in chunk, j != i, non-extra} D_hat_ij (F_j + beta C_i . R_j)
 // The chunk's j data sit in LDS; extra beads enter with zero force and
-// noise, so they contribute nothing and need no branch.
+// noise, so they contribute nothing and need no branch.  Coordinates and
+// coefficients are those of k_tea_pairs_sym, so both forms take the same
+// image of a pair half a box apart.
 // Splitting j into chunks gives ~10 work units per SIMD at 64 x 1040 beads,
 // against ~1 per SIMD for one thread per bead over the whole trajectory.
-template <int CHUNK, bool PERIODIC>
-__global__ void __launch_bounds__(TEA_TILE)
-    k_tea_pairs(mte_params P, DevTopo T, DevState S, const float4 *fxyz, const float4 *R, const float4 *ci,
-                const float *beta, const int4 *units, int chunk_stride, float4 *partial) {
-    __shared__ float4 sx[CHUNK], sf[CHUNK], sr[CHUNK];
-    const int4 u = units[blockIdx.x];   // traj, i0, j0, chunk index
+template <bool INT, int CHUNK>
+__device__ __forceinline__ void pair_chunk(const mte_params &P, const DevTopo &T, const DevState &S, const float4 *fxyz,
+                                           const float4 *R, const float4 *bc, int4 u, float4 *partial,
+                                           float4 (*jd)[CHUNK]) {
     const int base = T.tbase[u.x], n = T.tsize[u.x];
+    const float box = T.tbox[u.x];
+    const double ibox = INT ? 1.0 / (double)box : 0.0;
+    const PairCoef K = pair_coef(P, INT ? box * 0x1p-32f : 1.f);
     const int jn = min(CHUNK, n - u.z);
     for (int q = threadIdx.x; q < jn; q += TEA_TILE) {
-        const int jb = base + u.z + q;
-        float4 x = S.xyz[jb];
-        float4 f = fxyz[jb], r = R[jb];
-        if (T.extra[jb]) f = r = make_float4(0.f, 0.f, 0.f, 0.f);
-        sx[q] = x;
-        sf[q] = f;
-        sr[q] = r;
+        const PairBead v = pair_bead<INT>(S.xyz, fxyz, R, bc, base + u.z + q, true, ibox);
+        jd[0][q] = make_float4(v.x.x, v.x.y, v.x.z, v.F.x);
+        jd[1][q] = make_float4(v.F.y, v.F.z, v.R.x, v.R.y);
+        jd[2][q] = make_float4(v.R.z, v.C.x, v.C.y, v.C.z);
     }
     __syncthreads();
     const int li = u.y + threadIdx.x;
@@ -437,246 +742,45 @@ __global__ void __launch_bounds__(TEA_TILE)
     const int b = base + li;
     float3 acc = make_float3(0.f, 0.f, 0.f);
     if (!T.extra[b]) {
-        const float3 ri = f3(S.xyz[b]);
-        const float bt = beta[u.x];
-        const float4 cc = ci[b];
-        const float w = bt * bt;
-        const float cx = bt * rsq_fast(1.f + w * cc.x), cy = bt * rsq_fast(1.f + w * cc.y),
-                    cz = bt * rsq_fast(1.f + w * cc.z);
-        const float a = P.tea_a, ia = rcp_fast(P.tea_a);
-        const float box = T.tbox[u.x], ibox = inv_side(box);
-        for (int q = 0; q < jn; q++) {
-            const float4 xj = sx[q], Fj = sf[q], Rj = sr[q];
-            float3 d = sub3(f3(xj), ri);
-            if (PERIODIC) d = min_image_inv(d, box, ibox);
-            const float dx = d.x, dy = d.y, dz = d.z;
-            // the j == i slot (d = 0) and coincident beads stay finite through the clamp
-            // (extra beads carry zero F and R)
-            const float r2 = fmaxf(dx * dx + dy * dy + dz * dz, 1e-12f);
-            const float rinv = rsq_fast(r2);
-            // D_hat = cii I + crr e e^T (src/bdhitea_kernel.cu:38-58)
-            const RpyCoef c = rpy_select(r2, rinv, a, ia);
-            const float vx = fmaf(cx, Rj.x, Fj.x), vy = fmaf(cy, Rj.y, Fj.y), vz = fmaf(cz, Rj.z, Fj.z);
-            const float s = (c.crr * rinv * rinv) * (dx * vx + dy * vy + dz * vz);
-            acc.x = fmaf(s, dx, fmaf(c.cii, vx, acc.x));
-            acc.y = fmaf(s, dy, fmaf(c.cii, vy, acc.y));
-            acc.z = fmaf(s, dz, fmaf(c.cii, vz, acc.z));
-        }
+        const PairBead I = pair_bead<INT>(S.xyz, fxyz, R, bc, b, true, ibox);
+        float3 none = acc;
+        for (int q = 0; q < jn; q++) pair_block<INT, false>(K, I, jd[0][q], jd[1][q], jd[2][q], acc, none);
         const int self = li - u.z;   // position of i in this chunk, if any
         if (self >= 0 && self < jn) {
             // The loop took the j == i slot as a coincident bead: d = 0 leaves
             // only its cii (v_i) term, recomputed here from the same operands
             // and taken out again.
-            const float4 Fi = sf[self], Ri = sr[self];
-            const float r2 = 1e-12f, rinv = rsq_fast(r2);
-            const float cii = rpy_select(r2, rinv, a, ia).cii;
-            acc.x = fmaf(-cii, fmaf(cx, Ri.x, Fi.x), acc.x);
-            acc.y = fmaf(-cii, fmaf(cy, Ri.y, Fi.y), acc.y);
-            acc.z = fmaf(-cii, fmaf(cz, Ri.z, Fi.z), acc.z);
+            const float cii = fmaf(-0.28125f, K.r2min * rsq_fast(K.r2min) * K.ia, 1.f);
+            acc.x = fmaf(-cii, fmaf(I.C.x, I.R.x, I.F.x), acc.x);
+            acc.y = fmaf(-cii, fmaf(I.C.y, I.R.y, I.F.y), acc.y);
+            acc.z = fmaf(-cii, fmaf(I.C.z, I.R.z, I.F.z), acc.z);
         }
     }
-    partial[(size_t)u.w * chunk_stride + b] = make_float4(acc.x, acc.y, acc.z, 0.f);
+    partial[(size_t)u.w * T.nb + b] = make_float4(acc.x, acc.y, acc.z, 0.f);
 }
 
-// Pair sums with each (i, j) RPY block evaluated once for both beads.  Work
-// unit: (trajectory, 64-bead chunk I, 64-bead chunk J >= I), one
-// single-wave workgroup each, so the dispatcher balances units wave by
-// wave.  D_hat_ji = D_hat_ij, so the block serves
-//   i-side  D_hat_ij (F_j + beta C_i . R_j)  into partial slot J of bead i,
-//   j-side  D_hat_ij (F_i + beta C_j . R_i)  into partial slot I of bead j,
-// and slot c of a bead holds the sum over chunk c, as k_tea_pairs<64> writes
-// it (a unit may take two I chunks below J, I and I + 64: its lanes meet j
-// with both of their beads before g moves on, slot I of a j bead holds the
-// sum over both chunks and slot I + 1 zero).  Off the diagonal, lane l takes j = (l + s) mod 64 at step s: every
-// lane meets every j of the chunk once and no two lanes the same j in a
-// step.  The j-side sum of j travels with j in registers: after each step
-// the wave rotates it one lane down (DPP wave_rol:1, lane l takes lane l+1's
-// value), so at step s + 1 it sits in the lane that meets j next, and after
-// 64 steps in lane j.  A diagonal unit (I == J) is one-sided, as
-// k_tea_pairs.  j slots past the trajectory's end and extra beads carry zero
-// F and R, so their terms vanish; their sums are not stored (extra beads
-// store zero).
-constexpr int SYM_CHUNK = 64;
-template <bool PERIODIC>
-__global__ void __launch_bounds__(SYM_CHUNK)
-    k_tea_pairs_sym(mte_params P, DevTopo T, DevState S, const float4 *fxyz, const float4 *R, const float4 *ci,
-                    const float *beta, const int4 *units, int nunits, int chunk_stride, float4 *partial) {
-    // j data of each wave's block, packed as (x, F.x) (F.y, F.z, R.x, R.y)
-    // (R.z, beta C) and written twice, at q and q + 64, so that lane l reads
-    // slot l + s at step s with no wrap
-    __shared__ float4 jd[3][2 * SYM_CHUNK];
-    const int l = threadIdx.x;
-    const int ui = blockIdx.x;
-    const bool has = ui < nunits;
-    const int4 u = has ? units[ui] : make_int4(0, 0, 0, 0);
-    const int base = T.tbase[u.x], n = T.tsize[u.x];
-    const float bt = beta[u.x], w2 = bt * bt;
-    const float box = T.tbox[u.x], ibox = inv_side(box);
-    // beads of this lane in chunk I and, in a two-chunk unit (u.w = 2, both
-    // chunks below J), in chunk I + 64 ...
-    const int ni = u.w == 2 ? 2 : 1;
-    int bi[2];
-    bool vi[2], ei[2];
-    float3 xi[2], Fi[2], Ri[2], Ci[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int li = u.y + 64 * h + l;
-        bi[h] = base + li;
-        vi[h] = has && h < ni && li < n;
-        ei[h] = vi[h] && T.extra[bi[h]];
-        xi[h] = Fi[h] = Ri[h] = Ci[h] = make_float3(0.f, 0.f, 0.f);
-        if (vi[h]) {
-            xi[h] = f3(S.xyz[bi[h]]);
-            if (!ei[h]) {
-                Fi[h] = f3(fxyz[bi[h]]);
-                Ri[h] = f3(R[bi[h]]);
-                const float4 cc = ci[bi[h]];
-                Ci[h] = make_float3(bt * rsq_fast(1.f + w2 * cc.x), bt * rsq_fast(1.f + w2 * cc.y),
-                                    bt * rsq_fast(1.f + w2 * cc.z));
-            }
-        }
-    }
-    // ... and in chunk J, staged for the wave
-    const int lj = u.z + l, bj = base + lj;
-    const bool vj = has && lj < n;
-    const bool ej = vj && T.extra[bj];
-    {
-        float3 x = make_float3(0.f, 0.f, 0.f), F = x, Rj = x, C = x;
-        if (vj) {
-            x = f3(S.xyz[bj]);
-            if (!ej) {
-                F = f3(fxyz[bj]);
-                Rj = f3(R[bj]);
-                const float4 cc = ci[bj];
-                C = make_float3(bt * rsq_fast(1.f + w2 * cc.x), bt * rsq_fast(1.f + w2 * cc.y),
-                                bt * rsq_fast(1.f + w2 * cc.z));
-            }
-        }
-        const float4 d0 = make_float4(x.x, x.y, x.z, F.x), d1 = make_float4(F.y, F.z, Rj.x, Rj.y),
-                     d2 = make_float4(Rj.z, C.x, C.y, C.z);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            jd[0][l + h * SYM_CHUNK] = d0;
-            jd[1][l + h * SYM_CHUNK] = d1;
-            jd[2][l + h * SYM_CHUNK] = d2;
-        }
-    }
-    __syncthreads();
-    const float a = P.tea_a, ia = rcp_fast(P.tea_a);
-    float3 acc[2] = {make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f)}, g = acc[0];
-    const bool diag = u.y == u.z;
-    if (has && diag) {
-        if (vi[0] && !ei[0]) {
-            const int jn = min(SYM_CHUNK, n - u.z);
-            for (int q = 0; q < jn; q++) {
-                const float4 A = jd[0][q], B = jd[1][q], Cq = jd[2][q];
-                float3 d = make_float3(A.x - xi[0].x, A.y - xi[0].y, A.z - xi[0].z);
-                if (PERIODIC) d = min_image_inv(d, box, ibox);
-                const float r2 = fmaxf(d.x * d.x + d.y * d.y + d.z * d.z, 1e-12f);
-                const float rinv = rsq_fast(r2);
-                const RpyCoef c = rpy_select(r2, rinv, a, ia);
-                const float vx = fmaf(Ci[0].x, B.z, A.w), vy = fmaf(Ci[0].y, B.w, B.x), vz = fmaf(Ci[0].z, Cq.x, B.y);
-                const float sv = (c.crr * rinv * rinv) * (d.x * vx + d.y * vy + d.z * vz);
-                acc[0].x = fmaf(sv, d.x, fmaf(c.cii, vx, acc[0].x));
-                acc[0].y = fmaf(sv, d.y, fmaf(c.cii, vy, acc[0].y));
-                acc[0].z = fmaf(sv, d.z, fmaf(c.cii, vz, acc[0].z));
-            }
-            // the j == i slot (d = 0) left its cii v_i term: taken out again
-            const float r2 = 1e-12f, rinv = rsq_fast(r2);
-            const float cii = rpy_select(r2, rinv, a, ia).cii;
-            acc[0].x = fmaf(-cii, fmaf(Ci[0].x, Ri[0].x, Fi[0].x), acc[0].x);
-            acc[0].y = fmaf(-cii, fmaf(Ci[0].y, Ri[0].y, Fi[0].y), acc[0].y);
-            acc[0].z = fmaf(-cii, fmaf(Ci[0].z, Ri[0].z, Fi[0].z), acc[0].z);
-        }
-    } else if (has) {
-        const float4 *j0 = &jd[0][l], *j1 = &jd[1][l], *j2 = &jd[2][l];
-        // bead h of the lane against j: i-side into acc[h], j-side into g
-        auto pair = [&](auto far, int h, const float4 &A, const float4 &B, const float4 &Cq) {
-            float3 d = make_float3(A.x - xi[h].x, A.y - xi[h].y, A.z - xi[h].z);
-            if (PERIODIC) d = min_image_inv(d, box, ibox);
-            // (the clamp is the identity beyond 2a)
-            const float r2s = d.x * d.x + d.y * d.y + d.z * d.z;
-            const float r2 = decltype(far)::value ? r2s : fmaxf(r2s, 1e-12f);
-            const float rinv = rsq_fast(r2);
-            const RpyCoef c = decltype(far)::value ? rpy_far(rinv, a) : rpy_select(r2, rinv, a, ia);
-            const float cr = c.crr * rinv * rinv;
-            // i-side: F_j + beta C_i . R_j
-            const float vx = fmaf(Ci[h].x, B.z, A.w), vy = fmaf(Ci[h].y, B.w, B.x), vz = fmaf(Ci[h].z, Cq.x, B.y);
-            const float sv = cr * (d.x * vx + d.y * vy + d.z * vz);
-            acc[h].x = fmaf(sv, d.x, fmaf(c.cii, vx, acc[h].x));
-            acc[h].y = fmaf(sv, d.y, fmaf(c.cii, vy, acc[h].y));
-            acc[h].z = fmaf(sv, d.z, fmaf(c.cii, vz, acc[h].z));
-            // j-side: F_i + beta C_j . R_i (e e^T is even in e)
-            const float wx = fmaf(Cq.y, Ri[h].x, Fi[h].x), wy = fmaf(Cq.z, Ri[h].y, Fi[h].y),
-                        wz = fmaf(Cq.w, Ri[h].z, Fi[h].z);
-            const float sw = cr * (d.x * wx + d.y * wy + d.z * wz);
-            g.x = fmaf(sw, d.x, fmaf(c.cii, wx, g.x));
-            g.y = fmaf(sw, d.y, fmaf(c.cii, wy, g.y));
-            g.z = fmaf(sw, d.z, fmaf(c.cii, wz, g.z));
-        };
-        // each step: the lane's beads meet j together, then g moves on
-        auto sweep = [&](auto far, auto two) {
-            for (int s = 0; s < SYM_CHUNK; s++) {
-                const float4 A = j0[s], B = j1[s], Cq = j2[s];
-                pair(far, 0, A, B, Cq);
-                if (decltype(two)::value) pair(far, 1, A, B, Cq);
-                g.x = wave_rol1(g.x);
-                g.y = wave_rol1(g.y);
-                g.z = wave_rol1(g.z);
-            }
-        };
-        // Open boundaries: when the bounding boxes of the I beads and of
-        // chunk J lie more than 2a apart (with a margin over the rounding of
-        // r / a), every pair takes the far branch and the selection is
-        // skipped (same values).  Slots past the trajectory's end stand in
-        // as the chunk's first bead; a one-chunk unit counts its bead twice.
-        bool far = false;
-        if (!PERIODIC) {
-            const float4 xj = jd[0][vj ? l : 0];
-            const float3 xb = ni == 2 ? xi[1] : xi[0];
-            float lo[6] = {fminf(xi[0].x, xb.x), fminf(xi[0].y, xb.y), fminf(xi[0].z, xb.z), xj.x, xj.y, xj.z};
-            float hi[6] = {fmaxf(xi[0].x, xb.x), fmaxf(xi[0].y, xb.y), fmaxf(xi[0].z, xb.z), xj.x, xj.y, xj.z};
-#pragma unroll
-            for (int m = 1; m < SYM_CHUNK; m <<= 1)
-#pragma unroll
-                for (int k = 0; k < 6; k++) {
-                    lo[k] = fminf(lo[k], __shfl_xor(lo[k], m));
-                    hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], m));
-                }
-            const float gx = fmaxf(fmaxf(lo[3] - hi[0], lo[0] - hi[3]), 0.f);
-            const float gy = fmaxf(fmaxf(lo[4] - hi[1], lo[1] - hi[4]), 0.f);
-            const float gz = fmaxf(fmaxf(lo[5] - hi[2], lo[2] - hi[5]), 0.f);
-            const float lim = 2.002f * a;
-            far = __builtin_amdgcn_readfirstlane((int)(gx * gx + gy * gy + gz * gz > lim * lim)) != 0;
-        }
-        if (ni == 2) {
-            if (far) sweep(std::true_type{}, std::true_type{});
-            else sweep(std::false_type{}, std::true_type{});
-        } else {
-            if (far) sweep(std::true_type{}, std::false_type{});
-            else sweep(std::false_type{}, std::false_type{});
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-        if (vi[h])
-            partial[(size_t)(u.z / SYM_CHUNK) * chunk_stride + bi[h]] =
-                ei[h] ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(acc[h].x, acc[h].y, acc[h].z, 0.f);
-    if (vj && !diag) {
-        // a two-chunk unit's j-side sum covers both chunks: slot I holds
-        // it, slot I + 1 zero
-        partial[(size_t)(u.y / SYM_CHUNK) * chunk_stride + bj] = ej ? make_float4(0.f, 0.f, 0.f, 0.f)
-                                                                     : make_float4(g.x, g.y, g.z, 0.f);
-        if (ni == 2) partial[(size_t)(u.y / SYM_CHUNK + 1) * chunk_stride + bj] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+template <int CHUNK, bool PERIODIC>
+__global__ void __launch_bounds__(TEA_TILE)
+    k_tea_pairs(mte_params P, DevTopo T, DevState S, const float4 *fxyz, const float4 *R, const float4 *bc,
+                const int4 *units, float4 *partial) {
+    __shared__ float4 jd[3][CHUNK];
+    const int4 u = units[blockIdx.x];   // traj, i0, j0, chunk index
+    if (PERIODIC && T.tbox[u.x] > 0.f)
+        pair_chunk<true, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
+    else
+        pair_chunk<false, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
 }
 
 // Self term, chunk partials in fixed order, and the update of one bead
 // (integrateTea_kernel_unlisted, src/bdhitea_kernel.cu:148-213).
+// SYM: the partials of k_tea_pairs_sym (planes of x, y, z; the bead's j-side
+// slots, then its i-side slots), else the float4 slots of its trajectory's
+// chunks.
+template <bool SYM>
 __global__ void __launch_bounds__(TEA_TILE)
     k_tea_finish(mte_params P, DevTopo T, DevState Sin, DevState Sout, const float4 *fxyz, const float4 *fang,
-                 const float4 *R, const float4 *ci, const float *beta, const int *nchunks, int chunk_stride,
-                 const float4 *partial, uint4 *seeds, const float *noise, LatOffsets L) {
+                 const float4 *R, const float4 *ci, const float *beta, const int *nchunks, int jrun, int ioff,
+                 const float4 *partial4, uint4 *seeds, const float *noise, LatOffsets L) {
     const int b = blockIdx.x * TEA_TILE + threadIdx.x;
     if (b >= T.nb) return;
     const int t = T.tid[b];
@@ -688,25 +792,56 @@ __global__ void __launch_bounds__(TEA_TILE)
     float fx = fmaf(Ri.x, cx, Fi.x), fy = fmaf(Ri.y, cy, Fi.y), fz = fmaf(Ri.z, cz, Fi.z);
     // the bead's state is requested before the partial sums are added
     float4 x = Sin.xyz[b], an = Sin.ang[b];
-    const int nc = nchunks[t];
-    // partials four at a time: four loads in flight, then added in order
-    int c = 0;
-    for (; c + 4 <= nc; c += 4) {
-        float4 pp[4];
+    const size_t nb = T.nb;
+    if (SYM) {
+        const float *part = reinterpret_cast<const float *>(partial4) + b;
+        const int chunk = (b - T.tbase[t]) / SYM_CHUNK, nch = (T.tsize[t] + SYM_CHUNK - 1) / SYM_CHUNK;
+        // slots four at a time: twelve loads in flight, then added in order
+        auto add = [&](int c, int end) {
+            for (; c + 4 <= end; c += 4) {
+                float v[4][3];
 #pragma unroll
-        for (int u = 0; u < 4; u++) pp[u] = partial[(size_t)(c + u) * chunk_stride + b];
+                for (int u = 0; u < 4; u++)
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            fx += pp[u].x;
-            fy += pp[u].y;
-            fz += pp[u].z;
+                    for (int k = 0; k < 3; k++) v[u][k] = part[(3 * (size_t)(c + u) + k) * nb];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    fx += v[u][0];
+                    fy += v[u][1];
+                    fz += v[u][2];
+                }
+            }
+            for (; c < end; c++) {
+                const float *q = part + 3 * (size_t)c * nb;
+                const float v0 = q[0], v1 = q[nb], v2 = q[2 * nb];
+                fx += v0;
+                fy += v1;
+                fz += v2;
+            }
+        };
+        add(0, (chunk + 1) / 2);
+        add(ioff + (chunk & ~1) / jrun, ioff + (nch - 1) / jrun + 1);
+    } else {
+        const int nc = nchunks[t];
+        // partials four at a time: four loads in flight, then added in order
+        int c = 0;
+        for (; c + 4 <= nc; c += 4) {
+            float4 pp[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) pp[u] = partial4[(size_t)(c + u) * nb + b];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                fx += pp[u].x;
+                fy += pp[u].y;
+                fz += pp[u].z;
+            }
         }
-    }
-    for (; c < nc; c++) {
-        const float4 pp = partial[(size_t)c * chunk_stride + b];
-        fx += pp.x;
-        fy += pp.y;
-        fz += pp.z;
+        for (; c < nc; c++) {
+            const float4 pp = partial4[(size_t)c * nb + b];
+            fx += pp.x;
+            fy += pp.y;
+            fz += pp.z;
+        }
     }
     float4 ra;
     if (noise) {
@@ -1160,35 +1295,27 @@ hipError_t launch_tea_eps(mte_engine *e) {
     else
         hipLaunchKernelGGL(k_tea_eps<false>, dim3(e->ntiles), dim3(TEA_TILE), 0, e->stream, e->P, e->T,
                            e->S[e->cur], e->tiles, e->tea.ci, e->tea.eps);
-    hipLaunchKernelGGL(k_tea_beta, dim3(e->ntraj), dim3(256), 0, e->stream, e->P, e->T, e->tea.eps, e->tea.beta,
-                       e->tea.stats, e->tea.status);
+    hipLaunchKernelGGL(k_tea_beta, dim3(e->ntraj), dim3(256), 0, e->stream, e->P, e->T, e->tea.eps, e->tea.ci,
+                       e->tea.beta, e->tea.bc, e->tea.stats, e->tea.status);
     return hipGetLastError();
 }
 
 template <int CHUNK>
 static void launch_pairs_chunk(mte_engine *e) {
-    if (e->periodic)
-        hipLaunchKernelGGL((k_tea_pairs<CHUNK, true>), dim3(e->tea.nunits), dim3(TEA_TILE), 0, e->stream, e->P,
-                           e->T, e->S[e->cur], e->fxyz, e->tea.R, e->tea.ci, e->tea.beta, e->tea.units, e->nb,
-                           e->tea.partial);
-    else
-        hipLaunchKernelGGL((k_tea_pairs<CHUNK, false>), dim3(e->tea.nunits), dim3(TEA_TILE), 0, e->stream, e->P,
-                           e->T, e->S[e->cur], e->fxyz, e->tea.R, e->tea.ci, e->tea.beta, e->tea.units, e->nb,
-                           e->tea.partial);
+    auto kern = e->periodic ? k_tea_pairs<CHUNK, true> : k_tea_pairs<CHUNK, false>;
+    hipLaunchKernelGGL(kern, dim3(e->tea.nunits), dim3(TEA_TILE), 0, e->stream, e->P, e->T, e->S[e->cur], e->fxyz,
+                       e->tea.R, e->tea.bc, e->tea.units, e->tea.partial);
 }
 
 hipError_t launch_tea_pairs(mte_engine *e) {
     // the kernel's chunk must be the one the work units were built for
     if (e->tea.unit_chunk == MTE_TEA_SYMMETRIC) {
-        const int nwg = e->tea.nunits;
-        if (e->periodic)
-            hipLaunchKernelGGL(k_tea_pairs_sym<true>, dim3(nwg), dim3(SYM_CHUNK), 0, e->stream, e->P, e->T,
-                               e->S[e->cur], e->fxyz, e->tea.R, e->tea.ci, e->tea.beta, e->tea.units,
-                               e->tea.nunits, e->nb, e->tea.partial);
-        else
-            hipLaunchKernelGGL(k_tea_pairs_sym<false>, dim3(nwg), dim3(SYM_CHUNK), 0, e->stream, e->P, e->T,
-                               e->S[e->cur], e->fxyz, e->tea.R, e->tea.ci, e->tea.beta, e->tea.units,
-                               e->tea.nunits, e->nb, e->tea.partial);
+        auto kern = e->tea.split == 8   ? (e->periodic ? k_tea_pairs_sym<true, 8> : k_tea_pairs_sym<false, 8>)
+                    : e->tea.split == 4 ? (e->periodic ? k_tea_pairs_sym<true, 4> : k_tea_pairs_sym<false, 4>)
+                                        : (e->periodic ? k_tea_pairs_sym<true, 1> : k_tea_pairs_sym<false, 1>);
+        hipLaunchKernelGGL(kern, dim3(e->tea.nunits), dim3(SYM_CHUNK * e->tea.split), 0, e->stream, e->P, e->nb,
+                           e->S[e->cur].xyz, e->fxyz, e->tea.R, e->tea.bc, e->tea.pair_units, e->tea.jrun,
+                           e->tea.ioff, reinterpret_cast<float *>(e->tea.partial));
         return hipGetLastError();
     }
     if (e->tea.unit_chunk == MTE_TEA_MFMA) {
@@ -1211,9 +1338,10 @@ hipError_t launch_tea_pairs(mte_engine *e) {
 }
 
 hipError_t launch_tea_finish(mte_engine *e, const float *noise_step) {
-    hipLaunchKernelGGL(k_tea_finish, dim3((e->nb + TEA_TILE - 1) / TEA_TILE), dim3(TEA_TILE), 0, e->stream, e->P,
-                       e->T, e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.R, e->tea.ci, e->tea.beta,
-                       e->tea.nchunks, e->nb, e->tea.partial, e->seeds, noise_step, e->L);
+    auto kern = e->tea.unit_chunk == MTE_TEA_SYMMETRIC ? k_tea_finish<true> : k_tea_finish<false>;
+    hipLaunchKernelGGL(kern, dim3((e->nb + TEA_TILE - 1) / TEA_TILE), dim3(TEA_TILE), 0, e->stream, e->P, e->T,
+                       e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.R, e->tea.ci, e->tea.beta,
+                       e->tea.nchunks, e->tea.jrun, e->tea.ioff, e->tea.partial, e->seeds, noise_step, e->L);
     e->cur = 1 - e->cur;
     return hipGetLastError();
 }
