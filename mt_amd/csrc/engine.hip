@@ -238,20 +238,34 @@ hipError_t mte::upload_resident_order(mte_engine *e, const uint8_t *extra) {
 }
 
 // Work units of the one-pass epsilon kernel: every pair (I group, J group >=
-// I group) of 1024-bead groups of a trajectory, and its partial buffer.  Left
-// out (the two-sided kernel computes epsilon) when the buffer would exceed
-// EPS_PART_MAX_BYTES.
+// I group) of a trajectory's groups, and its partial buffer.  Left out (the
+// two-sided kernel computes epsilon) when the buffer would exceed
+// EPS_PART_MAX_BYTES.  Groups of 1024 beads (four chunks per wave) share the
+// j-side rotation and need the smaller buffer; 256 (one chunk per wave) where
+// those would be fewer than four workgroups per CU: 64 x 1040 beads, 192
+// workgroups of the large groups, take 351 us with them and 75 with the small.
 hipError_t mte::tea_build_eps_units(mte_engine *e) {
     std::vector<int4> units;
     int ngrp = 0;
-    for (int t = 0; t < e->ntraj; t++) {
-        const int n = (int)(e->off[t + 1] - e->off[t]);
-        const int g = (n + EPS_GROUP - 1) / EPS_GROUP;
-        ngrp = std::max(ngrp, g);
-        for (int i = 0; i < g; i++)
-            for (int j = i; j < g; j++) units.push_back(make_int4(t, i, j, 0));
+    size_t part = 0;
+    auto build = [&](int group) {
+        units.clear();
+        ngrp = 0;
+        for (int t = 0; t < e->ntraj; t++) {
+            const int n = (int)(e->off[t + 1] - e->off[t]);
+            const int g = (n + group - 1) / group;
+            ngrp = std::max(ngrp, g);
+            for (int i = 0; i < g; i++)
+                for (int j = i; j < g; j++) units.push_back(make_int4(t, i, j, 0));
+        }
+        e->tea.eps_group = group;
+        part = (size_t)2 * ngrp * 5 * e->nb;
+    };
+    build(EPS_GROUP_MAX);
+    if ((int64_t)units.size() < 4 * (int64_t)e->num_cus) {
+        build(EPS_GROUP_MIN);
+        if (part * sizeof(float) > EPS_PART_MAX_BYTES) build(EPS_GROUP_MAX);
     }
-    const size_t part = (size_t)2 * ngrp * 5 * e->nb;
     e->tune.tea_eps = MTE_TEA_EPS_TWOSIDED;
     if (units.empty() || part * sizeof(float) > EPS_PART_MAX_BYTES) return hipSuccess;
     hipError_t s;

@@ -55,17 +55,19 @@ struct TeaBuffers {
     float4 *rec = nullptr;
     int *rbead = nullptr;
     // epsilon with each pair evaluated once (k_tea_eps_sym): work units
-    // (traj, I group, J group >= I group) of 1024-bead groups, and the
-    // partial sums [side][group][5][nb]; null when they would not fit
+    // (traj, I group, J group >= I group) of groups of eps_group beads, and
+    // the partial sums [side][group][5][nb]; null when they would not fit
     int4 *eps_units = nullptr;
     int eps_nunits = 0;
     int eps_ngrp = 0;          // most groups of one trajectory
+    int eps_group = 0;         // EPS_GROUP_MIN or EPS_GROUP_MAX
     float *eps_part = nullptr;
 };
 
-// Beads per group of the one-pass epsilon kernel (16 chunks of 64) and the
-// largest partial-sum buffer it may take.
-constexpr int EPS_GROUP = 1024;
+// Beads per group of the one-pass epsilon kernel in small and large batches,
+// the 64-bead chunks that a wave takes in the latter, and the largest
+// partial-sum buffer.
+constexpr int EPS_GROUP_MIN = 256, EPS_GROUP_MAX = 1024, EPS_PER = 4;
 constexpr size_t EPS_PART_MAX_BYTES = size_t(6) << 30;
 
 // MTE_TEA_SYMMETRIC: J chunks that a unit takes at most.

@@ -44,18 +44,26 @@ __device__ __forceinline__ float wave_rol1(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x134, 0xF, 0xF, false));
 }
 
-// wave_rol1(v) + p, the rotation a DPP operand of the addition.
-__device__ __forceinline__ float wave_rol1_add(float v, float p) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x134, 0xF, 0xF, true)) + p;
+// Keeps a loop constant in a vector register: an FP32 operation with a scalar
+// operand issues at half rate (4 cycles per wave, measured, against 2).
+__device__ __forceinline__ float in_vgpr(float v) {
+    __asm__("" : "+v"(v));
+    return v;
 }
 
-// The far branch of rpy_select alone (r > 2a).
-__device__ __forceinline__ RpyCoef rpy_far(float rinv, float a) {
-    const float u1 = a * rinv, u2 = u1 * u1;
-    RpyCoef c;
-    c.cii = 0.75f * u1 * fmaf(0.66666666666666667f, u2, 1.f);
-    c.crr = 0.75f * u1 * fmaf(-2.f, u2, 1.f);
-    return c;
+// One coordinate of the pair loops: x itself, or (INT) its place in the
+// periodic box as a 32-bit integer (bit pattern), taken modulo the box in FP64.
+template <bool INT>
+__device__ __forceinline__ float pair_coord(float x, double ibox) {
+    if (!INT) return x;
+    double v = (double)x * ibox;
+    v -= rint(v);
+    // 1.5 2^52 leaves the rounded integer in the low mantissa word
+    return __int_as_float(__double2loint(fma(v, 4294967296.0, 6755399441055744.0)));
+}
+template <bool INT>
+__device__ __forceinline__ float pair_diff(float a, float b) {
+    return INT ? (float)(__float_as_int(a) - __float_as_int(b)) : a - b;
 }
 
 // Epsilon partials and ci of bead i over all j of its trajectory
@@ -134,10 +142,10 @@ __global__ void __launch_bounds__(TEA_TILE)
 // Epsilon partials and ci with each pair evaluated once.  The five sums of
 // k_tea_eps are even in e (cii^2, crr (2 cii + crr) e_a^2, 3 cii + crr
 // (ex + ey + ez)^2), so a pair adds the same terms to both beads.  Work unit:
-// (trajectory, 1024-bead group I, group J >= I), one workgroup of
-// EPS_WAVES waves; wave w takes chunks c = 16 I + w + h EPS_WAVES, h <
-// EPS_PER (64 beads each, one bead of each per lane) against each 64-bead
-// chunk c_J of group J in turn, staged in LDS:
+// (trajectory, group I of WAVES x PER chunks of 64 beads, group J >= I), one
+// workgroup of WAVES waves; wave w takes chunks c = WAVES (PER I + h) + w,
+// h < PER (one bead of each per lane) against each chunk c_J of group J in
+// turn, staged in LDS:
 //   c_J > c    both sides, lane l meeting j = (l + s) mod 64 at step s, the
 //              j-side sums carried along by a one-lane rotation (wave_rol1);
 //              when c_J lies above all of the wave's chunks, the lane's
@@ -146,165 +154,182 @@ __global__ void __launch_bounds__(TEA_TILE)
 //   c_J < c    nothing (that pair of chunks is the wave c_J's).
 // The waves' j-side sums of a chunk are added in wave order in LDS.  Output
 // (deterministic, no atomics): i-side sums of a bead of group H into
-// part[0][J][.] for J >= H, j-side sums into part[1][I][.] for I <= H; the
-// pair weight is 1 for two non-extra beads and 0 otherwise (WEIGHTED: some
-// bead of the batch is extra; without, every weight is 1 and none is formed).
-constexpr int EPS_CHUNKS = EPS_GROUP / 64;        // 64-bead chunks of a group
-constexpr int EPS_PER = 4;                        // chunks of a wave
-constexpr int EPS_WAVES = EPS_CHUNKS / EPS_PER;   // waves of a workgroup
-static_assert(EPS_CHUNKS % EPS_PER == 0 && EPS_WAVES >= 2, "chunks split over the waves; 128 threads stage c_J");
-template <bool PERIODIC, bool WEIGHTED>
-__global__ void __launch_bounds__(64 * EPS_WAVES)
-    k_tea_eps_sym(mte_params P, DevTopo T, DevState S, const int4 *units, int ngrp, float *part) {
-    __shared__ float4 jx[2 * 64];              // chunk c_J: x, weight; twice, no wrap
-    __shared__ float jred[EPS_WAVES][5][64];   // j-side sums of each wave
-    const int4 u = units[blockIdx.x];
-    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+// part[0][J][.] for J >= H, j-side sums into part[1][I][.] for I <= H.  A pair
+// counts for two non-extra beads (WEIGHTED: some bead of the batch is extra)
+// inside the trajectory: the weight, 0 or 1, multiplies 1 / r, of which every
+// far term holds a power, and the near terms themselves.
+//
+// With v = 1 / r^2, u = a / r (far branch) the terms are
+//   cii^2   = 9/16 a^2  v A^2            A = 1 + 2/3 a^2 v
+//   k e_x^2 = 9/16 a^2  v^2 B E  d_x^2   B = 1 - 2 a^2 v, E = 3 - 2/3 a^2 v
+//   3 cii + crr (e_x + e_y + e_z)^2 = 3/4 a  (1 / r) (3 A + B v (d_x + d_y + d_z)^2)
+// so the loop sums them without their constant factors and forms no unit
+// vector; lengths and minimum images are those of the pair kernel below.
+// Bound: VALU issue, 38 operations per pair and 64 lanes in a box, of them 32
+// FP32 adds and products, at a clock that falls to 2.2 GHz under them; four or
+// two chunks per wave, 4 or 6 waves per SIMD, take the same time.  Measured,
+// against unit vectors, per-pair constant factors and float minimum images:
+// eight periodic trajectories of 24k-40k beads (4.2e9 pairs) 4.48 -> 3.81 ms,
+// 64 x 1040 beads 351 -> 75 us (with the smaller groups, tea_build_eps_units).
+// Waves of a workgroup whose waves take `per` chunks.
+constexpr int eps_waves(int per) { return per == 1 ? 4 : EPS_GROUP_MAX / 64 / per; }
+// What a pair's terms need beside the beads, in loop units.
+struct EpsCoef {
+    float s2, c1, c2, c3, c4;   // a^2 and its multiples 2/3, -2, -2/3, 2
+    float near2, ia, r2min;     // (2a)^2 with its margin, 1 / a, the floor of r^2
+    float i0, i4;               // 1 / (9/16 a^2), 1 / (3/4 a)
+};
+
+// One pair's five terms: added to the sums t and, unless ONE_SIDE, to t2,
+// which takes the next lane's t2 first when SIDES is ROTATE (the j-side
+// rotation, done with the first of the lane's beads to meet this j).  WT: the
+// pair's weight ww is formed.
+enum EpsSides { ONE_SIDE, BOTH_SIDES, ROTATE };
+template <bool INT, bool WT, EpsSides SIDES>
+__device__ __forceinline__ void eps_pair(const EpsCoef &K, float3 xa, float wa, float4 xj, float (&t)[5],
+                                         float (&t2)[5]) {
+    const float dx = pair_diff<INT>(xj.x, xa.x), dy = pair_diff<INT>(xj.y, xa.y), dz = pair_diff<INT>(xj.z, xa.z);
+    // r2min (1e-12 nm^2) keeps coincident beads finite and is below the
+    // rounding of any other r^2
+    const float qx = dx * dx, qy = dy * dy, qz = fmaf(dz, dz, K.r2min);
+    const float r2 = (qx + qy) + qz;
+    const float ww = WT ? wa * xj.w : 1.f;
+    float rinv = rsq_fast(r2);
+    if (WT) rinv *= ww;
+    const float v = rinv * rinv;
+    const float A = fmaf(K.c1, v, 1.f), B = fmaf(K.c2, v, 1.f);
+    const float Bv = B * v, sd = (dx + dy) + dz;
+    float m = v * A, mA = A;                                             // cii^2 = m mA
+    float kk = Bv * (v * fmaf(K.c3, v, 3.f));                            // crr (2 cii + crr) / r^2
+    float h = rinv, hA = fmaf(Bv, sd * sd, fmaf(K.c4, v, 3.f));          // 3 cii + crr se^2 = h hA
+    if (__any(r2 <= K.near2)) {
+        __asm__ volatile("");   // a branch: the near form is not evaluated otherwise
+        const float rn = rsq_fast(r2), ra = r2 * rn * K.ia;
+        const bool nr = !(ra > 2.f);
+        const float cii = fmaf(-0.28125f, ra, 1.f), crr = 0.09375f * ra, vn = rn * rn;
+        m = nr ? ww * K.i0 * cii : m;
+        mA = nr ? cii : mA;
+        kk = nr ? ww * K.i0 * crr * fmaf(2.f, cii, crr) * vn : kk;
+        h = nr ? ww * K.i4 : h;
+        hA = nr ? fmaf(crr * vn, sd * sd, 3.f * cii) : hA;
+    }
+    t[0] = fmaf(m, mA, t[0]);
+    t[1] = fmaf(kk, qx, t[1]);
+    t[2] = fmaf(kk, qy, t[2]);
+    t[3] = fmaf(kk, qz, t[3]);
+    t[4] = fmaf(h, hA, t[4]);
+    if (SIDES != ONE_SIDE) {
+        constexpr bool ROT = SIDES == ROTATE;
+        t2[0] = fmaf(m, mA, ROT ? wave_rol1(t2[0]) : t2[0]);
+        t2[1] = fmaf(kk, qx, ROT ? wave_rol1(t2[1]) : t2[1]);
+        t2[2] = fmaf(kk, qy, ROT ? wave_rol1(t2[2]) : t2[2]);
+        t2[3] = fmaf(kk, qz, ROT ? wave_rol1(t2[3]) : t2[3]);
+        t2[4] = fmaf(h, hA, ROT ? wave_rol1(t2[4]) : t2[4]);
+    }
+}
+
+// The lane's N beads against every j of the staged chunk, both sides.
+template <bool INT, bool WT, int N>
+__device__ __forceinline__ void eps_sweep(const EpsCoef &K, const float4 *jl, const float3 *xi, const float *wi,
+                                          float (*ai)[5], float (&gj)[5]) {
+#pragma unroll 1
+    for (int s = 0; s < 64; s++) {
+        const float4 xj = jl[s];
+        eps_pair<INT, WT, ROTATE>(K, xi[0], wi[0], xj, ai[0], gj);
+#pragma unroll
+        for (int h = 1; h < N; h++) eps_pair<INT, WT, BOTH_SIDES>(K, xi[h], wi[h], xj, ai[h], gj);
+    }
+}
+
+template <bool INT, bool WEIGHTED, int PER>
+__device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, const DevState &S, int4 u, int ngrp,
+                                         float *part, float4 *jx, float (*jred)[5][64]) {
+    constexpr int WAVES = eps_waves(PER), CHUNKS = WAVES * PER;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), l = threadIdx.x % 64;
     const int base = T.tbase[u.x], n = T.tsize[u.x], nb = T.nb;
     const int nch = (n + 63) / 64;
-    // Lengths in the pair loop are in box units in a periodic box (positions
-    // x / box, so the minimum image is d - rint(d)) and in nm otherwise:
-    // sc is the unit's inverse, wf 1 where the image is taken.
     const float box = T.tbox[u.x];
-    const bool wrap = PERIODIC && box > 0.f;
-    const float sc = wrap ? inv_side(box) : 1.f, wf = wrap ? 1.f : 0.f;
-    const float a = P.tea_a * sc, ia = rcp_fast(P.tea_a) * (wrap ? box : 1.f);
-    const float r2min = 1e-12f * sc * sc;
+    const double ibox = INT ? 1.0 / (double)box : 0.0;
+    const float sc = INT ? box * 0x1p-32f : 1.f;   // nm per loop unit
+    const float a = P.tea_a / sc, s2 = a * a, lim = 2.002f * a;
+    EpsCoef K;
+    K.s2 = s2;
+    K.c1 = in_vgpr(0.66666666666666667f * s2);
+    K.c2 = in_vgpr(-2.f * s2);
+    K.c3 = in_vgpr(-0.66666666666666667f * s2);
+    K.c4 = in_vgpr(2.f * s2);
+    K.near2 = in_vgpr(lim * lim);
+    K.ia = sc * rcp_fast(P.tea_a);
+    K.r2min = in_vgpr(1e-12f / (sc * sc));
+    K.i0 = 1.f / (0.5625f * s2);
+    K.i4 = 1.f / (0.75f * a);
     // the lane's bead in each of the wave's chunks
-    int cI[EPS_PER], li[EPS_PER];
-    bool vi[EPS_PER];
-    float3 xi[EPS_PER];
-    float wi[EPS_PER], ai[EPS_PER][5];
+    int cI[PER];
+    bool vi[PER];
+    float3 xi[PER];
+    float wi[PER], ai[PER][5];
+    auto bead = [&](int li, float &wt) {
+        wt = 0.f;
+        if (li >= n) return make_float3(0.f, 0.f, 0.f);
+        const float3 x = f3(S.xyz[base + li]);
+        // a lost position (inf, NaN), which an integer cannot hold, spreads
+        // through the bead's weight as it would through r
+        const float lost = INT ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
+        wt = (T.extra[base + li] ? 0.f : 1.f) + lost;
+        return make_float3(pair_coord<INT>(x.x, ibox), pair_coord<INT>(x.y, ibox), pair_coord<INT>(x.z, ibox));
+    };
+    bool odd = false;   // a lost bead among the lane's own
 #pragma unroll
-    for (int h = 0; h < EPS_PER; h++) {
-        cI[h] = u.y * EPS_CHUNKS + w + h * EPS_WAVES;
-        li[h] = cI[h] * 64 + l;
-        vi[h] = li[h] < n;
-        xi[h] = make_float3(0.f, 0.f, 0.f);
-        wi[h] = 0.f;
-        if (vi[h]) {
-            const float3 x = f3(S.xyz[base + li[h]]);
-            xi[h] = make_float3(x.x * sc, x.y * sc, x.z * sc);
-            wi[h] = T.extra[base + li[h]] ? 0.f : 1.f;
-        }
+    for (int h = 0; h < PER; h++) {
+        cI[h] = u.y * CHUNKS + w + h * WAVES;
+        vi[h] = cI[h] * 64 + l < n;
+        xi[h] = bead(cI[h] * 64 + l, wi[h]);
+        odd |= !(fabsf(wi[h]) <= 1.f);
 #pragma unroll
         for (int k = 0; k < 5; k++) ai[h][k] = 0.f;
     }
-    const int c0 = u.z * EPS_CHUNKS, c1 = min(c0 + EPS_CHUNKS, nch);
-    // one pair's five terms p: added to the sums t; with t2 (both sides),
-    // t2 += p, after t2 takes the next lane's t2 when ROT (the j-side
-    // rotation, done with the first of the lane's beads to meet this j).  A
-    // wave with no pair inside 2a (margin over the rounding of r / a) keeps
-    // the far coefficients, which is the branch rpy_select picks for each of
-    // its pairs.  WT: the pair weights are formed (extra beads in the batch,
-    // or the padding of a trajectory's last chunk, whose slots have weight 0).
-    const float near2 = (2.002f * a) * (2.002f * a);
-    auto pair = [&](auto wt, auto rot, const float3 &xa, float wa, float4 xj, float *t, float *t2) {
-        constexpr bool WT = decltype(wt)::value, ROT = decltype(rot)::value;
-        float3 d = make_float3(xj.x - xa.x, xj.y - xa.y, xj.z - xa.z);
-        if (PERIODIC) {
-            d.x = fmaf(-wf, rintf(d.x), d.x);
-            d.y = fmaf(-wf, rintf(d.y), d.y);
-            d.z = fmaf(-wf, rintf(d.z), d.z);
-        }
-        const float r2 = fmaxf(d.x * d.x + d.y * d.y + d.z * d.z, r2min);
-        const float rinv = rsq_fast(r2);
-        RpyCoef c = rpy_far(rinv, a);
-        if (__any(r2 <= near2)) {
-            __asm__ volatile("");   // a branch: no speculation of the near form
-            const float ra = r2 * rinv * ia;
-            const bool nr = !(ra > 2.f);
-            c.cii = nr ? fmaf(-0.28125f, ra, 1.f) : c.cii;
-            c.crr = nr ? 0.09375f * ra : c.crr;
-        }
-        const float ww = WT ? wa * xj.w : 1.f;
-        const float ex = d.x * rinv, ey = d.y * rinv, ez = d.z * rinv;
-        const float cw = WT ? ww * c.cii : c.cii;
-        const float wcrr = WT ? ww * c.crr : c.crr;
-        const float k = wcrr * fmaf(2.f, c.cii, c.crr);
-        const float se = ex + ey + ez;
-        const float tall = fmaf(wcrr, se * se, 3.f * cw);
-        const float qx = ex * ex, qy = ey * ey, qz = ez * ez;
-        t[0] = fmaf(cw, c.cii, t[0]);
-        t[1] = fmaf(k, qx, t[1]);
-        t[2] = fmaf(k, qy, t[2]);
-        t[3] = fmaf(k, qz, t[3]);
-        t[4] += tall;
-        if (t2) {
-            t2[0] = fmaf(cw, c.cii, ROT ? wave_rol1(t2[0]) : t2[0]);
-            t2[1] = fmaf(k, qx, ROT ? wave_rol1(t2[1]) : t2[1]);
-            t2[2] = fmaf(k, qy, ROT ? wave_rol1(t2[2]) : t2[2]);
-            t2[3] = fmaf(k, qz, ROT ? wave_rol1(t2[3]) : t2[3]);
-            t2[4] = ROT ? wave_rol1_add(t2[4], tall) : t2[4] + tall;
-        }
-    };
-    const std::true_type yes{};
-    const std::false_type no{};
+    const bool wto = WEIGHTED || __any(odd);
+    const int c0 = u.z * CHUNKS, c1 = min(c0 + CHUNKS, nch);
+    float wj = 0.f;
     for (int cJ = c0; cJ < c1; cJ++) {
         if (threadIdx.x < 128) {
-            const int lj = cJ * 64 + (threadIdx.x % 64);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (lj < n) {
-                v = S.xyz[base + lj];
-                v.x *= sc;
-                v.y *= sc;
-                v.z *= sc;
-                v.w = T.extra[base + lj] ? 0.f : 1.f;
-            }
-            jx[threadIdx.x] = v;
+            const float3 x = bead(cJ * 64 + l, wj);
+            jx[threadIdx.x] = make_float4(x.x, x.y, x.z, wj);
         }
         __syncthreads();
+        const float4 *jl = jx + l;
         float gj[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
         // step s of a both-sided sweep: lane l meets j = (l + s) mod 64, its
         // gj the sums of that j (rotated in from lane l + 1, which held j at
         // the sweep's step s - 1; sweeps in a row continue the rotation).
-        // A chunk below c_J is full; c_J may be the padded last one.
-        bool two[EPS_PER], all = true;
+        // A chunk below c_J is full; c_J may be the padded last one, and its
+        // weights are formed there, or where a bead of it is lost.
+        const bool wtj = wto || (cJ + 1) * 64 > n || __any(!(fabsf(jx[l].w) <= 1.f));
+        int low = 0;   // the wave's chunks below c_J: the first `low`
 #pragma unroll
-        for (int h = 0; h < EPS_PER; h++) {
-            two[h] = cI[h] < nch && cJ > cI[h];
-            all = all && two[h];
-        }
-        const bool wtj = WEIGHTED || (cJ + 1) * 64 > n;
-        if (all) {
-            if (wtj)
-                for (int s = 0; s < 64; s++) {
-                    const float4 xj = jx[l + s];
-                    pair(yes, yes, xi[0], wi[0], xj, ai[0], gj);
+        for (int h = 0; h < PER; h++) low += cI[h] < nch && cJ > cI[h] ? 1 : 0;
+        if (low == PER) {
+            if (wtj) eps_sweep<INT, true, PER>(K, jl, xi, wi, ai, gj);
+            else eps_sweep<INT, false, PER>(K, jl, xi, wi, ai, gj);
+        } else if (PER > 1) {
 #pragma unroll
-                    for (int h = 1; h < EPS_PER; h++) pair(yes, no, xi[h], wi[h], xj, ai[h], gj);
-                }
-            else
-                for (int s = 0; s < 64; s++) {
-                    const float4 xj = jx[l + s];
-                    pair(no, yes, xi[0], wi[0], xj, ai[0], gj);
-#pragma unroll
-                    for (int h = 1; h < EPS_PER; h++) pair(no, no, xi[h], wi[h], xj, ai[h], gj);
-                }
-        } else {
-#pragma unroll
-            for (int h = 0; h < EPS_PER; h++)
-                if (two[h]) {
-                    if (wtj)
-                        for (int s = 0; s < 64; s++) pair(yes, yes, xi[h], wi[h], jx[l + s], ai[h], gj);
-                    else
-                        for (int s = 0; s < 64; s++) pair(no, yes, xi[h], wi[h], jx[l + s], ai[h], gj);
-                }
+            for (int h = 0; h < PER; h++)
+                if (h < low) eps_sweep<INT, true, 1>(K, jl, xi + h, wi + h, ai + h, gj);
         }
 #pragma unroll
-        for (int h = 0; h < EPS_PER; h++)
+        for (int h = 0; h < PER; h++)
             if (cI[h] < nch && cJ == cI[h]) {
-                // one-sided over the chunk's beads: no padding slot is met
+                // one-sided over the chunk's beads
                 const int jn = min(64, n - cJ * 64);
-                for (int q = 0; q < jn; q++)
-                    pair(std::integral_constant<bool, WEIGHTED>{}, no, xi[h], wi[h], jx[q], ai[h], nullptr);
-                if (!WEIGHTED || wi[h] != 0.f) {
-                    // the j == i slot entered as a coincident bead (d = 0):
-                    // cii^2 into the first sum and 3 cii into the last, taken out
-                    const float r2 = r2min, rinv = rsq_fast(r2);
-                    const float cii = rpy_select(r2, rinv, a, ia).cii;
-                    ai[h][0] = fmaf(-cii, cii, ai[h][0]);
-                    ai[h][4] = fmaf(-3.f, cii, ai[h][4]);
+#pragma unroll 1
+                for (int q = 0; q < jn; q++) eps_pair<INT, true, ONE_SIDE>(K, xi[h], wi[h], jx[q], ai[h], gj);
+                if (wi[h] != 0.f) {
+                    // the j == i slot entered as a coincident bead (r^2 =
+                    // r2min): cii^2 into the first sum and 3 cii into the
+                    // last, taken out
+                    const float cii = fmaf(-0.28125f, K.r2min * rsq_fast(K.r2min) * K.ia, 1.f);
+                    ai[h][0] = fmaf(-K.i0 * cii, cii, ai[h][0]);
+                    ai[h][4] = fmaf(-K.i4, 3.f * cii, ai[h][4]);
                 }
             }
         // after a multiple of 64 rotations lane l holds the sums of j =
@@ -312,33 +337,45 @@ __global__ void __launch_bounds__(64 * EPS_WAVES)
 #pragma unroll
         for (int k = 0; k < 5; k++) jred[w][k][(l + 63) & 63] = gj[k];
         __syncthreads();
-        for (int e = threadIdx.x; e < 5 * 64; e += 64 * EPS_WAVES) {
+        for (int e = threadIdx.x; e < 5 * 64; e += 64 * WAVES) {
             const int k = e / 64, q = e % 64;
             const int lj = cJ * 64 + q;
             if (lj < n) {
                 float sum = 0.f;
-                for (int v = 0; v < EPS_WAVES; v++) sum += jred[v][k][q];
-                part[(((size_t)1 * ngrp + u.y) * 5 + k) * nb + base + lj] = sum;
+                for (int v = 0; v < WAVES; v++) sum += jred[v][k][q];
+                part[(((size_t)1 * ngrp + u.y) * 5 + k) * nb + base + lj] = sum * (k < 4 ? 0.5625f * s2 : 0.75f * a);
             }
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int h = 0; h < EPS_PER; h++)
+    for (int h = 0; h < PER; h++)
         if (vi[h]) {
 #pragma unroll
-            for (int k = 0; k < 5; k++) part[(((size_t)0 * ngrp + u.z) * 5 + k) * nb + base + li[h]] = ai[h][k];
+            for (int k = 0; k < 5; k++)
+                part[(((size_t)0 * ngrp + u.z) * 5 + k) * nb + base + cI[h] * 64 + l] =
+                    ai[h][k] * (k < 4 ? 0.5625f * s2 : 0.75f * a);
         }
+}
+
+template <bool PERIODIC, bool WEIGHTED, int PER>
+__global__ void __launch_bounds__(64 * eps_waves(PER))
+    k_tea_eps_sym(mte_params P, DevTopo T, DevState S, const int4 *units, int ngrp, float *part) {
+    __shared__ float4 jx[2 * 64];              // chunk c_J: x, weight; twice, no wrap
+    __shared__ float jred[eps_waves(PER)][5][64];   // j-side sums of each wave
+    const int4 u = units[blockIdx.x];
+    if (PERIODIC && T.tbox[u.x] > 0.f) eps_unit<true, WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
+    else eps_unit<false, WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
 }
 
 // Per bead: the group sums of k_tea_eps_sym added in fixed order into ci and
 // eps, as k_tea_eps writes them.
 __global__ void __launch_bounds__(256)
-    k_tea_eps_reduce(DevTopo T, int ngrp, const float *part, float4 *ci, float *eps) {
+    k_tea_eps_reduce(DevTopo T, int group, int ngrp, const float *part, float4 *ci, float *eps) {
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= T.nb) return;
     const int t = T.tid[b], n = T.tsize[t];
-    const int h = (b - T.tbase[t]) / EPS_GROUP, g = (n + EPS_GROUP - 1) / EPS_GROUP;
+    const int h = (b - T.tbase[t]) / group, g = (n + group - 1) / group;
     const int nb = T.nb;
     // each of the five sums in the same order (groups h..g-1 of side 0, then
     // 0..h of side 1), the five advancing together so their loads overlap
@@ -420,13 +457,6 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Keeps a loop constant in a vector register: an FP32 operation with a scalar
-// operand issues at half rate (4 cycles per wave, measured, against 2).
-__device__ __forceinline__ float in_vgpr(float v) {
-    __asm__("" : "+v"(v));
-    return v;
-}
-
 // Pair sums with each (i, j) RPY block evaluated once for both beads.  Work
 // unit: (trajectory, I pair p: the 64-bead chunks 2p and 2p + 1, chunks J of a
 // range at or above 2p).  D_hat_ji = D_hat_ij, so a block serves
@@ -487,21 +517,6 @@ __device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float sc) {
     K.ia = sc * rcp_fast(P.tea_a);
     K.r2min = 1e-12f / (sc * sc);
     return K;
-}
-
-// One coordinate in loop units: x itself, or its place in the box as a
-// 32-bit integer (bit pattern), taken modulo the box in FP64.
-template <bool INT>
-__device__ __forceinline__ float pair_coord(float x, double ibox) {
-    if (!INT) return x;
-    double v = (double)x * ibox;
-    v -= rint(v);
-    // 1.5 2^52 leaves the rounded integer in the low mantissa word
-    return __int_as_float(__double2loint(fma(v, 4294967296.0, 6755399441055744.0)));
-}
-template <bool INT>
-__device__ __forceinline__ float pair_diff(float a, float b) {
-    return INT ? (float)(__float_as_int(a) - __float_as_int(b)) : a - b;
 }
 
 // Bead b (zeros where it is not valid); extra beads have zero F and R.
@@ -1281,14 +1296,24 @@ __global__ void __launch_bounds__(256)
     partial[(size_t)slot * chunk_stride + bi] = make_float4(f.x, f.y, f.z, 0.f);
 }
 
+template <int PER>
+static void launch_eps_per(mte_engine *e) {
+    auto kern = e->periodic ? (e->any_extra ? k_tea_eps_sym<true, true, PER> : k_tea_eps_sym<true, false, PER>)
+                            : (e->any_extra ? k_tea_eps_sym<false, true, PER> : k_tea_eps_sym<false, false, PER>);
+    hipLaunchKernelGGL(kern, dim3(e->tea.eps_nunits), dim3(64 * eps_waves(PER)), 0, e->stream, e->P, e->T, e->S[e->cur],
+                       e->tea.eps_units, e->tea.eps_ngrp, e->tea.eps_part);
+}
+static void launch_eps_units(mte_engine *e) {
+    if (e->tea.eps_group == EPS_GROUP_MIN) launch_eps_per<1>(e);
+    else launch_eps_per<EPS_PER>(e);
+}
+static_assert(EPS_GROUP_MIN == 64 * eps_waves(1), "a group is the workgroup's chunks");
+
 hipError_t launch_tea_eps(mte_engine *e) {
     if (e->tune.tea_eps == MTE_TEA_EPS_ONEPASS) {
-        auto kern = e->periodic ? (e->any_extra ? k_tea_eps_sym<true, true> : k_tea_eps_sym<true, false>)
-                                : (e->any_extra ? k_tea_eps_sym<false, true> : k_tea_eps_sym<false, false>);
-        hipLaunchKernelGGL(kern, dim3(e->tea.eps_nunits), dim3(64 * EPS_WAVES), 0, e->stream, e->P, e->T, e->S[e->cur],
-                           e->tea.eps_units, e->tea.eps_ngrp, e->tea.eps_part);
+        launch_eps_units(e);
         hipLaunchKernelGGL(k_tea_eps_reduce, dim3((e->nb + 255) / 256), dim3(256), 0, e->stream, e->T,
-                           e->tea.eps_ngrp, e->tea.eps_part, e->tea.ci, e->tea.eps);
+                           e->tea.eps_group, e->tea.eps_ngrp, e->tea.eps_part, e->tea.ci, e->tea.eps);
     } else if (e->periodic)
         hipLaunchKernelGGL(k_tea_eps<true>, dim3(e->ntiles), dim3(TEA_TILE), 0, e->stream, e->P, e->T,
                            e->S[e->cur], e->tiles, e->tea.ci, e->tea.eps);
