@@ -35,12 +35,11 @@ struct CellGeom {
 };
 
 // Cells of side >= `side` (searched K cells either way, so side = r / K covers
-// a radius r); a periodic box has at least 2K + 1 cells per side, in which
-// case the stencil spans the whole box.
+// a radius r).
 __device__ __forceinline__ CellGeom cell_geom(float box, float side, int K) {
     CellGeom g;
     if (box > 0.f) {
-        g.dims = max(2 * K + 1, (int)floorf(box / side));
+        g.dims = cell_dims(box, side, K);
         g.cs = box / (float)g.dims;
     } else {
         g.dims = 0;

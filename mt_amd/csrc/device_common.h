@@ -95,6 +95,19 @@ __device__ __forceinline__ float3 min_image_pre(float3 d, float L, float iL) {
 }
 __device__ __forceinline__ float3 sub3(float3 a, float3 b) { return make_float3(a.x - b.x, a.y - b.y, a.z - b.z); }
 
+// Cells per side of a periodic box for cells of side >= `side` searched K
+// cells either way (at least 2K + 1, where the stencil spans the whole box).
+// Every kernel that reads a cell table must count the cells as the kernel
+// that filled it did, but the fast division rounds otherwise where the
+// compiler knows `side` (672 nm / 12 nm came to 56 in one kernel and to 55 in
+// another): products decide, which round alike everywhere.
+__device__ __forceinline__ int cell_dims(float box, float side, int K) {
+    int n = (int)floorf(box / side);
+    if ((float)n * side > box) n--;
+    if ((float)(n + 1) * side <= box) n++;
+    return max(2 * K + 1, n);
+}
+
 // Periodic cell index: i in [-dims, 2 dims) wrapped into [0, dims) (a
 // neighbour stencil never reaches further), without an integer division.
 __device__ __forceinline__ int wrap_cell(int i, int dims) { return i < 0 ? i + dims : (i >= dims ? i - dims : i); }

@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(MLP_BLOCK)
     float A[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int cnt = 0;
     if (!T.extra[b]) {
-        const int dims = box > 0.f ? max(3, (int)floorf(box / MLP_RC)) : 0;
+        const int dims = box > 0.f ? cell_dims(box, MLP_RC, 1) : 0;
         const int4 me = C.cell[b];
         const uint32_t mask = (uint32_t)(C.tsize[t] - 1);
         const int toff = C.toff[t];

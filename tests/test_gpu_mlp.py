@@ -144,3 +144,28 @@ def test_trained_network_gains_over_free_draining():
     print(f"D tea {D['tea']:.5g} none {D['none']:.5g} mlp {D['mlp']:.5g}", flush=True)
     assert gap_none > 0.03
     assert gap_mlp < 0.5 * gap_none
+
+
+@pytest.mark.parametrize("box", [48.0, 264.0, 672.0, 768.0])
+def test_labels_across_the_boundary_of_a_whole_number_of_cells(box):
+    """Boxes that are multiples of the 12 nm search radius: the search must
+    count the cells per side as the table it reads did, or neighbours across
+    the boundary are lost."""
+    print(f"case MLP labels, box {box}", flush=True)
+    from mt_amd import lattice, topology
+    p = P.derive(dict(P.TEA))
+    rng = np.random.default_rng(3)
+    n = int(min(60, box ** 3 / 4000.0))
+    # dimers spread over the box and pairs of them on both sides of each face
+    cen = rng.uniform(0.0, box, (n, 3))
+    at = np.concatenate([cen, np.array([[1.0, 9.0, 9.0], [box - 4.0, 9.0, 9.0], [20.0, 0.5, 20.0],
+                                        [20.0, box - 6.0, 20.0], [30.0, 30.0, 1.0], [30.0, 30.0, box - 5.0]])])
+    a = lattice.free_dimers(len(at), 2000.0, rng, chain="Y")
+    a.xyz[0::2], a.xyz[1::2] = at - [0.0, 0.0, 2.0], at + [0.0, 0.0, 2.0]
+    b = topology.make_batch([a], [lattice.coords7(a, 0.0)], box=[box])
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    f, t = eng.mlp_local()
+    fo, to = M.local_features_targets(b.coords, b.off, b.extra, b.box, p.tea_a)
+    np.testing.assert_allclose(f, fo, atol=2e-5)   # positions of up to 768 nm: 2^-23 x 768 over 12 nm
+    np.testing.assert_allclose(t, to, rtol=1e-4, atol=1e-4 * np.abs(to).max())
+    eng.close()
