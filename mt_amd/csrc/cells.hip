@@ -25,37 +25,10 @@ namespace mte {
 constexpr int CELL_BLOCK = 64;
 constexpr int CAND_CAP = 128;   // candidates per bead within the candidate radius
 
-__device__ __forceinline__ uint32_t cell_hash(int cx, int cy, int cz) {
-    return ((uint32_t)cx * 73856093u) ^ ((uint32_t)cy * 19349663u) ^ ((uint32_t)cz * 83492791u);
-}
-
-struct CellGeom {
-    float cs;      // cell side
-    int dims;      // cells per side in a periodic box (0: open)
-};
-
-// Cells of side >= `side` (searched K cells either way, so side = r / K covers
-// a radius r).
-__device__ __forceinline__ CellGeom cell_geom(float box, float side, int K) {
-    CellGeom g;
-    if (box > 0.f) {
-        g.dims = cell_dims(box, side, K);
-        g.cs = box / (float)g.dims;
-    } else {
-        g.dims = 0;
-        g.cs = side;
-    }
-    return g;
-}
-
 __device__ __forceinline__ int3 cell_of(float3 r, float box, const CellGeom &g) {
-    if (g.dims > 0) {
-        const float wx = r.x - box * floorf(r.x / box), wy = r.y - box * floorf(r.y / box),
-                    wz = r.z - box * floorf(r.z / box);
-        return make_int3(min(g.dims - 1, (int)(wx / g.cs)), min(g.dims - 1, (int)(wy / g.cs)),
-                         min(g.dims - 1, (int)(wz / g.cs)));
-    }
-    return make_int3((int)floorf(r.x / g.cs), (int)floorf(r.y / g.cs), (int)floorf(r.z / g.cs));
+    const float x = cell_coord(r.x, box, g), y = cell_coord(r.y, box, g), z = cell_coord(r.z, box, g);
+    if (g.dims > 0) return make_int3(min(g.dims - 1, (int)x), min(g.dims - 1, (int)y), min(g.dims - 1, (int)z));
+    return make_int3((int)floorf(x), (int)floorf(y), (int)floorf(z));
 }
 
 // The bead's slot within its bucket comes from one atomic per bucket and

@@ -108,6 +108,26 @@ __device__ __forceinline__ int cell_dims(float box, float side, int K) {
     return max(2 * K + 1, n);
 }
 
+struct CellGeom {
+    float cs;      // cell side
+    int dims;      // cells per side in a periodic box (0: open)
+};
+__device__ __forceinline__ CellGeom cell_geom(float box, float side, int K) {
+    CellGeom g;
+    g.dims = box > 0.f ? cell_dims(box, side, K) : 0;
+    g.cs = g.dims > 0 ? box / (float)g.dims : side;
+    return g;
+}
+// A coordinate in cells from the origin (of the box, where it is periodic).
+__device__ __forceinline__ float cell_coord(float x, float box, const CellGeom &g) {
+    if (g.dims > 0) x -= box * floorf(x / box);
+    return x / g.cs;
+}
+
+// Bucket hash of a cell, masked to the table's size by the caller.
+__device__ __forceinline__ uint32_t cell_hash(int cx, int cy, int cz) {
+    return ((uint32_t)cx * 73856093u) ^ ((uint32_t)cy * 19349663u) ^ ((uint32_t)cz * 83492791u);
+}
 // Periodic cell index: i in [-dims, 2 dims) wrapped into [0, dims) (a
 // neighbour stencil never reaches further), without an integer division.
 __device__ __forceinline__ int wrap_cell(int i, int dims) { return i < 0 ? i + dims : (i >= dims ? i - dims : i); }

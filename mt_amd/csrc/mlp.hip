@@ -21,11 +21,15 @@
 #include "engine_internal.h"
 
 #include <mutex>
+#include <type_traits>
 
 namespace mte {
 
 constexpr int MLP_BLOCK = MLP_SEARCH_BLOCK;
+constexpr int MLP_LANES = 4;   // lanes per bead of the neighbour search
 constexpr float MLP_RC = 12.f, MLP_RIN = 8.f;
+constexpr float MLP_CELL = 2.f * MLP_RC + 0.02f;   // search cells: the margin is far above the rounding of a
+                                                   // bead's place in its cell
 // flat parameter offsets
 constexpr int OW1 = 0, OB1 = OW1 + MLP_IN * MLP_H, OW2 = OB1 + MLP_H, OB2 = OW2 + MLP_H * MLP_H, OW3 = OB2 + MLP_H,
               OB3 = OW3 + MLP_H * MLP_H, OW4 = OB3 + MLP_H, OB4 = OW4 + MLP_H * MLP_OUT;
@@ -42,118 +46,231 @@ __device__ __forceinline__ float taper(float r) {
 // ------------------------------------------------------------ features, labels
 constexpr int FEAT_BLK_NN = 8;   // neighbours per block of written features (24 floats: whole
                                  // float4 stores and whole 8-float MFMA operand slices)
-static_assert(3 * FEAT_BLK_NN % 8 == 0 && FEAT_BLK_NN % 4 == 0, "feature blocks");
-// The 27 bucket ranges of a search as [first, end) slots of the bucket-ordered
-// positions.  A trajectory's beads hold the slots [base, base + n) of its
-// buckets, so with trajectory-local indices of 16 bits (n < 65536) both ends
-// pack into one register.
+static_assert(3 * FEAT_BLK_NN % 8 == 0 && FEAT_BLK_NN % 4 == 0 && FEAT_BLK_NN * MLP_LANES == MLP_NN,
+              "feature blocks, one per lane of the bead");
+// A bucket's range as [first, end) slots of the bucket-ordered positions.  A
+// trajectory's beads hold the slots [base, base + n) of its buckets, so with
+// trajectory-local indices of 16 bits (n < 65536) both ends pack into one
+// word.
 template <typename JT>
-struct BucketRanges {
+struct BucketRange {
     using W = int2;
-    W v[27];
-    __device__ __forceinline__ void set(int o, int2 r, int) { v[o] = make_int2(r.x, r.x + r.y); }
-    __device__ __forceinline__ void clear(int o) { v[o] = make_int2(0, 0); }
+    __device__ __forceinline__ static W pack(int2 r, int) { return make_int2(r.x, r.x + r.y); }
+    __device__ __forceinline__ static W none() { return make_int2(0, 0); }
     __device__ __forceinline__ static int lo(W w, int) { return w.x; }
     __device__ __forceinline__ static int hi(W w, int) { return w.y; }
 };
 template <>
-struct BucketRanges<uint16_t> {
+struct BucketRange<uint16_t> {
     using W = uint32_t;
-    W v[27];
-    __device__ __forceinline__ void set(int o, int2 r, int base) {
+    __device__ __forceinline__ static W pack(int2 r, int base) {
         const uint32_t s = (uint32_t)(r.x - base);
-        v[o] = s | ((s + (uint32_t)r.y) << 16);
+        return s | ((s + (uint32_t)r.y) << 16);
     }
-    __device__ __forceinline__ void clear(int o) { v[o] = 0; }
+    __device__ __forceinline__ static W none() { return 0; }
     __device__ __forceinline__ static int lo(W w, int base) { return base + (int)(w & 0xffffu); }
     __device__ __forceinline__ static int hi(W w, int base) { return base + (int)(w >> 16); }
 };
 
-// Neighbour scan over the 27 cells of the hashed table (built with cell side
-// >= 12 nm, or 3 cells per side covering the whole box).  The 27 bucket
-// ranges are loaded up front; a bucket that two of the cells hash to is
-// visited once, and the candidates are streamed from the bucket-ordered
-// positions.  Every bead within 12 nm lies in one of the 27 cells, so
-// visiting their buckets (each once) sees it exactly once, and the distance
-// test rejects the beads of other cells sharing a bucket.  Keeps the 32
-// nearest (distance, then index) and sums the exact label over every
+// FP64 minimum and maximum of two keys (never NaN: the intrinsics would first
+// quiet both operands).
+__device__ __forceinline__ double key_min(double a, double b) {
+    double r;
+    __asm__("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double key_max(double a, double b) {
+    double r;
+    __asm__("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// kn into the ascending keys, slots K0 .. K1 - 1 of them: a slot takes the
+// middle one of its key, the key below and kn (from the top down).
+template <int K0, int K1>
+__device__ __forceinline__ void insert_key(double (&key)[MLP_NN], double kn) {
+#pragma unroll
+    for (int k = K1 - 1; k >= K0; k--) {
+        const double low = key_min(key[k], kn);
+        key[k] = k > 0 ? key_max(key[k - 1], low) : low;
+    }
+}
+// Index of the key at slot N part + u.
+template <int N>
+__device__ __forceinline__ int pick_key(const double (&key)[MLP_NN], int part, int u) {
+    const int j0 = __double2loint(key[u]), j1 = __double2loint(key[N + u]), j2 = __double2loint(key[2 * N + u]),
+              j3 = __double2loint(key[3 * N + u]);
+    return part & 2 ? (part & 1 ? j3 : j2) : (part & 1 ? j1 : j0);
+}
+
+// A value of the lane that differs in bit 0 (XOR = 1) or bit 1 (XOR = 2) of
+// its number, within the four lanes of a bead.
+template <int XOR>
+__device__ __forceinline__ int quad_swap(int v) {
+    return __builtin_amdgcn_mov_dpp(v, XOR == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true);   // quad_perm 1,0,3,2 / 2,3,0,1
+}
+template <int XOR>
+__device__ __forceinline__ double quad_swap(double v) {
+    return __hiloint2double(quad_swap<XOR>(__double2hiint(v)), quad_swap<XOR>(__double2loint(v)));
+}
+// The value of lane L of the bead's four.
+template <int L>
+__device__ __forceinline__ int quad_lane(int v) {
+    return __builtin_amdgcn_mov_dpp(v, L * 0x55, 0xF, 0xF, true);   // quad_perm L,L,L,L
+}
+template <int XOR>
+__device__ __forceinline__ float quad_swap(float v) {
+    return __int_as_float(quad_swap<XOR>(__float_as_int(v)));
+}
+
+// The first N keys of this lane and of the lane XOR of it, both ascending,
+// merged: the N smallest, ascending, in both lanes.  The smaller of key k
+// here and key N - 1 - k there are those N and a bitonic sequence.
+template <int XOR, int N>
+__device__ __forceinline__ void merge_keys(double (&key)[MLP_NN]) {
+#pragma unroll
+    for (int k = 0; k < N / 2; k++) {
+        const double a = key[k], b = key[N - 1 - k];
+        const double oa = quad_swap<XOR>(a), ob = quad_swap<XOR>(b);
+        key[k] = key_min(a, ob);
+        key[N - 1 - k] = key_min(b, oa);
+    }
+#pragma unroll
+    for (int d = N / 2; d > 0; d >>= 1)
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if ((k & d) == 0) {
+                const double a = key[k], b = key[k + d];
+                key[k] = key_min(a, b);
+                key[k + d] = key_max(a, b);
+            }
+}
+
+// Neighbour scan over eight cells of the hashed table.  Its cells are at
+// least twice the radius wide, so the sphere around a bead reaches at most
+// the cell on the nearer side in each direction (in a box of fewer than two
+// cells the bead's own cell is the whole side, and the second one the same).
+// The eight bucket ranges are loaded up front; a bucket that two of the cells
+// hash to is visited once, and the candidates are streamed from the
+// bucket-ordered positions.  Every bead within 12 nm lies in one of the
+// cells, so visiting their buckets (each once) sees it exactly once, and the
+// distance test rejects the beads of other cells sharing a bucket.  A dilute
+// bead's candidates are mostly those (the tables hold one bead per two
+// buckets): eight wide cells give 7 where 27 cells of the radius gave 13, for
+// eight range loads instead of 27; a tube bead's grow from 120 to 160.
+// Four lanes share a bead: each loads two of its ranges and visits every
+// fourth candidate (of four neighbouring slots, one cache line), then the four
+// sorted lists merge.  A tube's waves, few and each bound by its own
+// instructions (one wave per SIMD issues at half rate), thus become four times
+// as many with a quarter of the visits and insertions.  Keeps
+// the 32 nearest (distance, then index) and sums the exact label over every
 // neighbour within 12 nm (LABELS: only on check steps and for training data).
 // The 32 nearest live in registers as 64-bit keys (the squared distance's
 // float bits, which order as integers for non-negative floats, over the
-// trajectory-local index), ascending, empty slots all ones.  A candidate
-// that precedes the last key is inserted without branches: its place is the
-// count of smaller keys and every slot takes its own, its left neighbour's
-// or the new key.  A wave's lanes then never wait on one another's shift
-// loops, which on a crowded tube (60-130 candidates per lane, most of them
-// inserted) had made a wave run the longest lane's shifts for every
-// candidate.  JT selects the bucket-range packing (16-bit where every
+// trajectory-local index), ascending, empty slots at infinity.  Read as
+// doubles the keys order the same way (squared distances below 144 keep the
+// exponent finite), so a candidate that precedes the last key is inserted
+// with one FP64 minimum and one maximum per slot, 8 issue cycles where an
+// integer comparison and four selects take 20, and without branches: a
+// wave's lanes never wait on one another's shift loops, on a crowded tube
+// (60-130 candidates per lane, most of them inserted).
+// Measured per step, eight periodic systems of 24k-40k beads: 112 -> 45 us
+// (integer keys, 27 cells, one lane per bead: 112; FP64 keys 78; eight cells
+// 71; four lanes per bead 61; the dilute waves' own path 45); 8 x 1820 beads of
+// tubes alone 61 -> 22 us.  Bound by dependent loads (range, candidates,
+// neighbours) at three waves per SIMD: the keys take 64 of 168 registers.
+// JT selects the bucket-range packing (16-bit where every
 // trajectory has fewer than 65536 beads).
 // With fblk, a bead's features are written only up to the 24-float block
 // (8 neighbours) holding its last neighbour, and the number of blocks goes
 // to fblk: the step's network reads the rest as zeros, so in a dilute box
 // (a few neighbours within 12 nm) most of the 384 feature bytes per bead
 // never cross HBM.
+// Neighbours N part .. N part + N - 1 of a bead's sorted keys as features
+// (f: the bead's row; xyz: its trajectory's positions), zeros past the last.
+template <int N>
+__device__ __forceinline__ void write_features(const float4 *xyz, const double (&key)[MLP_NN], int part, int cnt,
+                                               float3 ri, float box, float ibox, float *f) {
+    const int k0 = N * part;
+    float4 xj[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        const int j = pick_key<N>(key, part, u);
+        xj[u] = k0 + u < cnt ? xyz[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float v[3 * N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        float3 d = make_float3(0.f, 0.f, 0.f);
+        if (k0 + u < cnt) {
+            d = min_image_pre(sub3(f3(xj[u]), ri), box, ibox);
+            constexpr float irc = 1.f / MLP_RC;   // features in units of the radius
+            d = make_float3(d.x * irc, d.y * irc, d.z * irc);
+        }
+        v[3 * u] = d.x;
+        v[3 * u + 1] = d.y;
+        v[3 * u + 2] = d.z;
+    }
+    float2 *o = reinterpret_cast<float2 *>(f + 3 * k0);
+#pragma unroll
+    for (int w = 0; w < 3 * N / 2; w++) o[w] = make_float2(v[2 * w], v[2 * w + 1]);
+}
+
 template <bool LABELS, typename JT>
-__global__ void __launch_bounds__(MLP_BLOCK)
+__global__ void __launch_bounds__(MLP_BLOCK * MLP_LANES, 3)
     k_mlp_local(mte_params P, DevTopo T, DevState S, CellTables C, const int2 *blocks, float *feat, float *targ,
                 uint8_t *fblk) {
-    using Ranges = BucketRanges<JT>;
-    // the lane's non-empty bucket ranges, in bucket order, for the walk over
-    // its candidates
-    __shared__ typename Ranges::W srg[27 * MLP_BLOCK];
+    using Range = BucketRange<JT>;
+    __shared__ typename Range::W srg[MLP_BLOCK][8];   // the beads' bucket ranges
     const int2 blk = blocks[blockIdx.x];
     const int t = blk.x;
     const int base = T.tbase[t];
-    const int b = base + blk.y * MLP_BLOCK + threadIdx.x;
-    if (b >= base + T.tsize[t]) return;
-    uint64_t key[MLP_NN];
+    const int lb = threadIdx.x / MLP_LANES, part = threadIdx.x % MLP_LANES;
+    const int b = base + blk.y * MLP_BLOCK + lb;
+    if (b >= base + T.tsize[t]) return;   // all four lanes of a bead
+    double key[MLP_NN];
 #pragma unroll
-    for (int k = 0; k < MLP_NN; k++) key[k] = ~0ull;
+    for (int k = 0; k < MLP_NN; k++) key[k] = __hiloint2double(0x7ff00000, 0);
     const float box = T.tbox[t], ibox = inv_side(box);
     const float3 ri = f3(S.xyz[b]);
     float A[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int cnt = 0;
     if (!T.extra[b]) {
-        const int dims = box > 0.f ? cell_dims(box, MLP_RC, 1) : 0;
         const int4 me = C.cell[b];
+        const CellGeom geo = cell_geom(box, MLP_CELL, 0);
+        const int dims = geo.dims;
         const uint32_t mask = (uint32_t)(C.tsize[t] - 1);
         const int toff = C.toff[t];
         const float ia = 1.f / P.tea_a;
-        // own cell first, then faces, edges, corners: the nearest neighbours
-        // come early and later candidates mostly fail the 32nd-distance test
-        constexpr int ORD[27] = {13, 4, 10, 12, 14, 16, 22, 1, 3, 5, 7, 9, 11, 15, 17, 19, 21, 23, 25,
-                                 0, 2, 6, 8, 18, 20, 24, 26};
-        int bk[27];
-#pragma unroll
-        for (int o = 0; o < 27; o++) {
-            const int c = ORD[o];
-            int cx = me.x + c % 3 - 1, cy = me.y + (c / 3) % 3 - 1, cz = me.z + c / 9 - 1;
-            if (dims > 0) {
-                cx = wrap_cell(cx, dims);
-                cy = wrap_cell(cy, dims);
-                cz = wrap_cell(cz, dims);
-            }
-            const uint32_t h = ((uint32_t)cx * 73856093u) ^ ((uint32_t)cy * 19349663u) ^ ((uint32_t)cz * 83492791u);
-            bk[o] = toff + (int)(h & mask);
-        }
-        Ranges rg;
-#pragma unroll
-        for (int o = 0; o < 27; o++) rg.set(o, C.range[bk[o]], base);
-        // a bucket two cells hash to is visited once: a 64-bit filter on the
-        // low bucket bits, and the full comparison only when it hits
-        uint64_t seen = 1ull << (bk[0] & 63);
-#pragma unroll
-        for (int o = 1; o < 27; o++) {
-            const uint64_t bit = 1ull << (bk[o] & 63);
-            if (seen & bit) {
-                bool dup = false;
-#pragma unroll
-                for (int k = 0; k < o; k++) dup |= bk[k] == bk[o];
-                if (dup) rg.clear(o);
-            }
-            seen |= bit;
-        }
-        auto visit = [&](const float4 pj) {
+        // the cell on the nearer side: the bead's place from its cell's lower
+        // face, in cells (taken modulo the box, so it does not matter where
+        // the table kernel's rounding put a bead on a face)
+        const float ics = 1.f / geo.cs, fdims = (float)dims, idims = dims > 0 ? 1.f / fdims : 0.f;
+        auto nearer = [&](float x, int cell) {
+            float u = x * ics - (float)cell;
+            u -= fdims * rintf((u - 0.5f) * idims);
+            const int n = u < 0.5f ? cell - 1 : cell + 1;
+            return dims > 0 ? wrap_cell(n, dims) : n;
+        };
+        const int nx = nearer(ri.x, me.x), ny = nearer(ri.y, me.y), nz = nearer(ri.z, me.z);
+        // this lane's two cells: x and y by its part, own and nearer z; cells
+        // are numbered part and part + 4
+        const int cx = part & 1 ? nx : me.x, cy = part & 2 ? ny : me.y;
+        const int b0 = toff + (int)(cell_hash(cx, cy, me.z) & mask), b1 = toff + (int)(cell_hash(cx, cy, nz) & mask);
+        const int2 r0 = C.range[b0], r1 = C.range[b1];
+        // a bucket that two cells hash to is visited for the first of them
+        bool dup0 = false, dup1 = false;
+        auto against = [&](int q, int o0, int o1) {   // the buckets of part q's two cells
+            dup0 |= q < part && o0 == b0;
+            dup1 |= o0 == b1 || (q < part && o1 == b1);
+        };
+        against(0, quad_lane<0>(b0), quad_lane<0>(b1));
+        against(1, quad_lane<1>(b0), quad_lane<1>(b1));
+        against(2, quad_lane<2>(b0), quad_lane<2>(b1));
+        against(3, quad_lane<3>(b0), quad_lane<3>(b1));
+        const int n0 = dup0 ? 0 : r0.y, n1 = dup1 ? 0 : r1.y;
+        // a candidate; SMALL: the lane has at most 8, so its first 8 slots do
+        auto visit = [&](auto small, const float4 pj) {
             const int jw = __float_as_int(pj.w);
             const int j = jw & 0x7fffffff;
             const float3 d = min_image_pre(make_float3(pj.x - ri.x, pj.y - ri.y, pj.z - ri.z), box, ibox);
@@ -181,117 +298,123 @@ __global__ void __launch_bounds__(MLP_BLOCK)
                     for (int y = 0; y < 3; y++) A[3 * x + y] += w * (crr * e[x] * e[y] + (x == y ? cii : 0.f));
             }
             // 32 nearest, ordered by (r2, j)
-            const uint64_t kn = ((uint64_t)__float_as_uint(r2) << 32) | (uint32_t)(j - base);
-            if (kn < key[MLP_NN - 1]) {
+            const double kn = __hiloint2double(__float_as_int(r2), j - base);
+            if (decltype(small)::value) {
+                insert_key<0, 8>(key, kn);
+                cnt++;
+            } else if (kn < key[MLP_NN - 1]) {
                 // slots in chunks of 8, a chunk only where some lane of the
-                // wave holds a key in it (the rest are all ones and stay so):
-                // a dilute wave touches one chunk.  Sorted keys: slot k keeps
-                // its key if that is below kn, else takes kn when the key
-                // below is below kn, else the key below; from the top down,
-                // each comparison serves two slots.
-                constexpr int CH = 8;
-                bool used[MLP_NN / CH];
-#pragma unroll
-                for (int c = 0; c < MLP_NN / CH; c++) used[c] = c == 0 || __any(cnt >= CH * c);
-#pragma unroll
-                for (int c = MLP_NN / CH - 1; c >= 0; c--)
-                    if (used[c]) {
-#pragma unroll
-                        for (int k = CH * (c + 1) - 1; k >= CH * c; k--) {
-                            const bool keep = key[k] < kn;
-                            const uint64_t below = k > 0 ? key[k - 1] : kn;
-                            const bool below_lt = k > 0 && below < kn;
-                            key[k] = keep ? key[k] : (below_lt ? kn : below);
-                        }
-                    }
+                // wave holds a key in it (the rest are empty and stay so)
+                const bool u1 = __any(cnt >= 8), u2 = __any(cnt >= 16), u3 = __any(cnt >= 24);
+                if (u3) insert_key<24, 32>(key, kn);
+                if (u2) insert_key<16, 24>(key, kn);
+                if (u1) insert_key<8, 16>(key, kn);
+                insert_key<0, 8>(key, kn);
                 cnt = min(cnt + 1, MLP_NN);
             }
         };
-        // the non-empty ranges, in bucket order, and their candidate count
-        int nne = 0, total = 0;
+        constexpr int PF = 4;
+        if (!__any(n0 + n1 > 8)) {
+            // a dilute wave: each lane visits its own two ranges, the first
+            // four candidates requested together (a lane past its last one
+            // requests the bead itself)
+            const int own = n0 + n1, o1 = r1.x - n0;
+            float4 pf[PF];
 #pragma unroll
-        for (int o = 0; o < 27; o++) {
-            const int q0 = Ranges::lo(rg.v[o], base), q1 = Ranges::hi(rg.v[o], base);
-            if (q1 > q0) {
-                srg[nne * MLP_BLOCK + threadIdx.x] = rg.v[o];
-                nne++;
-                total += q1 - q0;
-            }
-        }
-        // One flat walk over the lane's candidates (buckets in order, each
-        // bucket's in slot order), the loads PF candidates ahead of the
-        // visits (pf[k % PF] holds candidate k; the cursor q, in range r,
-        // is the next candidate to request).  A wave then runs as many
-        // iterations as its lane with the most candidates, not the sum over
-        // buckets of each bucket's longest lane.
-        int r = 0, q = 0, qend = 0;
-        if (nne > 0) {
-            const typename Ranges::W w = srg[threadIdx.x];
-            q = Ranges::lo(w, base);
-            qend = Ranges::hi(w, base);
-        }
-        auto advance = [&]() {
-            if (++q == qend && ++r < nne) {
-                const typename Ranges::W w = srg[r * MLP_BLOCK + threadIdx.x];
-                q = Ranges::lo(w, base);
-                qend = Ranges::hi(w, base);
-            }
-        };
-        constexpr int PF = 2;   // 3 and 4 measured no faster
-        float4 pf[PF];
+            for (int k0 = 0; k0 < 8; k0 += PF) {
+                if (!__any(own > k0)) break;
 #pragma unroll
-        for (int u = 0; u < PF; u++) pf[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (u < total) {
-                pf[u] = C.spos[q];
-                advance();
-            }
-        for (int k = 0; k < total; k += PF) {
-#pragma unroll
-            for (int u = 0; u < PF; u++)
-                if (k + u < total) {
-                    const float4 pj = pf[u];
-                    if (k + u + PF < total) {
-                        pf[u] = C.spos[q];
-                        advance();
-                    }
-                    visit(pj);
+                for (int u = 0; u < PF; u++) {
+                    const int k = k0 + u;
+                    pf[u] = C.spos[k < n0 ? r0.x + k : k < own ? o1 + k : b];
                 }
+#pragma unroll
+                for (int u = 0; u < PF; u++)
+                    if (k0 + u < own) visit(std::true_type{}, pf[u]);
+            }
+        } else {
+            srg[lb][part] = dup0 ? Range::none() : Range::pack(r0, base);
+            srg[lb][part + 4] = dup1 ? Range::none() : Range::pack(r1, base);
+            // the four lanes are of one wave: its LDS accesses only must keep their order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            int total = n0 + n1;
+            total += quad_swap<1>(total);
+            total += quad_swap<2>(total);
+            // One flat walk over every fourth of the bead's candidates (buckets
+            // in order, each bucket's in slot order), the loads PF candidates
+            // ahead of the visits (pf[k % PF] holds candidate k; the cursor q, in
+            // range r, is the next one to request).  A lane past its last
+            // candidate requests that one again: with no branch around the
+            // loads, the wait before a visit leaves the later ones in flight.
+            int r = 0, q = Range::lo(srg[lb][0], base), qend = Range::hi(srg[lb][0], base);
+            int last = q;
+            auto step = [&](int by) {
+                q += by;
+                while (q >= qend && r < 7) {
+                    const int over = q - qend;
+                    r++;
+                    q = Range::lo(srg[lb][r], base) + over;
+                    qend = Range::hi(srg[lb][r], base);
+                }
+                last = q < qend ? q : last;
+            };
+            step(part);
+            const int mine = (total - part + MLP_LANES - 1) / MLP_LANES;   // candidates of this lane
+            if (mine <= 0) last = b;   // none: any slot of the trajectory
+            float4 pf[PF];
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                pf[u] = C.spos[last];
+                step(MLP_LANES);
+            }
+            for (int k = 0; k < mine; k += PF) {
+#pragma unroll
+                for (int u = 0; u < PF; u++) {
+                    const float4 pj = pf[u];
+                    pf[u] = C.spos[last];
+                    step(MLP_LANES);
+                    if (k + u < mine) visit(std::false_type{}, pj);
+                }
+            }
         }
+        // the four lists into one, which all four lanes hold; the keys of a
+        // wave whose beads have at most 8 or 16 neighbours fill that many slots
+        const int c1 = cnt + quad_swap<1>(cnt), all = c1 + quad_swap<2>(c1);
+        if (!__any(all > 8)) {
+            merge_keys<1, 8>(key);
+            merge_keys<2, 8>(key);
+        } else if (!__any(all > 16)) {
+            merge_keys<1, 16>(key);
+            merge_keys<2, 16>(key);
+        } else {
+            merge_keys<1, MLP_NN>(key);
+            merge_keys<2, MLP_NN>(key);
+        }
+        cnt = min(all, MLP_NN);
+        if (LABELS)
+#pragma unroll
+            for (int c = 0; c < 9; c++) {
+                A[c] += quad_swap<1>(A[c]);
+                A[c] += quad_swap<2>(A[c]);
+            }
     }
     if (feat) {
-        // a block of eight neighbours (24 floats, six float4 stores) at a
-        // time, their positions requested together
-        float4 *f = reinterpret_cast<float4 *>(feat + (size_t)b * MLP_IN);
+        // each lane a block of eight neighbours (24 floats), their positions
+        // requested together
         const int nblk = (cnt + FEAT_BLK_NN - 1) / FEAT_BLK_NN;
-        if (fblk) fblk[b] = (uint8_t)nblk;
-#pragma unroll
-        for (int k0 = 0; k0 < MLP_NN; k0 += FEAT_BLK_NN) {
-            if (fblk && k0 >= FEAT_BLK_NN * nblk) break;
-            float4 xj[FEAT_BLK_NN];
-#pragma unroll
-            for (int u = 0; u < FEAT_BLK_NN; u++)
-                xj[u] = k0 + u < cnt ? S.xyz[base + (int)(uint32_t)key[k0 + u]] : make_float4(0.f, 0.f, 0.f, 0.f);
-            float v[3 * FEAT_BLK_NN];
-#pragma unroll
-            for (int u = 0; u < FEAT_BLK_NN; u++) {
-                float3 d = make_float3(0.f, 0.f, 0.f);
-                if (k0 + u < cnt) {
-                    d = min_image_pre(sub3(f3(xj[u]), ri), box, ibox);
-                    constexpr float irc = 1.f / MLP_RC;   // features in units of the radius
-                    d = make_float3(d.x * irc, d.y * irc, d.z * irc);
-                }
-                v[3 * u] = d.x;
-                v[3 * u + 1] = d.y;
-                v[3 * u + 2] = d.z;
-            }
-#pragma unroll
-            for (int w = 0; w < 3 * FEAT_BLK_NN / 4; w++)
-                f[3 * k0 / 4 + w] = make_float4(v[4 * w], v[4 * w + 1], v[4 * w + 2], v[4 * w + 3]);
+        if (fblk && part == 0) fblk[b] = (uint8_t)nblk;
+        if (fblk && !__any(nblk > 1)) {
+            // a dilute wave's one block, two neighbours per lane
+            if (nblk > 0)
+                write_features<FEAT_BLK_NN / MLP_LANES>(S.xyz + base, key, part, cnt, ri, box, ibox,
+                                                        feat + (size_t)b * MLP_IN);
+        } else if (!fblk || part < nblk) {
+            write_features<FEAT_BLK_NN>(S.xyz + base, key, part, cnt, ri, box, ibox, feat + (size_t)b * MLP_IN);
         }
     }
-    if (LABELS) {
+    if (LABELS && part == 0) {
 #pragma unroll
         for (int q = 0; q < 9; q++) targ[(size_t)b * MLP_OUT + q] = A[q];
     }
@@ -1114,14 +1237,14 @@ __global__ void __launch_bounds__(256) k_mlp_round(const float *w, float *wi, in
 // ------------------------------------------------------------------ launchers
 static inline int blocks(int n, int bs) { return (n + bs - 1) / bs; }
 
-hipError_t launch_mlp_cells(mte_engine *e) { return build_cells(e, MLP_RC, 1); }
+hipError_t launch_mlp_cells(mte_engine *e) { return build_cells(e, MLP_CELL, 0); }
 
 hipError_t launch_mlp_local(mte_engine *e, float *feat, float *targ, bool build_tables, uint8_t *fblk) {
     if (build_tables) {
         const hipError_t s = launch_mlp_cells(e);
         if (s != hipSuccess) return s;
     }
-    const dim3 grid(e->mlp.nblocks), block(MLP_BLOCK);
+    const dim3 grid(e->mlp.nblocks), block(MLP_BLOCK * MLP_LANES);
     const int2 *bl = e->mlp.blocks;
     const bool narrow = e->nmax < 65536;   // trajectory-local indices and bucket ends fit 16 bits
     if (targ && narrow)

@@ -169,3 +169,25 @@ def test_labels_across_the_boundary_of_a_whole_number_of_cells(box):
     np.testing.assert_allclose(f, fo, atol=2e-5)   # positions of up to 768 nm: 2^-23 x 768 over 12 nm
     np.testing.assert_allclose(t, to, rtol=1e-4, atol=1e-4 * np.abs(to).max())
     eng.close()
+
+
+@pytest.mark.parametrize("box", [0.0, 36.0, 47.9, 50.0, 73.0])
+@pytest.mark.parametrize("dimers", [1, 40, 150])
+def test_search_over_few_cells_and_crowded_beads(box, dimers):
+    """Features and labels where a box holds one, two or three search cells a
+    side, from a lone dimer to beads with more than 32 neighbours within 12
+    nm (both paths of the search and every merge of its four lanes)."""
+    print(f"case MLP search, box {box}, {dimers} dimers", flush=True)
+    from mt_amd import lattice, topology
+    p = P.derive(dict(P.TEA))
+    rng = np.random.default_rng(7)
+    a = lattice.free_dimers(dimers, 2000.0, rng, chain="Y")
+    cen = rng.uniform(0.0, box or 36.0, (dimers, 3))
+    a.xyz[0::2], a.xyz[1::2] = cen - [0.0, 0.0, 2.0], cen + [0.0, 0.0, 2.0]
+    b = topology.make_batch([a, a], [lattice.coords7(a, 0.1, rng) for _ in range(2)], box=[box, box])
+    eng = Engine(p, b.copy(), max_lj=400, mode=MODE_STREAMED)
+    f, t = eng.mlp_local()
+    fo, to = M.local_features_targets(b.coords, b.off, b.extra, b.box, p.tea_a)
+    np.testing.assert_allclose(f, fo, atol=5e-6)   # positions of up to 80 nm: 2^-24 x 80 over 12 nm
+    np.testing.assert_allclose(t, to, rtol=2e-5, atol=2e-5 * max(np.abs(to).max(), 1e-3))
+    eng.close()
