@@ -1,6 +1,6 @@
 // bead_physics.h -- per-bead force and energy evaluation, shared by the
 // streamed kernels (state in HBM) and the resident kernel (state in LDS).
-// An accessor type supplies neighbour data by global bead index.
+// An accessor type supplies neighbour data by a handle, a list type the handles.
 //
 // Restates compute_kernel (src/compute_cuda.cu:32-525) and energy_kernel
 // (:676-911) in attachment-point form; see device_common.h.
@@ -18,6 +18,7 @@ struct Own {
     float fi, theta, psi;
     float box;   // periodic side of the bead's trajectory (0: open)
     float ibox;  // inv_side(box)
+    int flags;   // packed (FL_*)
 };
 __device__ __forceinline__ void set_box(Own &o, float L) {
     o.box = L;
@@ -25,7 +26,8 @@ __device__ __forceinline__ void set_box(Own &o, float L) {
 }
 
 // trig = (sin theta, cos theta, sin psi, cos psi) of the bead.
-__device__ __forceinline__ Own make_own_trig(float4 xyz, float4 ang, float4 fn, float4 fp1, float4 fp2, float4 trig) {
+__device__ __forceinline__ Own make_own_trig(float4 xyz, float4 ang, float4 fn, float4 fp1, float4 fp2, float4 trig,
+                                             int flags) {
     Own o;
     o.r = f3(xyz);
     o.n = f3(fn);
@@ -37,38 +39,15 @@ __device__ __forceinline__ Own make_own_trig(float4 xyz, float4 ang, float4 fn, 
     o.uphi = make_float3(trig.w * trig.y, trig.z * trig.y, -trig.x);
     o.uth = make_float2(-trig.z, trig.w);
     o.box = o.ibox = 0.f;
+    o.flags = flags;
     return o;
 }
 
-__device__ __forceinline__ Own make_own(float4 xyz, float4 ang, float4 fn, float4 fp1, float4 fp2) {
-    Own o;
-    o.r = f3(xyz);
-    o.n = f3(fn);
-    o.a1 = f3(fp1);
-    o.a2 = f3(fp2);
-    o.fi = ang.x;
-    o.theta = ang.y;
-    o.psi = ang.z;
-    float st, ct, sp, cp;
-    sincos_fast(ang.y, &st, &ct);
-    sincos_fast(ang.z, &sp, &cp);
-    o.uphi = make_float3(cp * ct, sp * ct, -st);
-    o.uth = make_float2(-sp, cp);
-    o.box = o.ibox = 0.f;
-    return o;
-}
-
-// Bending torques of a harmonic or longitudinal pair (:156-177, :271-295).
-__device__ __forceinline__ void bending(const mte_params &P, float rm, float th0, const Own &I, float4 aj,
-                                        float F[6]) {
-    const float psiji = aj.z - I.psi, thetaji = aj.y - I.theta, fiji = aj.x - I.fi;
-    // rm > 0: F += B sin(d - d0); rm < 0: F -= B sin(-d - d0).  One branch-free
-    // form with s = +-1 (exact sign flips: the same values), since the two
-    // monomers of a dimer sit in neighbouring lanes and take opposite signs.
-    const float sg = rm > 0.f ? 1.f : -1.f;
-    F[5] += sg * P.B_psi * sin_fast_near0(sg * psiji - P.psi_0);
-    F[3] += sg * P.B_fi * sin_fast_near0(sg * fiji - P.fi_0);
-    F[4] += sg * P.B_theta * sin_fast_near0(sg * thetaji - th0);
+__device__ __forceinline__ Own make_own(float4 xyz, float4 ang, float4 fn, float4 fp1, float4 fp2, int flags) {
+    float4 trig;
+    sincos_fast(ang.y, &trig.x, &trig.y);
+    sincos_fast(ang.z, &trig.z, &trig.w);
+    return make_own_trig(xyz, ang, fn, fp1, fp2, trig, flags);
 }
 
 // Per-bead flags packed into xyz.w when a trajectory's state is staged in LDS.
@@ -78,20 +57,33 @@ __device__ __forceinline__ int pack_flags(const DevTopo &T, int b) {
     return (T.mon_type[b] ? FL_MON : 0) | (T.gtp[b] == 1 ? FL_GTP1 : 0) | (T.on_tub[b] == 0 ? FL_OFFTUB : 0);
 }
 
-// A trajectory's bead data staged in LDS, by local index: position with the
-// packed flags in w, and the rotated offsets with the Euler angles in w
-// (n|fi, p1|theta, p2|psi).
+// Neighbour data by a handle that the list entry gives.  In LDS, four arrays
+// hold per bead its position with the packed flags in w, and the rotated
+// offsets with the Euler angles in w (n|fi, p1|theta, p2|psi); the handle is
+// the LDS address of the bead's position, and n, p1, p2 are the distances of
+// the other arrays from that one.
+typedef float v4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint32_t lds_addr(const void *p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+__device__ __forceinline__ float4 lds_f4(uint32_t a) {
+    const v4f v = *(const __attribute__((address_space(3))) v4f *)(uintptr_t)a;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
 struct LdsAcc {
-    const float4 *x, *n, *p1, *p2;
-    __device__ __forceinline__ float4 xyz(int j) const { return x[j]; }
-    __device__ __forceinline__ float4 ang(int j) const { return make_float4(n[j].w, p1[j].w, p2[j].w, 0.f); }
-    __device__ __forceinline__ float4 fn(int j) const { return n[j]; }
-    __device__ __forceinline__ float4 fp1(int j) const { return p1[j]; }
-    __device__ __forceinline__ float4 fp2(int j) const { return p2[j]; }
-    __device__ __forceinline__ int flags(int j) const { return __float_as_int(x[j].w); }
-    __device__ __forceinline__ int mon(int j) const { return flags(j) & FL_MON; }
-    __device__ __forceinline__ bool gtp1(int j) const { return (flags(j) & FL_GTP1) != 0; }
-    __device__ __forceinline__ bool offtub(int j) const { return (flags(j) & FL_OFFTUB) != 0; }
+    uint32_t x, n, p1, p2;   // x: address of the position array
+    static constexpr int SCALE = sizeof(float4);
+    __device__ __forceinline__ LdsAcc(const float4 *lx, const float4 *ln, const float4 *l1, const float4 *l2)
+        : x(lds_addr(lx)), n(in_vgpr(lds_addr(ln) - lds_addr(lx))), p1(in_vgpr(lds_addr(l1) - lds_addr(lx))),
+          p2(in_vgpr(lds_addr(l2) - lds_addr(lx))) {}
+    __device__ __forceinline__ uint32_t origin() const { return x; }
+    __device__ __forceinline__ float4 xyz(uint32_t h) const { return lds_f4(h); }
+    __device__ __forceinline__ float4 fn(uint32_t h) const { return lds_f4(h + n); }
+    __device__ __forceinline__ float4 lat(uint32_t h, bool p2nd) const { return lds_f4(h + (p2nd ? p2 : p1)); }
+    __device__ __forceinline__ float3 angles(float4 fnj, uint32_t h) const {
+        return make_float3(fnj.w, lds_f4(h + p1).w, lds_f4(h + p2).w);
+    }
+    __device__ __forceinline__ int flags(float4 xj, uint32_t) const { return __float_as_int(xj.w); }
 };
 
 // Stages beads [0, n) of the trajectory starting at global bead `base` into
@@ -114,150 +106,202 @@ __device__ __forceinline__ void stage_state(const DevTopo &T, const DevState &S,
     }
 }
 
-// Neighbour lists held in the k-major global arrays of bead b, with entry
-// indices taken relative to `base` (0: global indices, the streamed kernels;
-// the trajectory's first bead: local indices, the resident kernel).
+// Neighbour lists held in the k-major global arrays of bead b.  The handle of
+// global bead j is origin + SCALE (j - base): its index, or the LDS address of
+// its position.
+template <int SCALE>
 struct GlobalLists {
     const DevTopo &T;
     int b, base;
-    __device__ __forceinline__ int harm() const {
-        const int h = T.harm[b];
-        return h >= 0 ? h - 2 * base : -1;
-    }
+    uint32_t origin;
+    __device__ __forceinline__ int harm() const { return T.harm[b]; }
     __device__ __forceinline__ int nlon() const { return T.lon_n[b]; }
-    __device__ __forceinline__ int lon(int k) const { return T.lon[k * T.nb + b] - 2 * base; }
+    __device__ __forceinline__ int lon(int k) const { return T.lon[k * T.nb + b]; }
     __device__ __forceinline__ int nlat() const { return T.lat_n[b]; }
-    __device__ __forceinline__ int lat(int k) const { return T.lat[k * T.nb + b] - 2 * base; }
+    __device__ __forceinline__ int lat(int k) const { return T.lat[k * T.nb + b]; }
+    __device__ __forceinline__ uint32_t handle(int j) const { return origin + (uint32_t)((j - base) * SCALE); }
+    __device__ __forceinline__ uint32_t ref(int e) const { return handle(ent_j(e)); }
     __device__ __forceinline__ int nlj() const { return T.lj_n[b]; }
-    __device__ __forceinline__ int lj(int k) const { return T.lj[k * T.nb + b] - base; }
+    __device__ __forceinline__ uint32_t lj(int k) const { return handle(T.lj[k * T.nb + b]); }
 };
 
-// Position of a bead's k-th LJ neighbour; a list format that stores
-// something other than the neighbour's index provides its own overload.
-template <class Acc, class Lists>
-__device__ __forceinline__ float4 lj_xyz(const Acc &A, const Lists &Ls, int k) {
-    return A.xyz(Ls.lj(k));
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// What a bead's bonds add up to: force, and the moments about the bead of
+// its bonds at the axial offset (M, to be crossed with n) and at the lateral
+// ones (Tq).  A bond's torque is a x f with a its offset; the three angular
+// components are the torque's along u_phi, u_theta, u_psi, taken once.
+struct BondSum {
+    float3 F, M, Tq;
+    float3 bend;   // fi, theta, psi
+};
+__device__ __forceinline__ float3 cross_add(float3 a, float3 f, float3 t) {
+    return make_float3(fmaf(a.y, f.z, fmaf(-a.z, f.y, t.x)), fmaf(a.z, f.x, fmaf(-a.x, f.z, t.y)),
+                       fmaf(a.x, f.y, fmaf(-a.y, f.x, t.z)));
 }
 
-// LJ repulsion over the list; the cutoff test selects the force (no branch
-// around the accumulation), and periodic and open boxes get separate loops,
-// as do runs with and without the regularization cap (a uniform choice: the
-// cap's reciprocal square root is not paid per pair when it is off).
+// Bending torques of a harmonic or longitudinal pair (:156-177, :271-295):
+// rm > 0: F += B sin(d - d0); rm < 0: F -= B sin(-d - d0), one form for both
+// since sin is odd: B sin(d - s d0), s = rm / 2 = +-1.
+__device__ __forceinline__ void bending(const ForceK &K, float rm, float th_h, const Own &I, float3 aj, float3 &bend) {
+    const float3 s = sin3(make_float3(fmaf(-rm, K.fi_h, aj.x - I.fi), fmaf(-rm, th_h, aj.y - I.theta),
+                                      fmaf(-rm, K.psi_h, aj.z - I.psi)));
+    bend.x = fmaf(K.Bfi, s.x, bend.x);
+    bend.y = fmaf(K.Bth, s.y, bend.y);
+    bend.z = fmaf(K.Bpsi, s.z, bend.z);
+}
+
+// |g|^2, above zero (1e-30 nm^2 is below the rounding of any other gap): its
+// reciprocal root is finite, and a closed gap's force is 0 times it.
+__device__ __forceinline__ float gap2(float3 g) { return fmaf(g.x, g.x, fmaf(g.y, g.y, fmaf(g.z, g.z, 1e-30f))); }
+
+// dU/dr over r of a Morse bond (d = 2 A D, na = -A log2 e) with its barrier.
+__device__ __forceinline__ float bond_slope(float d2, float na, float d, bool barrier, float br, float bk, float bc) {
+    const float inv = rsq_fast(d2), dr = d2 * inv;
+    const float e = exp2_fast(na * dr);
+    float s = d * fmaf(-e, e, e);
+    if (__any(barrier)) {   // rare: a branch, where the compiler would select
+        const float x = dr - br;
+        s = barrier ? fmaf(bc * x, exp2_fast(bk * (x * x)), s) : s;
+    }
+    return s * inv;
+}
+
+template <bool PERIODIC>
+__device__ __forceinline__ float3 separation(const Own &I, float4 xj) {
+    const float3 d = sub3(I.r, f3(xj));
+    if (!PERIODIC) return d;
+    return min_image_inv(d, I.box, I.ibox);
+}
+
+// 1 for r2 < LJ_CUT^2, else 0 (NaN: 0), by a fused product and clamp: below
+// the cutoff 2^100 (LJ_CUT^2 - r2) is at least 2^81.  Two 2-cycle operations
+// per pair with the product, where comparing and selecting take 4 each.
+__device__ __forceinline__ float below_cut(float r2, float nscale, float offset) {
+    return __builtin_amdgcn_fmed3f(fmaf(nscale, r2, offset), 0.f, 1.f);
+}
+
+// LJ repulsion over the list; the cutoff test scales the force (no branch
+// around the accumulation), and runs with and without the regularization cap
+// get separate loops (a uniform choice: the cap's reciprocal square root is
+// not paid per pair when it is off).
 template <bool PERIODIC, bool REG, class Acc, class Lists>
-__device__ __forceinline__ void lj_sum(const mte_params &P, const Acc &A, const Lists &Ls, const Own &I, float F[6]) {
+__device__ __forceinline__ void lj_sum(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I, float3 &F) {
     const int nlj = Ls.nlj();
-    const float s6 = 6.f * (P.ljscale * P.ljsigma6);
-    // REGULARIZATION (src/compute_cuda.cu:482-486): the pair force s r is
-    // capped at gammaR r_mon / dt, i.e. s at that over r (r_mon = 2 nm)
-    const float cap = P.gammaR * 2.f / P.dt;
-    float fx = F[0], fy = F[1], fz = F[2];   // same accumulation order, scalar registers
+    const float nscale = in_vgpr(-0x1p100f), offset = in_vgpr(LJ_CUT * LJ_CUT * 0x1p100f);
+    float3 f = make_float3(0.f, 0.f, 0.f);   // without K.lj6, unless REG
     auto pair = [&](float4 xj) {
-        float3 d = sub3(I.r, f3(xj));
-        if (PERIODIC) d = min_image_inv(d, I.box, I.ibox);   // called with I.box > 0
+        const float3 d = separation<PERIODIC>(I, xj);
         const float r2 = d.x * d.x + d.y * d.y + d.z * d.z;
         const float inv = rcp_fast(r2);
         const float inv2 = inv * inv;
-        float s = r2 < LJ_CUT * LJ_CUT ? s6 * (inv2 * inv2) : 0.f;
-        if (REG) s = fminf(s, cap * rsq_fast(r2));
-        fx += s * d.x;
-        fy += s * d.y;
-        fz += s * d.z;
+        float s = below_cut(r2, nscale, offset) * (inv2 * inv2);
+        // REGULARIZATION (src/compute_cuda.cu:482-486): the pair force s r is
+        // capped at gammaR r_mon / dt, i.e. s at that over r (r_mon = 2 nm)
+        if (REG) s = fminf(K.lj6 * s, K.lj_cap * rsq_fast(r2));
+        f.x = fmaf(s, d.x, f.x);
+        f.y = fmaf(s, d.y, f.y);
+        f.z = fmaf(s, d.z, f.z);
     };
     // four entries and their positions requested before the first is used
     // (one wait for the four gathers rather than one each), then summed in
     // list order
     int k = 0;
     for (; k + 4 <= nlj; k += 4) {
-        const float4 x0 = lj_xyz(A, Ls, k), x1 = lj_xyz(A, Ls, k + 1), x2 = lj_xyz(A, Ls, k + 2),
-                     x3 = lj_xyz(A, Ls, k + 3);
+        const float4 x0 = A.xyz(Ls.lj(k)), x1 = A.xyz(Ls.lj(k + 1)), x2 = A.xyz(Ls.lj(k + 2)), x3 = A.xyz(Ls.lj(k + 3));
         pair(x0);
         pair(x1);
         pair(x2);
         pair(x3);
     }
-    for (; k < nlj; k++) pair(lj_xyz(A, Ls, k));
-    F[0] = fx;
-    F[1] = fy;
-    F[2] = fz;
-}
-template <bool PERIODIC, class Acc, class Lists>
-__device__ __forceinline__ void lj_forces(const mte_params &P, const Acc &A, const Lists &Ls, const Own &I,
-                                          float F[6]) {
-    if (P.lj_regularize) lj_sum<PERIODIC, true>(P, A, Ls, I, F);
-    else lj_sum<PERIODIC, false>(P, A, Ls, I, F);
+    for (; k < nlj; k++) pair(A.xyz(Ls.lj(k)));
+    const float s6 = REG ? 1.f : K.lj6;
+    F = make_float3(fmaf(s6, f.x, F.x), fmaf(s6, f.y, F.y), fmaf(s6, f.z, F.z));
 }
 
-// Force and torque on bead b (an accessor index, as are the list entries);
-// wall_z is Parameters.zs of the bead's trajectory.
-template <class Acc, class Lists>
-__device__ __forceinline__ void bead_force(const mte_params &P, const Acc &A, const Lists &Ls, int b, float wall_z,
-                                           const Own &I, float F[6]) {
-#pragma unroll
-    for (int q = 0; q < 6; q++) F[q] = 0.f;
+// Force and torque on a bead; wall_z is Parameters.zs of its trajectory.
+template <bool PERIODIC, class Acc, class Lists>
+__device__ __forceinline__ void bead_force(const ForceK &K, const Acc &A, const Lists &Ls, float wall_z, const Own &I,
+                                           float F[6]) {
+    BondSum S;
+    S.F = S.M = S.Tq = S.bend = make_float3(0.f, 0.f, 0.f);
+    const bool gtp = (I.flags & FL_GTP1) != 0, off = K.barrier && (I.flags & FL_OFFTUB) != 0;
+    // an axial bond with force slope s over its gap g
+    auto axial = [&](float rm, float s, float3 g) {
+        const float3 f = scale3(-s, g);
+        S.F = make_float3(S.F.x + f.x, S.F.y + f.y, S.F.z + f.z);
+        S.M = make_float3(fmaf(rm, f.x, S.M.x), fmaf(rm, f.y, S.M.y), fmaf(rm, f.z, S.M.z));
+    };
+    auto axial_gap = [&](float rm, float4 xj, float4 nj) {
+        const float3 d = separation<PERIODIC>(I, xj);
+        return make_float3(fmaf(rm, I.n.x + nj.x, d.x), fmaf(rm, I.n.y + nj.y, d.y), fmaf(rm, I.n.z + nj.z, d.z));
+    };
     // harmonic (intra-dimer spring + bending), :70-182
-    const int h = Ls.harm();
-    if (h >= 0) {
-        const int j = ent_j(h);
-        const float rm = ent_f(h) ? RMON : -RMON;
-        const float3 nj = f3(A.fn(j));
-        const Grad G = gap_grad(min_image_pre(sub3(I.r, f3(A.xyz(j))), I.box, I.ibox), scale3(rm, I.n), scale3(-rm, nj), I.uphi, I.uth);
-#pragma unroll
-        for (int q = 0; q < 6; q++) F[q] -= P.C * G.g[q];
-        if (G.dr < ANGLE_CUT) {
-            const float th0 = A.gtp1(b) ? P.theta0_gtp : P.theta0_gdp;
-            bending(P, rm, th0, I, A.ang(j), F);
-        }
+    const int eh = Ls.harm();
+    if (eh >= 0) {
+        const uint32_t j = Ls.ref(eh);
+        const float rm = ent_f(eh) ? RMON : -RMON;
+        const float4 xj = A.xyz(j), nj = A.fn(j);
+        const float3 g = axial_gap(rm, xj, nj);
+        axial(rm, K.C, g);
+        if (gap2(g) < ANGLE_CUT * ANGLE_CUT)
+            bending(K, rm, gtp ? K.th_gtp_h : K.th_gdp_h, I, A.angles(nj, j), S.bend);
     }
     // longitudinal Morse + barrier + bending, :189-299
     const int nlon = Ls.nlon();
     for (int k = 0; k < nlon; k++) {
         const int e = Ls.lon(k);
-        const int j = ent_j(e);
+        const uint32_t j = Ls.ref(e);
         const float rm = ent_f(e) ? RMON : -RMON;
-        const float4 xj = A.xyz(j);
-        const Grad G = gap_grad(min_image_pre(sub3(I.r, f3(xj)), I.box, I.ibox), scale3(rm, I.n), scale3(-rm, f3(A.fn(j))), I.uphi, I.uth);
-        float dUdr = (G.dr == 0.f) ? 0.f : dmorse(P.D_long, P.A_long, G.dr) * G.inv;
-        if (P.barrier && A.offtub(b) && A.offtub(j) && G.dr != 0.f)
-            dUdr += dbarr(P.a_barr_long, P.r_barr_long, P.w_barr_long, G.dr) * G.inv;
-#pragma unroll
-        for (int q = 0; q < 6; q++) F[q] -= dUdr * G.g[q];
-        if (G.dr < ANGLE_CUT) {
-            const int last = (I.r.z > xj.z) ? b : j;
-            const float th0 = A.gtp1(last) ? P.theta0_gtp : P.theta0_gdp;
-            bending(P, rm, th0, I, A.ang(j), F);
+        const float4 xj = A.xyz(j), nj = A.fn(j);
+        const float3 g = axial_gap(rm, xj, nj);
+        const float d2 = gap2(g);
+        const int fj = A.flags(xj, j);
+        axial(rm, bond_slope(d2, K.lon_a, K.lon_d, off && (fj & FL_OFFTUB), K.lonb_r, K.lonb_k, K.lonb_c), g);
+        if (d2 < ANGLE_CUT * ANGLE_CUT) {
+            const bool gl = (I.r.z > xj.z) ? gtp : (fj & FL_GTP1) != 0;   // theta0 of the bead with larger z
+            bending(K, rm, gl ? K.th_gtp_h : K.th_gdp_h, I, A.angles(nj, j), S.bend);
         }
     }
     // lateral Morse + barrier with seam weakening, :304-466
     const int nlat = Ls.nlat();
     for (int k = 0; k < nlat; k++) {
         const int e = Ls.lat(k);
-        const int j = ent_j(e);
-        const int sw = ent_f(e);
+        const uint32_t j = Ls.ref(e);
+        const bool sw = ent_f(e) != 0;
         const float3 a = sw ? I.a1 : I.a2;
-        const float3 bj = f3(sw ? A.fp2(j) : A.fp1(j));
-        const Grad G = gap_grad(min_image_pre(sub3(I.r, f3(A.xyz(j))), I.box, I.ibox), a, bj, I.uphi, I.uth);
+        const float4 xj = A.xyz(j), bj = A.lat(j, sw);
+        const float3 d = separation<PERIODIC>(I, xj);
+        const float3 g = make_float3(d.x + (a.x - bj.x), d.y + (a.y - bj.y), d.z + (a.z - bj.z));
+        const int fj = A.flags(xj, j);
         // seam bonds (monomer types differ) are weakened by seam_coeff (:447-452)
-        const float Dl = A.mon(b) != A.mon(j) ? P.D_lat / P.seam_coeff : P.D_lat;
-        float dUdr = (G.dr == 0.f) ? 0.f : dmorse(Dl, P.A_lat, G.dr) * G.inv;
-        if (P.barrier && A.offtub(b) && A.offtub(j) && G.dr != 0.f)
-            dUdr += dbarr(P.a_barr_lat, P.r_barr_lat, P.w_barr_lat, G.dr) * G.inv;
-#pragma unroll
-        for (int q = 0; q < 6; q++) F[q] -= dUdr * G.g[q];
+        const float dl = (fj ^ I.flags) & FL_MON ? K.seam_d : K.lat_d;
+        const float s = bond_slope(gap2(g), K.lat_a, dl, off && (fj & FL_OFFTUB), K.latb_r, K.latb_k, K.latb_c);
+        const float3 f = scale3(-s, g);
+        S.F = make_float3(S.F.x + f.x, S.F.y + f.y, S.F.z + f.z);
+        S.Tq = cross_add(a, f, S.Tq);
     }
     // LJ repulsion r^-6 below the hard 6 nm cutoff, :470-495
-    if (P.lj_on) {
-        if (I.box > 0.f) lj_forces<true>(P, A, Ls, I, F);
-        else lj_forces<false>(P, A, Ls, I, F);
+    if (K.lj_on) {
+        if (K.lj_reg) lj_sum<PERIODIC, true>(K, A, Ls, I, S.F);
+        else lj_sum<PERIODIC, false>(K, A, Ls, I, S.F);
     }
+    const float3 t = cross_add(I.n, S.M, S.Tq);
+    F[0] = S.F.x;
+    F[1] = S.F.y;
+    F[2] = S.F.z;
+    F[3] = fmaf(I.uphi.x, t.x, fmaf(I.uphi.y, t.y, fmaf(I.uphi.z, t.z, S.bend.x)));
+    F[4] = fmaf(I.uth.x, t.x, fmaf(I.uth.y, t.y, S.bend.y));
+    F[5] = t.z + S.bend.z;
     // cylindrical and end walls, :497-517
-    if (P.is_wall) {
-        const float z = I.r.z, lb = P.rep_leftborder, zt = wall_z + lb;
-        if (z < lb) F[2] += P.rep_eps * fabsf(z - lb);
-        else if (z > zt) F[2] += -P.rep_eps * fabsf(z - zt);
+    if (K.is_wall) {
+        const float z = I.r.z, lb = K.wall_left, zt = wall_z + lb;
+        if (z < lb) F[2] += K.wall_eps * fabsf(z - lb);
+        else if (z > zt) F[2] += -K.wall_eps * fabsf(z - zt);
         const float rad2 = I.r.x * I.r.x + I.r.y * I.r.y;
-        if (rad2 > P.rep_r * P.rep_r) {
+        if (rad2 > K.wall_r * K.wall_r) {
             const float rad = sqrtf(rad2);
-            const float coeff = -P.rep_eps * (rad - P.rep_r);
+            const float coeff = -K.wall_eps * (rad - K.wall_r);
             F[0] += I.r.x / rad * coeff;
             F[1] += I.r.y / rad * coeff;
         }
@@ -336,18 +380,12 @@ __device__ __forceinline__ void bead_energy(const mte_params &P, const DevTopo &
 }
 
 // Euler-Maruyama update of one mobile bead, src/compute_cuda.cu:955-961.
-__device__ __forceinline__ void em_update(const mte_params &P, const float F[6], float4 rx, float4 ra, float4 &x,
+__device__ __forceinline__ void em_update(const ForceK &K, const float F[6], float4 rx, float4 ra, float4 &x,
                                           float4 &a) {
-    const float dtg = P.dt / P.gammaR;
-    const float dta = P.dt / (P.gammaTheta * P.alpha);
-    const float dtt = P.dt / P.gammaTheta;
-    const float vta = P.varTheta * sqrtf(P.freeze_temp / P.alpha);
-    x.x += dtg * F[0] + P.varR * rx.x;
-    x.y += dtg * F[1] + P.varR * rx.y;
-    x.z += dtg * F[2] + P.varR * rx.z;
-    a.x += dta * F[3] + vta * ra.x;          // fi
-    a.z += dta * F[5] + vta * ra.y;          // psi
-    a.y += dtt * F[4] + P.varTheta * ra.z;   // theta
+    x.x += fmaf(K.dtg, F[0], K.vR * rx.x);
+    x.y += fmaf(K.dtg, F[1], K.vR * rx.y);
+    x.z += fmaf(K.dtg, F[2], K.vR * rx.z);
+    em_angles(K, F[3], F[4], F[5], ra, a);
 }
 
 }  // namespace mte

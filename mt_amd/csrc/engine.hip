@@ -425,6 +425,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
         return code;
     };
     e->P = *params;
+    e->K = force_constants(e->P);
     e->O = *opt;
     if (e->O.max_lj <= 0) e->O.max_lj = 64;
     if (e->O.max_lj > 1023) { e->err = "mte_create: max_lj must be at most 1023"; return bail(MTE_ERR_ARG); }

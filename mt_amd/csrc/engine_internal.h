@@ -141,6 +141,7 @@ struct ResidentPlan {
 
 struct mte_engine {
     mte_params P{};
+    mte::ForceK K{};                 // P's constants as the kernels use them
     mte_options O{};
     int nb = 0, ntraj = 0;
     int nmax = 0;            // beads in the largest trajectory

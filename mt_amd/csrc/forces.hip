@@ -34,6 +34,11 @@ struct GlobalAcc {
     __device__ __forceinline__ float4 fn(int j) const { return S.fn[j]; }
     __device__ __forceinline__ float4 fp1(int j) const { return S.fp1[j]; }
     __device__ __forceinline__ float4 fp2(int j) const { return S.fp2[j]; }
+    // as bead_force reads them: the handle is the bead's index
+    static constexpr int SCALE = 1;
+    __device__ __forceinline__ float4 lat(int j, bool p2nd) const { return (p2nd ? S.fp2 : S.fp1)[j]; }
+    __device__ __forceinline__ float3 angles(float4, int j) const { return f3(S.ang[j]); }
+    __device__ __forceinline__ int flags(float4, int j) const { return pack_flags(T, j); }
 };
 
 __global__ void __launch_bounds__(STREAM_BLOCK) k_frames(DevState S, int nb, LatOffsets L) {
@@ -50,9 +55,9 @@ __global__ void __launch_bounds__(STREAM_BLOCK) k_frames(DevState S, int nb, Lat
 // Force + Euler-Maruyama step.  Reads Sin, writes Sout (both positions and
 // rotated offsets), advances the HybridTaus states of mobile beads only
 // (src/compute_cuda.cu:949-953) unless noise is injected.
-template <int BS>
+template <int BS, bool PERIODIC>
 __global__ void __launch_bounds__(BS)
-    k_step_plain(mte_params P, DevTopo T, DevState Sin, DevState Sout, uint4 *seeds, const float *noise,
+    k_step_plain(ForceK K, DevTopo T, DevState Sin, DevState Sout, uint4 *seeds, const float *noise,
                  LatOffsets L) {
     const int b = xcd_bead(BS);
     if (b >= T.nb) return;
@@ -67,10 +72,10 @@ __global__ void __launch_bounds__(BS)
         Sout.fp2[b] = Sin.fp2[b];
         return;
     }
-    Own I = make_own(x, a, Sin.fn[b], Sin.fp1[b], Sin.fp2[b]);
-    set_box(I, T.tbox[T.tid[b]]);
+    Own I = make_own(x, a, Sin.fn[b], Sin.fp1[b], Sin.fp2[b], pack_flags(T, b));
+    if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
     float F[6];
-    bead_force(P, GlobalAcc{Sin, T}, GlobalLists{T, b, 0}, b, P.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
+    bead_force<PERIODIC>(K, GlobalAcc{Sin, T}, GlobalLists<1>{T, b, 0, 0}, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
     float4 rx, ra;
     if (noise) {
         const float *nz = noise + 6 * (size_t)b;
@@ -84,7 +89,7 @@ __global__ void __launch_bounds__(BS)
         ra = normals4(s);
         seeds[b + T.nb] = s;
     }
-    em_update(P, F, rx, ra, x, a);
+    em_update(K, F, rx, ra, x, a);
     float4 n, p1, p2;
     frame_vectors(a.x, a.y, a.z, L, n, p1, p2);
     Sout.xyz[b] = x;
@@ -103,42 +108,45 @@ struct TeaDraw {
     float4 *R;   // nullptr: no draw
 };
 
+// One bead's share of it.
+__device__ __forceinline__ void tea_draw(const TeaDraw &D, float var, int b, bool extra) {
+    float4 r;
+    if (D.noise) {
+        const float *nz = D.noise + 6 * (size_t)b;
+        r = make_float4(nz[0], nz[1], nz[2], 0.f);
+    } else {
+        uint4 s = D.seeds[b];
+        r = normals4(s);
+        D.seeds[b] = s;
+    }
+    D.R[b] = extra ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
+}
+
 // Forces (compute_kernel semantics; extra beads get zero), optionally with
 // the TEA random forces.
-template <int BS>
+template <int BS, bool PERIODIC>
 __global__ void __launch_bounds__(BS)
-    k_forces(mte_params P, DevTopo T, DevState S, float4 *fxyz, float4 *fang, TeaDraw D) {
+    k_forces(ForceK K, DevTopo T, DevState S, float4 *fxyz, float4 *fang, TeaDraw D) {
     const int b = xcd_bead(BS);
     if (b >= T.nb) return;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (!T.extra[b]) {
-        Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b]);
-        set_box(I, T.tbox[T.tid[b]]);
-        bead_force(P, GlobalAcc{S, T}, GlobalLists{T, b, 0}, b, P.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
+        Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b], pack_flags(T, b));
+        if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
+        bead_force<PERIODIC>(K, GlobalAcc{S, T}, GlobalLists<1>{T, b, 0, 0}, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) {
-        const float var = sqrtf(2.0f * KB * P.temp * P.gammaR / P.dt);
-        float4 r;
-        if (D.noise) {
-            const float *nz = D.noise + 6 * (size_t)b;
-            r = make_float4(nz[0], nz[1], nz[2], 0.f);
-        } else {
-            uint4 s = D.seeds[b];
-            r = normals4(s);
-            D.seeds[b] = s;
-        }
-        D.R[b] = T.extra[b] ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
-    }
+    if (D.R) tea_draw(D, K.vF, b, T.extra[b]);
 }
 
 // The same forces with the bead's whole trajectory staged in LDS (positions,
 // rotated offsets, angles and flags of every bead), one workgroup per
 // 256-bead tile of a trajectory: neighbour data are read from LDS instead of
 // gathered from L2 per pair.  For trajectories that fit (forces_lds_bytes).
+template <bool PERIODIC>
 __global__ void __launch_bounds__(FORCE_TILE)
-    k_forces_lds(mte_params P, DevTopo T, DevState S, const int2 *tiles, float4 *fxyz, float4 *fang, TeaDraw D) {
+    k_forces_lds(ForceK K, DevTopo T, DevState S, const int2 *tiles, float4 *fxyz, float4 *fang, TeaDraw D) {
     extern __shared__ float4 lds[];
     const int2 tl = tiles[blockIdx.x];
     const int t = tl.x, base = T.tbase[t], n = T.tsize[t];
@@ -151,25 +159,15 @@ __global__ void __launch_bounds__(FORCE_TILE)
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (!T.extra[b]) {
         const float4 fn = ln[i], f1 = l1[i], f2 = l2[i];
-        Own I = make_own(lx[i], make_float4(fn.w, f1.w, f2.w, 0.f), fn, f1, f2);
-        set_box(I, T.tbox[t]);
-        bead_force(P, LdsAcc{lx, ln, l1, l2}, GlobalLists{T, b, base}, i, P.is_wall ? T.zs[t] : 0.f, I, F);
+        const float4 x = lx[i];
+        Own I = make_own(x, make_float4(fn.w, f1.w, f2.w, 0.f), fn, f1, f2, __float_as_int(x.w));
+        if (PERIODIC) set_box(I, T.tbox[t]);
+        const LdsAcc A(lx, ln, l1, l2);
+        bead_force<PERIODIC>(K, A, GlobalLists<LdsAcc::SCALE>{T, b, base, A.origin()}, K.is_wall ? T.zs[t] : 0.f, I, F);
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) {
-        const float var = sqrtf(2.0f * KB * P.temp * P.gammaR / P.dt);
-        float4 r;
-        if (D.noise) {
-            const float *nz = D.noise + 6 * (size_t)b;
-            r = make_float4(nz[0], nz[1], nz[2], 0.f);
-        } else {
-            uint4 s = D.seeds[b];
-            r = normals4(s);
-            D.seeds[b] = s;
-        }
-        D.R[b] = T.extra[b] ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
-    }
+    if (D.R) tea_draw(D, K.vF, b, T.extra[b]);
 }
 
 // Dynamic LDS of k_forces_lds for trajectories of up to nmax beads.
@@ -182,7 +180,7 @@ __global__ void __launch_bounds__(BS)
     if (b >= T.nb) return;
     float U[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (!T.extra[b]) {
-        Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b]);
+        Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b], 0);
         set_box(I, T.tbox[T.tid[b]]);
         bead_energy(P, T, GlobalAcc{S, T}, b, I, U);
     }
@@ -212,18 +210,6 @@ __global__ void __launch_bounds__(256) k_traj_sum(DevTopo T, const double *en, d
 static inline int grid_for(int n, int bs = STREAM_BLOCK) { return (n + bs - 1) / bs; }
 // Grid of a kernel that takes its beads through xcd_bead: a multiple of 8.
 static inline int grid_xcd(int n, int bs) { return 8 * ((grid_for(n, bs) + 7) / 8); }
-
-// Launch of a per-bead kernel template at the tuned workgroup size.
-#define MTE_LAUNCH_BS(KERNEL, e, ...)                                                                              \
-    do {                                                                                                           \
-        const int bs_ = (e)->tune.stream_block;                                                                    \
-        if (bs_ == 64)                                                                                             \
-            hipLaunchKernelGGL(KERNEL<64>, dim3(grid_xcd((e)->nb, 64)), dim3(64), 0, (e)->stream, __VA_ARGS__);   \
-        else if (bs_ == 128)                                                                                       \
-            hipLaunchKernelGGL(KERNEL<128>, dim3(grid_xcd((e)->nb, 128)), dim3(128), 0, (e)->stream, __VA_ARGS__); \
-        else                                                                                                       \
-            hipLaunchKernelGGL(KERNEL<256>, dim3(grid_xcd((e)->nb, 256)), dim3(256), 0, (e)->stream, __VA_ARGS__); \
-    } while (0)
 
 // The updater's tubule classification (mt_length, src/updater.cpp:164-205)
 // on the device: a bead is on the tubule when rad_lo < sqrt(x^2 + y^2) <
@@ -259,23 +245,41 @@ hipError_t launch_frames(mte_engine *e, int buf) {
     return hipGetLastError();
 }
 
+// Batches with a periodic box take the kernels with the minimum image; there
+// an open trajectory's separations are unchanged (side and inverse zero).
+template <bool PERIODIC>
+static void step_plain(mte_engine *e, const float *noise_step) {
+    const int bs = e->tune.stream_block;
+    const dim3 grid(grid_xcd(e->nb, bs)), block(bs);
+    auto k = bs == 64 ? k_step_plain<64, PERIODIC> : bs == 128 ? k_step_plain<128, PERIODIC> : k_step_plain<256, PERIODIC>;
+    hipLaunchKernelGGL(k, grid, block, 0, e->stream, e->K, e->T, e->S[e->cur], e->S[1 - e->cur], e->seeds, noise_step,
+                       e->L);
+}
 hipError_t launch_step_plain(mte_engine *e, const float *noise_step) {
-    MTE_LAUNCH_BS(k_step_plain, e, e->P, e->T, e->S[e->cur], e->S[1 - e->cur], e->seeds, noise_step, e->L);
+    if (e->periodic) step_plain<true>(e, noise_step);
+    else step_plain<false>(e, noise_step);
     e->cur = 1 - e->cur;
     return hipGetLastError();
 }
 
-static hipError_t launch_forces_draw(mte_engine *e, TeaDraw D) {
+template <bool PERIODIC>
+static hipError_t forces_draw(mte_engine *e, TeaDraw D) {
     if (e->tune.forces == MTE_FORCES_LDS && e->forces_lds > 0) {
-        const hipError_t s = hipFuncSetAttribute((const void *)k_forces_lds,
+        const hipError_t s = hipFuncSetAttribute((const void *)k_forces_lds<PERIODIC>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)e->forces_lds);
         if (s != hipSuccess) return s;
-        hipLaunchKernelGGL(k_forces_lds, dim3(e->ntiles), dim3(FORCE_TILE), e->forces_lds, e->stream, e->P, e->T,
-                           e->S[e->cur], e->tiles, e->fxyz, e->fang, D);
+        hipLaunchKernelGGL(k_forces_lds<PERIODIC>, dim3(e->ntiles), dim3(FORCE_TILE), e->forces_lds, e->stream, e->K,
+                           e->T, e->S[e->cur], e->tiles, e->fxyz, e->fang, D);
     } else {
-        MTE_LAUNCH_BS(k_forces, e, e->P, e->T, e->S[e->cur], e->fxyz, e->fang, D);
+        const int bs = e->tune.stream_block;
+        const dim3 grid(grid_xcd(e->nb, bs)), block(bs);
+        auto k = bs == 64 ? k_forces<64, PERIODIC> : bs == 128 ? k_forces<128, PERIODIC> : k_forces<256, PERIODIC>;
+        hipLaunchKernelGGL(k, grid, block, 0, e->stream, e->K, e->T, e->S[e->cur], e->fxyz, e->fang, D);
     }
     return hipGetLastError();
+}
+static hipError_t launch_forces_draw(mte_engine *e, TeaDraw D) {
+    return e->periodic ? forces_draw<true>(e, D) : forces_draw<false>(e, D);
 }
 
 hipError_t launch_forces(mte_engine *e) { return launch_forces_draw(e, TeaDraw{nullptr, nullptr, nullptr}); }
@@ -285,7 +289,9 @@ hipError_t launch_forces_tea(mte_engine *e, const float *noise_step) {
 }
 
 hipError_t launch_energies(mte_engine *e) {
-    MTE_LAUNCH_BS(k_energies, e, e->P, e->T, e->S[e->cur], e->en_bead);
+    const int bs = e->tune.stream_block;
+    auto k = bs == 64 ? k_energies<64> : bs == 128 ? k_energies<128> : k_energies<256>;
+    hipLaunchKernelGGL(k, dim3(grid_xcd(e->nb, bs)), dim3(bs), 0, e->stream, e->P, e->T, e->S[e->cur], e->en_bead);
     hipLaunchKernelGGL(k_traj_sum, dim3(e->ntraj), dim3(256), 0, e->stream, e->T, e->en_bead, e->en_traj);
     return hipGetLastError();
 }

@@ -691,7 +691,7 @@ __global__ void __launch_bounds__(NET_THREADS)
 }
 
 struct MlpStepArgs {
-    mte_params P;
+    ForceK K;
     DevTopo T;
     DevState Sin, Sout;
     const float4 *fxyz, *fang, *ci;
@@ -741,7 +741,7 @@ __device__ __forceinline__ MlpIn mlp_load(const MlpStepArgs &A, int b) {
 }
 
 __device__ __forceinline__ void mlp_integrate(const MlpStepArgs &A, int b, const float y[MLP_OUT], const MlpIn &in) {
-    const mte_params &P = A.P;
+    const ForceK &K = A.K;
     const DevTopo &T = A.T;
     float4 x = in.x, an = in.an;
     float4 n4 = in.n4, p1 = in.p1, p2 = in.p2;
@@ -781,20 +781,14 @@ __device__ __forceinline__ void mlp_integrate(const MlpStepArgs &A, int b, const
             A.seeds[b + T.nb] = s;
         }
         const float4 F = in.F;
-        const float dtg = P.dt / P.gammaR;
         const float d0 = F.x + G[0] * F.x + G[1] * F.y + G[2] * F.z;
         const float d1 = F.y + G[3] * F.x + G[4] * F.y + G[5] * F.z;
         const float d2 = F.z + G[6] * F.x + G[7] * F.y + G[8] * F.z;
         const float n0 = Lc[0] * rx.x, n1 = Lc[1] * rx.x + Lc[2] * rx.y, n2 = Lc[3] * rx.x + Lc[4] * rx.y + Lc[5] * rx.z;
-        x.x += dtg * d0 + P.varR * n0;
-        x.y += dtg * d1 + P.varR * n1;
-        x.z += dtg * d2 + P.varR * n2;
-        const float4 fa = in.fa;
-        const float dta = P.dt / (P.gammaTheta * P.alpha), dtt = P.dt / P.gammaTheta;
-        const float vta = P.varTheta * sqrtf(P.freeze_temp / P.alpha);
-        an.x += dta * fa.x + vta * ra.x;
-        an.z += dta * fa.z + vta * ra.y;
-        an.y += dtt * fa.y + P.varTheta * ra.z;
+        x.x += fmaf(K.dtg, d0, K.vR * n0);
+        x.y += fmaf(K.dtg, d1, K.vR * n1);
+        x.z += fmaf(K.dtg, d2, K.vR * n2);
+        em_angles(K, in.fa.x, in.fa.y, in.fa.z, ra, an);
         frame_vectors(an.x, an.y, an.z, A.L, n4, p1, p2);
     } else if (A.yout) {
         for (int q = 0; q < MLP_OUT; q++) A.yout[(size_t)b * MLP_OUT + q] = 0.f;
@@ -1284,7 +1278,7 @@ hipError_t launch_mlp_forward(mte_engine *e, const float *feat, int n, float *ou
 hipError_t launch_mlp_step(mte_engine *e, const float *noise_step, float *yout) {
     hipError_t s = net_lds_attr((const void *)k_mlp_step);
     if (s != hipSuccess) return s;
-    MlpStepArgs A{e->P, e->T, e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.ci, e->tea.beta,
+    MlpStepArgs A{e->K, e->T, e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.ci, e->tea.beta,
                   e->seeds, noise_step, yout, e->mlp.nbad, e->L};
     hipLaunchKernelGGL(k_mlp_step, dim3(net_blocks(e, e->nb)), dim3(NET_THREADS), NET_IMG_BYTES, e->stream,
                        reinterpret_cast<const u32x4 *>(e->mlp.img), e->mlp.feat, e->mlp.fblk, A);

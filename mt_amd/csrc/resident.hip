@@ -4,9 +4,9 @@
 // One workgroup owns one trajectory.  LDS holds, per bead, the position and
 // the three rotated offsets with the Euler angles packed into their spare
 // lanes (64 B), plus the bead's neighbour lists compacted into a uint16 CSR
-// (bonds: local index << 1 | flag; LJ: 16 x local index, the neighbour's
-// byte offset among the positions) whose places are sized for the full lists, so a
-// distance-filtered list and its later refill share one layout.  Each
+// (the LDS address of the neighbour's position; bonds: with their flag in bit
+// 0) whose places are sized for the full lists, so a distance-filtered list
+// and its later refill share one layout.  Each
 // thread owns PT beads and keeps their two HybridTaus states in registers.
 // A launch runs every step up to the next
 // list-rebuild boundary (LJPairsUpdateFreq steps; 100 in the batched
@@ -16,6 +16,15 @@
 //   forces + Euler-Maruyama for own beads, every operand from LDS
 //   -> barrier -> own new state to LDS -> barrier.
 // The arithmetic is bead_force / em_update, the code the streamed step runs.
+//
+// What bounds it: the vector operations, about 3 cycles each, of 16 waves on
+// four SIMDs (256 tubes of 1040 beads, a workgroup per CU); of a step the LJ
+// sums take some 30 %, the normals 20 %, the bonds 27 %, the frames 9 %.  So
+// the operations were cut: quotients and halves taken on the host (ForceK),
+// torques summed as vectors and projected once, lists with ready LDS
+// addresses, LJ lists padded to the groups they are summed in, fewer
+// operations per HybridTaus draw, no minimum image in open batches: 713 ->
+// 575 us per 100 steps, one tube of 312 beads 435 -> 343 us.
 // If a trajectory's lists do not fit the LDS left over, that workgroup reads
 // them from the global k-major arrays instead (same results, slower).
 #include "bead_physics.h"
@@ -61,46 +70,59 @@ __device__ __forceinline__ int pack_counts(int h, int nlon, int nlat, int nlj) {
     return (h ? 1 : 0) | (nlon << 1) | (nlat << 5) | (nlj << 10);
 }
 
-// Lists compacted in LDS: packed entries with local indices (LJ entries as
-// byte offsets), the encoding bead_force reads through LdsAcc.
+// Lists compacted in LDS at ent[off]: the LDS address of the neighbour's
+// position (LdsAcc's handle), a bond's flag in bit 0.  Made once per launch
+// by threads that keep their bead's state: the harmonic entry itself, and the
+// addresses of the others.
 struct LdsLists {
-    const uint16_t *e;
-    int off, cnt;
-    __device__ __forceinline__ int h() const { return cnt & 1; }
-    __device__ __forceinline__ int harm() const { return h() ? (int)e[off] : -1; }
+    int eh, cnt;
+    uint32_t alon, alat, alj;
+    __device__ __forceinline__ static int at(uint32_t a, int k) {
+        return *(const __attribute__((address_space(3))) uint16_t *)(uintptr_t)(a + 2 * k);
+    }
+    __device__ __forceinline__ LdsLists(const uint16_t *ent, int off, int c) : cnt(c) {
+        const uint32_t a = lds_addr(ent) + 2 * off;
+        eh = c & 1 ? at(a, 0) : -1;
+        alon = a + 2 * (c & 1);
+        alat = alon + 2 * nlon();
+        alj = alat + 2 * nlat();
+    }
+    __device__ __forceinline__ int harm() const { return eh; }
     __device__ __forceinline__ int nlon() const { return (cnt >> 1) & 15; }
-    __device__ __forceinline__ int lon(int k) const { return e[off + h() + k]; }
+    __device__ __forceinline__ int lon(int k) const { return at(alon, k); }
     __device__ __forceinline__ int nlat() const { return (cnt >> 5) & 31; }
-    __device__ __forceinline__ int lat(int k) const { return e[off + h() + nlon() + k]; }
-    __device__ __forceinline__ int nlj() const { return (cnt >> 10) & 1023; }
-    __device__ __forceinline__ int lj(int k) const { return e[off + h() + nlon() + nlat() + k]; }
+    __device__ __forceinline__ int lat(int k) const { return at(alat, k); }
+    __device__ __forceinline__ uint32_t ref(int e) const { return e & 0xfff0; }
+    __device__ __forceinline__ int nlj() const { return cnt >> 10; }
+    __device__ __forceinline__ uint32_t lj(int k) const { return at(alj, k); }
 };
-// LJ entries in LDS hold the neighbour's byte offset in the position array
-// (16 times its local index), so reading its position takes no scaling.
-__device__ __forceinline__ float4 lj_xyz(const LdsAcc &A, const LdsLists &Ls, int k) {
-    return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(A.x) + Ls.lj(k));
+
+// A bead's state as LDS holds it: position (w: packed flags), rotated offsets
+// with the Euler angles in w (n|fi, p1|theta, p2|psi).
+struct BeadState {
+    float4 x, n, p1, p2;
+};
+__device__ __forceinline__ BeadState load_state(const LdsAcc &A, int i) {
+    const uint32_t h = A.origin() + i * LdsAcc::SCALE;
+    return {A.xyz(h), A.fn(h), A.lat(h, false), A.lat(h, true)};
+}
+// The state at position x with angles a; trig = (sin theta, cos theta, sin
+// psi, cos psi).
+__device__ __forceinline__ BeadState new_state(float4 x, float4 a, const LatOffsets &L, float4 &trig) {
+    const Frame f = make_frame(a.x, a.y, a.z, L);
+    trig = make_float4(f.st, f.ct, f.sp, f.cp);
+    return {x, make_float4(f.n.x, f.n.y, f.n.z, a.x), make_float4(f.p1.x, f.p1.y, f.p1.z, a.y),
+            make_float4(f.p2.x, f.p2.y, f.p2.z, a.z)};
 }
 
-// Writes a bead's new state to LDS; returns (sin theta, cos theta, sin psi,
-// cos psi) for the owner's next force evaluation.
-__device__ __forceinline__ float4 store_state(float4 *lx, float4 *ln, float4 *l1, float4 *l2, int i, float4 x,
-                                              float4 a, const LatOffsets &L) {
-    const Rot R = make_rot(a.x, a.y, a.z);
-    float3 v = R.apply(0.f, 0.f, 1.f);
-    float4 n = make_float4(v.x, v.y, v.z, 0.f);
-    v = R.apply(L.p1x, L.p1y, L.p1z);
-    float4 p1 = make_float4(v.x, v.y, v.z, 0.f);
-    v = R.apply(L.p2x, L.p2y, L.p2z);
-    float4 p2 = make_float4(v.x, v.y, v.z, 0.f);
-    n.w = a.x;   // fi
-    p1.w = a.y;  // theta
-    p2.w = a.z;  // psi
-    lx[i] = x;
-    ln[i] = n;
-    l1[i] = p1;
-    l2[i] = p2;
-    return make_float4(R.st, R.ct, R.sp, R.cp);
-}
+// What a thread carries from step to step for each of its beads.
+template <int PT>
+struct Lanes {
+    bool mob[PT];
+    int ib[PT];             // local index
+    uint4 s0[PT], s1[PT];   // HybridTaus states
+    float4 trig[PT];
+};
 
 // The step loop over steps [first, nsteps).  FILTERED: the LJ lists in LDS
 // hold only the pairs within FILTER_R at step `first`; each mobile bead's
@@ -110,56 +132,85 @@ __device__ __forceinline__ float4 store_state(float4 *lx, float4 *ln, float4 *l1
 // force evaluation (dropped pairs contribute exactly zero force until then,
 // so the sums are those over the full lists) and go on unfiltered.
 // Returns nsteps when every step ran.
-template <int PT, bool FILTERED, class Lists, class MakeLists>
-__device__ __forceinline__ int run_steps(const mte_params &P, const DevTopo &T, const LdsAcc &A, int t, float4 *lx,
-                                         float4 *ln, float4 *l1, float4 *l2, const bool mob[PT], uint4 s0[PT],
-                                         uint4 s1[PT], float4 trig[PT], const float *noise, int first, int nsteps,
-                                         const LatOffsets &L, const MakeLists &make_lists, int *flags, float4 *rbuf,
-                                         int own_slot, int help_slot, const int ib[PT]) {
+//
+// A step has two phases, one before each barrier: forces and update from the
+// old state in LDS, and the stores of the new one.  With one bead per thread
+// the new frame belongs to the first phase, the normals of the next step,
+// which need no neighbour, to the second (drawn while the stores drain), and
+// the thread keeps its bead's state and list position in registers.  Several
+// beads per thread leave no registers for that: state read back from LDS,
+// normals drawn where they are used, frames made before they are stored.
+template <int PT, bool FILTERED, bool PERIODIC, class Lists, class MakeLists>
+__device__ __forceinline__ int run_steps(const ForceK &K0, const DevTopo &T, const LdsAcc &A, int t, float4 *lx,
+                                         float4 *ln, float4 *l1, float4 *l2, Lanes<PT> &W, const float *noise,
+                                         int first, int nsteps, const LatOffsets &L0, const MakeLists &make_lists,
+                                         int *flags, float4 *rbuf, int own_slot, int help_slot) {
     const int base = T.tbase[t], nb = T.nb;
-    const float box = T.tbox[t];
-    const float wall_z = P.is_wall ? T.zs[t] : 0.f;
+    const float box = PERIODIC ? T.tbox[t] : 0.f, ibox = inv_side(box);
+    constexpr bool KEEP = PT == 1;
+    ForceK K = K0;
+    LatOffsets L = L0;
+    if (KEEP) {   // constants used several times a step: 2 cycles an operation, 4 with a scalar operand
+        for (float *c : {&K.dtg, &K.vR, &K.fi_h, &K.psi_h, &K.lat_d, &K.seam_d, &L.p1x, &L.p1y, &L.p1z}) *c = in_vgpr(*c);
+    }
+    const float wall_z = K.is_wall ? T.zs[t] : 0.f;
     float3 xr[PT];
 #pragma unroll
-    for (int k = 0; k < PT; k++) xr[k] = FILTERED && mob[k] ? f3(lx[ib[k]]) : make_float3(0.f, 0.f, 0.f);
+    for (int k = 0; k < PT; k++) xr[k] = FILTERED && W.mob[k] ? f3(lx[W.ib[k]]) : make_float3(0.f, 0.f, 0.f);
+    BeadState st;     // KEEP: the bead's state
+    float4 rx1, ra1;  // and its next normals
+    if (KEEP && W.mob[0]) {
+        st = load_state(A, W.ib[0]);
+        if (!noise) {
+            rx1 = normals4(W.s0[0]);
+            ra1 = normals4(W.s1[0]);
+        }
+    }
+    const Lists own = make_lists(W.ib[0], base + W.ib[0], KEEP && W.mob[0]);
     for (int s = first; s < nsteps; s++) {
         float4 nx[PT], na[PT];
         bool moved = false;
 #pragma unroll
         for (int k = 0; k < PT; k++) {
-            if (!mob[k]) continue;
-            const int i = ib[k];
+            if (!W.mob[k]) continue;
+            const int i = W.ib[k];
             const int b = base + i;
-            float4 x = lx[i];
-            float4 a = make_float4(ln[i].w, l1[i].w, l2[i].w, 0.f);
-            Own I = make_own_trig(x, a, ln[i], l1[i], l2[i], trig[k]);
-            set_box(I, box);
+            const BeadState B = KEEP ? st : load_state(A, i);
+            float4 x = B.x, a = make_float4(B.n.w, B.p1.w, B.p2.w, 0.f);
+            Own I = make_own_trig(x, a, B.n, B.p1, B.p2, W.trig[k], __float_as_int(x.w));
+            if (PERIODIC) I.box = box, I.ibox = ibox;
             float F[6];
-            const Lists Ls = make_lists(i, b);
-            bead_force(P, A, Ls, i, wall_z, I, F);
+            bead_force<PERIODIC>(K, A, KEEP ? own : make_lists(i, b, true), wall_z, I, F);
             float4 rx, ra;
             if (noise) {
                 const float *nz = noise + (size_t)s * 6 * nb + 6 * (size_t)b;
                 rx = make_float4(nz[0], nz[1], nz[2], 0.f);
                 ra = make_float4(nz[3], nz[4], nz[5], 0.f);
+            } else if (KEEP) {
+                rx = rx1;
+                ra = ra1;
             } else if (k == 1 && own_slot >= 0) {   // drawn by the helper (PT == 2)
                 rx = rbuf[((s & 1) * RNG_SLOTS + own_slot) * 2];
                 ra = rbuf[((s & 1) * RNG_SLOTS + own_slot) * 2 + 1];
             } else {
-                rx = normals4(s0[k]);
-                ra = normals4(s1[k]);
+                rx = normals4(W.s0[k]);
+                ra = normals4(W.s1[k]);
             }
-            em_update(P, F, rx, ra, x, a);
-            nx[k] = x;   // w keeps the packed flags
-            na[k] = a;
+            em_update(K, F, rx, ra, x, a);
+            if (KEEP) {
+                st = new_state(x, a, L, W.trig[k]);   // x.w keeps the packed flags
+            } else {
+                nx[k] = x;
+                na[k] = a;
+            }
             if (FILTERED) {
                 const float dx = x.x - xr[k].x, dy = x.y - xr[k].y, dz = x.z - xr[k].z;
                 moved |= dx * dx + dy * dy + dz * dz >= SKIN_HALF * SKIN_HALF;
             }
         }
         if (PT == 2 && help_slot >= 0 && s + 1 < nsteps) {   // the owner's draws of the next step
-            rbuf[(((s + 1) & 1) * RNG_SLOTS + help_slot) * 2] = normals4(s0[PT - 1]);
-            rbuf[(((s + 1) & 1) * RNG_SLOTS + help_slot) * 2 + 1] = normals4(s1[PT - 1]);
+            rbuf[(((s + 1) & 1) * RNG_SLOTS + help_slot) * 2] = normals4(W.s0[PT - 1]);
+            rbuf[(((s + 1) & 1) * RNG_SLOTS + help_slot) * 2 + 1] = normals4(W.s1[PT - 1]);
         }
         if (FILTERED && moved) flags[s & 1] = 1;
         __syncthreads();
@@ -167,8 +218,17 @@ __device__ __forceinline__ int run_steps(const mte_params &P, const DevTopo &T, 
         if (FILTERED && threadIdx.x == 0) flags[(s + 1) & 1] = 0;   // read at the next step, after its barrier
 #pragma unroll
         for (int k = 0; k < PT; k++) {
-            if (!mob[k]) continue;
-            trig[k] = store_state(lx, ln, l1, l2, ib[k], nx[k], na[k], L);
+            if (!W.mob[k]) continue;
+            const int i = W.ib[k];
+            if (!KEEP) st = new_state(nx[k], na[k], L, W.trig[k]);
+            lx[i] = st.x;
+            ln[i] = st.n;
+            l1[i] = st.p1;
+            l2[i] = st.p2;
+            if (KEEP && !noise && s + 1 < nsteps && !left) {   // (after leaving, the next call draws them)
+                rx1 = normals4(W.s0[0]);
+                ra1 = normals4(W.s1[0]);
+            }
         }
         __syncthreads();
         if (left) return s + 1;   // uniform: every thread read the same flag
@@ -176,9 +236,9 @@ __device__ __forceinline__ int run_steps(const mte_params &P, const DevTopo &T, 
     return nsteps;
 }
 
-template <int PT, int MAXT>
+template <int PT, int MAXT, bool PERIODIC>
 __global__ void __launch_bounds__(MAXT)
-    k_resident(mte_params P, DevTopo T, DevState S, uint4 *seeds, const float *noise, int nsteps, LatOffsets L,
+    k_resident(ForceK K, float ljpairscutoff, DevTopo T, DevState S, uint4 *seeds, const float *noise, int nsteps, LatOffsets L,
                int stride, int entry_cap, const int *order) {
     extern __shared__ float4 lds[];
     // A rebuild that ran out of list capacity stops the dynamics: the state
@@ -201,30 +261,26 @@ __global__ void __launch_bounds__(MAXT)
     const int nb = T.nb;
     if (threadIdx.x == 0) flags[0] = 0;
     stage_state(T, S, base, n, lx, ln, l1, l2);
-    bool mob[PT];
-    uint4 s0[PT], s1[PT];
-    float4 trig[PT];
-    int ib[PT];   // the bead of each of this thread's lane slots (order: immobile beads last)
+    Lanes<PT> W;   // this thread's lane slots (order: immobile beads last)
     int lcnt[PT];   // its list counts, packed as in hcnt (requested with the bead's state)
 #pragma unroll
     for (int k = 0; k < PT; k++) {
         const int slot = threadIdx.x + k * blockDim.x;
         const int i = slot < n ? order[base + slot] : slot;
-        ib[k] = i;
+        W.ib[k] = i;
         const int b = base + i;
-        mob[k] = i < n && !T.fixed[b] && !T.extra[b];
+        W.mob[k] = i < n && !T.fixed[b] && !T.extra[b];
         lcnt[k] = 0;
-        if (mob[k])
-            lcnt[k] = pack_counts(T.harm[b] >= 0, T.lon_n[b], T.lat_n[b], P.lj_on ? T.lj_n[b] : 0);
-        trig[k] = make_float4(0.f, 1.f, 0.f, 1.f);
-        if (mob[k]) {
+        if (W.mob[k])
+            lcnt[k] = pack_counts(T.harm[b] >= 0, T.lon_n[b], T.lat_n[b], K.lj_on ? T.lj_n[b] : 0);
+        if (W.mob[k]) {
             const float4 a = S.ang[b];
-            sincos_fast(a.y, &trig[k].x, &trig[k].y);
-            sincos_fast(a.z, &trig[k].z, &trig[k].w);
+            sincos_fast(a.y, &W.trig[k].x, &W.trig[k].y);
+            sincos_fast(a.z, &W.trig[k].z, &W.trig[k].w);
         }
-        if (mob[k] && !noise) {
-            s0[k] = seeds[b];
-            s1[k] = seeds[b + nb];
+        if (W.mob[k] && !noise) {
+            W.s0[k] = seeds[b];
+            W.s1[k] = seeds[b + nb];
         }
     }
     // noise offload roles (two beads per thread, drawn noise); the first
@@ -234,7 +290,7 @@ __global__ void __launch_bounds__(MAXT)
     // (flags[0] was cleared before the first barrier; the skin test clears it
     // again in fill before its first use)
     __syncthreads();
-    if (PT == 2 && threadIdx.x >= 256 && mob[PT - 1]) flags[0] = 1;
+    if (PT == 2 && threadIdx.x >= 256 && W.mob[PT - 1]) flags[0] = 1;
     __syncthreads();
     const bool tail_busy = flags[0] != 0;
     auto offloaded = [&](int tt) {
@@ -248,15 +304,15 @@ __global__ void __launch_bounds__(MAXT)
         if (!T.fixed[b] && !T.extra[b]) {
             help_slot = rng_slot(owner);
             help_b = b;
-            s0[PT - 1] = seeds[b];
-            s1[PT - 1] = seeds[b + nb];
-            rbuf[help_slot * 2] = normals4(s0[PT - 1]);   // step 0's draws (parity 0)
-            rbuf[help_slot * 2 + 1] = normals4(s1[PT - 1]);
+            W.s0[PT - 1] = seeds[b];
+            W.s1[PT - 1] = seeds[b + nb];
+            rbuf[help_slot * 2] = normals4(W.s0[PT - 1]);   // step 0's draws (parity 0)
+            rbuf[help_slot * 2 + 1] = normals4(W.s1[PT - 1]);
         }
     }
     __syncthreads();
-    const LdsAcc A{lx, ln, l1, l2};
-    const float box = T.tbox[t], ibox = inv_side(box);
+    const LdsAcc A(lx, ln, l1, l2);
+    const float box = PERIODIC ? T.tbox[t] : 0.f, ibox = inv_side(box);
     // LJ entries of bead i kept in LDS: all of them (rf2 == 0), or those
     // within sqrt(rf2) of it now.
     auto lj_keep = [lx, box, ibox](int i, int j, float rf2) {
@@ -269,13 +325,14 @@ __global__ void __launch_bounds__(MAXT)
     // through a block scan into hoff.  Returns the number of entries.  Every
     // later fill writes at these offsets (a filtered list uses a prefix of
     // its bead's place), so the layout is computed once per launch.
+    auto handle = [&](int j) { return A.origin() + (uint32_t)((j - base) * LdsAcc::SCALE); };
     auto layout = [&]() {
         for (int i = threadIdx.x; i < n; i += blockDim.x) hoff[i] = 0;   // immobile beads use no lists
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < PT; k++) {
-            if (!mob[k]) continue;
-            const int i = ib[k], hc = lcnt[k];
+            if (!W.mob[k]) continue;
+            const int i = W.ib[k], hc = lcnt[k];
             hcnt[i] = hc;
             hoff[i] = (hc & 1) + ((hc >> 1) & 15) + ((hc >> 5) & 31) + (hc >> 10);
         }
@@ -325,14 +382,15 @@ __global__ void __launch_bounds__(MAXT)
     auto fill = [&](float rf2) {
 #pragma unroll
         for (int kk = 0; kk < PT; kk++) {
-            if (!mob[kk]) continue;
-            const int i = ib[kk], b = base + i;
+            if (!W.mob[kk]) continue;
+            const int i = W.ib[kk], b = base + i;
             const int hc = hcnt[i];
             const int h = hc & 1, nlon = (hc >> 1) & 15, nlat = (hc >> 5) & 31;
             const int nbond = h + nlon + nlat;
             const int o0 = hoff[i];
             const int nall = (i + 1 < n ? hoff[i + 1] : nent) - o0;
             int o = o0, nlj = 0;
+            int spare[3] = {0, 0, 0}, nspare = 0;   // the last three dropped
             for (int k0 = 0; k0 < nall; k0 += FILL_BATCH) {
                 int v[FILL_BATCH];
 #pragma unroll
@@ -348,13 +406,29 @@ __global__ void __launch_bounds__(MAXT)
                 for (int u = 0; u < FILL_BATCH; u++) {
                     const int k = k0 + u;
                     if (k < nbond) {
-                        ent[o++] = (uint16_t)((((v[u] >> 1) - base) << 1) | (v[u] & 1));
-                    } else if (k < nall && lj_keep(i, v[u] - base, rf2)) {
-                        ent[o++] = (uint16_t)((v[u] - base) * (int)sizeof(float4));
-                        nlj++;
+                        ent[o++] = (uint16_t)(handle(ent_j(v[u])) | ent_f(v[u]));
+                    } else if (k < nall) {
+                        if (lj_keep(i, v[u] - base, rf2)) {
+                            ent[o++] = (uint16_t)handle(v[u]);
+                            nlj++;
+                        } else {
+                            spare[2] = spare[1];
+                            spare[1] = spare[0];
+                            spare[0] = v[u];
+                            nspare++;
+                        }
                     }
                 }
             }
+            // Dropped entries, which contribute nothing, fill the list up to
+            // a multiple of the four that lj_sum takes at once: a remainder
+            // runs one entry at a time, for the whole wave.
+#pragma unroll
+            for (int u = 0; u < 3; u++)
+                if ((nlj & 3) != 0 && u < nspare) {
+                    ent[o++] = (uint16_t)handle(spare[u]);
+                    nlj++;
+                }
             hcnt[i] = (hc & 1023) | (nlj << 10);
         }
         if (threadIdx.x == 0) flags[0] = flags[1] = 0;
@@ -366,22 +440,23 @@ __global__ void __launch_bounds__(MAXT)
     nent = layout();
     const bool use_lds = nent <= entry_cap;
     if (use_lds) {
-        const bool filter = P.lj_on && P.ljpairscutoff > FILTER_R;
+        const bool filter = K.lj_on && ljpairscutoff > FILTER_R;
         fill(filter ? FILTER_R * FILTER_R : 0.f);
-        auto mk = [&](int i, int) { return LdsLists{ent, hoff[i], hcnt[i]}; };
+        auto mk = [&](int i, int, bool lists) { return LdsLists(ent, lists ? hoff[i] : 0, lists ? hcnt[i] : 0); };
         int s = 0;
         if (filter) {
-            s = run_steps<PT, true, LdsLists>(P, T, A, t, lx, ln, l1, l2, mob, s0, s1, trig, noise, 0, nsteps, L, mk,
-                                              flags, rbuf, own_slot, help_slot, ib);
+            s = run_steps<PT, true, PERIODIC, LdsLists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk,
+                                              flags, rbuf, own_slot, help_slot);
             if (s < nsteps) fill(0.f);   // a bead left its skin: the full lists from step s on
         }
         if (s < nsteps)
-            run_steps<PT, false, LdsLists>(P, T, A, t, lx, ln, l1, l2, mob, s0, s1, trig, noise, s, nsteps, L, mk,
-                                           flags, rbuf, own_slot, help_slot, ib);
+            run_steps<PT, false, PERIODIC, LdsLists>(K, T, A, t, lx, ln, l1, l2, W, noise, s, nsteps, L, mk,
+                                           flags, rbuf, own_slot, help_slot);
     } else {
-        auto mk = [&](int, int b) { return GlobalLists{T, b, base}; };
-        run_steps<PT, false, GlobalLists>(P, T, A, t, lx, ln, l1, l2, mob, s0, s1, trig, noise, 0, nsteps, L, mk,
-                                          flags, rbuf, own_slot, help_slot, ib);
+        using Lists = GlobalLists<LdsAcc::SCALE>;
+        auto mk = [&](int, int b, bool) { return Lists{T, b, base, A.origin()}; };
+        run_steps<PT, false, PERIODIC, Lists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk,
+                                          flags, rbuf, own_slot, help_slot);
     }
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int b = base + i;
@@ -396,15 +471,15 @@ __global__ void __launch_bounds__(MAXT)
     }
 #pragma unroll
     for (int k = 0; k < PT; k++) {
-        if (mob[k] && !noise && !(k == 1 && own_slot >= 0)) {   // an offloaded bead's state is the helper's
-            const int b = base + ib[k];
-            seeds[b] = s0[k];
-            seeds[b + nb] = s1[k];
+        if (W.mob[k] && !noise && !(k == 1 && own_slot >= 0)) {   // an offloaded bead's state is the helper's
+            const int b = base + W.ib[k];
+            seeds[b] = W.s0[k];
+            seeds[b + nb] = W.s1[k];
         }
     }
     if (help_b >= 0) {
-        seeds[help_b] = s0[PT - 1];
-        seeds[help_b + nb] = s1[PT - 1];
+        seeds[help_b] = W.s0[PT - 1];
+        seeds[help_b + nb] = W.s1[PT - 1];
     }
 }
 
@@ -420,7 +495,7 @@ bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     if (e->P.tea_on || pt < 1 || pt > RES_MAX_PT) return false;
     int nmax = 0;
     for (int t = 0; t < e->ntraj; t++) nmax = std::max<int>(nmax, (int)(e->off[t + 1] - e->off[t]));
-    if (nmax > 4096) return false;   // uint16 list entries (LJ entries: 16 x the local index)
+    if (nmax > 4096) return false;   // uint16 list entries (16 x the local index: the position array is at LDS address 0)
     int lds_limit = 0;
     if (hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device) != hipSuccess)
         return false;
@@ -452,25 +527,31 @@ bool resident_fits(const mte_engine *e, ResidentPlan *plan) {
     return false;
 }
 
-template <int PT, int MAXT>
+template <int PT, int MAXT, bool PERIODIC>
 static hipError_t launch_pt(mte_engine *e, int nsteps, const float *noise) {
     const ResidentPlan &pl = e->rplan;
-    hipError_t s = hipFuncSetAttribute((const void *)k_resident<PT, MAXT>,
+    hipError_t s = hipFuncSetAttribute((const void *)k_resident<PT, MAXT, PERIODIC>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
     if (s != hipSuccess) return s;
-    hipLaunchKernelGGL((k_resident<PT, MAXT>), dim3(e->ntraj), dim3(pl.threads), pl.lds_bytes, e->stream, e->P,
-                       e->T, e->S[e->cur], e->seeds, noise, nsteps, e->L, pl.max_beads, pl.entry_cap, e->res_order);
+    hipLaunchKernelGGL((k_resident<PT, MAXT, PERIODIC>), dim3(e->ntraj), dim3(pl.threads), pl.lds_bytes, e->stream, e->K,
+                       e->P.ljpairscutoff, e->T, e->S[e->cur], e->seeds, noise, nsteps, e->L, pl.max_beads, pl.entry_cap, e->res_order);
     return hipGetLastError();
 }
 
-hipError_t launch_resident(mte_engine *e, int nsteps, const float *noise) {
-    const ResidentPlan &pl = e->rplan;
-    switch (pl.per_thread) {
-    case 1: return launch_pt<1, RES_MAX_THREADS>(e, nsteps, noise);
-    case 2: return launch_pt<2, RES_MULTI_THREADS>(e, nsteps, noise);
-    case 3: return launch_pt<3, RES_MULTI_THREADS>(e, nsteps, noise);
+template <bool PERIODIC>
+static hipError_t launch_box(mte_engine *e, int nsteps, const float *noise) {
+    switch (e->rplan.per_thread) {
+    case 1: return launch_pt<1, RES_MAX_THREADS, PERIODIC>(e, nsteps, noise);
+    case 2: return launch_pt<2, RES_MULTI_THREADS, PERIODIC>(e, nsteps, noise);
+    case 3: return launch_pt<3, RES_MULTI_THREADS, PERIODIC>(e, nsteps, noise);
     default: return hipErrorInvalidValue;
     }
+}
+
+// Batches with a periodic box take the kernels with the minimum image; there
+// an open trajectory's separations are unchanged (side and inverse zero).
+hipError_t launch_resident(mte_engine *e, int nsteps, const float *noise) {
+    return e->periodic ? launch_box<true>(e, nsteps, noise) : launch_box<false>(e, nsteps, noise);
 }
 
 }  // namespace mte

@@ -44,13 +44,6 @@ __device__ __forceinline__ float wave_rol1(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x134, 0xF, 0xF, false));
 }
 
-// Keeps a loop constant in a vector register: an FP32 operation with a scalar
-// operand issues at half rate (4 cycles per wave, measured, against 2).
-__device__ __forceinline__ float in_vgpr(float v) {
-    __asm__("" : "+v"(v));
-    return v;
-}
-
 // One coordinate of the pair loops: x itself, or (INT) its place in the
 // periodic box as a 32-bit integer (bit pattern), taken modulo the box in FP64.
 template <bool INT>
@@ -793,7 +786,7 @@ __global__ void __launch_bounds__(TEA_TILE)
 // chunks.
 template <bool SYM>
 __global__ void __launch_bounds__(TEA_TILE)
-    k_tea_finish(mte_params P, DevTopo T, DevState Sin, DevState Sout, const float4 *fxyz, const float4 *fang,
+    k_tea_finish(ForceK K, DevTopo T, DevState Sin, DevState Sout, const float4 *fxyz, const float4 *fang,
                  const float4 *R, const float4 *ci, const float *beta, const int *nchunks, int jrun, int ioff,
                  const float4 *partial4, uint4 *seeds, const float *noise, LatOffsets L) {
     const int b = blockIdx.x * TEA_TILE + threadIdx.x;
@@ -869,16 +862,11 @@ __global__ void __launch_bounds__(TEA_TILE)
     }
     float4 n4 = Sin.fn[b], p1 = Sin.fp1[b], p2 = Sin.fp2[b];
     if (!T.fixed[b] && !T.extra[b]) {
-        const float mult = P.dt / P.gammaR;
-        x.x = fmaf(mult, fx, x.x);
-        x.y = fmaf(mult, fy, x.y);
-        x.z = fmaf(mult, fz, x.z);
+        x.x = fmaf(K.dtg, fx, x.x);
+        x.y = fmaf(K.dtg, fy, x.y);
+        x.z = fmaf(K.dtg, fz, x.z);
         const float4 fa = fang[b];
-        const float dta = P.dt / (P.gammaTheta * P.alpha), dtt = P.dt / P.gammaTheta;
-        const float vta = P.varTheta * sqrtf(P.freeze_temp / P.alpha);
-        an.x += dta * fa.x + vta * ra.x;            // fi
-        an.z += dta * fa.z + vta * ra.y;            // psi
-        an.y += dtt * fa.y + P.varTheta * ra.z;     // theta
+        em_angles(K, fa.x, fa.y, fa.z, ra, an);
         frame_vectors(an.x, an.y, an.z, L, n4, p1, p2);
     }
     Sout.xyz[b] = x;
@@ -1364,7 +1352,7 @@ hipError_t launch_tea_pairs(mte_engine *e) {
 
 hipError_t launch_tea_finish(mte_engine *e, const float *noise_step) {
     auto kern = e->tea.unit_chunk == MTE_TEA_SYMMETRIC ? k_tea_finish<true> : k_tea_finish<false>;
-    hipLaunchKernelGGL(kern, dim3((e->nb + TEA_TILE - 1) / TEA_TILE), dim3(TEA_TILE), 0, e->stream, e->P, e->T,
+    hipLaunchKernelGGL(kern, dim3((e->nb + TEA_TILE - 1) / TEA_TILE), dim3(TEA_TILE), 0, e->stream, e->K, e->T,
                        e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.R, e->tea.ci, e->tea.beta,
                        e->tea.nchunks, e->tea.jrun, e->tea.ioff, e->tea.partial, e->seeds, noise_step, e->L);
     e->cur = 1 - e->cur;
