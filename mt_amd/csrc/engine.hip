@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "engine_internal.h"
+#include "stage.h"
 
 using namespace mte;
 
@@ -330,9 +331,29 @@ static void generate_seeds(int32_t seed, size_t nwords, uint32_t *out) {
 
 namespace mte {
 // The list-capacity flags into the host's pinned, device-mapped words.
-__global__ void k_publish_flags(const int *overflow, const int *frozen, int *out) {
+// Position and angle arrays as mte_coord records (seven words: x, y, z, fi,
+// theta, psi, 0) in pinned host memory: four consecutive words per thread, so
+// that a wave's store is one run of 1 KB over the bus.
+__global__ void __launch_bounds__(256) k_pack_coords(const float4 *xyz, const float4 *ang, int words, float *out) {
+    const int w0 = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (w0 >= words) return;
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int w = min(w0 + u, words - 1), b = w / 7, c = w - 7 * b;
+        v[u] = c == 6 ? 0.f : reinterpret_cast<const float *>(c < 3 ? xyz + b : ang + b)[c < 3 ? c : c - 3];
+    }
+    if (w0 + 4 <= words) {
+        *reinterpret_cast<float4 *>(out + w0) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+        for (int u = 0; w0 + u < words; u++) out[w0 + u] = v[u];
+    }
+}
+
+__global__ void k_publish_flags(const int *overflow, const int *frozen, const int *tea, int *out) {
     out[0] = *(volatile const int *)overflow;
     out[1] = *(volatile const int *)frozen;
+    out[2] = tea ? *(volatile const int *)tea : 0;
 }
 }  // namespace mte
 
@@ -408,6 +429,7 @@ int mte_destroy(mte_engine *e) {
         if (p) (void)hipFree(p);
     if (e->noise) (void)hipFree(e->noise);
     if (e->stream) (void)hipStreamDestroy(e->stream);
+    if (e->stage_user) StagePool::get().drop_user(e->device);
     delete e;
     return MTE_OK;
 }
@@ -461,6 +483,8 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
         e->err = "mte_create: stream creation failed";
         return bail(MTE_ERR_HIP);
     }
+    StagePool::get().add_user(e->device);
+    e->stage_user = true;
     if (noalloc_scratch_init(e->device, &e->noalloc) != hipSuccess) {
         e->err = "mte_create: hipGetSymbolAddress failed for the inference staging array";
         return bail(MTE_ERR_HIP);
@@ -597,13 +621,13 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
         e->err = "mte_create: memset failed";
         return bail(MTE_ERR_HIP);
     }
-    if (hipHostMalloc((void **)&e->flags_host, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) !=
+    if (hipHostMalloc((void **)&e->flags_host, 3 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) !=
             hipSuccess ||
         hipHostGetDevicePointer((void **)&e->flags_dev, e->flags_host, 0) != hipSuccess) {
         e->err = "mte_create: pinned allocation failed for the list-capacity flags";
         return bail(MTE_ERR_HIP);
     }
-    e->flags_host[0] = e->flags_host[1] = 0;
+    e->flags_host[0] = e->flags_host[1] = e->flags_host[2] = 0;
     if (e->P.tea_on && hipMemsetAsync(e->tea.status, 0, sizeof(int), e->stream) != hipSuccess) {
         e->err = "mte_create: memset failed";
         return bail(MTE_ERR_HIP);
@@ -749,14 +773,26 @@ int mte_set_state(mte_engine *e, const mte_coord *r) {
 int mte_get_state(mte_engine *e, mte_coord *r) {
     if (!e || !r) return MTE_ERR_ARG;
     HIPCHK(hipSetDevice(e->device));
-    std::vector<float4> xyz(e->nb), ang(e->nb);
-    HIPCHK(hipMemcpyAsync(xyz.data(), e->S[e->cur].xyz, sizeof(float4) * e->nb, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipMemcpyAsync(ang.data(), e->S[e->cur].ang, sizeof(float4) * e->nb, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
-    for (int b = 0; b < e->nb; b++) {
-        r[b].x = xyz[b].x; r[b].y = xyz[b].y; r[b].z = xyz[b].z;
-        r[b].fi = ang[b].x; r[b].theta = ang[b].y; r[b].psi = ang[b].z; r[b].w = 0.f;
+    Stage st(e->device, e->stream);
+    const DevState S = e->S[e->cur];
+    if (!st.pinned()) {
+        std::vector<float4> xyz(e->nb), ang(e->nb);
+        HIPCHK(st.to_host(xyz.data(), S.xyz, sizeof(float4) * e->nb));
+        HIPCHK(st.to_host(ang.data(), S.ang, sizeof(float4) * e->nb));
+        HIPCHK(st.finish());
+        for (int b = 0; b < e->nb; b++)
+            r[b] = mte_coord{xyz[b].x, xyz[b].y, xyz[b].z, ang[b].x, ang[b].y, ang[b].z, 0.f};
+        return MTE_OK;
     }
+    // records straight from the device's arrays to the pinned slots
+    constexpr size_t step = STAGE_SLOT / (4 * sizeof(mte_coord)) * (4 * sizeof(mte_coord));
+    HIPCHK(st.produce(r, sizeof(mte_coord) * e->nb, step, [&](char *p, size_t o, size_t m) {
+        const int words = (int)(m / sizeof(float)), b0 = (int)(o / sizeof(mte_coord));
+        hipLaunchKernelGGL(mte::k_pack_coords, dim3((words + 1023) / 1024), dim3(256), 0, e->stream, S.xyz + b0,
+                           S.ang + b0, words, (float *)p);
+        return hipGetLastError();
+    }));
+    HIPCHK(st.finish());
     return MTE_OK;
 }
 
@@ -832,6 +868,7 @@ int mte_get_step(const mte_engine *e, int64_t *step) {
 // in place of two device-to-host copies and a synchronisation of their own.
 static hipError_t publish_flags(mte_engine *e) {
     hipLaunchKernelGGL(mte::k_publish_flags, dim3(1), dim3(1), 0, e->stream, e->T.overflow, e->T.frozen,
+                       e->P.tea_on ? e->tea.status : nullptr,
                        e->flags_dev);
     return hipGetLastError();
 }
@@ -888,9 +925,9 @@ int mte_rebuild_lists(mte_engine *e) {
 }
 
 static int check_tea(mte_engine *e) {
-    int st = 0;
-    HIPCHK(hipMemcpyAsync(&st, e->tea.status, sizeof(int), hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(publish_flags(e));
     HIPCHK(hipStreamSynchronize(e->stream));
+    const int st = ((volatile int *)e->flags_host)[2];
     if (st) {
         (void)hipMemsetAsync(e->tea.status, 0, sizeof(int), e->stream);
         char buf[160];
@@ -1223,10 +1260,7 @@ int mte_tea_ci(mte_engine *e, float *ci) {
 static int need_mlp(mte_engine *e) {
     if (!e) return MTE_ERR_ARG;
     if (!e->P.tea_on) return fail(e, MTE_ERR_STATE, "MLP-HI needs TEA parameters (tea_on, tea_a)");
-    std::vector<float> box(e->ntraj);
-    if (hipMemcpy(box.data(), e->T.tbox, sizeof(float) * e->ntraj, hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(e, MTE_ERR_HIP, "need_mlp: box download failed");
-    for (float L : box)
+    for (float L : e->box_h)
         if (L > 0.f && L < 36.f) return fail(e, MTE_ERR_ARG, "MLP-HI needs periodic boxes of at least 36 nm");
     return MTE_OK;
 }
@@ -1289,8 +1323,10 @@ int mte_mlp_get_weights(mte_engine *e, float *w, int64_t n) {
     int rc = need_mlp(e);
     if (rc) return rc;
     if (!w || n != MLP_NPARAM) return fail(e, MTE_ERR_ARG, "mte_mlp_get_weights: expected MTE_MLP_NPARAM weights");
-    HIPCHK(hipMemcpyAsync(w, e->mlp.w, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    HIPCHK(hipSetDevice(e->device));
+    Stage st(e->device, e->stream);
+    HIPCHK(st.to_host(w, e->mlp.w, sizeof(float) * MLP_NPARAM));
+    HIPCHK(st.finish());
     return MTE_OK;
 }
 
@@ -1299,11 +1335,10 @@ int mte_mlp_local(mte_engine *e, float *features, float *labels) {
     if (rc) return rc;
     HIPCHK(hipSetDevice(e->device));
     HIPCHK(launch_mlp_local(e, e->mlp.feat, e->mlp.targ));
-    if (features)
-        HIPCHK(hipMemcpyAsync(features, e->mlp.feat, sizeof(float) * MLP_IN * e->nb, hipMemcpyDeviceToHost, e->stream));
-    if (labels)
-        HIPCHK(hipMemcpyAsync(labels, e->mlp.targ, sizeof(float) * MLP_OUT * e->nb, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    Stage st(e->device, e->stream);
+    if (features) HIPCHK(st.to_host(features, e->mlp.feat, sizeof(float) * MLP_IN * e->nb));
+    if (labels) HIPCHK(st.to_host(labels, e->mlp.targ, sizeof(float) * MLP_OUT * e->nb));
+    HIPCHK(st.finish());
     return MTE_OK;
 }
 
@@ -1314,10 +1349,11 @@ int mte_mlp_forward(mte_engine *e, const float *features, int64_t n, float *out)
     HIPCHK(hipSetDevice(e->device));
     rc = mlp_reserve(e, n);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(e->mlp.x, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
+    Stage st(e->device, e->stream);
+    HIPCHK(st.to_device(e->mlp.x, features, sizeof(float) * MLP_IN * n));
     HIPCHK(launch_mlp_forward(e, e->mlp.x, (int)n, e->mlp.y));
-    HIPCHK(hipMemcpyAsync(out, e->mlp.y, sizeof(float) * MLP_OUT * n, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    HIPCHK(st.to_host(out, e->mlp.y, sizeof(float) * MLP_OUT * n));
+    HIPCHK(st.finish());
     return MTE_OK;
 }
 
@@ -1345,13 +1381,14 @@ int mte_mlp_loss_grad(mte_engine *e, const float *features, const float *labels,
     if (!features || !labels || n <= 0) return fail(e, MTE_ERR_ARG, "mte_mlp_loss_grad: bad arguments");
     HIPCHK(hipSetDevice(e->device));
     if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, 1))) return rc;
-    HIPCHK(hipMemcpyAsync(e->mlp.x, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
-    HIPCHK(hipMemcpyAsync(e->mlp.t, labels, sizeof(float) * MLP_OUT * n, hipMemcpyHostToDevice, e->stream));
-    HIPCHK(launch_mlp_grad(e, e->mlp.x, e->mlp.t, (int)n, e->mlp.loss, 0.f, 0));
-    if (grad) HIPCHK(hipMemcpyAsync(grad, e->mlp.grad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, e->stream));
     double l = 0.0;
-    HIPCHK(hipMemcpyAsync(&l, e->mlp.loss, sizeof(double), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    Stage st(e->device, e->stream);
+    HIPCHK(st.to_device(e->mlp.x, features, sizeof(float) * MLP_IN * n));
+    HIPCHK(st.to_device(e->mlp.t, labels, sizeof(float) * MLP_OUT * n));
+    HIPCHK(launch_mlp_grad(e, e->mlp.x, e->mlp.t, (int)n, e->mlp.loss, 0.f, 0));
+    if (grad) HIPCHK(st.to_host(grad, e->mlp.grad, sizeof(float) * MLP_NPARAM));
+    HIPCHK(st.to_host(&l, e->mlp.loss, sizeof(double)));
+    HIPCHK(st.finish());
     if (loss) *loss = l;
     return MTE_OK;
 }
@@ -1368,8 +1405,9 @@ int mte_mlp_train(mte_engine *e, const float *features, const float *labels, int
     // slices, and the losses come back together at the end
     if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, iters))) return rc;
     float *X = e->mlp.x, *Y = e->mlp.t;
-    HIPCHK(hipMemcpyAsync(X, features, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, e->stream));
-    HIPCHK(hipMemcpyAsync(Y, labels, sizeof(float) * MLP_OUT * n, hipMemcpyHostToDevice, e->stream));
+    Stage st(e->device, e->stream);
+    HIPCHK(st.to_device(X, features, sizeof(float) * MLP_IN * n));
+    HIPCHK(st.to_device(Y, labels, sizeof(float) * MLP_OUT * n));
     int64_t pos = 0;
     for (int it = 0; it < iters; it++) {
         if (pos + batch > n) pos = 0;
@@ -1377,9 +1415,8 @@ int mte_mlp_train(mte_engine *e, const float *features, const float *labels, int
         pos += batch;
     }
     HIPCHK(launch_mlp_pack(e));
-    if (losses && iters > 0)
-        HIPCHK(hipMemcpyAsync(losses, e->mlp.loss, sizeof(double) * iters, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    if (losses && iters > 0) HIPCHK(st.to_host(losses, e->mlp.loss, sizeof(double) * iters));
+    HIPCHK(st.finish());
     return MTE_OK;
 }
 

@@ -174,10 +174,11 @@ struct mte_engine {
     size_t forces_lds = 0;     // > 0: forces by k_forces_lds with this much dynamic LDS
     int rb_traj_threads = 0;   // > 0: list rebuilds by k_rebuild_traj with this workgroup size
     size_t rb_traj_lds = 0;    // and this much dynamic LDS
-    // {overflow, frozen} copied by k_publish_flags at the end of a run into
+    // {overflow, frozen, TEA status} copied by k_publish_flags at the end of a run into
     // pinned, device-mapped host memory, so that the run's one stream
     // synchronisation also delivers them (flags_dev is its device address).
     int *flags_host = nullptr, *flags_dev = nullptr;
+    bool stage_user = false;         // counted among the staging pool's engines
     mte::TeaBuffers tea;
     mte::CellTables cells;
     bool use_cells = false;

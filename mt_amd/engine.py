@@ -192,7 +192,7 @@ class Engine:
         self._chk(self.lib.mte_set_state(self.h, _p(c)))
 
     def get_state(self):
-        c = np.zeros((self.nb, 7), np.float32)
+        c = np.empty((self.nb, 7), np.float32)
         self._chk(self.lib.mte_get_state(self.h, _p(c)))
         return c
 
@@ -319,19 +319,19 @@ class Engine:
         self._chk(self.lib.mte_mlp_set_weights(self.h, _p(w), w.size))
 
     def mlp_get_weights(self):
-        w = np.zeros(MLP_NPARAM, np.float32)
+        w = np.empty(MLP_NPARAM, np.float32)
         self._chk(self.lib.mte_mlp_get_weights(self.h, _p(w), w.size))
         return w
 
     def mlp_local(self):
-        f = np.zeros((self.nb, MLP_IN), np.float32)
-        t = np.zeros((self.nb, MLP_OUT), np.float32)
+        f = np.empty((self.nb, MLP_IN), np.float32)
+        t = np.empty((self.nb, MLP_OUT), np.float32)
         self._chk(self.lib.mte_mlp_local(self.h, _p(f), _p(t)))
         return f, t
 
     def mlp_forward(self, feat):
         x = np.ascontiguousarray(feat, np.float32)
-        out = np.zeros((len(x), MLP_OUT), np.float32)
+        out = np.empty((len(x), MLP_OUT), np.float32)
         self._chk(self.lib.mte_mlp_forward(self.h, _p(x), len(x), _p(out)))
         return out
 
@@ -347,7 +347,7 @@ class Engine:
         x = np.ascontiguousarray(feat, np.float32)
         t = np.ascontiguousarray(targ, np.float32)
         loss = ctypes.c_double()
-        g = np.zeros(MLP_NPARAM, np.float32)
+        g = np.empty(MLP_NPARAM, np.float32)
         self._chk(self.lib.mte_mlp_loss_grad(self.h, _p(x), _p(t), len(x), ctypes.byref(loss), _p(g)))
         return loss.value, g
 
