@@ -121,8 +121,64 @@ struct GlobalLists {
     __device__ __forceinline__ int lat(int k) const { return T.lat[k * T.nb + b]; }
     __device__ __forceinline__ uint32_t handle(int j) const { return origin + (uint32_t)((j - base) * SCALE); }
     __device__ __forceinline__ uint32_t ref(int e) const { return handle(ent_j(e)); }
-    __device__ __forceinline__ int nlj() const { return T.lj_n[b]; }
-    __device__ __forceinline__ uint32_t lj(int k) const { return handle(T.lj[k * T.nb + b]); }
+    // The LJ entries in order: four(h0, h1, h2, h3) for each four of them,
+    // one(h) for each of the rest.
+    template <class Four, class One>
+    __device__ __forceinline__ void lj(const Four &four, const One &one) const {
+        const int n = T.lj_n[b];
+        auto at = [&](int k) { return handle(T.lj[(size_t)k * T.nb + b]); };
+        int k = 0;
+        for (; k + 4 <= n; k += 4) four(at(k), at(k + 1), at(k + 2), at(k + 3));
+        for (; k < n; k++) one(at(k));
+    }
+};
+
+// The same lists, for one force evaluation: what most beads need (the counts,
+// one longitudinal, two lateral and the first LJ entries) is requested at
+// once when the lists are made, before the bead's state.  Read where they are
+// used, each count and entry is one more trip to memory that nothing overlaps
+// (64 tubes of 1040 beads: k_forces_lds 14.6 -> 12.5 us, one tube of 312 beads
+// 7.7 -> 5.7, 4 periodic systems of 122646 beads: k_step_plain 11.1 -> 10.1).
+// Slots beyond a count hold no entry but exist.
+constexpr int LJ_AHEAD = 4;
+template <int SCALE>
+struct AheadLists {
+    const DevTopo &T;
+    int b, base;
+    uint32_t origin;
+    int eh, cl, ct, cj, elon, elat0, elat1, elj[LJ_AHEAD];
+    __device__ __forceinline__ AheadLists(const DevTopo &T, int b, int base, uint32_t origin)
+        : T(T), b(b), base(base), origin(origin), eh(T.harm[b]), cl(T.lon_n[b]), ct(T.lat_n[b]), cj(T.lj_n[b]),
+          elon(T.lon[b]), elat0(T.lat[b]), elat1(T.lat[T.nb + b]) {
+#pragma unroll
+        for (int u = 0; u < LJ_AHEAD; u++) elj[u] = T.lj[(size_t)min(u, T.max_lj - 1) * T.nb + b];
+    }
+    __device__ __forceinline__ int harm() const { return eh; }
+    __device__ __forceinline__ int nlon() const { return cl; }
+    __device__ __forceinline__ int lon(int k) const { return k == 0 ? elon : T.lon[k * T.nb + b]; }
+    __device__ __forceinline__ int nlat() const { return ct; }
+    __device__ __forceinline__ int lat(int k) const { return k == 0 ? elat0 : k == 1 ? elat1 : T.lat[k * T.nb + b]; }
+    __device__ __forceinline__ uint32_t handle(int j) const { return origin + (uint32_t)((j - base) * SCALE); }
+    __device__ __forceinline__ uint32_t ref(int e) const { return handle(ent_j(e)); }
+    // the next four entries are requested before the current ones' positions
+    template <class Four, class One>
+    __device__ __forceinline__ void lj(const Four &four, const One &one) const {
+        uint32_t h[LJ_AHEAD];
+#pragma unroll
+        for (int u = 0; u < LJ_AHEAD; u++) h[u] = handle(elj[u]);
+        int k = 0;
+        for (; k + LJ_AHEAD <= cj; k += LJ_AHEAD) {
+            int e[LJ_AHEAD];
+#pragma unroll
+            for (int u = 0; u < LJ_AHEAD; u++) e[u] = T.lj[(size_t)min(k + LJ_AHEAD + u, cj - 1) * T.nb + b];
+            four(h[0], h[1], h[2], h[3]);
+#pragma unroll
+            for (int u = 0; u < LJ_AHEAD; u++) h[u] = handle(e[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < LJ_AHEAD - 1; u++)
+            if (k + u < cj) one(h[u]);
+    }
 };
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -187,7 +243,6 @@ __device__ __forceinline__ float below_cut(float r2, float nscale, float offset)
 // not paid per pair when it is off).
 template <bool PERIODIC, bool REG, class Acc, class Lists>
 __device__ __forceinline__ void lj_sum(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I, float3 &F) {
-    const int nlj = Ls.nlj();
     const float nscale = in_vgpr(-0x1p100f), offset = in_vgpr(LJ_CUT * LJ_CUT * 0x1p100f);
     float3 f = make_float3(0.f, 0.f, 0.f);   // without K.lj6, unless REG
     auto pair = [&](float4 xj) {
@@ -203,18 +258,17 @@ __device__ __forceinline__ void lj_sum(const ForceK &K, const Acc &A, const List
         f.y = fmaf(s, d.y, f.y);
         f.z = fmaf(s, d.z, f.z);
     };
-    // four entries and their positions requested before the first is used
-    // (one wait for the four gathers rather than one each), then summed in
-    // list order
-    int k = 0;
-    for (; k + 4 <= nlj; k += 4) {
-        const float4 x0 = A.xyz(Ls.lj(k)), x1 = A.xyz(Ls.lj(k + 1)), x2 = A.xyz(Ls.lj(k + 2)), x3 = A.xyz(Ls.lj(k + 3));
-        pair(x0);
-        pair(x1);
-        pair(x2);
-        pair(x3);
-    }
-    for (; k < nlj; k++) pair(A.xyz(Ls.lj(k)));
+    // four positions requested before the first is used (one wait for the four
+    // gathers rather than one each), then summed in list order
+    Ls.lj(
+        [&](uint32_t h0, uint32_t h1, uint32_t h2, uint32_t h3) {
+            const float4 x0 = A.xyz(h0), x1 = A.xyz(h1), x2 = A.xyz(h2), x3 = A.xyz(h3);
+            pair(x0);
+            pair(x1);
+            pair(x2);
+            pair(x3);
+        },
+        [&](uint32_t h) { pair(A.xyz(h)); });
     const float s6 = REG ? 1.f : K.lj6;
     F = make_float3(fmaf(s6, f.x, F.x), fmaf(s6, f.y, F.y), fmaf(s6, f.z, F.z));
 }
@@ -386,6 +440,29 @@ __device__ __forceinline__ void em_update(const ForceK &K, const float F[6], flo
     x.y += fmaf(K.dtg, F[1], K.vR * rx.y);
     x.z += fmaf(K.dtg, F[2], K.vR * rx.z);
     em_angles(K, F[3], F[4], F[5], ra, a);
+}
+
+// Random-force draw for TEA steps, fused into the force pass: every bead
+// draws sqrt(2 kB T gammaR / dt) xi from its xyz stream
+// (integrateTea_prepare, src/bdhitea_kernel.cu:16-36).
+struct TeaDraw {
+    uint4 *seeds;
+    const float *noise;
+    float4 *R;   // nullptr: no draw
+};
+
+// One bead's share of it.
+__device__ __forceinline__ void tea_draw(const TeaDraw &D, float var, int b, bool extra) {
+    float4 r;
+    if (D.noise) {
+        const float *nz = D.noise + 6 * (size_t)b;
+        r = make_float4(nz[0], nz[1], nz[2], 0.f);
+    } else {
+        uint4 s = D.seeds[b];
+        r = normals4(s);
+        D.seeds[b] = s;
+    }
+    D.R[b] = extra ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
 }
 
 }  // namespace mte

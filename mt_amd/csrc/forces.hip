@@ -72,10 +72,11 @@ __global__ void __launch_bounds__(BS)
         Sout.fp2[b] = Sin.fp2[b];
         return;
     }
+    const AheadLists<1> Ls(T, b, 0, 0);
     Own I = make_own(x, a, Sin.fn[b], Sin.fp1[b], Sin.fp2[b], pack_flags(T, b));
     if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
     float F[6];
-    bead_force<PERIODIC>(K, GlobalAcc{Sin, T}, GlobalLists<1>{T, b, 0, 0}, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
+    bead_force<PERIODIC>(K, GlobalAcc{Sin, T}, Ls, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
     float4 rx, ra;
     if (noise) {
         const float *nz = noise + 6 * (size_t)b;
@@ -99,29 +100,6 @@ __global__ void __launch_bounds__(BS)
     Sout.fp2[b] = p2;
 }
 
-// Random-force draw for TEA steps, fused into the force pass: every bead
-// draws sqrt(2 kB T gammaR / dt) xi from its xyz stream
-// (integrateTea_prepare, src/bdhitea_kernel.cu:16-36).
-struct TeaDraw {
-    uint4 *seeds;
-    const float *noise;
-    float4 *R;   // nullptr: no draw
-};
-
-// One bead's share of it.
-__device__ __forceinline__ void tea_draw(const TeaDraw &D, float var, int b, bool extra) {
-    float4 r;
-    if (D.noise) {
-        const float *nz = D.noise + 6 * (size_t)b;
-        r = make_float4(nz[0], nz[1], nz[2], 0.f);
-    } else {
-        uint4 s = D.seeds[b];
-        r = normals4(s);
-        D.seeds[b] = s;
-    }
-    D.R[b] = extra ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
-}
-
 // Forces (compute_kernel semantics; extra beads get zero), optionally with
 // the TEA random forces.
 template <int BS, bool PERIODIC>
@@ -131,9 +109,10 @@ __global__ void __launch_bounds__(BS)
     if (b >= T.nb) return;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (!T.extra[b]) {
+        const AheadLists<1> Ls(T, b, 0, 0);
         Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b], pack_flags(T, b));
         if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
-        bead_force<PERIODIC>(K, GlobalAcc{S, T}, GlobalLists<1>{T, b, 0, 0}, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
+        bead_force<PERIODIC>(K, GlobalAcc{S, T}, Ls, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
@@ -151,19 +130,19 @@ __global__ void __launch_bounds__(FORCE_TILE)
     const int2 tl = tiles[blockIdx.x];
     const int t = tl.x, base = T.tbase[t], n = T.tsize[t];
     float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n;
+    const LdsAcc A(lx, ln, l1, l2);
+    const int i = tl.y + threadIdx.x, b = base + min(i, n - 1);
+    const AheadLists<LdsAcc::SCALE> Ls(T, b, base, A.origin());
     stage_state(T, S, base, n, lx, ln, l1, l2);
     __syncthreads();
-    const int i = tl.y + threadIdx.x;
     if (i >= n) return;
-    const int b = base + i;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (!T.extra[b]) {
         const float4 fn = ln[i], f1 = l1[i], f2 = l2[i];
         const float4 x = lx[i];
         Own I = make_own(x, make_float4(fn.w, f1.w, f2.w, 0.f), fn, f1, f2, __float_as_int(x.w));
         if (PERIODIC) set_box(I, T.tbox[t]);
-        const LdsAcc A(lx, ln, l1, l2);
-        bead_force<PERIODIC>(K, A, GlobalLists<LdsAcc::SCALE>{T, b, base, A.origin()}, K.is_wall ? T.zs[t] : 0.f, I, F);
+        bead_force<PERIODIC>(K, A, Ls, K.is_wall ? T.zs[t] : 0.f, I, F);
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi

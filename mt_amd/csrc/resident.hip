@@ -93,8 +93,13 @@ struct LdsLists {
     __device__ __forceinline__ int nlat() const { return (cnt >> 5) & 31; }
     __device__ __forceinline__ int lat(int k) const { return at(alat, k); }
     __device__ __forceinline__ uint32_t ref(int e) const { return e & 0xfff0; }
-    __device__ __forceinline__ int nlj() const { return cnt >> 10; }
-    __device__ __forceinline__ uint32_t lj(int k) const { return at(alj, k); }
+    template <class Four, class One>
+    __device__ __forceinline__ void lj(const Four &four, const One &one) const {
+        const int n = cnt >> 10;
+        int k = 0;
+        for (; k + 4 <= n; k += 4) four(at(alj, k), at(alj, k + 1), at(alj, k + 2), at(alj, k + 3));
+        for (; k < n; k++) one(at(alj, k));
+    }
 };
 
 // A bead's state as LDS holds it: position (w: packed flags), rotated offsets
