@@ -250,6 +250,9 @@ hipError_t upload_resident_order(mte_engine *e, const uint8_t *extra);
 int resident_mobile_max(const mte_engine *e, const uint8_t *extra);
 hipError_t launch_tea_pairs(mte_engine *e);
 hipError_t launch_tea_finish(mte_engine *e, const float *noise_step);
+// The end of a step and the forces of the next in one launch.
+bool tea_turn_fits(const mte_engine *e);
+hipError_t launch_tea_turn(mte_engine *e, const float *noise_step, const float *noise_next);
 hipError_t launch_resident(mte_engine *e, int nsteps, const float *noise);
 bool resident_fits(const mte_engine *e, ResidentPlan *plan);
 // Resident plan with `pt` beads per thread; false if the batch cannot use it.

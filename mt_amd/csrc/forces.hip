@@ -10,17 +10,6 @@ namespace mte {
 // engine's tuning (64, 128 or 256).
 constexpr int STREAM_BLOCK = 256;
 
-// Bead of this thread in a grid of 8 x nb8 workgroups (grid_xcd).  The
-// dispatcher hands workgroup k to XCD k mod 8, so workgroup k takes the
-// (k / 8)-th block of the (k mod 8)-th eighth of the beads: each XCD works
-// on a contiguous eighth, whose trajectories' state then stays in that
-// XCD's L2 while their neighbours are gathered.  The bead a thread computes
-// does not change any result.
-__device__ __forceinline__ int xcd_bead(int bs) {
-    const int nb8 = (int)gridDim.x >> 3;
-    return (((int)blockIdx.x & 7) * nb8 + ((int)blockIdx.x >> 3)) * bs + (int)threadIdx.x;
-}
-
 constexpr int FORCE_TILE = 256;   // k_forces_lds: beads per workgroup (the 256-bead tiles of e->tiles)
 
 struct GlobalAcc {
@@ -123,11 +112,17 @@ __global__ void __launch_bounds__(BS)
 // rotated offsets, angles and flags of every bead), one workgroup per
 // 256-bead tile of a trajectory: neighbour data are read from LDS instead of
 // gathered from L2 per pair.  For trajectories that fit (forces_lds_bytes).
+// Bounded by the staging, five times each bead of a 1040-bead trajectory: its
+// tiles go to one XCD, whose L2 then serves all but the first (64 tubes: 12.5
+// -> 9.6 us with the update kernel's beads and the pair units in the same
+// eighths, tea_build_units).
 template <bool PERIODIC>
 __global__ void __launch_bounds__(FORCE_TILE)
-    k_forces_lds(ForceK K, DevTopo T, DevState S, const int2 *tiles, float4 *fxyz, float4 *fang, TeaDraw D) {
+    k_forces_lds(ForceK K, DevTopo T, DevState S, const int2 *tiles, int ntiles, float4 *fxyz, float4 *fang, TeaDraw D) {
     extern __shared__ float4 lds[];
-    const int2 tl = tiles[blockIdx.x];
+    const int tile = xcd_block();   // a trajectory's tiles share one L2
+    if (tile >= ntiles) return;
+    const int2 tl = tiles[tile];
     const int t = tl.x, base = T.tbase[t], n = T.tsize[t];
     float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n;
     const LdsAcc A(lx, ln, l1, l2);
@@ -187,8 +182,6 @@ __global__ void __launch_bounds__(256) k_traj_sum(DevTopo T, const double *en, d
 }
 
 static inline int grid_for(int n, int bs = STREAM_BLOCK) { return (n + bs - 1) / bs; }
-// Grid of a kernel that takes its beads through xcd_bead: a multiple of 8.
-static inline int grid_xcd(int n, int bs) { return 8 * ((grid_for(n, bs) + 7) / 8); }
 
 // The updater's tubule classification (mt_length, src/updater.cpp:164-205)
 // on the device: a bead is on the tubule when rad_lo < sqrt(x^2 + y^2) <
@@ -247,8 +240,8 @@ static hipError_t forces_draw(mte_engine *e, TeaDraw D) {
         const hipError_t s = hipFuncSetAttribute((const void *)k_forces_lds<PERIODIC>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)e->forces_lds);
         if (s != hipSuccess) return s;
-        hipLaunchKernelGGL(k_forces_lds<PERIODIC>, dim3(e->ntiles), dim3(FORCE_TILE), e->forces_lds, e->stream, e->K,
-                           e->T, e->S[e->cur], e->tiles, e->fxyz, e->fang, D);
+        hipLaunchKernelGGL(k_forces_lds<PERIODIC>, dim3(grid_xcd(e->ntiles, 1)), dim3(FORCE_TILE), e->forces_lds,
+                           e->stream, e->K, e->T, e->S[e->cur], e->tiles, e->ntiles, e->fxyz, e->fang, D);
     } else {
         const int bs = e->tune.stream_block;
         const dim3 grid(grid_xcd(e->nb, bs)), block(bs);

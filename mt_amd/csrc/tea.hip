@@ -16,6 +16,7 @@
 // LDS, FP32 partial sums per chunk reduced in fixed order by the finish kernel,
 // which adds the self term and integrates.  Each (i, j) block costs one rsqrt
 // and ~35 FP32 operations: the product is VALU-bound.
+#include "bead_physics.h"
 #include "engine_internal.h"
 #include <type_traits>
 
@@ -779,64 +780,68 @@ __global__ void __launch_bounds__(TEA_TILE)
         pair_chunk<false, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
 }
 
-// Self term, chunk partials in fixed order, and the update of one bead
-// (integrateTea_kernel_unlisted, src/bdhitea_kernel.cu:148-213).
+// What the update of a bead adds up and moves, k_tea_finish and k_tea_turn.
+struct TeaMove {
+    const float4 *fxyz, *fang, *R, *ci;
+    const float *beta;
+    const int *nchunks;
+    int jrun, ioff;
+    const float4 *partial;
+    uint4 *seeds;
+};
+
+// Self term, chunk partials in fixed order, and the update of bead b of
+// trajectory t (integrateTea_kernel_unlisted, src/bdhitea_kernel.cu:148-213).
 // SYM: the partials of k_tea_pairs_sym (planes of x, y, z; the bead's j-side
 // slots, then its i-side slots), else the float4 slots of its trajectory's
 // chunks.
 template <bool SYM>
-__global__ void __launch_bounds__(TEA_TILE)
-    k_tea_finish(ForceK K, DevTopo T, DevState Sin, DevState Sout, const float4 *fxyz, const float4 *fang,
-                 const float4 *R, const float4 *ci, const float *beta, const int *nchunks, int jrun, int ioff,
-                 const float4 *partial4, uint4 *seeds, const float *noise, LatOffsets L) {
-    const int b = blockIdx.x * TEA_TILE + threadIdx.x;
-    if (b >= T.nb) return;
-    const int t = T.tid[b];
-    const float bt = beta[t];
-    const float4 cc = ci[b], Fi = fxyz[b], Ri = R[b];
+__device__ __forceinline__ void tea_move(const ForceK &K, const DevTopo &T, const DevState &Sin, const TeaMove &M,
+                                         const float *noise, const LatOffsets &L, int b, int t, float4 &x, float4 &an,
+                                         float4 &n4, float4 &p1, float4 &p2) {
+    const float bt = M.beta[t];
+    const float4 cc = M.ci[b], Fi = M.fxyz[b], Ri = M.R[b];
     const float w = bt * bt;
     // C_i = 1/sqrt(1 + beta^2 ci) per row (eq. 19)
     const float cx = rsq_fast(1.f + w * cc.x), cy = rsq_fast(1.f + w * cc.y), cz = rsq_fast(1.f + w * cc.z);
     float fx = fmaf(Ri.x, cx, Fi.x), fy = fmaf(Ri.y, cy, Fi.y), fz = fmaf(Ri.z, cz, Fi.z);
     // the bead's state is requested before the partial sums are added
-    float4 x = Sin.xyz[b], an = Sin.ang[b];
+    x = Sin.xyz[b];
+    an = Sin.ang[b];
     const size_t nb = T.nb;
     if (SYM) {
-        const float *part = reinterpret_cast<const float *>(partial4) + b;
+        const float *part = reinterpret_cast<const float *>(M.partial) + b;
         const int chunk = (b - T.tbase[t]) / SYM_CHUNK, nch = (T.tsize[t] + SYM_CHUNK - 1) / SYM_CHUNK;
-        // slots four at a time: twelve loads in flight, then added in order
-        auto add = [&](int c, int end) {
-            for (; c + 4 <= end; c += 4) {
-                float v[4][3];
+        // the j-side slots, then the i-side ones, eight at a time: 24 loads in
+        // flight, then added in order (of a last group, those that exist)
+        const int nj = (chunk + 1) / 2, i0 = M.ioff + (chunk & ~1) / M.jrun;
+        const int ns = nj + (nch - 1) / M.jrun + 1 - (chunk & ~1) / M.jrun;
+        for (int c = 0; c < ns; c += 8) {
+            float v[8][3];
 #pragma unroll
-                for (int u = 0; u < 4; u++)
+            for (int u = 0; u < 8; u++) {
+                const int q = min(c + u, ns - 1);
+                const float *p = part + 3 * (size_t)(q < nj ? q : i0 + q - nj) * nb;
 #pragma unroll
-                    for (int k = 0; k < 3; k++) v[u][k] = part[(3 * (size_t)(c + u) + k) * nb];
+                for (int k = 0; k < 3; k++) v[u][k] = p[k * nb];
+            }
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < 8; u++) {
+                if (c + u < ns) {
                     fx += v[u][0];
                     fy += v[u][1];
                     fz += v[u][2];
                 }
             }
-            for (; c < end; c++) {
-                const float *q = part + 3 * (size_t)c * nb;
-                const float v0 = q[0], v1 = q[nb], v2 = q[2 * nb];
-                fx += v0;
-                fy += v1;
-                fz += v2;
-            }
-        };
-        add(0, (chunk + 1) / 2);
-        add(ioff + (chunk & ~1) / jrun, ioff + (nch - 1) / jrun + 1);
+        }
     } else {
-        const int nc = nchunks[t];
+        const int nc = M.nchunks[t];
         // partials four at a time: four loads in flight, then added in order
         int c = 0;
         for (; c + 4 <= nc; c += 4) {
             float4 pp[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) pp[u] = partial4[(size_t)(c + u) * nb + b];
+            for (int u = 0; u < 4; u++) pp[u] = M.partial[(size_t)(c + u) * nb + b];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 fx += pp[u].x;
@@ -845,7 +850,7 @@ __global__ void __launch_bounds__(TEA_TILE)
             }
         }
         for (; c < nc; c++) {
-            const float4 pp = partial4[(size_t)c * nb + b];
+            const float4 pp = M.partial[(size_t)c * nb + b];
             fx += pp.x;
             fy += pp.y;
             fz += pp.z;
@@ -856,24 +861,85 @@ __global__ void __launch_bounds__(TEA_TILE)
         const float *q = noise + 6 * (size_t)b;
         ra = make_float4(q[3], q[4], q[5], 0.f);
     } else {
-        uint4 s = seeds[b + T.nb];
+        uint4 s = M.seeds[b + T.nb];
         ra = normals4(s);
-        seeds[b + T.nb] = s;
+        M.seeds[b + T.nb] = s;
     }
-    float4 n4 = Sin.fn[b], p1 = Sin.fp1[b], p2 = Sin.fp2[b];
+    n4 = Sin.fn[b];
+    p1 = Sin.fp1[b];
+    p2 = Sin.fp2[b];
     if (!T.fixed[b] && !T.extra[b]) {
         x.x = fmaf(K.dtg, fx, x.x);
         x.y = fmaf(K.dtg, fy, x.y);
         x.z = fmaf(K.dtg, fz, x.z);
-        const float4 fa = fang[b];
+        const float4 fa = M.fang[b];
         em_angles(K, fa.x, fa.y, fa.z, ra, an);
         frame_vectors(an.x, an.y, an.z, L, n4, p1, p2);
     }
-    Sout.xyz[b] = x;
-    Sout.ang[b] = an;
-    Sout.fn[b] = n4;
-    Sout.fp1[b] = p1;
-    Sout.fp2[b] = p2;
+}
+__device__ __forceinline__ void store_bead(const DevState &S, int b, float4 x, float4 an, float4 n4, float4 p1,
+                                           float4 p2) {
+    S.xyz[b] = x;
+    S.ang[b] = an;
+    S.fn[b] = n4;
+    S.fp1[b] = p1;
+    S.fp2[b] = p2;
+}
+
+template <bool SYM>
+__global__ void __launch_bounds__(TEA_TILE)
+    k_tea_finish(ForceK K, DevTopo T, DevState Sin, DevState Sout, TeaMove M, const float *noise, LatOffsets L) {
+    const int b = xcd_bead(TEA_TILE);
+    if (b >= T.nb) return;
+    float4 x, an, n4, p1, p2;
+    tea_move<SYM>(K, T, Sin, M, noise, L, b, T.tid[b], x, an, n4, p1, p2);
+    store_bead(Sout, b, x, an, n4, p1, p2);
+}
+
+// The end of one step and the forces of the next in one launch, a workgroup
+// per trajectory and a thread per bead: each moves its bead and stages it in
+// LDS, then the new forces and random forces are formed from there.  Bounded,
+// as the two kernels it stands for, by trips to memory, not by bytes or
+// operations: it saves a launch, their second reading of every state and the
+// wait between them.  One tube of 312 beads: 7.6 us, for 5.7 of forces and 4.2
+// of update.  The lists are requested before the bead is moved.
+constexpr int TURN_THREADS = 640;
+template <bool PERIODIC>
+__global__ void __launch_bounds__(TURN_THREADS)
+    k_tea_turn(ForceK K, DevTopo T, DevState Sin, DevState Sout, TeaMove M, const float *noise, TeaDraw D,
+               float4 *fxyz, float4 *fang, LatOffsets L) {
+    extern __shared__ float4 lds[];
+    const int t = xcd_block();   // through the L2 that the pair kernel left its partials in
+    if (t >= T.ntraj) return;
+    const int base = T.tbase[t], n = T.tsize[t];
+    float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n;
+    const LdsAcc A(lx, ln, l1, l2);
+    const float wall_z = K.is_wall ? T.zs[t] : 0.f;
+    const int i = threadIdx.x, b = base + min(i, n - 1);
+    const AheadLists<LdsAcc::SCALE> Ls(T, b, base, A.origin());
+    float4 x, an, n4, p1, p2;
+    bool extra = false;
+    if (i < n) {
+        extra = T.extra[b];
+        tea_move<true>(K, T, Sin, M, noise, L, b, t, x, an, n4, p1, p2);
+        store_bead(Sout, b, x, an, n4, p1, p2);
+        x.w = __int_as_float(pack_flags(T, b));
+        lx[i] = x;
+        ln[i] = make_float4(n4.x, n4.y, n4.z, an.x);
+        l1[i] = make_float4(p1.x, p1.y, p1.z, an.y);
+        l2[i] = make_float4(p2.x, p2.y, p2.z, an.z);
+        tea_draw(D, K.vF, b, extra);
+    }
+    __syncthreads();
+    if (i >= n) return;
+    float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (!extra) {
+        Own I = make_own(x, an, n4, p1, p2, __float_as_int(x.w));
+        if (PERIODIC) set_box(I, T.tbox[t]);
+        bead_force<PERIODIC>(K, A, Ls, wall_z, I, F);
+    }
+    fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
+    fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
 }
 
 // ------------------------------------------------------------------ MFMA
@@ -1350,11 +1416,35 @@ hipError_t launch_tea_pairs(mte_engine *e) {
     return hipGetLastError();
 }
 
+static TeaMove tea_move_args(const mte_engine *e) {
+    return TeaMove{e->fxyz, e->fang,    e->tea.R,    e->tea.ci,      e->tea.beta, e->tea.nchunks,
+                   e->tea.jrun, e->tea.ioff, e->tea.partial, e->seeds};
+}
+
 hipError_t launch_tea_finish(mte_engine *e, const float *noise_step) {
     auto kern = e->tea.unit_chunk == MTE_TEA_SYMMETRIC ? k_tea_finish<true> : k_tea_finish<false>;
-    hipLaunchKernelGGL(kern, dim3((e->nb + TEA_TILE - 1) / TEA_TILE), dim3(TEA_TILE), 0, e->stream, e->K, e->T,
-                       e->S[e->cur], e->S[1 - e->cur], e->fxyz, e->fang, e->tea.R, e->tea.ci, e->tea.beta,
-                       e->tea.nchunks, e->tea.jrun, e->tea.ioff, e->tea.partial, e->seeds, noise_step, e->L);
+    hipLaunchKernelGGL(kern, dim3(grid_xcd(e->nb, TEA_TILE)), dim3(TEA_TILE), 0, e->stream, e->K, e->T, e->S[e->cur],
+                       e->S[1 - e->cur], tea_move_args(e), noise_step, e->L);
+    e->cur = 1 - e->cur;
+    return hipGetLastError();
+}
+
+// k_tea_turn serves the symmetric pair kernel's partials, with forces from
+// LDS, for trajectories of up to 640 beads: a workgroup's one bead per thread
+// then costs less than the launch it saves (per 100 steps, two kernels -> one:
+// 1, 8 and 64 tubes of 520 beads 1700 -> 1598, 1754 -> 1593 and 3063 -> 2850
+// us, of 624 beads 1723 -> 1633, 1762 -> 1607 and 3364 -> 3185; of 780 beads
+// 1766 -> 1806, 2012 -> 2040 and 4100 -> 3985: the two keep more CUs busy).
+bool tea_turn_fits(const mte_engine *e) {
+    return e->tea.unit_chunk == MTE_TEA_SYMMETRIC && e->tune.forces == MTE_FORCES_LDS && e->forces_lds > 0 &&
+           e->nmax <= TURN_THREADS;
+}
+
+hipError_t launch_tea_turn(mte_engine *e, const float *noise_step, const float *noise_next) {
+    auto kern = e->periodic ? k_tea_turn<true> : k_tea_turn<false>;
+    hipLaunchKernelGGL(kern, dim3(grid_xcd(e->ntraj, 1)), dim3(((e->nmax + 63) / 64) * 64), e->forces_lds, e->stream,
+                       e->K, e->T, e->S[e->cur], e->S[1 - e->cur], tea_move_args(e), noise_step,
+                       TeaDraw{e->seeds, noise_next, e->tea.R}, e->fxyz, e->fang, e->L);
     e->cur = 1 - e->cur;
     return hipGetLastError();
 }
