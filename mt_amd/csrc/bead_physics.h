@@ -254,10 +254,11 @@ __device__ __forceinline__ float below_cut(float r2, float nscale, float offset)
 // around the accumulation), and runs with and without the regularization cap
 // get separate loops (a uniform choice: the cap's reciprocal square root is
 // not paid per pair when it is off).
+// Without the regularization the sum is to be scaled by K.lj6 (lj_scale).
 template <bool PERIODIC, bool REG, class Acc, class Lists>
-__device__ __forceinline__ void lj_sum(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I, float3 &F) {
+__device__ __forceinline__ float3 lj_sum_as(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I) {
     const float nscale = in_vgpr(-0x1p100f), offset = in_vgpr(LJ_CUT * LJ_CUT * 0x1p100f);
-    float3 f = make_float3(0.f, 0.f, 0.f);   // without K.lj6, unless REG
+    float3 f = make_float3(0.f, 0.f, 0.f);
     auto pair = [&](float4 xj) {
         const float3 d = separation<PERIODIC>(I, xj);
         const float r2 = d.x * d.x + d.y * d.y + d.z * d.z;
@@ -282,14 +283,17 @@ __device__ __forceinline__ void lj_sum(const ForceK &K, const Acc &A, const List
             pair(x3);
         },
         [&](uint32_t h) { pair(A.xyz(h)); });
-    const float s6 = REG ? 1.f : K.lj6;
-    F = make_float3(fmaf(s6, f.x, F.x), fmaf(s6, f.y, F.y), fmaf(s6, f.z, F.z));
+    return f;
 }
-
-// Force and torque on a bead; wall_z is Parameters.zs of its trajectory.
 template <bool PERIODIC, class Acc, class Lists>
-__device__ __forceinline__ void bead_force(const ForceK &K, const Acc &A, const Lists &Ls, float wall_z, const Own &I,
-                                           float F[6]) {
+__device__ __forceinline__ float3 lj_sum(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I) {
+    return K.lj_reg ? lj_sum_as<PERIODIC, true>(K, A, Ls, I) : lj_sum_as<PERIODIC, false>(K, A, Ls, I);
+}
+__device__ __forceinline__ float lj_scale(const ForceK &K) { return K.lj_reg ? 1.f : K.lj6; }
+
+// The bonds of a bead.
+template <bool PERIODIC, class Acc, class Lists>
+__device__ __forceinline__ BondSum bond_forces(const ForceK &K, const Acc &A, const Lists &Ls, const Own &I) {
     BondSum S;
     S.F = S.M = S.Tq = S.bend = make_float3(0.f, 0.f, 0.f);
     const bool gtp = (I.flags & FL_GTP1) != 0, off = K.barrier && (I.flags & FL_OFFTUB) != 0;
@@ -348,11 +352,11 @@ __device__ __forceinline__ void bead_force(const ForceK &K, const Acc &A, const 
         S.F = make_float3(S.F.x + f.x, S.F.y + f.y, S.F.z + f.z);
         S.Tq = cross_add(a, f, S.Tq);
     }
-    // LJ repulsion r^-6 below the hard 6 nm cutoff, :470-495
-    if (K.lj_on) {
-        if (K.lj_reg) lj_sum<PERIODIC, true>(K, A, Ls, I, S.F);
-        else lj_sum<PERIODIC, false>(K, A, Ls, I, S.F);
-    }
+    return S;
+}
+
+// Their force and torque.
+__device__ __forceinline__ void bond_total(const BondSum &S, const Own &I, float F[6]) {
     const float3 t = cross_add(I.n, S.M, S.Tq);
     F[0] = S.F.x;
     F[1] = S.F.y;
@@ -360,19 +364,38 @@ __device__ __forceinline__ void bead_force(const ForceK &K, const Acc &A, const 
     F[3] = fmaf(I.uphi.x, t.x, fmaf(I.uphi.y, t.y, fmaf(I.uphi.z, t.z, S.bend.x)));
     F[4] = fmaf(I.uth.x, t.x, fmaf(I.uth.y, t.y, S.bend.y));
     F[5] = t.z + S.bend.z;
+}
+
+// Adds the LJ sum (:470-495) and the walls; wall_z is Parameters.zs of the
+// bead's trajectory.
+__device__ __forceinline__ void add_lj_walls(const ForceK &K, float3 lj, float wall_z, const float3 r, float F[6]) {
+    if (K.lj_on) {
+        const float s6 = lj_scale(K);
+        F[0] = fmaf(s6, lj.x, F[0]);
+        F[1] = fmaf(s6, lj.y, F[1]);
+        F[2] = fmaf(s6, lj.z, F[2]);
+    }
     // cylindrical and end walls, :497-517
     if (K.is_wall) {
-        const float z = I.r.z, lb = K.wall_left, zt = wall_z + lb;
+        const float z = r.z, lb = K.wall_left, zt = wall_z + lb;
         if (z < lb) F[2] += K.wall_eps * fabsf(z - lb);
         else if (z > zt) F[2] += -K.wall_eps * fabsf(z - zt);
-        const float rad2 = I.r.x * I.r.x + I.r.y * I.r.y;
+        const float rad2 = r.x * r.x + r.y * r.y;
         if (rad2 > K.wall_r * K.wall_r) {
             const float rad = sqrtf(rad2);
             const float coeff = -K.wall_eps * (rad - K.wall_r);
-            F[0] += I.r.x / rad * coeff;
-            F[1] += I.r.y / rad * coeff;
+            F[0] += r.x / rad * coeff;
+            F[1] += r.y / rad * coeff;
         }
     }
+}
+
+template <bool PERIODIC, class Acc, class Lists>
+__device__ __forceinline__ void bead_force(const ForceK &K, const Acc &A, const Lists &Ls, float wall_z, const Own &I,
+                                           float F[6]) {
+    bond_total(bond_forces<PERIODIC>(K, A, Ls, I), I, F);
+    const float3 lj = K.lj_on ? lj_sum<PERIODIC>(K, A, Ls, I) : make_float3(0.f, 0.f, 0.f);
+    add_lj_walls(K, lj, wall_z, I.r, F);
 }
 
 // Energies in the energy_kernel convention (:676-911): U_harm, U_long,

@@ -131,6 +131,7 @@ struct MlpBuffers {
 // Resident-mode launch plan: trajectories grouped by workgroup.
 struct ResidentPlan {
     int threads = 0;        // workgroup size
+    bool helped = false;    // a second thread for every bead (run_steps_helped)
     int per_thread = 0;     // beads per thread
     int max_beads = 0;      // largest trajectory
     size_t lds_bytes = 0;

@@ -74,8 +74,9 @@ __device__ __forceinline__ int pack_counts(int h, int nlon, int nlat, int nlj) {
 // position (LdsAcc's handle), a bond's flag in bit 0.  Made once per launch
 // by threads that keep their bead's state: the harmonic entry itself, and the
 // addresses of the others.
+template <bool HELD>
 struct LdsLists {
-    int eh, cnt;
+    int eh, cnt, elon, elat0, elat1;   // the harmonic entry; HELD: the first longitudinal and two lateral ones
     uint32_t alon, alat, alj;
     __device__ __forceinline__ static int at(uint32_t a, int k) {
         return *(const __attribute__((address_space(3))) uint16_t *)(uintptr_t)(a + 2 * k);
@@ -86,12 +87,15 @@ struct LdsLists {
         alon = a + 2 * (c & 1);
         alat = alon + 2 * nlon();
         alj = alat + 2 * nlat();
+        elon = HELD && nlon() > 0 ? at(alon, 0) : 0;
+        elat0 = HELD && nlat() > 0 ? at(alat, 0) : 0;
+        elat1 = HELD && nlat() > 1 ? at(alat, 1) : 0;
     }
     __device__ __forceinline__ int harm() const { return eh; }
     __device__ __forceinline__ int nlon() const { return (cnt >> 1) & 15; }
-    __device__ __forceinline__ int lon(int k) const { return at(alon, k); }
+    __device__ __forceinline__ int lon(int k) const { return HELD && k == 0 ? elon : at(alon, k); }
     __device__ __forceinline__ int nlat() const { return (cnt >> 5) & 31; }
-    __device__ __forceinline__ int lat(int k) const { return at(alat, k); }
+    __device__ __forceinline__ int lat(int k) const { return HELD && k == 0 ? elat0 : HELD && k == 1 ? elat1 : at(alat, k); }
     __device__ __forceinline__ uint32_t ref(int e) const { return e & 0xfff0; }
     template <class Four, class One>
     __device__ __forceinline__ void lj(const Four &four, const One &one) const {
@@ -241,7 +245,94 @@ __device__ __forceinline__ int run_steps(const ForceK &K0, const DevTopo &T, con
     return nsteps;
 }
 
-template <int PT, int MAXT, bool PERIODIC>
+// The step loop with two waves to each 64 beads: thread t < nmain owns bead
+// W.ib[0] as in run_steps<1, ...>, thread t + nmain helps it.  The helper sums
+// the bead's LJ forces while the owner sums its bonds, and draws its next
+// normals while the owner moves it; both pass through xbuf (per main thread
+// the LJ sum and two pairs of normals by step parity).  The sums are added as
+// run_steps adds them: the same values.  `drawn`: the helper has drawn the
+// normals of step `first` already.
+constexpr int XBUF_F4 = 5;
+template <bool FILTERED, bool PERIODIC, class Lists, class MakeLists>
+__device__ __forceinline__ int run_steps_helped(const ForceK &K0, const DevTopo &T, const LdsAcc &A, int t, float4 *lx,
+                                                float4 *ln, float4 *l1, float4 *l2, Lanes<1> &W, const float *noise,
+                                                int first, int nsteps, const LatOffsets &L0,
+                                                const MakeLists &make_lists, int *flags, float4 *xbuf, int nmain,
+                                                bool drawn) {
+    const int base = T.tbase[t], nb = T.nb;
+    const float box = PERIODIC ? T.tbox[t] : 0.f, ibox = inv_side(box);
+    ForceK K = K0;
+    LatOffsets L = L0;
+    for (float *c : {&K.dtg, &K.vR, &K.fi_h, &K.psi_h, &K.lat_d, &K.seam_d, &L.p1x, &L.p1y, &L.p1z}) *c = in_vgpr(*c);
+    const float wall_z = K.is_wall ? T.zs[t] : 0.f;
+    const bool helper = (int)threadIdx.x >= nmain;   // uniform in a wave
+    const int main_t = threadIdx.x - (helper ? nmain : 0);
+    float4 *xlj = xbuf + main_t, *xrx = xbuf + nmain + main_t, *xra = xbuf + 3 * nmain + main_t;   // normals: + parity nmain
+    const int i = W.ib[0], b = base + i;
+    const bool mob = W.mob[0];
+    const Lists own = make_lists(i, b, mob);
+    BeadState st{};
+    if (mob) st = load_state(A, i);
+    const float3 xr = f3(st.x);
+    auto draw = [&](int s) {
+        xrx[(s & 1) * nmain] = normals4(W.s0[0]);
+        xra[(s & 1) * nmain] = normals4(W.s1[0]);
+    };
+    if (helper && mob && !noise && !drawn) draw(first);
+    for (int s = first; s < nsteps; s++) {
+        float F[6];
+        if (mob) {
+            Own I;
+            if (helper) {
+                if (K.lj_on) {
+                    I.r = f3(lds_f4(A.origin() + i * LdsAcc::SCALE));
+                    I.box = box, I.ibox = ibox;
+                    const float3 f = lj_sum<PERIODIC>(K, A, own, I);
+                    *xlj = make_float4(f.x, f.y, f.z, 0.f);
+                }
+            } else {
+                const float4 a = make_float4(st.n.w, st.p1.w, st.p2.w, 0.f);
+                I = make_own_trig(st.x, a, st.n, st.p1, st.p2, W.trig[0], __float_as_int(st.x.w));
+                if (PERIODIC) I.box = box, I.ibox = ibox;
+                bond_total(bond_forces<PERIODIC>(K, A, own, I), I, F);
+            }
+        }
+        __syncthreads();
+        if (FILTERED && threadIdx.x == 0) flags[(s + 1) & 1] = 0;   // all have read it (after the last step's end)
+        if (mob) {
+            if (helper) {
+                if (!noise && s + 1 < nsteps) draw(s + 1);
+            } else {
+                add_lj_walls(K, f3(*xlj), wall_z, f3(st.x), F);
+                float4 rx, ra;
+                if (noise) {
+                    const float *nz = noise + (size_t)s * 6 * nb + 6 * (size_t)b;
+                    rx = make_float4(nz[0], nz[1], nz[2], 0.f);
+                    ra = make_float4(nz[3], nz[4], nz[5], 0.f);
+                } else {
+                    rx = xrx[(s & 1) * nmain];
+                    ra = xra[(s & 1) * nmain];
+                }
+                float4 x = st.x, a = make_float4(st.n.w, st.p1.w, st.p2.w, 0.f);
+                em_update(K, F, rx, ra, x, a);
+                st = new_state(x, a, L, W.trig[0]);   // x.w keeps the packed flags
+                lx[i] = st.x;
+                ln[i] = st.n;
+                l1[i] = st.p1;
+                l2[i] = st.p2;
+                if (FILTERED) {
+                    const float dx = x.x - xr.x, dy = x.y - xr.y, dz = x.z - xr.z;
+                    if (dx * dx + dy * dy + dz * dz >= SKIN_HALF * SKIN_HALF) flags[s & 1] = 1;
+                }
+            }
+        }
+        __syncthreads();
+        if (FILTERED && flags[s & 1] != 0) return s + 1;   // uniform: every thread reads the same flag
+    }
+    return nsteps;
+}
+
+template <int PT, int MAXT, bool PERIODIC, bool HELPED = false>
 __global__ void __launch_bounds__(MAXT)
     k_resident(ForceK K, float ljpairscutoff, DevTopo T, DevState S, uint4 *seeds, const float *noise, int nsteps, LatOffsets L,
                int stride, int entry_cap, const int *order) {
@@ -260,7 +351,11 @@ __global__ void __launch_bounds__(MAXT)
     int *hcnt = hoff + stride;
     int *scan = hcnt + stride;
     int *flags = scan + SCAN_INTS;
-    uint16_t *ent = reinterpret_cast<uint16_t *>(flags + FLAG_INTS);
+    static_assert(!HELPED || PT == 1, "a helper serves one bead");
+    const int nmain = HELPED ? blockDim.x / 2 : blockDim.x;   // threads that own beads
+    const bool helper = HELPED && (int)threadIdx.x >= nmain;
+    float4 *xbuf = reinterpret_cast<float4 *>(flags + FLAG_INTS);
+    uint16_t *ent = reinterpret_cast<uint16_t *>(xbuf + (HELPED ? XBUF_F4 * nmain : 0));
     const int t = blockIdx.x;
     const int base = T.tbase[t], n = T.tsize[t];
     const int nb = T.nb;
@@ -270,7 +365,7 @@ __global__ void __launch_bounds__(MAXT)
     int lcnt[PT];   // its list counts, packed as in hcnt (requested with the bead's state)
 #pragma unroll
     for (int k = 0; k < PT; k++) {
-        const int slot = threadIdx.x + k * blockDim.x;
+        const int slot = (helper ? threadIdx.x - nmain : threadIdx.x) + k * blockDim.x;
         const int i = slot < n ? order[base + slot] : slot;
         W.ib[k] = i;
         const int b = base + i;
@@ -336,7 +431,7 @@ __global__ void __launch_bounds__(MAXT)
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < PT; k++) {
-            if (!W.mob[k]) continue;
+            if (!W.mob[k] || helper) continue;
             const int i = W.ib[k], hc = lcnt[k];
             hcnt[i] = hc;
             hoff[i] = (hc & 1) + ((hc >> 1) & 15) + ((hc >> 5) & 31) + (hc >> 10);
@@ -387,7 +482,7 @@ __global__ void __launch_bounds__(MAXT)
     auto fill = [&](float rf2) {
 #pragma unroll
         for (int kk = 0; kk < PT; kk++) {
-            if (!W.mob[kk]) continue;
+            if (!W.mob[kk] || helper) continue;
             const int i = W.ib[kk], b = base + i;
             const int hc = hcnt[i];
             const int h = hc & 1, nlon = (hc >> 1) & 15, nlat = (hc >> 5) & 31;
@@ -447,20 +542,34 @@ __global__ void __launch_bounds__(MAXT)
     if (use_lds) {
         const bool filter = K.lj_on && ljpairscutoff > FILTER_R;
         fill(filter ? FILTER_R * FILTER_R : 0.f);
-        auto mk = [&](int i, int, bool lists) { return LdsLists(ent, lists ? hoff[i] : 0, lists ? hcnt[i] : 0); };
+        using LL = LdsLists<PT == 1>;
+        auto mk = [&](int i, int, bool lists) { return LL(ent, lists ? hoff[i] : 0, lists ? hcnt[i] : 0); };
         int s = 0;
         if (filter) {
-            s = run_steps<PT, true, PERIODIC, LdsLists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk,
-                                              flags, rbuf, own_slot, help_slot);
+            if constexpr (HELPED)
+                s = run_steps_helped<true, PERIODIC, LL>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk, flags,
+                                                         xbuf, nmain, false);
+            else
+                s = run_steps<PT, true, PERIODIC, LL>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk, flags, rbuf,
+                                                      own_slot, help_slot);
             if (s < nsteps) fill(0.f);   // a bead left its skin: the full lists from step s on
         }
-        if (s < nsteps)
-            run_steps<PT, false, PERIODIC, LdsLists>(K, T, A, t, lx, ln, l1, l2, W, noise, s, nsteps, L, mk,
-                                           flags, rbuf, own_slot, help_slot);
+        if (s < nsteps) {
+            if constexpr (HELPED)
+                run_steps_helped<false, PERIODIC, LL>(K, T, A, t, lx, ln, l1, l2, W, noise, s, nsteps, L, mk, flags, xbuf,
+                                                      nmain, s > 0);
+            else
+                run_steps<PT, false, PERIODIC, LL>(K, T, A, t, lx, ln, l1, l2, W, noise, s, nsteps, L, mk, flags, rbuf,
+                                                   own_slot, help_slot);
+        }
     } else {
         using Lists = GlobalLists<LdsAcc::SCALE>;
         auto mk = [&](int, int b, bool) { return Lists{T, b, base, A.origin()}; };
-        run_steps<PT, false, PERIODIC, Lists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk,
+        if constexpr (HELPED)
+            run_steps_helped<false, PERIODIC, Lists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk, flags, xbuf,
+                                                     nmain, false);
+        else
+            run_steps<PT, false, PERIODIC, Lists>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk,
                                           flags, rbuf, own_slot, help_slot);
     }
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -476,7 +585,7 @@ __global__ void __launch_bounds__(MAXT)
     }
 #pragma unroll
     for (int k = 0; k < PT; k++) {
-        if (W.mob[k] && !noise && !(k == 1 && own_slot >= 0)) {   // an offloaded bead's state is the helper's
+        if (W.mob[k] && !noise && (!HELPED || helper) && !(k == 1 && own_slot >= 0)) {   // an offloaded bead's state is the helper's
             const int b = base + W.ib[k];
             seeds[b] = W.s0[k];
             seeds[b + nb] = W.s1[k];
@@ -494,7 +603,14 @@ static size_t fixed_lds_bytes(int nmax) {
 }
 
 // Launch plan with pt beads per thread (pt = 1 allows up to 1024 threads,
-// 2 and 3 up to 768 so the multi-bead kernels keep their registers).
+// 2 and 3 up to 768 so the multi-bead kernels keep their registers).  Where
+// the mobile beads fill at most half the largest workgroup, every bead gets a
+// second thread (run_steps_helped): a wave alone on its SIMD spends 7500
+// cycles on a step, most of them waiting, and the idle half of the workgroup
+// takes the two longest independent parts of it.  Per 100 steps, through the
+// API: 1, 256 and 700 tubes of 312 beads 390 -> 288, 514 -> 422 and 1323 ->
+// 1057 us, 1 and 512 tubes of 520 beads (494 mobile) 370 -> 327 and 1079 ->
+// 1000.
 bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     *plan = ResidentPlan{};
     if (e->P.tea_on || pt < 1 || pt > RES_MAX_PT) return false;
@@ -504,7 +620,9 @@ bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     int lds_limit = 0;
     if (hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device) != hipSuccess)
         return false;
-    const size_t fixed = fixed_lds_bytes(nmax);
+    const int nmain = std::min(((nmax + 63) / 64) * 64, RES_MAX_THREADS / 2);
+    const bool helped = pt == 1 && e->res_mobile_max <= nmain;
+    const size_t fixed = fixed_lds_bytes(nmax) + (helped ? (size_t)XBUF_F4 * sizeof(float4) * nmain : 0);
     if (fixed + (size_t)MIN_ENTRIES_PER_BEAD * 2 * nmax > (size_t)lds_limit) return false;
     int threads = (nmax + pt - 1) / pt;
     threads = ((threads + 63) / 64) * 64;
@@ -516,9 +634,11 @@ bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     // second-pass beads then leave idle waves on the third SIMD for the
     // noise offload.
     if (pt == 2 && nmax > RES_MULTI_THREADS) threads = RES_MULTI_THREADS;
+    if (helped) threads = 2 * nmain;
     if (threads > (pt == 1 ? RES_MAX_THREADS : RES_MULTI_THREADS)) return false;
     plan->threads = threads;
     plan->per_thread = pt;
+    plan->helped = helped;
     plan->max_beads = nmax;
     plan->lds_bytes = (size_t)lds_limit & ~(size_t)15;
     plan->entry_cap = (int)std::min<size_t>((plan->lds_bytes - fixed) / 2, 1u << 30);
@@ -532,13 +652,13 @@ bool resident_fits(const mte_engine *e, ResidentPlan *plan) {
     return false;
 }
 
-template <int PT, int MAXT, bool PERIODIC>
+template <int PT, int MAXT, bool PERIODIC, bool HELPED = false>
 static hipError_t launch_pt(mte_engine *e, int nsteps, const float *noise) {
     const ResidentPlan &pl = e->rplan;
-    hipError_t s = hipFuncSetAttribute((const void *)k_resident<PT, MAXT, PERIODIC>,
+    hipError_t s = hipFuncSetAttribute((const void *)k_resident<PT, MAXT, PERIODIC, HELPED>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
     if (s != hipSuccess) return s;
-    hipLaunchKernelGGL((k_resident<PT, MAXT, PERIODIC>), dim3(e->ntraj), dim3(pl.threads), pl.lds_bytes, e->stream, e->K,
+    hipLaunchKernelGGL((k_resident<PT, MAXT, PERIODIC, HELPED>), dim3(e->ntraj), dim3(pl.threads), pl.lds_bytes, e->stream, e->K,
                        e->P.ljpairscutoff, e->T, e->S[e->cur], e->seeds, noise, nsteps, e->L, pl.max_beads, pl.entry_cap, e->res_order);
     return hipGetLastError();
 }
@@ -546,7 +666,9 @@ static hipError_t launch_pt(mte_engine *e, int nsteps, const float *noise) {
 template <bool PERIODIC>
 static hipError_t launch_box(mte_engine *e, int nsteps, const float *noise) {
     switch (e->rplan.per_thread) {
-    case 1: return launch_pt<1, RES_MAX_THREADS, PERIODIC>(e, nsteps, noise);
+    case 1:
+        return e->rplan.helped ? launch_pt<1, RES_MAX_THREADS, PERIODIC, true>(e, nsteps, noise)
+                               : launch_pt<1, RES_MAX_THREADS, PERIODIC>(e, nsteps, noise);
     case 2: return launch_pt<2, RES_MULTI_THREADS, PERIODIC>(e, nsteps, noise);
     case 3: return launch_pt<3, RES_MULTI_THREADS, PERIODIC>(e, nsteps, noise);
     default: return hipErrorInvalidValue;

@@ -1,0 +1,43 @@
+"""The resident kernel with a second thread for every bead (at most 512 mobile
+beads per trajectory) against two beads per thread, bit for bit: the helper
+only sums and draws what the owner would, and the sums are added in the same
+order.  At the edges: one dimer row, a workgroup of whole and of partly filled
+waves, the last size with helpers and the first without (494 and 520 mobile
+beads), several lengths in a batch, open and periodic; drawn noise (the same
+final streams), and injected noise with a bead thrown out of its skin in the
+middle and at the last step, so that the lists are refilled."""
+import numpy as np
+import pytest
+
+from mt_amd.engine import Engine, MODE_RESIDENT
+from tests.helpers import base_params, noise, uneven_batch
+
+pytestmark = pytest.mark.gpu
+NSTEPS = 60
+
+
+def _run(b, pt, nz):
+    eng = Engine(base_params(), b.copy(), max_lj=64, mode=MODE_RESIDENT)
+    eng.set_tuning(resident_per_thread=pt)
+    if nz is not None:
+        eng.set_noise(nz)
+    eng.run(NSTEPS)
+    out = eng.get_state(), eng.get_rng().copy()
+    eng.close()
+    return out
+
+
+@pytest.mark.parametrize("lengths,side", [((1,), 0.0), ((12,), 0.0), ((20,), 0.0), ((21,), 0.0),
+                                          ((19, 2, 7), 0.0), ((12, 5), 200.0)])
+@pytest.mark.parametrize("kick", [None, 30, NSTEPS - 1])
+def test_helped_equals_two_per_thread(lengths, side, kick):
+    print(f"case helped resident steps, lengths {lengths}, side {side}, kick {kick}", flush=True)
+    b = uneven_batch(lengths=lengths, n_free=(0,) * len(lengths))
+    b.box = np.full(len(lengths), side, np.float32)
+    nz = None
+    if kick is not None:
+        nz = noise(np.random.default_rng(9), NSTEPS, b.nb)
+        nz[kick, b.nb // 2, 0] += 70.0   # about 1 nm (varR is 0.0149 nm)
+    got, want = _run(b, 1, nz), _run(b, 2, nz)
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(got[0], want[0])
