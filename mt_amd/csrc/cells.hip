@@ -6,9 +6,7 @@
 // :913-940), O(N^2) per trajectory.  Here the rebuild is:
 //   1. assign: cell coordinates floor(x / cs) per bead (wrapped in periodic
 //      boxes), hashed into a per-trajectory table of 2^k buckets; count;
-//   2. scan: one exclusive scan over the buckets of all trajectories (whose
-//      tables and beads are both laid out trajectory after trajectory)
-//      turns bucket counts into first slots;
+//   2. ranges: every bucket gets as many consecutive slots as it has beads;
 //   3. scatter: beads into bucket order (counting sort), with their
 //      positions copied into that order for the searches;
 //   4. search: each bead visits the 27 neighbouring cells, keeps the beads of
@@ -31,14 +29,16 @@ __device__ __forceinline__ int3 cell_of(float3 r, float box, const CellGeom &g) 
     return make_int3((int)floorf(x), (int)floorf(y), (int)floorf(z));
 }
 
-// The bead's slot within its bucket comes from one atomic per bucket and
-// wave: the wave's lanes are grouped by bucket (one round per distinct
-// bucket, scalar work), each group's first lane adds the group's size, and
-// the lanes of a group take consecutive slots from the returned count.
-// Neighbouring beads of a microtubule share cells, so most of a wave's
-// lanes fall in a few buckets.  The order of the beads within a bucket is
-// not fixed (nor was it with one atomic per bead); every user of the tables
-// orders what it finds there by bead index or by distance.
+// The bead's slot within its bucket comes from the atomic that counts it.
+// Neighbouring beads of a microtubule share cells: while the first lane left
+// has at least ASSIGN_GROUP lanes of its bucket, that group takes one atomic,
+// its first lane adding the group's size and its lanes taking consecutive
+// slots from the returned count.  Below that a round costs the wave more than
+// the atomics it saves, but the two monomers of a free dimer, neighbouring
+// lanes, are still joined.  The order of the beads within a bucket is not
+// fixed; every user of the tables orders what it finds there by bead index or
+// by distance.
+constexpr int ASSIGN_GROUP = 8;
 __global__ void __launch_bounds__(256)
     k_cell_assign(DevTopo T, DevState S, CellTables C, float side, int K) {
     const int b = blockIdx.x * 256 + threadIdx.x;
@@ -52,18 +52,27 @@ __global__ void __launch_bounds__(256)
         bucket = C.toff[t] + (int)(cell_hash(c.x, c.y, c.z) & (uint32_t)(C.tsize[t] - 1));
         C.cell[b] = make_int4(c.x, c.y, c.z, bucket);
     }
+    for (int t = b; t < T.ntraj; t += 256 * (int)gridDim.x) C.cursor[CELL_CURSOR_STRIDE * t] = T.tbase[t];   // for k_cell_ranges
     const int lane = threadIdx.x & 63;
-    uint64_t todo = __ballot(valid), group = 0;
+    uint64_t todo = __ballot(valid), group = valid ? 1ull << lane : 0;
     int leader = lane;
     while (todo) {
         const int l0 = __ffsll((unsigned long long)todo) - 1;
         const int kb = __builtin_amdgcn_readlane(bucket, l0);
         const uint64_t m = __ballot(valid && bucket == kb);
+        if (__popcll(m) < ASSIGN_GROUP) break;
         if (valid && bucket == kb) {
             leader = l0;
             group = m;
         }
         todo &= ~m;
+    }
+    if ((todo >> lane) & 1) {
+        const int other = __builtin_amdgcn_update_dpp(0, bucket, 0xB1, 0xf, 0xf, true);   // lane ^ 1
+        if (other == bucket && ((todo >> (lane ^ 1)) & 1)) {
+            leader = lane & ~1;
+            group = 3ull << leader;
+        }
     }
     int first = 0;
     if (valid && lane == leader) first = atomicAdd(&C.count[bucket], __popcll(group));
@@ -71,101 +80,64 @@ __global__ void __launch_bounds__(256)
     if (valid) C.rank[b] = first + __popcll(group & ((1ull << lane) - 1ull));
 }
 
-// Exclusive scan of the bucket counts over ALL trajectories at once.  Each
-// trajectory's buckets follow the previous trajectory's, and its beads follow
-// the previous trajectory's beads, so the global prefix of bucket k is
-// directly the first slot of that bucket (tbase[t] + the local prefix).
-// Three passes: per-block sums, a scan of the block sums, the in-block scan.
-constexpr int SCAN_T = 256, SCAN_PER = CELL_SCAN_SPAN / SCAN_T;
-
-__global__ void __launch_bounds__(SCAN_T) k_scan_partial(const int *count, int n, int *bsum) {
-    __shared__ int red[SCAN_T];
-    const int g0 = blockIdx.x * CELL_SCAN_SPAN + threadIdx.x;   // lanes read consecutive buckets
-    int s = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_PER; k++)
-        if (g0 + k * SCAN_T < n) s += count[g0 + k * SCAN_T];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int d = SCAN_T / 2; d > 0; d >>= 1) {
-        if (threadIdx.x < d) red[threadIdx.x] += red[threadIdx.x + d];
-        __syncthreads();
+// Slots of the buckets: each workgroup sums and scans the counts of
+// CELL_SCAN_SPAN buckets in LDS and takes that many slots from the cursor of
+// their trajectory with one atomic (a span of small tables: one for each),
+// so a trajectory's beads hold the slots [tbase, tbase + n).  Which of them a
+// span gets depends on the order the workgroups arrive in; no user of the
+// tables looks beyond a bucket's range.  (A scan over all buckets, in bucket order, took three
+// launches: 17 us for 2^20 buckets, this one
+// 6.)  Bounded by the bytes, 16 per bucket, and by the cursors: atomics on one
+// cache line from all XCDs take about 10 ns each, so a cursor has a line of
+// its own and a span is 4096 buckets (1024: 13.5 us).
+constexpr int SCAN_T = CELL_SCAN_SPAN / 4;   // four buckets to a thread: whole 16-byte loads and stores
+static_assert(CELL_TABLE_MIN % 4 == 0, "the tables, and so the buckets, come in whole fours");
+static_assert(CELL_SCAN_SPAN / CELL_TABLE_MIN + 1 <= SCAN_T, "a thread for each table in a span");
+__global__ void __launch_bounds__(SCAN_T) k_cell_ranges(CellTables C) {
+    __shared__ int wsum[SCAN_T / 64], shift[SCAN_T], first[SCAN_T];   // per table in the span: slot shift, first bucket
+    __shared__ int4 before[SCAN_T + 1];                               // beads of the span before each bucket
+    const int n = C.total, g0 = blockIdx.x * CELL_SCAN_SPAN, g = g0 + 4 * (int)threadIdx.x;
+    const int t0 = C.span_traj[blockIdx.x], nt = C.span_traj[blockIdx.x + 1] - t0 + 1;   // tables that reach into the span
+    int4 v = make_int4(0, 0, 0, 0);
+    if (g < n) {
+        v = *reinterpret_cast<const int4 *>(C.count + g);
+        *reinterpret_cast<int4 *>(C.count + g) = make_int4(0, 0, 0, 0);   // ready for the next build's counting atomics
     }
-    if (threadIdx.x == 0) bsum[blockIdx.x] = red[0];
+    const int s = v.x + v.y + v.z + v.w;
+    // exclusive prefix of the threads' sums: lanes by shuffles, then the waves
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int inc = s;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += u;
+    }
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    int acc = inc - s;
+#pragma unroll
+    for (int w = 0; w < SCAN_T / 64; w++) acc += w < wv ? wsum[w] : 0;
+    const int4 p = make_int4(acc, acc + v.x, acc + v.x + v.y, acc + v.x + v.y + v.z);
+    before[threadIdx.x] = p;
+    if (threadIdx.x == SCAN_T - 1) before[SCAN_T].x = acc + s;
+    __syncthreads();
+    if ((int)threadIdx.x < nt) {
+        const int t = t0 + threadIdx.x;
+        const int lo = max(0, C.toff[t] - g0), hi = min(CELL_SCAN_SPAN, C.toff[t] + C.tsize[t] - g0);
+        const int *bf = reinterpret_cast<const int *>(before);
+        if (lo < hi) shift[threadIdx.x] = atomicAdd(&C.cursor[CELL_CURSOR_STRIDE * t], bf[hi] - bf[lo]) - bf[lo];
+        first[threadIdx.x] = lo;
+    }
+    __syncthreads();
+    if (g >= n) return;
+    int q = 0;   // the table of the thread's four buckets
+    while (q + 1 < nt && first[q + 1] <= 4 * (int)threadIdx.x) q++;
+    const int sh = shift[q];
+    int4 *out = reinterpret_cast<int4 *>(C.range + g);
+    out[0] = make_int4(sh + p.x, v.x, sh + p.y, v.y);
+    out[1] = make_int4(sh + p.z, v.z, sh + p.w, v.w);
 }
 
-// In-place exclusive scan of the nblk block sums (one workgroup).
-__global__ void __launch_bounds__(1024) k_scan_top(int *bsum, int nblk) {
-    __shared__ int part[1024];
-    int carry = 0;
-    for (int c0 = 0; c0 < nblk; c0 += 1024) {
-        const int i = c0 + threadIdx.x;
-        const int v = i < nblk ? bsum[i] : 0;
-        part[threadIdx.x] = v;
-        __syncthreads();
-        for (int d = 1; d < 1024; d <<= 1) {
-            const int u = threadIdx.x >= (unsigned)d ? part[threadIdx.x - d] : 0;
-            __syncthreads();
-            part[threadIdx.x] += u;
-            __syncthreads();
-        }
-        if (i < nblk) bsum[i] = carry + part[threadIdx.x] - v;
-        const int tot = part[1023];
-        __syncthreads();
-        carry += tot;
-    }
-}
-
-// Packed (first slot, count) ranges of the buckets (for the scatter and the
-// searches).  The span's counts pass through LDS
-// so that global loads and stores are coalesced (lane-consecutive buckets)
-// while each thread scans a contiguous run of SCAN_PER; one pad word per 16
-// keeps a run's reads off shared banks.
-__device__ __forceinline__ int scan_pad(int i) { return i + (i >> 4); }
-__global__ void __launch_bounds__(SCAN_T) k_scan_apply(CellTables C) {
-    __shared__ int part[SCAN_T];
-    __shared__ int cnt[CELL_SCAN_SPAN + CELL_SCAN_SPAN / 16], st[CELL_SCAN_SPAN + CELL_SCAN_SPAN / 16];
-    const int n = C.total;
-    const int g0 = blockIdx.x * CELL_SCAN_SPAN;
-#pragma unroll
-    for (int k = 0; k < SCAN_PER; k++) {
-        const int idx = k * SCAN_T + threadIdx.x;
-        cnt[scan_pad(idx)] = g0 + idx < n ? C.count[g0 + idx] : 0;
-        if (g0 + idx < n) C.count[g0 + idx] = 0;   // ready for the next build's counting atomics
-    }
-    __syncthreads();
-    const int run = threadIdx.x * SCAN_PER;
-    int v[SCAN_PER];
-    int s = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_PER; k++) {
-        v[k] = cnt[scan_pad(run + k)];
-        s += v[k];
-    }
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int d = 1; d < SCAN_T; d <<= 1) {
-        const int u = threadIdx.x >= (unsigned)d ? part[threadIdx.x - d] : 0;
-        __syncthreads();
-        part[threadIdx.x] += u;
-        __syncthreads();
-    }
-    int acc = C.bsum[blockIdx.x] + part[threadIdx.x] - s;
-#pragma unroll
-    for (int k = 0; k < SCAN_PER; k++) {
-        st[scan_pad(run + k)] = acc;
-        acc += v[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < SCAN_PER; k++) {
-        const int idx = k * SCAN_T + threadIdx.x;
-        if (g0 + idx < n) C.range[g0 + idx] = make_int2(st[scan_pad(idx)], cnt[scan_pad(idx)]);
-    }
-}
-
-// Counting-sort scatter; also the bucket-ordered positions the searches
-// stream through (w = bead index, bit 31 set for extra beads).
 __global__ void __launch_bounds__(256) k_cell_scatter(DevTopo T, DevState S, CellTables C) {
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= T.nb) return;
@@ -255,12 +227,9 @@ hipError_t build_cells(mte_engine *e, float side, int K) {
     const CellTables &C = e->cells;
     const int gb = (e->nb + 255) / 256;
     // the bucket counts are zero here: set at creation, and cleared by
-    // k_scan_apply once it has read them
+    // k_cell_ranges once it has read them
     hipLaunchKernelGGL(k_cell_assign, dim3(gb), dim3(256), 0, e->stream, e->T, e->S[e->cur], C, side, K);
-    const int nblk = (C.total + CELL_SCAN_SPAN - 1) / CELL_SCAN_SPAN;
-    hipLaunchKernelGGL(k_scan_partial, dim3(nblk), dim3(SCAN_T), 0, e->stream, C.count, C.total, C.bsum);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, e->stream, C.bsum, nblk);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nblk), dim3(SCAN_T), 0, e->stream, C);
+    hipLaunchKernelGGL(k_cell_ranges, dim3((C.total + CELL_SCAN_SPAN - 1) / CELL_SCAN_SPAN), dim3(SCAN_T), 0, e->stream, C);
     hipLaunchKernelGGL(k_cell_scatter, dim3(gb), dim3(256), 0, e->stream, e->T, e->S[e->cur], C);
     return hipGetLastError();
 }

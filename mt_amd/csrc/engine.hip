@@ -658,29 +658,39 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
             std::vector<int> toff(nt), tsz(nt);
             int total = 0;
             for (int t = 0; t < nt; t++) {
-                int s = 64;
+                int s = CELL_TABLE_MIN;
                 while (s < 2 * tsize[t]) s <<= 1;
                 toff[t] = total;
                 tsz[t] = s;
                 total += s;
             }
+            // the first table that reaches into each span of k_cell_ranges;
+            // the entry after the last span, and so the last table of each
+            std::vector<int> span;
+            for (int64_t g = 0, t = 0; g < total; g += CELL_SCAN_SPAN) {
+                while (toff[t] + tsz[t] <= g) t++;
+                span.push_back((int)t);
+            }
+            span.push_back(nt - 1);
             CellTables &C = e->cells;
-            int *p_toff, *p_tsz;
+            int *p_toff, *p_tsz, *p_span;
             if (dalloc(e, &p_toff, nt) != hipSuccess || dalloc(e, &p_tsz, nt) != hipSuccess ||
                 dalloc(e, &C.count, total) != hipSuccess || dalloc(e, &C.rank, nb) != hipSuccess ||
                 dalloc(e, &C.cell, nb) != hipSuccess ||
                 dalloc(e, &C.sorted, nb) != hipSuccess || dalloc(e, &C.range, total) != hipSuccess ||
                 dalloc(e, &C.spos, nb) != hipSuccess ||
-                dalloc(e, &C.bsum, (total + CELL_SCAN_SPAN - 1) / CELL_SCAN_SPAN) != hipSuccess) {
+                dalloc(e, &C.cursor, (size_t)CELL_CURSOR_STRIDE * nt) != hipSuccess || dalloc(e, &p_span, span.size()) != hipSuccess) {
                 e->err = "mte_create: hipMalloc failed for cell tables";
                 return bail(MTE_ERR_HIP);
             }
             C.toff = p_toff;
             C.tsize = p_tsz;
+            C.span_traj = p_span;
             C.total = total;
             if (hipMemsetAsync(C.count, 0, sizeof(int) * (size_t)total, e->stream) != hipSuccess ||
                 hipMemcpyAsync(p_toff, toff.data(), sizeof(int) * nt, hipMemcpyHostToDevice, e->stream) != hipSuccess ||
-                hipMemcpyAsync(p_tsz, tsz.data(), sizeof(int) * nt, hipMemcpyHostToDevice, e->stream) != hipSuccess) {
+                hipMemcpyAsync(p_tsz, tsz.data(), sizeof(int) * nt, hipMemcpyHostToDevice, e->stream) != hipSuccess ||
+                hipMemcpyAsync(p_span, span.data(), sizeof(int) * span.size(), hipMemcpyHostToDevice, e->stream) != hipSuccess) {
                 e->err = "mte_create: upload failed for cell tables";
                 return bail(MTE_ERR_HIP);
             }

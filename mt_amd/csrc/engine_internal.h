@@ -90,11 +90,14 @@ struct CellTables {
     int *rank = nullptr;         // per bead: its place among the beads of its bucket
     int *sorted = nullptr;       // beads in bucket order
     float4 *spos = nullptr;      // per slot: position of the bead there, w = its index (bit 31: extra)
-    int *bsum = nullptr;         // scan partials, one per CELL_SCAN_SPAN buckets
+    int *cursor = nullptr;       // per trajectory: first free slot while ranges are given out
+    const int *span_traj = nullptr;   // first trajectory in each CELL_SCAN_SPAN buckets (and the last one)
     int total = 0;               // buckets over all trajectories
 };
-// Buckets per block of the global bucket scan (cells.hip).
+// Buckets per workgroup of k_cell_ranges (cells.hip).
 constexpr int CELL_SCAN_SPAN = 4096;
+constexpr int CELL_TABLE_MIN = 64;   // buckets of the smallest table
+constexpr int CELL_CURSOR_STRIDE = 32;   // words between cursors: a cache line each
 
 // MLP-HI network and work buffers (mlp.hip).
 constexpr int MLP_NN = 32, MLP_IN = 96, MLP_H = 128, MLP_OUT = 9;
