@@ -9,12 +9,13 @@
 //   2. ranges: every bucket gets as many consecutive slots as it has beads;
 //   3. scatter: beads into bucket order (counting sort), with their
 //      positions copied into that order for the searches;
-//   4. search: each bead visits the 27 neighbouring cells, keeps the beads of
-//      exactly those cells within the candidate radius, sorts the candidates
-//      by index and runs the reference's per-pair tests on them in that
-//      order, so the lists come out identical to the all-pairs scan (same
-//      entries, same order).
-// A hash collision only adds beads that the exact cell check then rejects.
+//   4. search: each bead visits the buckets of the 27 neighbouring cells,
+//      keeps the beads within the candidate radius, sorts the candidates by
+//      index and runs the reference's per-pair tests on them in that order,
+//      so the lists come out identical to the all-pairs scan (same entries,
+//      same order).
+// A hash collision only adds beads that the distance rejects, or that have
+// been met already.
 #include "engine_internal.h"
 #include "rebuild_common.h"
 
@@ -22,6 +23,9 @@ namespace mte {
 
 constexpr int CELL_BLOCK = 64;
 constexpr int CAND_CAP = 128;   // candidates per bead within the candidate radius
+// A lane's buffer: one more, and lanes in banks of their own (an odd number of words).
+template <class JT>
+constexpr int CAND_STRIDE = CAND_CAP + (sizeof(JT) == 2 ? 2 : 1);
 
 __device__ __forceinline__ int3 cell_of(float3 r, float box, const CellGeom &g) {
     const float x = cell_coord(r.x, box, g), y = cell_coord(r.y, box, g), z = cell_coord(r.z, box, g);
@@ -85,11 +89,11 @@ __global__ void __launch_bounds__(256)
 // their trajectory with one atomic (a span of small tables: one for each),
 // so a trajectory's beads hold the slots [tbase, tbase + n).  Which of them a
 // span gets depends on the order the workgroups arrive in; no user of the
-// tables looks beyond a bucket's range.  (A scan over all buckets, in bucket order, took three
-// launches: 17 us for 2^20 buckets, this one
-// 6.)  Bounded by the bytes, 16 per bucket, and by the cursors: atomics on one
-// cache line from all XCDs take about 10 ns each, so a cursor has a line of
-// its own and a span is 4096 buckets (1024: 13.5 us).
+// tables looks beyond a bucket's range.  (A scan over all buckets, in bucket
+// order, took three launches and 17 us for 2^20 buckets, this one 6.)  Bounded
+// by the bytes, 16 per bucket, and by the cursors: atomics on one cache line
+// from all XCDs take about 10 ns each, so a cursor has a line of its own and
+// a span is 4096 buckets (1024: 13.5 us).
 constexpr int SCAN_T = CELL_SCAN_SPAN / 4;   // four buckets to a thread: whole 16-byte loads and stores
 static_assert(CELL_TABLE_MIN % 4 == 0, "the tables, and so the buckets, come in whole fours");
 static_assert(CELL_SCAN_SPAN / CELL_TABLE_MIN + 1 <= SCAN_T, "a thread for each table in a span");
@@ -142,17 +146,20 @@ __global__ void __launch_bounds__(256) k_cell_scatter(DevTopo T, DevState S, Cel
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= T.nb) return;
     const int slot = C.range[C.cell[b].w].x + C.rank[b];
-    C.sorted[slot] = b;
     const float4 x = S.xyz[b];
     C.spos[slot] = make_float4(x.x, x.y, x.z, __int_as_float(b | (T.extra[b] ? (int)0x80000000 : 0)));
 }
-
-// Candidates of bead b: beads of the (2K+1)^3 neighbouring cells (of side
-// >= radius / K) within `radius` (minimum image), as local indices in
-// ascending order.  Returns the count, or -1 when more than CAND_CAP were
-// found.
-__device__ int gather_candidates(const DevTopo &T, const DevState &S, const CellTables &C, int b, float radius,
-                                 int K, int *cand) {
+// Candidates of a bead: the beads of the (2K + 1)^3 cells about it that lie
+// within the radius, in ascending index; -1 if there are more than CAND_CAP.
+// Bounded by trips to memory: a tube's wave, one of few on its CU, visits 27
+// cells of up to a dozen beads.  So the ranges of a plane's cells (K = 2: of a
+// row's) are requested together, then four positions at a time, each with its
+// bead's index.  A bucket that a hash collision shows twice, or one that holds
+// other cells' beads too, needs no cell check: what lies within the radius is
+// a candidate, once.
+template <int K, class JT>
+__device__ __forceinline__ int gather_candidates(const DevTopo &T, const DevState &S, const CellTables &C, int b,
+                                                 float radius, JT *cand) {
     const int t = T.tid[b], base = T.tbase[t];
     const float box = T.tbox[t], ibox = inv_side(box);
     const CellGeom g = cell_geom(box, radius / K, K);
@@ -160,59 +167,79 @@ __device__ int gather_candidates(const DevTopo &T, const DevState &S, const Cell
     const float3 ri = f3(S.xyz[b]);
     const float r2max = radius * radius;
     const uint32_t mask = (uint32_t)(C.tsize[t] - 1);
+    const int toff = C.toff[t];
+    constexpr int W = 2 * K + 1, ROWS = K == 1 ? W : 1, NC = ROWS * W;   // cells whose ranges are requested together
     int n = 0;
-    for (int dz = -K; dz <= K; dz++)
-        for (int dy = -K; dy <= K; dy++)
-            for (int dx = -K; dx <= K; dx++) {
-                int cx = me.x + dx, cy = me.y + dy, cz = me.z + dz;
-                if (g.dims > 0) {
-                    cx = wrap_cell(cx, g.dims);
-                    cy = wrap_cell(cy, g.dims);
-                    cz = wrap_cell(cz, g.dims);
-                }
-                const int bucket = C.toff[t] + (int)(cell_hash(cx, cy, cz) & mask);
-                const int2 rg = C.range[bucket];
-                const int s0 = rg.x, s1 = rg.x + rg.y;
-                for (int q = s0; q < s1; q++) {
-                    const int j = C.sorted[q];
-                    if (j == b) continue;
-                    const int4 cj = C.cell[j];
-                    if (cj.x != cx || cj.y != cy || cj.z != cz) continue;
-                    const float3 d = min_image_pre(sub3(ri, f3(S.xyz[j])), box, ibox);
-                    if (d.x * d.x + d.y * d.y + d.z * d.z >= r2max) continue;
-                    if (n >= CAND_CAP) return -1;
-                    // insertion keeps the candidates sorted by index
-                    int k = n++;
-                    const int lj = j - base;
-                    while (k > 0 && cand[k - 1] > lj) {
-                        cand[k] = cand[k - 1];
-                        k--;
-                    }
-                    cand[k] = lj;
-                }
+    bool over = false;
+    auto test = [&](float4 pj) {
+        const int j = __float_as_int(pj.w) & 0x7fffffff;
+        const float3 d = min_image_pre(sub3(ri, f3(pj)), box, ibox);
+        if (j == b || d.x * d.x + d.y * d.y + d.z * d.z >= r2max || over) return;
+        // insertion keeps the candidates sorted by index, each once
+        const int lj = j - base;
+        int k = n;
+        for (; k > 0 && (int)cand[k - 1] > lj; k--) cand[k] = cand[k - 1];
+        if (k > 0 && (int)cand[k - 1] == lj) {
+            for (; k < n; k++) cand[k] = cand[k + 1];
+        } else {
+            cand[k] = (JT)lj;
+            over = ++n > CAND_CAP;
+        }
+    };
+    for (int r0 = 0; r0 < W * W; r0 += ROWS) {
+        int2 rg[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int r = r0 + c / W;
+            int cx = me.x + c % W - K, cy = me.y + r % W - K, cz = me.z + r / W - K;
+            if (g.dims > 0) {
+                cx = wrap_cell(cx, g.dims);
+                cy = wrap_cell(cy, g.dims);
+                cz = wrap_cell(cz, g.dims);
             }
-    return n;
+            rg[c] = C.range[toff + (int)(cell_hash(cx, cy, cz) & mask)];
+        }
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            for (int q = 0; q < rg[c].y; q += 4) {
+                float4 p[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) p[u] = C.spos[rg[c].x + min(q + u, rg[c].y - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (q + u < rg[c].y) test(p[u]);
+            }
+        }
+    }
+    return over ? -1 : n;
 }
 
+template <int K, class JT>
 __global__ void __launch_bounds__(CELL_BLOCK)
-    k_rebuild_cells(mte_params P, DevTopo T, DevState S, CellTables C, float radius, int K, int do_lj,
-                    int do_bonded) {
-    __shared__ int cand_all[CELL_BLOCK * CAND_CAP];
+    k_rebuild_cells(mte_params P, DevTopo T, DevState S, CellTables C, float radius, int do_lj, int do_bonded) {
+    __shared__ JT cand_all[CELL_BLOCK * CAND_STRIDE<JT>];
     const int b = blockIdx.x * CELL_BLOCK + threadIdx.x;
     if (b >= T.nb) return;
     const int t = T.tid[b], base = T.tbase[t];
     RebuildOwn o = rebuild_own(S.xyz[b], S.fn[b], S.fp1[b], S.fp2[b], T.mon_type[b], T.harm_raw[b], b - base, b,
                                base, T.tbox[t]);
     if (!T.extra[b]) {
-        int *cand = cand_all + threadIdx.x * CAND_CAP;
-        const int n = gather_candidates(T, S, C, b, radius, K, cand);
+        JT *cand = cand_all + threadIdx.x * CAND_STRIDE<JT>;
+        const int n = gather_candidates<K>(T, S, C, b, radius, cand);
         if (n < 0) {
             o.ovf = 1;
-        } else {
+        } else if (n > 0) {
+            // the next candidate's data are requested before the current one's tests
+            auto bead = [&](int k) { return base + (int)cand[min(k, n - 1)]; };
+            int j = bead(0);
+            float4 x = S.xyz[j], fn = S.fn[j], f1 = S.fp1[j], f2 = S.fp2[j];
+            int mt = T.mon_type[j];
             for (int k = 0; k < n; k++) {
-                const int j = base + cand[k];
-                rebuild_pair(T, o, cand[k], S.xyz[j], S.fn[j], S.fp1[j], S.fp2[j], T.mon_type[j], P.ljpairscutoff,
-                             do_lj, do_bonded);
+                const int jn = bead(k + 1);
+                const float4 xn = S.xyz[jn], fnn = S.fn[jn], f1n = S.fp1[jn], f2n = S.fp2[jn];
+                const int mtn = T.mon_type[jn];
+                rebuild_pair(T, o, j - base, x, fn, f1, f2, mt, P.ljpairscutoff, do_lj, do_bonded);
+                j = jn, x = xn, fn = fnn, f1 = f1n, f2 = f2n, mt = mtn;
             }
         }
     }
@@ -242,8 +269,12 @@ hipError_t launch_rebuild_cells(mte_engine *e) {
     const int K = e->tune.cell_stencil == 2 ? 2 : 1;
     hipError_t s = build_cells(e, radius / K, K);
     if (s != hipSuccess) return s;
-    hipLaunchKernelGGL(k_rebuild_cells, dim3((e->nb + CELL_BLOCK - 1) / CELL_BLOCK), dim3(CELL_BLOCK), 0, e->stream,
-                       e->P, e->T, e->S[e->cur], e->cells, radius, K, do_lj, do_bonded);
+    // 16-bit candidates where a trajectory's indices fit: half the LDS, twice the waves on a CU
+    const bool small = e->nmax <= 65536;
+    auto kern = K == 2 ? (small ? k_rebuild_cells<2, uint16_t> : k_rebuild_cells<2, int>)
+                       : (small ? k_rebuild_cells<1, uint16_t> : k_rebuild_cells<1, int>);
+    hipLaunchKernelGGL(kern, dim3((e->nb + CELL_BLOCK - 1) / CELL_BLOCK), dim3(CELL_BLOCK), 0, e->stream, e->P, e->T,
+                       e->S[e->cur], e->cells, radius, do_lj, do_bonded);
     return hipGetLastError();
 }
 

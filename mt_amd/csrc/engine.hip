@@ -677,7 +677,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
             if (dalloc(e, &p_toff, nt) != hipSuccess || dalloc(e, &p_tsz, nt) != hipSuccess ||
                 dalloc(e, &C.count, total) != hipSuccess || dalloc(e, &C.rank, nb) != hipSuccess ||
                 dalloc(e, &C.cell, nb) != hipSuccess ||
-                dalloc(e, &C.sorted, nb) != hipSuccess || dalloc(e, &C.range, total) != hipSuccess ||
+                dalloc(e, &C.range, total) != hipSuccess ||
                 dalloc(e, &C.spos, nb) != hipSuccess ||
                 dalloc(e, &C.cursor, (size_t)CELL_CURSOR_STRIDE * nt) != hipSuccess || dalloc(e, &p_span, span.size()) != hipSuccess) {
                 e->err = "mte_create: hipMalloc failed for cell tables";

@@ -88,7 +88,6 @@ struct CellTables {
     int2 *range = nullptr;       // per bucket: first slot, bead count
     int4 *cell = nullptr;        // per bead: cell coordinates, bucket
     int *rank = nullptr;         // per bead: its place among the beads of its bucket
-    int *sorted = nullptr;       // beads in bucket order
     float4 *spos = nullptr;      // per slot: position of the bead there, w = its index (bit 31: extra)
     int *cursor = nullptr;       // per trajectory: first free slot while ranges are given out
     const int *span_traj = nullptr;   // first trajectory in each CELL_SCAN_SPAN buckets (and the last one)
