@@ -156,7 +156,10 @@ __global__ void __launch_bounds__(256) k_cell_scatter(DevTopo T, DevState S, Cel
 // row's) are requested together, then four positions at a time, each with its
 // bead's index.  A bucket that a hash collision shows twice, or one that holds
 // other cells' beads too, needs no cell check: what lies within the radius is
-// a candidate, once.
+// a candidate (met twice, it stands there twice, side by side once sorted, and
+// the caller takes it once).  Up to 32 are sorted in registers.  4 periodic
+// systems of 122646 beads: 188 us with three gathers per bead and an insertion
+// sort in LDS, 108 with the requests together, 61 with the sort.
 template <int K, class JT>
 __device__ __forceinline__ int gather_candidates(const DevTopo &T, const DevState &S, const CellTables &C, int b,
                                                  float radius, JT *cand) {
@@ -171,19 +174,27 @@ __device__ __forceinline__ int gather_candidates(const DevTopo &T, const DevStat
     constexpr int W = 2 * K + 1, ROWS = K == 1 ? W : 1, NC = ROWS * W;   // cells whose ranges are requested together
     int n = 0;
     bool over = false;
+    // the n entries of the buffer in ascending order, each once; their number
+    auto ordered = [](JT *cand, int n) {
+        for (int i = 1; i < n; i++) {
+            const JT v = cand[i];
+            int k = i;
+            for (; k > 0 && cand[k - 1] > v; k--) cand[k] = cand[k - 1];
+            cand[k] = v;
+        }
+        int m = 0;
+        for (int i = 0; i < n; i++)
+            if (m == 0 || cand[i] != cand[m - 1]) cand[m++] = cand[i];
+        return m;
+    };
     auto test = [&](float4 pj) {
         const int j = __float_as_int(pj.w) & 0x7fffffff;
         const float3 d = min_image_pre(sub3(ri, f3(pj)), box, ibox);
         if (j == b || d.x * d.x + d.y * d.y + d.z * d.z >= r2max || over) return;
-        // insertion keeps the candidates sorted by index, each once
-        const int lj = j - base;
-        int k = n;
-        for (; k > 0 && (int)cand[k - 1] > lj; k--) cand[k] = cand[k - 1];
-        if (k > 0 && (int)cand[k - 1] == lj) {
-            for (; k < n; k++) cand[k] = cand[k + 1];
-        } else {
-            cand[k] = (JT)lj;
-            over = ++n > CAND_CAP;
+        cand[n++] = (JT)(j - base);
+        if (n > CAND_CAP) {   // full: too many, unless some have been met twice
+            n = ordered(cand, n);
+            over = n > CAND_CAP;
         }
     };
     for (int r0 = 0; r0 < W * W; r0 += ROWS) {
@@ -211,7 +222,10 @@ __device__ __forceinline__ int gather_candidates(const DevTopo &T, const DevStat
             }
         }
     }
-    return over ? -1 : n;
+    if (over) return -1;
+    if (n > SORT_W) return ordered(cand, n);
+    sort_cands<SORT_W>(cand, 1, n);
+    return n;
 }
 
 template <int K, class JT>
@@ -238,6 +252,7 @@ __global__ void __launch_bounds__(CELL_BLOCK)
                 const int jn = bead(k + 1);
                 const float4 xn = S.xyz[jn], fnn = S.fn[jn], f1n = S.fp1[jn], f2n = S.fp2[jn];
                 const int mtn = T.mon_type[jn];
+                if (k + 1 < n && jn == j) continue;   // met twice: once more in the next turn
                 rebuild_pair(T, o, j - base, x, fn, f1, f2, mt, P.ljpairscutoff, do_lj, do_bonded);
                 j = jn, x = xn, fn = fnn, f1 = f1n, f2 = f2n, mt = mtn;
             }

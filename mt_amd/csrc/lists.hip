@@ -283,34 +283,6 @@ __device__ __forceinline__ void scan_cands(const float4 *sm, const float4 *glo, 
     }
 }
 
-// The lane's nc <= TRAJ_CAND candidates in ascending order: a bitonic
-// network over SORT_W registers (padding sorts last), with no dependent LDS
-// accesses.
-constexpr int SORT_W = 32;
-static_assert(TRAJ_CAND <= SORT_W, "the sorting network covers the candidate buffer");
-__device__ __forceinline__ void sort_cands(uint16_t *mine, int stride, int nc) {
-    uint32_t v[SORT_W];
-#pragma unroll
-    for (int q = 0; q < SORT_W; q++) v[q] = (q < TRAJ_CAND && q < nc) ? mine[q * stride] : 0xffffu;
-#pragma unroll
-    for (int k = 2; k <= SORT_W; k <<= 1)
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1)
-#pragma unroll
-            for (int i = 0; i < SORT_W; i++) {
-                const int l = i ^ j;
-                if (l > i) {
-                    const uint32_t a = min(v[i], v[l]), b = max(v[i], v[l]);
-                    const bool up = (i & k) == 0;
-                    v[i] = up ? a : b;
-                    v[l] = up ? b : a;
-                }
-            }
-#pragma unroll
-    for (int q = 0; q < TRAJ_CAND; q++)
-        if (q < nc) mine[q * stride] = (uint16_t)v[q];
-}
-
 // The same rebuild with one workgroup per trajectory and the whole
 // trajectory in LDS (positions, rotated offsets, monomer types, a uint16
 // candidate buffer per lane), used when the largest trajectory fits
@@ -367,7 +339,7 @@ __global__ void __launch_bounds__(TRAJ_THREADS)
                     rebuild_pair(T, o, jj, sx[jj], float4{}, float4{}, float4{}, 0, P.ljpairscutoff, do_lj, false);
             };
             if (nc <= TRAJ_CAND) {
-                sort_cands(mine, stride, nc);
+                sort_cands<TRAJ_CAND>(mine, stride, nc);
                 for (int q = 0; q < nc; q++) pair(mine[q * stride]);
             } else {
                 for (int jj = 0; jj < n; jj++) {

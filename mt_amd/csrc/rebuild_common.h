@@ -121,4 +121,32 @@ __device__ __forceinline__ void rebuild_finish(const DevTopo &T, const RebuildOw
     if (o.ovf) atomicOr(T.overflow, 1);
 }
 
+// The lane's nc <= CAP candidates in ascending order: a bitonic network over
+// SORT_W registers (padding sorts last), with no dependent LDS accesses.
+constexpr int SORT_W = 32;
+template <int CAP, class CandT>
+__device__ __forceinline__ void sort_cands(CandT *mine, int stride, int nc) {
+    static_assert(CAP <= SORT_W, "the sorting network covers the candidates");
+    uint32_t v[SORT_W];
+#pragma unroll
+    for (int q = 0; q < SORT_W; q++) v[q] = (q < CAP && q < nc) ? (uint32_t)mine[q * stride] : 0xffffffffu;
+#pragma unroll
+    for (int k = 2; k <= SORT_W; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+            for (int i = 0; i < SORT_W; i++) {
+                const int l = i ^ j;
+                if (l > i) {
+                    const uint32_t a = min(v[i], v[l]), b = max(v[i], v[l]);
+                    const bool up = (i & k) == 0;
+                    v[i] = up ? a : b;
+                    v[l] = up ? b : a;
+                }
+            }
+#pragma unroll
+    for (int q = 0; q < CAP; q++)
+        if (q < nc) mine[q * stride] = (CandT)v[q];
+}
+
 }  // namespace mte
