@@ -11,19 +11,6 @@ namespace mte {
 
 __device__ __forceinline__ float3 scale3(float s, float3 v) { return make_float3(s * v.x, s * v.y, s * v.z); }
 
-// Bead of this thread in a grid of 8 x nb8 workgroups (grid_xcd).  The
-// dispatcher hands workgroup k to XCD k mod 8, so workgroup k takes the
-// (k / 8)-th block of the (k mod 8)-th eighth of the beads: each XCD works
-// on a contiguous eighth, whose trajectories' state then stays in that
-// XCD's L2 while their neighbours are gathered.  The bead a thread computes
-// does not change any result.
-__device__ __forceinline__ int xcd_block() {
-    return ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
-}
-__device__ __forceinline__ int xcd_bead(int bs) { return xcd_block() * bs + (int)threadIdx.x; }
-// The grid of such a kernel over n items, bs to a workgroup: a multiple of 8.
-inline int grid_xcd(int n, int bs) { return 8 * (((n + bs - 1) / bs + 7) / 8); }
-
 // Own-bead quantities needed for the angular gradients.
 struct Own {
     float3 r, n, a1, a2, uphi;

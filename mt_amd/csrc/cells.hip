@@ -45,7 +45,7 @@ __device__ __forceinline__ int3 cell_of(float3 r, float box, const CellGeom &g) 
 constexpr int ASSIGN_GROUP = 8;
 __global__ void __launch_bounds__(256)
     k_cell_assign(DevTopo T, DevState S, CellTables C, float side, int K) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
+    const int b = xcd_bead(256);
     const bool valid = b < T.nb;
     int bucket = -1;
     if (valid) {
@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(256)
         bucket = C.toff[t] + (int)(cell_hash(c.x, c.y, c.z) & (uint32_t)(C.tsize[t] - 1));
         C.cell[b] = make_int4(c.x, c.y, c.z, bucket);
     }
-    for (int t = b; t < T.ntraj; t += 256 * (int)gridDim.x) C.cursor[CELL_CURSOR_STRIDE * t] = T.tbase[t];   // for k_cell_ranges
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < T.ntraj; t += 256 * (int)gridDim.x) C.cursor[CELL_CURSOR_STRIDE * t] = T.tbase[t];   // for k_cell_ranges
     const int lane = threadIdx.x & 63;
     uint64_t todo = __ballot(valid), group = valid ? 1ull << lane : 0;
     int leader = lane;
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(SCAN_T) k_cell_ranges(CellTables C) {
 }
 
 __global__ void __launch_bounds__(256) k_cell_scatter(DevTopo T, DevState S, CellTables C) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
+    const int b = xcd_bead(256);
     if (b >= T.nb) return;
     const int slot = C.range[C.cell[b].w].x + C.rank[b];
     const float4 x = S.xyz[b];
@@ -159,7 +159,8 @@ __global__ void __launch_bounds__(256) k_cell_scatter(DevTopo T, DevState S, Cel
 // a candidate (met twice, it stands there twice, side by side once sorted, and
 // the caller takes it once).  Up to 32 are sorted in registers.  4 periodic
 // systems of 122646 beads: 188 us with three gathers per bead and an insertion
-// sort in LDS, 108 with the requests together, 61 with the sort.
+// sort in LDS, 108 with the requests together, 61 with the sort, 53 with each
+// XCD on its own eighth of the beads, whose tables then stay in its L2.
 template <int K, class JT>
 __device__ __forceinline__ int gather_candidates(const DevTopo &T, const DevState &S, const CellTables &C, int b,
                                                  float radius, JT *cand) {
@@ -232,7 +233,7 @@ template <int K, class JT>
 __global__ void __launch_bounds__(CELL_BLOCK)
     k_rebuild_cells(mte_params P, DevTopo T, DevState S, CellTables C, float radius, int do_lj, int do_bonded) {
     __shared__ JT cand_all[CELL_BLOCK * CAND_STRIDE<JT>];
-    const int b = blockIdx.x * CELL_BLOCK + threadIdx.x;
+    const int b = xcd_bead(CELL_BLOCK);
     if (b >= T.nb) return;
     const int t = T.tid[b], base = T.tbase[t];
     RebuildOwn o = rebuild_own(S.xyz[b], S.fn[b], S.fp1[b], S.fp2[b], T.mon_type[b], T.harm_raw[b], b - base, b,
@@ -267,7 +268,7 @@ float candidate_radius(const mte_params &P) {
 
 hipError_t build_cells(mte_engine *e, float side, int K) {
     const CellTables &C = e->cells;
-    const int gb = (e->nb + 255) / 256;
+    const int gb = grid_xcd(e->nb, 256);
     // the bucket counts are zero here: set at creation, and cleared by
     // k_cell_ranges once it has read them
     hipLaunchKernelGGL(k_cell_assign, dim3(gb), dim3(256), 0, e->stream, e->T, e->S[e->cur], C, side, K);
@@ -288,7 +289,7 @@ hipError_t launch_rebuild_cells(mte_engine *e) {
     const bool small = e->nmax <= 65536;
     auto kern = K == 2 ? (small ? k_rebuild_cells<2, uint16_t> : k_rebuild_cells<2, int>)
                        : (small ? k_rebuild_cells<1, uint16_t> : k_rebuild_cells<1, int>);
-    hipLaunchKernelGGL(kern, dim3((e->nb + CELL_BLOCK - 1) / CELL_BLOCK), dim3(CELL_BLOCK), 0, e->stream, e->P, e->T,
+    hipLaunchKernelGGL(kern, dim3(grid_xcd(e->nb, CELL_BLOCK)), dim3(CELL_BLOCK), 0, e->stream, e->P, e->T,
                        e->S[e->cur], e->cells, radius, do_lj, do_bonded);
     return hipGetLastError();
 }

@@ -318,6 +318,19 @@ __device__ __forceinline__ float4 normals4(uint4 &s) {
     return o;
 }
 
+// Bead of this thread in a grid of 8 x nb8 workgroups (grid_xcd).  The
+// dispatcher hands workgroup k to XCD k mod 8, so workgroup k takes the
+// (k / 8)-th block of the (k mod 8)-th eighth of the beads: each XCD works
+// on a contiguous eighth, whose trajectories' state then stays in that
+// XCD's L2 while their neighbours are gathered.  The bead a thread computes
+// does not change any result.
+__device__ __forceinline__ int xcd_block() {
+    return ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+}
+__device__ __forceinline__ int xcd_bead(int bs) { return xcd_block() * bs + (int)threadIdx.x; }
+// The grid of such a kernel over n items, bs to a workgroup: a multiple of 8.
+inline int grid_xcd(int n, int bs) { return 8 * (((n + bs - 1) / bs + 7) / 8); }
+
 // Constants of the force field and the integrator as the kernels use them,
 // derived once on the host: per step and bead, quotients of the parameters
 // (with the scaling and fix-ups a division expands to) would be taken anew.
