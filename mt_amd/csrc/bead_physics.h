@@ -50,13 +50,6 @@ __device__ __forceinline__ Own make_own(float4 xyz, float4 ang, float4 fn, float
     return make_own_trig(xyz, ang, fn, fp1, fp2, trig, flags);
 }
 
-// Per-bead flags packed into xyz.w when a trajectory's state is staged in LDS.
-constexpr int FL_MON = 1, FL_GTP1 = 2, FL_OFFTUB = 4;
-
-__device__ __forceinline__ int pack_flags(const DevTopo &T, int b) {
-    return (T.mon_type[b] ? FL_MON : 0) | (T.gtp[b] == 1 ? FL_GTP1 : 0) | (T.on_tub[b] == 0 ? FL_OFFTUB : 0);
-}
-
 // Neighbour data by a handle that the list entry gives.  In LDS, four arrays
 // hold per bead its position with the packed flags in w, and the rotated
 // offsets with the Euler angles in w (n|fi, p1|theta, p2|psi); the handle is
@@ -93,7 +86,7 @@ __device__ __forceinline__ void stage_state(const DevTopo &T, const DevState &S,
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int b = base + i;
         float4 x = S.xyz[b];
-        x.w = __int_as_float(pack_flags(T, b));
+        x.w = __int_as_float(T.flags[b]);
         const float4 a = S.ang[b];
         float4 fn = S.fn[b], f1 = S.fp1[b], f2 = S.fp2[b];
         fn.w = a.x;

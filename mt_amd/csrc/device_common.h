@@ -49,11 +49,16 @@ struct DevTopo {
     uint8_t *extra;
     const int *mon_type;
     int *gtp, *on_tub;
+    uint8_t *flags;       // the five per-bead flags (FL_*), packed by k_pack_flags
     const float *zs;
     const float *tbox;    // trajectory -> periodic box side (0: open boundaries)
     int *overflow;        // set to 1 by a rebuild that ran out of list capacity
     int *frozen;          // steps the resident kernel left undone because `overflow` was set
 };
+
+// Per-bead flags: monomer type, GTP state 1, off the tubule, fixed, extra.
+constexpr int FL_MON = 1, FL_GTP1 = 2, FL_OFFTUB = 4, FL_FIXED = 8, FL_EXTRA = 16;
+__device__ __forceinline__ bool is_mobile(int flags) { return (flags & (FL_FIXED | FL_EXTRA)) == 0; }
 
 // One buffer of bead state: positions, angles and the rotated offsets.
 struct DevState {

@@ -563,7 +563,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
     }
     ALLOC(p_tid, nb) ALLOC(p_tbase, nt) ALLOC(p_tsize, nt) ALLOC(p_harm, nb) ALLOC(p_harm_raw, nb)
     ALLOC(T.lon_n, nb) ALLOC(T.lon, (size_t)MAXLON * nb) ALLOC(T.lat_n, nb) ALLOC(T.lat, (size_t)MAXLAT * nb)
-    ALLOC(T.lj_n, nb) ALLOC(T.lj, (size_t)T.max_lj * nb) ALLOC(p_fixed, nb) ALLOC(p_extra, nb) ALLOC(p_mon, nb)
+    ALLOC(T.lj_n, nb) ALLOC(T.lj, (size_t)T.max_lj * nb) ALLOC(p_fixed, nb) ALLOC(p_extra, nb) ALLOC(T.flags, nb) ALLOC(p_mon, nb)
     ALLOC(p_gtp, nb) ALLOC(p_ont, nb) ALLOC(p_zs, nt) ALLOC(p_box, nt) ALLOC(T.overflow, 1) ALLOC(T.frozen, 1) ALLOC(e->tiles, tiles.size())
     ALLOC(e->rb_order, nb) ALLOC(e->res_order, nb) ALLOC(e->mtl_counts, nt) ALLOC(e->mtl_flags, nb)
     for (int k = 0; k < 2; k++) {
@@ -611,6 +611,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
     UP(p_fixed, fixed.data(), nb) UP(p_extra, extra.data(), nb) UP(p_mon, mon.data(), nb)
     UP(p_gtp, gtp.data(), nb) UP(p_ont, ont.data(), nb) UP(p_zs, zs.data(), nt)
     UP(p_box, box.data(), nt)
+    if (launch_pack_flags(e) != hipSuccess) { e->err = "mte_create: launch failed"; return bail(MTE_ERR_HIP); }
     UP(e->tiles, tiles.data(), tiles.size()) UP(e->seeds, seeds.data(), seeds.size())
     std::vector<int> order(nb);   // rebuild order: index order until a state arrives (mte_set_state)
     for (int t = 0; t < nt; t++)
@@ -846,6 +847,7 @@ int mte_set_flags(mte_engine *e, const uint8_t *extra, const int32_t *gtp, const
     }
     if (gtp) HIPCHK(hipMemcpyAsync(e->T.gtp, gtp, sizeof(int) * e->nb, hipMemcpyHostToDevice, e->stream));
     if (on_tubule) HIPCHK(hipMemcpyAsync(e->T.on_tub, on_tubule, sizeof(int) * e->nb, hipMemcpyHostToDevice, e->stream));
+    HIPCHK(launch_pack_flags(e));
     HIPCHK(hipStreamSynchronize(e->stream));
     return MTE_OK;
 }

@@ -225,6 +225,7 @@ hipError_t launch_rebuild_order(mte_engine *e);
 size_t forces_lds_bytes(int nmax);
 hipError_t launch_mt_length(mte_engine *e, float rad_hi, float rad_lo, float cos_min, int apply);
 bool rebuild_traj_plan(int nmax, int lds_limit, int *threads, size_t *lds);
+hipError_t launch_pack_flags(mte_engine *e);
 hipError_t launch_rebuild_cells(mte_engine *e);
 // The cell tables of the MLP-HI feature search, then the search
 // itself (which builds the tables first unless build_tables is false).

@@ -732,7 +732,7 @@ __device__ __forceinline__ MlpIn mlp_load(const MlpStepArgs &A, int b) {
     v.fa = A.fang[b];
     v.cc = A.ci[b];
     v.bt = A.beta[T.tid[b]];
-    v.mobile = !T.fixed[b] && !T.extra[b];
+    v.mobile = is_mobile(T.flags[b]);
     if (!A.noise) {
         v.s0 = A.seeds[b];
         v.s1 = A.seeds[b + T.nb];

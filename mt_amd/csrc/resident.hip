@@ -369,7 +369,7 @@ __global__ void __launch_bounds__(MAXT)
         const int i = slot < n ? order[base + slot] : slot;
         W.ib[k] = i;
         const int b = base + i;
-        W.mob[k] = i < n && !T.fixed[b] && !T.extra[b];
+        W.mob[k] = i < n && is_mobile(T.flags[b]);
         lcnt[k] = 0;
         if (W.mob[k])
             lcnt[k] = pack_counts(T.harm[b] >= 0, T.lon_n[b], T.lat_n[b], K.lj_on ? T.lj_n[b] : 0);
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(MAXT)
     int help_slot = -1, help_b = -1;
     if (owner >= 0 && offloaded(owner)) {
         const int b = base + order[base + owner + blockDim.x];   // the owner's second-pass bead
-        if (!T.fixed[b] && !T.extra[b]) {
+        if (is_mobile(T.flags[b])) {
             help_slot = rng_slot(owner);
             help_b = b;
             W.s0[PT - 1] = seeds[b];

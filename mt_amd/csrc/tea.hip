@@ -868,7 +868,7 @@ __device__ __forceinline__ void tea_move(const ForceK &K, const DevTopo &T, cons
     n4 = Sin.fn[b];
     p1 = Sin.fp1[b];
     p2 = Sin.fp2[b];
-    if (!T.fixed[b] && !T.extra[b]) {
+    if (is_mobile(T.flags[b])) {
         x.x = fmaf(K.dtg, fx, x.x);
         x.y = fmaf(K.dtg, fy, x.y);
         x.z = fmaf(K.dtg, fz, x.z);
@@ -918,12 +918,12 @@ __global__ void __launch_bounds__(TURN_THREADS)
     const int i = threadIdx.x, b = base + min(i, n - 1);
     const AheadLists<LdsAcc::SCALE> Ls(T, b, base, A.origin());
     float4 x, an, n4, p1, p2;
-    bool extra = false;
+    const int flags = T.flags[b];
+    const bool extra = (flags & FL_EXTRA) != 0;
     if (i < n) {
-        extra = T.extra[b];
         tea_move<true>(K, T, Sin, M, noise, L, b, t, x, an, n4, p1, p2);
         store_bead(Sout, b, x, an, n4, p1, p2);
-        x.w = __int_as_float(pack_flags(T, b));
+        x.w = __int_as_float(flags);
         lx[i] = x;
         ln[i] = make_float4(n4.x, n4.y, n4.z, an.x);
         l1[i] = make_float4(p1.x, p1.y, p1.z, an.y);
