@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(256)
 // so a trajectory's beads hold the slots [tbase, tbase + n).  Which of them a
 // span gets depends on the order the workgroups arrive in; no user of the
 // tables looks beyond a bucket's range.  (A scan over all buckets, in bucket
-// order, took three launches and 17 us for 2^20 buckets, this one 6.)  Bounded
+// order, took three launches and 17 us for 851968 buckets, this one 6.)  Bounded
 // by the bytes, 16 per bucket, and by the cursors: atomics on one cache line
 // from all XCDs take about 10 ns each, so a cursor has a line of its own and
 // a span is 4096 buckets (1024: 13.5 us).
