@@ -347,15 +347,15 @@ __global__ void __launch_bounds__(MAXT)
     }
     float4 *lx = lds, *ln = lds + stride, *l1 = lds + 2 * stride, *l2 = lds + 3 * stride;
     float4 *rbuf = lds + STATE_ARRAYS * stride;
-    int *hoff = reinterpret_cast<int *>(rbuf + RNG_F4);
-    int *hcnt = hoff + stride;
-    int *scan = hcnt + stride;
-    int *flags = scan + SCAN_INTS;
     static_assert(!HELPED || PT == 1, "a helper serves one bead");
     const int nmain = HELPED ? blockDim.x / 2 : blockDim.x;   // threads that own beads
     const bool helper = HELPED && (int)threadIdx.x >= nmain;
-    float4 *xbuf = reinterpret_cast<float4 *>(flags + FLAG_INTS);
-    uint16_t *ent = reinterpret_cast<uint16_t *>(xbuf + (HELPED ? XBUF_F4 * nmain : 0));
+    float4 *xbuf = rbuf + RNG_F4;
+    int *hoff = reinterpret_cast<int *>(xbuf + (HELPED ? XBUF_F4 * nmain : 0));
+    int *hcnt = hoff + stride;
+    int *scan = hcnt + stride;
+    int *flags = scan + SCAN_INTS;
+    uint16_t *ent = reinterpret_cast<uint16_t *>(flags + FLAG_INTS);
     const int t = blockIdx.x;
     const int base = T.tbase[t], n = T.tsize[t];
     const int nb = T.nb;
