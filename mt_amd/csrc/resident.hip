@@ -337,14 +337,7 @@ __global__ void __launch_bounds__(MAXT)
     k_resident(ForceK K, float ljpairscutoff, DevTopo T, DevState S, uint4 *seeds, const float *noise, int nsteps, LatOffsets L,
                int stride, int entry_cap, const int *order) {
     extern __shared__ float4 lds[];
-    // A rebuild that ran out of list capacity stops the dynamics: the state
-    // and RNG streams stay at that rebuild's step, and the host reports the
-    // error with the steps not taken (every thread returns before any
-    // barrier).
-    if (*(volatile const int *)T.overflow) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(T.frozen, nsteps);
-        return;
-    }
+    const int overflow = *(volatile const int *)T.overflow;
     float4 *lx = lds, *ln = lds + stride, *l1 = lds + 2 * stride, *l2 = lds + 3 * stride;
     float4 *rbuf = lds + STATE_ARRAYS * stride;
     static_assert(!HELPED || PT == 1, "a helper serves one bead");
@@ -362,26 +355,32 @@ __global__ void __launch_bounds__(MAXT)
     if (threadIdx.x == 0) flags[0] = 0;
     stage_state(T, S, base, n, lx, ln, l1, l2);
     Lanes<PT> W;   // this thread's lane slots (order: immobile beads last)
-    int lcnt[PT];   // its list counts, packed as in hcnt (requested with the bead's state)
+    int lcnt[PT];   // its list counts, packed as in hcnt
+    // everything a bead needs is requested at once, of the trajectory's last
+    // bead where a slot has none, before its flags tell whether it is mobile
 #pragma unroll
     for (int k = 0; k < PT; k++) {
         const int slot = (helper ? threadIdx.x - nmain : threadIdx.x) + k * blockDim.x;
-        const int i = slot < n ? order[base + slot] : slot;
-        W.ib[k] = i;
-        const int b = base + i;
-        W.mob[k] = i < n && is_mobile(T.flags[b]);
-        lcnt[k] = 0;
-        if (W.mob[k])
-            lcnt[k] = pack_counts(T.harm[b] >= 0, T.lon_n[b], T.lat_n[b], K.lj_on ? T.lj_n[b] : 0);
-        if (W.mob[k]) {
-            const float4 a = S.ang[b];
-            sincos_fast(a.y, &W.trig[k].x, &W.trig[k].y);
-            sincos_fast(a.z, &W.trig[k].z, &W.trig[k].w);
-        }
-        if (W.mob[k] && !noise) {
+        const int i = order[base + min(slot, n - 1)], b = base + i;
+        const int fl = T.flags[b], h = T.harm[b], c0 = T.lon_n[b], c1 = T.lat_n[b], c2 = T.lj_n[b];
+        const float4 a = S.ang[b];
+        if (!noise) {
             W.s0[k] = seeds[b];
             W.s1[k] = seeds[b + nb];
         }
+        W.ib[k] = i;
+        W.mob[k] = slot < n && is_mobile(fl);
+        lcnt[k] = W.mob[k] ? pack_counts(h >= 0, c0, c1, K.lj_on ? c2 : 0) : 0;
+        sincos_fast(a.y, &W.trig[k].x, &W.trig[k].y);
+        sincos_fast(a.z, &W.trig[k].z, &W.trig[k].w);
+    }
+    // A rebuild that ran out of list capacity stops the dynamics: the state
+    // and RNG streams stay at that rebuild's step, and the host reports the
+    // error with the steps not taken (every thread returns before any
+    // barrier).
+    if (overflow) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(T.frozen, nsteps);
+        return;
     }
     // noise offload roles (two beads per thread, drawn noise); the first
     // wave offloads too only when a later second-pass wave of the first SIMD
