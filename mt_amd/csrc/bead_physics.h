@@ -468,7 +468,7 @@ struct TeaDraw {
 };
 
 // One bead's share of it.
-__device__ __forceinline__ void tea_draw(const TeaDraw &D, float var, int b, bool extra) {
+__device__ __forceinline__ float4 tea_draw(const TeaDraw &D, float var, int b, bool extra) {
     float4 r;
     if (D.noise) {
         const float *nz = D.noise + 6 * (size_t)b;
@@ -478,7 +478,7 @@ __device__ __forceinline__ void tea_draw(const TeaDraw &D, float var, int b, boo
         r = normals4(s);
         D.seeds[b] = s;
     }
-    D.R[b] = extra ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
+    return extra ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(r.x * var, r.y * var, r.z * var, 0.f);
 }
 
 }  // namespace mte

@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(BS)
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
+    if (D.R) D.R[b] = tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
 }
 
 // The same forces with the bead's whole trajectory staged in LDS (positions,
@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(FORCE_TILE)
     }
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
+    if (D.R) D.R[b] = tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
 }
 
 // Dynamic LDS of k_forces_lds for trajectories of up to nmax beads.

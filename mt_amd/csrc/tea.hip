@@ -790,15 +790,14 @@ struct TeaMove {
     uint4 *seeds;
 };
 
-// Self term, chunk partials in fixed order, and the update of bead b of
-// trajectory t (integrateTea_kernel_unlisted, src/bdhitea_kernel.cu:148-213).
+// Self term and chunk partials in fixed order, of bead b of trajectory t, and
+// the bead's state (integrateTea_kernel_unlisted, src/bdhitea_kernel.cu:148-213).
 // SYM: the partials of k_tea_pairs_sym (planes of x, y, z; the bead's j-side
 // slots, then its i-side slots), else the float4 slots of its trajectory's
 // chunks.
 template <bool SYM>
-__device__ __forceinline__ void tea_move(const ForceK &K, const DevTopo &T, const DevState &Sin, const TeaMove &M,
-                                         const float *noise, const LatOffsets &L, int b, int t, float4 &x, float4 &an,
-                                         float4 &n4, float4 &p1, float4 &p2) {
+__device__ __forceinline__ float3 tea_sum(const DevTopo &T, const DevState &Sin, const TeaMove &M, int b, int t, float4 &x,
+                                          float4 &an, float4 &n4, float4 &p1, float4 &p2) {
     const float bt = M.beta[t];
     const float4 cc = M.ci[b], Fi = M.fxyz[b], Ri = M.R[b];
     const float w = bt * bt;
@@ -808,6 +807,9 @@ __device__ __forceinline__ void tea_move(const ForceK &K, const DevTopo &T, cons
     // the bead's state is requested before the partial sums are added
     x = Sin.xyz[b];
     an = Sin.ang[b];
+    n4 = Sin.fn[b];
+    p1 = Sin.fp1[b];
+    p2 = Sin.fp2[b];
     const size_t nb = T.nb;
     if (SYM) {
         const float *part = reinterpret_cast<const float *>(M.partial) + b;
@@ -856,26 +858,29 @@ __device__ __forceinline__ void tea_move(const ForceK &K, const DevTopo &T, cons
             fz += pp.z;
         }
     }
-    float4 ra;
+    return make_float3(fx, fy, fz);
+}
+// The angular normals of a bead, and its update by the sum f.
+__device__ __forceinline__ float4 tea_angles(const DevTopo &T, const TeaMove &M, const float *noise, int b) {
     if (noise) {
         const float *q = noise + 6 * (size_t)b;
-        ra = make_float4(q[3], q[4], q[5], 0.f);
-    } else {
-        uint4 s = M.seeds[b + T.nb];
-        ra = normals4(s);
-        M.seeds[b + T.nb] = s;
+        return make_float4(q[3], q[4], q[5], 0.f);
     }
-    n4 = Sin.fn[b];
-    p1 = Sin.fp1[b];
-    p2 = Sin.fp2[b];
-    if (is_mobile(T.flags[b])) {
-        x.x = fmaf(K.dtg, fx, x.x);
-        x.y = fmaf(K.dtg, fy, x.y);
-        x.z = fmaf(K.dtg, fz, x.z);
-        const float4 fa = M.fang[b];
-        em_angles(K, fa.x, fa.y, fa.z, ra, an);
-        frame_vectors(an.x, an.y, an.z, L, n4, p1, p2);
-    }
+    uint4 s = M.seeds[b + T.nb];
+    const float4 ra = normals4(s);
+    M.seeds[b + T.nb] = s;
+    return ra;
+}
+__device__ __forceinline__ void tea_update(const ForceK &K, const TeaMove &M, const LatOffsets &L, int b, int flags,
+                                           float3 f, float4 ra, float4 &x, float4 &an, float4 &n4, float4 &p1,
+                                           float4 &p2) {
+    if (!is_mobile(flags)) return;
+    x.x = fmaf(K.dtg, f.x, x.x);
+    x.y = fmaf(K.dtg, f.y, x.y);
+    x.z = fmaf(K.dtg, f.z, x.z);
+    const float4 fa = M.fang[b];
+    em_angles(K, fa.x, fa.y, fa.z, ra, an);
+    frame_vectors(an.x, an.y, an.z, L, n4, p1, p2);
 }
 __device__ __forceinline__ void store_bead(const DevState &S, int b, float4 x, float4 an, float4 n4, float4 p1,
                                            float4 p2) {
@@ -892,52 +897,78 @@ __global__ void __launch_bounds__(TEA_TILE)
     const int b = xcd_bead(TEA_TILE);
     if (b >= T.nb) return;
     float4 x, an, n4, p1, p2;
-    tea_move<SYM>(K, T, Sin, M, noise, L, b, T.tid[b], x, an, n4, p1, p2);
+    const float3 f = tea_sum<SYM>(T, Sin, M, b, T.tid[b], x, an, n4, p1, p2);
+    tea_update(K, M, L, b, T.flags[b], f, tea_angles(T, M, noise, b), x, an, n4, p1, p2);
     store_bead(Sout, b, x, an, n4, p1, p2);
 }
 
 // The end of one step and the forces of the next in one launch, a workgroup
 // per trajectory and a thread per bead: each moves its bead and stages it in
 // LDS, then the new forces and random forces are formed from there.  Bounded,
-// as the two kernels it stands for, by trips to memory, not by bytes or
-// operations: it saves a launch, their second reading of every state and the
-// wait between them.  One tube of 312 beads: 7.6 us, for 5.7 of forces and 4.2
-// of update.  The lists are requested before the bead is moved.
-constexpr int TURN_THREADS = 640;
-template <bool PERIODIC>
-__global__ void __launch_bounds__(TURN_THREADS)
+// as the two kernels it stands for, by waiting, not by bytes or operations:
+// it saves a launch, their second reading of every state and the wait between
+// them.  The lists are requested before the bead is moved.
+// HELPED: a second thread per bead, in another wave, draws both its normals
+// while the sums come in, and sums its LJ forces beside its bonds; the sums
+// are added in the same order.
+// One tube of 312 beads: 5.7 us of forces and 4.2 of update apart, 7.3 in one,
+// 5.9 helped.
+constexpr int TURN_THREADS = 640, TURN_HELPED = 512;   // beads at most
+template <bool PERIODIC, bool HELPED>
+__global__ void __launch_bounds__(HELPED ? 2 * TURN_HELPED : TURN_THREADS)
     k_tea_turn(ForceK K, DevTopo T, DevState Sin, DevState Sout, TeaMove M, const float *noise, TeaDraw D,
                float4 *fxyz, float4 *fang, LatOffsets L) {
     extern __shared__ float4 lds[];
     const int t = xcd_block();   // through the L2 that the pair kernel left its partials in
     if (t >= T.ntraj) return;
     const int base = T.tbase[t], n = T.tsize[t];
-    float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n;
+    float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n, *xb = l2 + n;   // xb: from the helpers
     const LdsAcc A(lx, ln, l1, l2);
     const float wall_z = K.is_wall ? T.zs[t] : 0.f;
-    const int i = threadIdx.x, b = base + min(i, n - 1);
+    const int nmain = HELPED ? blockDim.x / 2 : blockDim.x;
+    const bool helper = HELPED && (int)threadIdx.x >= nmain;
+    const int i = threadIdx.x - (helper ? nmain : 0), b = base + min(i, n - 1);
     const AheadLists<LdsAcc::SCALE> Ls(T, b, base, A.origin());
-    float4 x, an, n4, p1, p2;
     const int flags = T.flags[b];
     const bool extra = (flags & FL_EXTRA) != 0;
+    float4 x, an, n4, p1, p2, R;   // R: the next random force
+    float3 f;
     if (i < n) {
-        tea_move<true>(K, T, Sin, M, noise, L, b, t, x, an, n4, p1, p2);
+        if (!helper) f = tea_sum<true>(T, Sin, M, b, t, x, an, n4, p1, p2);
+        if (helper) xb[i] = tea_angles(T, M, noise, b);
+        if (!HELPED || helper) R = tea_draw(D, K.vF, b, extra);
+    }
+    if (HELPED) __syncthreads();
+    if (i < n && !helper) {
+        tea_update(K, M, L, b, flags, f, HELPED ? xb[i] : tea_angles(T, M, noise, b), x, an, n4, p1, p2);
         store_bead(Sout, b, x, an, n4, p1, p2);
         x.w = __int_as_float(flags);
         lx[i] = x;
         ln[i] = make_float4(n4.x, n4.y, n4.z, an.x);
         l1[i] = make_float4(p1.x, p1.y, p1.z, an.y);
         l2[i] = make_float4(p2.x, p2.y, p2.z, an.z);
-        tea_draw(D, K.vF, b, extra);
     }
     __syncthreads();
-    if (i >= n) return;
+    // written once the bead has been moved: its sum has read the last one
+    if (i < n && (!HELPED || helper)) D.R[b] = R;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (!extra) {
-        Own I = make_own(x, an, n4, p1, p2, __float_as_int(x.w));
-        if (PERIODIC) set_box(I, T.tbox[t]);
-        bead_force<PERIODIC>(K, A, Ls, wall_z, I, F);
+    if (i < n && !extra) {
+        if (helper) {
+            Own I;
+            I.r = f3(lx[i]);
+            if (PERIODIC) set_box(I, T.tbox[t]);
+            const float3 lj = K.lj_on ? lj_sum<PERIODIC>(K, A, Ls, I) : make_float3(0.f, 0.f, 0.f);
+            xb[i] = make_float4(lj.x, lj.y, lj.z, 0.f);
+        } else {
+            Own I = make_own(x, an, n4, p1, p2, flags);
+            if (PERIODIC) set_box(I, T.tbox[t]);
+            if (HELPED) bond_total(bond_forces<PERIODIC>(K, A, Ls, I), I, F);
+            else bead_force<PERIODIC>(K, A, Ls, wall_z, I, F);
+        }
     }
+    if (HELPED) __syncthreads();
+    if (i >= n || helper) return;
+    if (HELPED && !extra) add_lj_walls(K, f3(xb[i]), wall_z, f3(x), F);
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
 }
@@ -1435,16 +1466,22 @@ hipError_t launch_tea_finish(mte_engine *e, const float *noise_step) {
 // 1, 8 and 64 tubes of 520 beads 1700 -> 1598, 1754 -> 1593 and 3063 -> 2850
 // us, of 624 beads 1723 -> 1633, 1762 -> 1607 and 3364 -> 3185; of 780 beads
 // 1766 -> 1806, 2012 -> 2040 and 4100 -> 3985: the two keep more CUs busy).
+// Where two threads per bead fit, they do (64 and 1 tubes of 312 beads 1742 ->
+// 1623 and 1386 -> 1298).
 bool tea_turn_fits(const mte_engine *e) {
     return e->tea.unit_chunk == MTE_TEA_SYMMETRIC && e->tune.forces == MTE_FORCES_LDS && e->forces_lds > 0 &&
            e->nmax <= TURN_THREADS;
 }
 
 hipError_t launch_tea_turn(mte_engine *e, const float *noise_step, const float *noise_next) {
-    auto kern = e->periodic ? k_tea_turn<true> : k_tea_turn<false>;
-    hipLaunchKernelGGL(kern, dim3(grid_xcd(e->ntraj, 1)), dim3(((e->nmax + 63) / 64) * 64), e->forces_lds, e->stream,
-                       e->K, e->T, e->S[e->cur], e->S[1 - e->cur], tea_move_args(e), noise_step,
-                       TeaDraw{e->seeds, noise_next, e->tea.R}, e->fxyz, e->fang, e->L);
+    const bool helped = e->nmax <= TURN_HELPED;
+    auto kern = helped ? (e->periodic ? k_tea_turn<true, true> : k_tea_turn<false, true>)
+                       : (e->periodic ? k_tea_turn<true, false> : k_tea_turn<false, false>);
+    const int threads = ((e->nmax + 63) / 64) * 64 * (helped ? 2 : 1);
+    const size_t lds = e->forces_lds + (helped ? sizeof(float4) * e->nmax : 0);   // at most 40 KB
+    hipLaunchKernelGGL(kern, dim3(grid_xcd(e->ntraj, 1)), dim3(threads), lds, e->stream, e->K, e->T, e->S[e->cur],
+                       e->S[1 - e->cur], tea_move_args(e), noise_step, TeaDraw{e->seeds, noise_next, e->tea.R}, e->fxyz,
+                       e->fang, e->L);
     e->cur = 1 - e->cur;
     return hipGetLastError();
 }

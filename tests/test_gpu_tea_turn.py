@@ -2,8 +2,9 @@
 640 beads) against the same steps with separate force and update kernels, which
 add the same terms in the same order: the same random streams, and states that
 differ by at most one rounding at 150 nm (1.5e-5) per step.  Sizes at the edges: one
-dimer row, a wave's edge, the largest trajectory of the fused kernel and the
-first beyond it; batches of several lengths, open, periodic and mixed, drawn
+dimer row, the largest trajectory with a helper thread per bead (494) and the
+first without (520), the largest of the fused kernel (624) and the first
+beyond it; batches of several lengths, open, periodic and mixed, drawn
 and injected noise, across a tensor refresh."""
 import numpy as np
 import pytest
@@ -28,7 +29,7 @@ def _run(b, forces, nz, steps):
 
 
 @pytest.mark.parametrize("lengths,boxes", [
-    ((1,), (0.0,)), ((24,), (0.0,)), ((25, 3), (0.0, 0.0)), ((12, 1, 24), (0.0, 0.0, 0.0)),
+    ((1,), (0.0,)), ((19, 2), (0.0, 0.0)), ((20,), (0.0,)), ((24,), (0.0,)), ((25, 3), (0.0, 0.0)), ((12, 1, 24), (0.0, 0.0, 0.0)),
     ((12, 5), (150.0, 0.0)), ((5, 12, 1, 2, 3, 4, 6, 7, 8), (150.0,) * 9)])
 @pytest.mark.parametrize("injected", [False, True])
 def test_fused_turn_equals_separate_kernels(lengths, boxes, injected):
