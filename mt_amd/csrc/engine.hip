@@ -742,6 +742,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
             !rebuild_traj_plan(nmax, lds_limit, &e->rb_traj_threads, &e->rb_traj_lds))
             e->rb_traj_threads = 0;
         // forces with the trajectory staged in LDS when it fits
+        e->lds_limit = lds_limit;
         e->forces_lds = forces_lds_bytes(nmax) <= (size_t)lds_limit ? forces_lds_bytes(nmax) : 0;
         e->tune.forces = e->forces_lds > 0 ? MTE_FORCES_LDS : MTE_FORCES_GLOBAL;
     }

@@ -181,6 +181,7 @@ struct mte_engine {
     // pinned, device-mapped host memory, so that the run's one stream
     // synchronisation also delivers them (flags_dev is its device address).
     int *flags_host = nullptr, *flags_dev = nullptr;
+    int lds_limit = 0;               // LDS bytes a workgroup may have
     bool stage_user = false;         // counted among the staging pool's engines
     mte::TeaBuffers tea;
     mte::CellTables cells;

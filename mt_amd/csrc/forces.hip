@@ -116,8 +116,13 @@ __global__ void __launch_bounds__(BS)
 // tiles go to one XCD, whose L2 then serves all but the first (64 tubes: 12.5
 // -> 9.6 us with the update kernel's beads and the pair units in the same
 // eighths, tea_build_units).
-template <bool PERIODIC>
-__global__ void __launch_bounds__(FORCE_TILE)
+// HELPED: a second thread per bead, in another wave, draws its random force and
+// sums its LJ forces beside its bonds (about one wave per SIMD otherwise, each
+// bound by its own waits: 64 tubes of 1040 beads 9.3 -> 8.0 us, 100 steps of 1
+// and 8 such tubes 1882 -> 1711 and 2354 -> 2192); the sums are added in the
+// same order.
+template <bool PERIODIC, bool HELPED>
+__global__ void __launch_bounds__(HELPED ? 2 * FORCE_TILE : FORCE_TILE)
     k_forces_lds(ForceK K, DevTopo T, DevState S, const int2 *tiles, int ntiles, float4 *fxyz, float4 *fang, TeaDraw D) {
     extern __shared__ float4 lds[];
     const int tile = xcd_block();   // a trajectory's tiles share one L2
@@ -126,26 +131,45 @@ __global__ void __launch_bounds__(FORCE_TILE)
     const int t = tl.x, base = T.tbase[t], n = T.tsize[t];
     float4 *lx = lds, *ln = lds + n, *l1 = ln + n, *l2 = l1 + n;
     const LdsAcc A(lx, ln, l1, l2);
-    const int i = tl.y + threadIdx.x, b = base + min(i, n - 1);
+    const bool helper = HELPED && threadIdx.x >= FORCE_TILE;
+    const int q = threadIdx.x - (helper ? FORCE_TILE : 0);
+    float4 *xlj = l2 + n + q;   // HELPED: the helper's LJ sum
+    const int i = tl.y + q, b = base + min(i, n - 1);
     const AheadLists<LdsAcc::SCALE> Ls(T, b, base, A.origin());
     stage_state(T, S, base, n, lx, ln, l1, l2);
     __syncthreads();
-    if (i >= n) return;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const float4 x = lx[i];
-    const int flags = __float_as_int(x.w);
-    if (!(flags & FL_EXTRA)) {
-        const float4 fn = ln[i], f1 = l1[i], f2 = l2[i];
-        Own I = make_own(x, make_float4(fn.w, f1.w, f2.w, 0.f), fn, f1, f2, flags);
-        if (PERIODIC) set_box(I, T.tbox[t]);
-        bead_force<PERIODIC>(K, A, Ls, K.is_wall ? T.zs[t] : 0.f, I, F);
+    const float wall_z = K.is_wall ? T.zs[t] : 0.f;
+    Own I;
+    bool extra = true;
+    if (i < n) {
+        const float4 x = lx[i];
+        const int flags = __float_as_int(x.w);
+        extra = (flags & FL_EXTRA) != 0;
+        if (helper) {
+            I.r = f3(x);
+            if (PERIODIC) set_box(I, T.tbox[t]);
+            float3 lj = make_float3(0.f, 0.f, 0.f);
+            if (!extra && K.lj_on) lj = lj_sum<PERIODIC>(K, A, Ls, I);
+            *xlj = make_float4(lj.x, lj.y, lj.z, 0.f);
+        } else if (!extra) {
+            const float4 fn = ln[i], f1 = l1[i], f2 = l2[i];
+            I = make_own(x, make_float4(fn.w, f1.w, f2.w, 0.f), fn, f1, f2, flags);
+            if (PERIODIC) set_box(I, T.tbox[t]);
+            if (HELPED) bond_total(bond_forces<PERIODIC>(K, A, Ls, I), I, F);
+            else bead_force<PERIODIC>(K, A, Ls, wall_z, I, F);
+        }
+        if (D.R && (!HELPED || helper)) D.R[b] = tea_draw(D, K.vF, b, extra);
     }
+    if (HELPED) __syncthreads();
+    if (i >= n || helper) return;
+    if (HELPED && !extra) add_lj_walls(K, f3(*xlj), wall_z, I.r, F);
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
     fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) D.R[b] = tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
 }
 
-// Dynamic LDS of k_forces_lds for trajectories of up to nmax beads.
+// Dynamic LDS of k_forces_lds for trajectories of up to nmax beads, without
+// the helpers' sums.
 size_t forces_lds_bytes(int nmax) { return (size_t)4 * sizeof(float4) * nmax; }
 
 template <int BS>
@@ -258,11 +282,14 @@ hipError_t launch_step_plain(mte_engine *e, const float *noise_step) {
 template <bool PERIODIC>
 static hipError_t forces_draw(mte_engine *e, TeaDraw D) {
     if (e->tune.forces == MTE_FORCES_LDS && e->forces_lds > 0) {
-        const hipError_t s = hipFuncSetAttribute((const void *)k_forces_lds<PERIODIC>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)e->forces_lds);
+        const size_t helped_lds = e->forces_lds + sizeof(float4) * FORCE_TILE;
+        const bool helped = helped_lds <= (size_t)e->lds_limit;   // up to 2496 beads
+        auto k = helped ? k_forces_lds<PERIODIC, true> : k_forces_lds<PERIODIC, false>;
+        const size_t lds = helped ? helped_lds : e->forces_lds;
+        const hipError_t s = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (s != hipSuccess) return s;
-        hipLaunchKernelGGL(k_forces_lds<PERIODIC>, dim3(grid_xcd(e->ntiles, 1)), dim3(FORCE_TILE), e->forces_lds,
-                           e->stream, e->K, e->T, e->S[e->cur], e->tiles, e->ntiles, e->fxyz, e->fang, D);
+        hipLaunchKernelGGL(k, dim3(grid_xcd(e->ntiles, 1)), dim3(helped ? 2 * FORCE_TILE : FORCE_TILE), lds, e->stream, e->K,
+                           e->T, e->S[e->cur], e->tiles, e->ntiles, e->fxyz, e->fang, D);
     } else {
         const int bs = e->tune.stream_block;
         const dim3 grid(grid_xcd(e->nb, bs)), block(bs);

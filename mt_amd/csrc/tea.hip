@@ -1463,9 +1463,9 @@ hipError_t launch_tea_finish(mte_engine *e, const float *noise_step) {
 // k_tea_turn serves the symmetric pair kernel's partials, with forces from
 // LDS, for trajectories of up to 640 beads: a workgroup's one bead per thread
 // then costs less than the launch it saves (per 100 steps, two kernels -> one:
-// 1, 8 and 64 tubes of 520 beads 1700 -> 1598, 1754 -> 1593 and 3063 -> 2850
-// us, of 624 beads 1723 -> 1633, 1762 -> 1607 and 3364 -> 3185; of 780 beads
-// 1766 -> 1806, 2012 -> 2040 and 4100 -> 3985: the two keep more CUs busy).
+// 1, 8 and 64 tubes of 520 beads 1571 -> 1600, 1621 -> 1560 and 2906 -> 2768
+// us, of 624 beads 1591 -> 1589, 1641 -> 1582 and 3194 -> 3058; of 780 beads
+// 1631 -> 1760, 1878 -> 2031 and 3863 -> 4013: the two keep more CUs busy).
 // Where two threads per bead fit, they do (64 and 1 tubes of 312 beads 1742 ->
 // 1623 and 1386 -> 1298).
 bool tea_turn_fits(const mte_engine *e) {
