@@ -47,8 +47,8 @@ __global__ void __launch_bounds__(STREAM_BLOCK) k_frames(DevState S, int nb, Lat
 // A second thread per bead, in another wave, draws its normals and sums its LJ
 // forces beside its bonds; the sums are added in the order of one thread.  A
 // bead's work is a chain of dependent waits, and a thread per bead leaves too
-// few waves to cover them (blocks of 256: 100 steps of 4546 beads 752 -> 644
-// us, of 66184 beads 870 -> 763; 200 steps of 169880 beads 2286 -> 1990).
+// few waves to cover them (blocks of 256: 100 steps of 3982 beads 752 -> 644
+// us, of 45436 beads 870 -> 763; 200 steps of 122646 beads 2256 -> 1974).
 template <int BS, bool PERIODIC>
 __global__ void __launch_bounds__(2 * BS)
     k_step_plain(ForceK K, DevTopo T, DevState Sin, DevState Sout, uint4 *seeds, const float *noise,
@@ -120,22 +120,46 @@ __global__ void __launch_bounds__(2 * BS)
 
 // Forces (compute_kernel semantics; extra beads get zero), optionally with
 // the TEA random forces.
+// The helper thread of k_step_plain again (100 MLP-HI steps of 262426 beads 19.43
+// -> 19.32 ms; 50 TEA steps of 3982 beads 1613 -> 1542 us).
 template <int BS, bool PERIODIC>
-__global__ void __launch_bounds__(BS)
+__global__ void __launch_bounds__(2 * BS)
     k_forces(ForceK K, DevTopo T, DevState S, float4 *fxyz, float4 *fang, TeaDraw D) {
-    const int b = xcd_bead(BS);
-    if (b >= T.nb) return;
+    __shared__ float4 xlj[BS];
+    const bool helper = threadIdx.x >= BS;
+    const int q = threadIdx.x - (helper ? BS : 0), b = xcd_block() * BS + q;
+    const bool valid = b < T.nb;
+    const int flags = valid ? T.flags[b] : FL_EXTRA;
+    const bool extra = (flags & FL_EXTRA) != 0;
+    float3 r;
     float F[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const int flags = T.flags[b];
-    if (!(flags & FL_EXTRA)) {
+    if (!extra) {
         const AheadLists<1> Ls(T, b, 0, 0);
-        Own I = make_own(S.xyz[b], S.ang[b], S.fn[b], S.fp1[b], S.fp2[b], flags);
-        if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
-        bead_force<PERIODIC>(K, GlobalAcc{S, T}, Ls, K.is_wall ? T.zs[T.tid[b]] : 0.f, I, F);
+        const GlobalAcc A{S, T};
+        const float4 x = S.xyz[b];
+        r = f3(x);
+        Own I;
+        if (helper) {
+            I.r = r;
+            if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
+            if (D.R) D.R[b] = tea_draw(D, K.vF, b, false);
+            if (K.lj_on) {
+                const float3 lj = lj_sum<PERIODIC>(K, A, Ls, I);
+                xlj[q] = make_float4(lj.x, lj.y, lj.z, 0.f);
+            }
+        } else {
+            I = make_own(x, S.ang[b], S.fn[b], S.fp1[b], S.fp2[b], flags);
+            if (PERIODIC) set_box(I, T.tbox[T.tid[b]]);
+            bond_total(bond_forces<PERIODIC>(K, A, Ls, I), I, F);
+        }
+    } else if (valid && helper && D.R) {
+        D.R[b] = tea_draw(D, K.vF, b, true);
     }
+    __syncthreads();
+    if (!valid || helper) return;
+    if (!extra) add_lj_walls(K, f3(xlj[q]), K.is_wall ? T.zs[T.tid[b]] : 0.f, r, F);
     fxyz[b] = make_float4(F[0], F[1], F[2], 0.f);
-    fang[b] = make_float4(F[3], F[4], F[5], 0.f);   // fi, theta, psi
-    if (D.R) D.R[b] = tea_draw(D, K.vF, b, (flags & FL_EXTRA) != 0);
+    fang[b] = make_float4(F[3], F[4], F[5], 0.f);
 }
 
 // The same forces with the bead's whole trajectory staged in LDS (positions,
@@ -322,7 +346,7 @@ static hipError_t forces_draw(mte_engine *e, TeaDraw D) {
                            e->T, e->S[e->cur], e->tiles, e->ntiles, e->fxyz, e->fang, D);
     } else {
         const int bs = e->tune.stream_block;
-        const dim3 grid(grid_xcd(e->nb, bs)), block(bs);
+        const dim3 grid(grid_xcd(e->nb, bs)), block(2 * bs);
         auto k = bs == 64 ? k_forces<64, PERIODIC> : bs == 128 ? k_forces<128, PERIODIC> : k_forces<256, PERIODIC>;
         hipLaunchKernelGGL(k, grid, block, 0, e->stream, e->K, e->T, e->S[e->cur], e->fxyz, e->fang, D);
     }
