@@ -477,7 +477,11 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
         if (!(e->box_h[t] >= 0.f)) { e->err = "mte_create: periodic box side must be >= 0"; return bail(MTE_ERR_ARG); }
         if (e->box_h[t] > 0.f) e->periodic = true;
     }
-    e->tune.stream_block = 256;
+    // The smallest of the three ends a block's wait for its slowest list soonest
+    // (64 / 128 / 256, two threads a bead: 200 plain steps of 122646 beads 1875 /
+    // 1939 / 1988 us, 100 of 512948 3198 / 3252 / 3361; 100 MLP-HI steps of 262426
+    // 19.23 / 19.26 / 19.32 ms; 50 TEA steps of 3982 1547 / 1517 / 1542 us).
+    e->tune.stream_block = 64;
     e->tune.tea_chunk = 0;   // set when TEA's work units are built
     e->tune.cell_stencil = 1;
     e->device = opt->device;
