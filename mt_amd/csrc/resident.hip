@@ -609,7 +609,9 @@ static size_t fixed_lds_bytes(int nmax) {
 // takes the two longest independent parts of it.  Per 100 steps, through the
 // API: 1, 256 and 700 tubes of 312 beads 390 -> 288, 514 -> 422 and 1323 ->
 // 1057 us, 1 and 512 tubes of 520 beads (494 mobile) 370 -> 327 and 1079 ->
-// 1000.
+// 1000, 256 of 910 beads (500 mobile) 431 with two beads per thread, 365.
+// From 922 beads on the LDS has no room for the helpers' buffer: one bead per
+// thread alone (64 tubes of 1040 beads, 500 mobile: 405 with two, 394).
 bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     *plan = ResidentPlan{};
     if (e->P.tea_on || pt < 1 || pt > RES_MAX_PT) return false;
@@ -620,9 +622,11 @@ bool resident_plan_for(const mte_engine *e, int pt, ResidentPlan *plan) {
     if (hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device) != hipSuccess)
         return false;
     const int nmain = std::min(((nmax + 63) / 64) * 64, RES_MAX_THREADS / 2);
-    const bool helped = pt == 1 && e->res_mobile_max <= nmain;
-    const size_t fixed = fixed_lds_bytes(nmax) + (helped ? (size_t)XBUF_F4 * sizeof(float4) * nmain : 0);
-    if (fixed + (size_t)MIN_ENTRIES_PER_BEAD * 2 * nmax > (size_t)lds_limit) return false;
+    auto room = [&](size_t fixed) { return fixed + (size_t)MIN_ENTRIES_PER_BEAD * 2 * nmax <= (size_t)lds_limit; };
+    const size_t alone = fixed_lds_bytes(nmax), with_xbuf = alone + (size_t)XBUF_F4 * sizeof(float4) * nmain;
+    const bool helped = pt == 1 && e->res_mobile_max <= nmain && room(with_xbuf);
+    const size_t fixed = helped ? with_xbuf : alone;
+    if (!room(fixed)) return false;
     int threads = (nmax + pt - 1) / pt;
     threads = ((threads + 63) / 64) * 64;
     // One bead per thread also covers a trajectory longer than the largest

@@ -41,3 +41,16 @@ def test_helped_equals_two_per_thread(lengths, side, kick):
     got, want = _run(b, 1, nz), _run(b, 2, nz)
     np.testing.assert_array_equal(got[1], want[1])
     np.testing.assert_array_equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("length", [35, 36, 48])
+def test_one_per_thread_when_the_helpers_find_no_room(length):
+    """Long trajectories, mostly immobile: 500 mobile beads of 910 (the last
+    such tube whose LDS holds the helpers' buffer), of 936 (the first without)
+    and of 1248 (the longest that one bead per thread takes)."""
+    print(f"case one bead per thread, 500 mobile beads, length {length}", flush=True)
+    b = uneven_batch(lengths=(length,), n_free=(0,))
+    b.fixed[500:] = 1
+    got, want = _run(b, 1, None), _run(b, 2, None)
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(got[0], want[0])
