@@ -327,7 +327,9 @@ __device__ __forceinline__ int run_steps_helped(const ForceK &K0, const DevTopo 
             }
         }
         __syncthreads();
-        if (FILTERED && flags[s & 1] != 0) return s + 1;   // uniform: every thread reads the same flag
+        // uniform: set before the barrier, and next written after the barrier
+        // of the following step or, when this returns, never again
+        if (FILTERED && flags[s & 1] != 0) return s + 1;
     }
     return nsteps;
 }
@@ -387,7 +389,7 @@ __global__ void __launch_bounds__(MAXT)
     // has work (its lanes past the mobile beads hold the immobile ones)
     const int m2 = n - (int)blockDim.x;
     // (flags[0] was cleared before the first barrier; the skin test clears it
-    // again in fill before its first use)
+    // again before its first use)
     __syncthreads();
     if (PT == 2 && threadIdx.x >= 256 && W.mob[PT - 1]) flags[0] = 1;
     __syncthreads();
@@ -530,7 +532,6 @@ __global__ void __launch_bounds__(MAXT)
                 }
             hcnt[i] = (hc & 1023) | (nlj << 10);
         }
-        if (threadIdx.x == 0) flags[0] = flags[1] = 0;
         __syncthreads();
     };
     // The full lists decide between LDS and global lists; in LDS, the LJ
@@ -545,6 +546,11 @@ __global__ void __launch_bounds__(MAXT)
         auto mk = [&](int i, int, bool lists) { return LL(ent, lists ? hoff[i] : 0, lists ? hcnt[i] : 0); };
         int s = 0;
         if (filter) {
+            // Cleared once, before the loop that reads them, and not again at
+            // the refill, where waves of the helped loop may still be reading
+            // the flag that ended it (after that step's last barrier).
+            if (threadIdx.x == 0) flags[0] = flags[1] = 0;
+            __syncthreads();
             if constexpr (HELPED)
                 s = run_steps_helped<true, PERIODIC, LL>(K, T, A, t, lx, ln, l1, l2, W, noise, 0, nsteps, L, mk, flags,
                                                          xbuf, nmain, false);

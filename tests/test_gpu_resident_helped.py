@@ -54,3 +54,27 @@ def test_one_per_thread_when_the_helpers_find_no_room(length):
     got, want = _run(b, 1, None), _run(b, 2, None)
     np.testing.assert_array_equal(got[1], want[1])
     np.testing.assert_array_equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("length,out,leaves", [(12, 4.0, 4), (12, 3.5, 5), (20, 4.0, 5), (20, 3.5, 6)])
+def test_drawn_noise_goes_on_across_a_refill(length, out, leaves):
+    """A bead set `out` nm off its place springs back and leaves its skin
+    (0.75 nm from where the launch began) at step `leaves`, even or odd, in the
+    middle of the launch: the lists are refilled and the helper's normals,
+    drawn a step ahead, are used from there on, none twice and none skipped."""
+    print(f"case helped resident steps, refill at step {leaves} of {length}", flush=True)
+    b = uneven_batch(lengths=(length,), n_free=(0,))
+    k = b.nb // 2
+    r = b.coords[k, :2].copy()
+    b.coords[k, :2] += out * r / np.hypot(*r)
+    eng = Engine(base_params(), b.copy(), max_lj=64, mode=MODE_RESIDENT)
+    eng.set_tuning(resident_per_thread=2)
+    moved = []
+    for _ in range(leaves + 1):
+        eng.run(1)
+        moved.append(np.linalg.norm(eng.get_state()[:, :3] - b.coords[:, :3], axis=1).max())
+    eng.close()
+    assert moved[-1] > 0.76 > 0.74 > max(moved[:-1])   # well clear of 0.75 either way
+    got, want = _run(b, 1, None), _run(b, 2, None)
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(got[0], want[0])
