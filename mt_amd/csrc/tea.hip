@@ -55,9 +55,16 @@ __device__ __forceinline__ float pair_coord(float x, double ibox) {
     // 1.5 2^52 leaves the rounded integer in the low mantissa word
     return __int_as_float(__double2loint(fma(v, 4294967296.0, 6755399441055744.0)));
 }
+// Integer places apart, wrapped to the nearest image: the subtraction is
+// unsigned, where wrapping is defined (a signed one does not compile in the
+// constant expression below).
+__host__ __device__ constexpr int wrap_diff(uint32_t a, uint32_t b) { return (int)(a - b); }
+static_assert(wrap_diff(0x7fffffffu, 0x80000000u) == -1 && wrap_diff(0x80000000u, 0x7fffffffu) == 1 &&
+                  wrap_diff(0u, 0x80000000u) == INT32_MIN && wrap_diff(5u, 7u) == -2,
+              "differences across the faces of the box wrap");
 template <bool INT>
 __device__ __forceinline__ float pair_diff(float a, float b) {
-    return INT ? (float)(__float_as_int(a) - __float_as_int(b)) : a - b;
+    return INT ? (float)wrap_diff(__float_as_uint(a), __float_as_uint(b)) : a - b;
 }
 
 // Epsilon partials and ci of bead i over all j of its trajectory
