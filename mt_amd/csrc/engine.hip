@@ -419,6 +419,11 @@ static void flush_timers(mte_engine *e) {
     e->ev_pool.insert(e->ev_pool.end(), done.begin(), done.end());
 }
 
+static void clear_graphs(mte_engine *e) {
+    for (auto &kv : e->graphs) (void)hipGraphExecDestroy(kv.second);
+    e->graphs.clear();
+}
+
 extern "C" {
 
 const char *mte_last_error(const mte_engine *e) { return e ? e->err.c_str() : g_create_error.c_str(); }
@@ -839,7 +844,12 @@ int mte_set_flags(mte_engine *e, const uint8_t *extra, const int32_t *gtp, const
             return fail(e, MTE_ERR_STATE, "mte_set_flags: no resident plan fits the new flags");
         }
         HIPCHK(hipMemcpyAsync(e->T.extra, x.data(), e->nb, hipMemcpyHostToDevice, e->stream));
-        e->any_extra = std::any_of(x.begin(), x.end(), [](uint8_t v) { return v != 0; });
+        const bool any = std::any_of(x.begin(), x.end(), [](uint8_t v) { return v != 0; });
+        if (any != e->any_extra) {   // captured steps hold the epsilon kernel of the old flags
+            HIPCHK(hipStreamSynchronize(e->stream));
+            clear_graphs(e);
+        }
+        e->any_extra = any;
         HIPCHK(upload_resident_order(e, x.data()));
         HIPCHK(hipStreamSynchronize(e->stream));
         if (plan_ok) {
@@ -1507,11 +1517,6 @@ int mte_kernel_time(mte_engine *e, const char *name, double *total_ms, int64_t *
 }  // extern "C"
 
 // ------------------------------------------------------------------ tuning
-static void clear_graphs(mte_engine *e) {
-    for (auto &kv : e->graphs) (void)hipGraphExecDestroy(kv.second);
-    e->graphs.clear();
-}
-
 int mte_get_tuning(const mte_engine *e, mte_tuning *t) {
     if (!e || !t) return MTE_ERR_ARG;
     *t = e->tune;
