@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(TEA_TILE)
 //              j-side sums carried along by a one-lane rotation (wave_rol1);
 //              when c_J lies above all of the wave's chunks, the lane's
 //              beads meet the same j together and share the rotation,
-//   c_J = c    one-sided over the chunk, the j == i term taken out after,
+//   c_J = c    one-sided over the chunk, the j == i term at weight 0,
 //   c_J < c    nothing (that pair of chunks is the wave c_J's).
 // The waves' j-side sums of a chunk are added in wave order in LDS.  Output
 // (deterministic, no atomics): i-side sums of a bead of group H into
@@ -320,18 +320,13 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
 #pragma unroll
         for (int h = 0; h < PER; h++)
             if (cI[h] < nch && cJ == cI[h]) {
-                // one-sided over the chunk's beads
+                // one-sided over the chunk's beads, the bead itself (q == l)
+                // at weight 0: what a coincident bead of weight 1 adds, taken
+                // out afterwards, outgrows the sums where a is small
                 const int jn = min(64, n - cJ * 64);
 #pragma unroll 1
-                for (int q = 0; q < jn; q++) eps_pair<INT, true, ONE_SIDE>(K, xi[h], wi[h], jx[q], ai[h], gj);
-                if (wi[h] != 0.f) {
-                    // the j == i slot entered as a coincident bead (r^2 =
-                    // r2min): cii^2 into the first sum and 3 cii into the
-                    // last, taken out
-                    const float cii = fmaf(-0.28125f, K.r2min * rsq_fast(K.r2min) * K.ia, 1.f);
-                    ai[h][0] = fmaf(-K.i0 * cii, cii, ai[h][0]);
-                    ai[h][4] = fmaf(-K.i4, 3.f * cii, ai[h][4]);
-                }
+                for (int q = 0; q < jn; q++)
+                    eps_pair<INT, true, ONE_SIDE>(K, xi[h], q == l ? 0.f : wi[h], jx[q], ai[h], gj);
             }
         // after a multiple of 64 rotations lane l holds the sums of j =
         // (l + 63) mod 64; with none, gj is zero

@@ -152,3 +152,33 @@ def test_eps_sums_at_group_edges(ntraj, box, extra):
     keep = b.extra == 0
     np.testing.assert_allclose(ci[keep], want_ci[keep], rtol=1e-5, atol=1e-6)
     eng.close()
+
+
+# a from none (free draining) over radii below the clamp of coincident beads
+# (1e-6 nm) to the usual one
+RADII = [0.0, 1e-8, 1e-4, 0.02, 2.0]
+
+
+@pytest.mark.parametrize("a", RADII)
+@pytest.mark.parametrize("box", [0.0, 300.0])
+def test_eps_sums_of_any_radius(a, box):
+    """Epsilon and ci hold no trace of the bead itself, however small the
+    other beads' terms are."""
+    print(f"case TEA eps, a={a}, box={box}", flush=True)
+    p = P.derive(dict(P.TEA, tea_epsilon_freq=1, tea_capricious=False))
+    p.tea_a = a
+    b = _dimers((97, 20), box, 7)
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    eng.set_tuning(tea_chunk=TEA_SYMMETRIC)
+    eng.set_noise(np.zeros((1, b.nb, 6), np.float32))
+    eng.run(1)
+    eps, beta = eng.tea_stats()
+    ci = eng.tea_ci().astype(np.float64)
+    eng.close()
+    p.tea_a = max(a, 1e-30)   # (the FP64 sums divide by it; a^2 is below any float)
+    want_eps, want_ci = _eps_ci(p, b)
+    # FP32 sums of up to 200 positive terms
+    np.testing.assert_allclose(eps, want_eps, rtol=1e-5, atol=1e-25)
+    np.testing.assert_allclose(ci, want_ci, rtol=1e-5, atol=1e-37)
+    if a <= 1e-8:
+        np.testing.assert_array_equal(beta, 0.5)   # |a_TEA| < 1e-7
