@@ -504,14 +504,18 @@ struct PairBead {
 };
 // sc: nm per loop unit.
 __device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float sc) {
-    const float a = P.tea_a / sc, lim = 2.002f * a;
+    const float a = P.tea_a / sc, a1 = fmaxf(P.tea_a, 1e-15f);
+    // Coincident beads are taken apart to 1e-6 nm, or to a where that is less:
+    // they are near ones (r <= 2a) for every radius, 0 among them, where the
+    // far coefficients are infinite or undefined.
+    const float am = a1 / sc, lim = 2.002f * am;
     PairCoef K;
     K.k1 = in_vgpr(0.75f * a);
     K.k3 = in_vgpr(0.5f * a * a * a);
     K.k5 = in_vgpr(-1.5f * a * a * a);
     K.near2 = in_vgpr(lim * lim);
-    K.ia = sc * rcp_fast(P.tea_a);
-    K.r2min = 1e-12f / (sc * sc);
+    K.ia = sc * rcp_fast(a1);
+    K.r2min = fminf(1e-12f / (sc * sc), am * am);
     return K;
 }
 

@@ -182,3 +182,29 @@ def test_eps_sums_of_any_radius(a, box):
     np.testing.assert_allclose(ci, want_ci, rtol=1e-5, atol=1e-37)
     if a <= 1e-8:
         np.testing.assert_array_equal(beta, 0.5)   # |a_TEA| < 1e-7
+
+
+@pytest.mark.parametrize("a", RADII)
+@pytest.mark.parametrize("box", [0.0, 300.0])
+@pytest.mark.parametrize("chunk", [64, 128, 256, TEA_SYMMETRIC])
+def test_pair_sums_of_any_radius(a, box, chunk):
+    """The one-sided kernels meet the bead itself, at distance 0, and take it
+    out: for every radius."""
+    print(f"case TEA pairs, a={a}, box={box}, chunk={chunk}", flush=True)
+    p = P.derive(dict(P.TEA, tea_epsilon_freq=1, tea_capricious=False, dt=1000.0, LJPairsCutoff=8.0))
+    p.tea_a = a
+    b = _dimers((97, 20), box, 7)
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    eng.set_tuning(tea_chunk=chunk)
+    F = eng.forces()[:, :3].astype(np.float64)
+    eng.set_noise(np.zeros((1, b.nb, 6), np.float32))
+    eng.run(1)
+    moved = eng.get_state()[:, :3].astype(np.float64) - b.coords[:, :3].astype(np.float64)
+    eng.close()
+    p.tea_a = max(a, 1e-30)
+    want = p.dt / p.gammaR * _drift(p, b, F)
+    ok = np.isfinite(want[:, 0])
+    assert ok.mean() > 0.99
+    # the sums' FP32 rounding (1e-5 of the largest move) and the state's own
+    tol = 1e-5 * np.abs(want[ok]).max() + 2 * 2.0 ** -24 * np.abs(b.coords[:, :3]).max()
+    assert np.abs(moved - want)[ok].max() <= tol
