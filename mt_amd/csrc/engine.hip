@@ -481,6 +481,7 @@ int mte_create(const mte_params *params, const mte_topology *topo, const mte_opt
     for (int t = 0; t < nt; t++) {
         if (!(e->box_h[t] >= 0.f)) { e->err = "mte_create: periodic box side must be >= 0"; return bail(MTE_ERR_ARG); }
         if (e->box_h[t] > 0.f) e->periodic = true;
+        e->box_max = std::max(e->box_max, e->box_h[t]);
     }
     // The smallest of the three ends a block's wait for its slowest list soonest
     // (64 / 128 / 256, two threads a bead: 200 plain steps of 122646 beads 1875 /

@@ -171,6 +171,7 @@ struct mte_engine {
     int *res_order = nullptr;  // per trajectory: local bead at each resident lane slot (immobile beads last)
     std::vector<uint8_t> fixed_h;   // host copy of the fixed flags (the resident lane order)
     std::vector<float> box_h;        // and of the periodic box sides
+    float box_max = 0.f;             // the longest of them
     int res_mobile_max = 0;          // most mobile beads in one trajectory (the resident plan)
     bool any_extra = false;          // some bead is flagged extra (TEA's epsilon weights are needed)
     int *mtl_counts = nullptr, *mtl_flags = nullptr;   // mte_mt_length: per trajectory, per bead

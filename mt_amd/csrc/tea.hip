@@ -45,11 +45,29 @@ __device__ __forceinline__ float wave_rol1(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x134, 0xF, 0xF, false));
 }
 
-// One coordinate of the pair loops: x itself, or (INT) its place in the
+// How the pair loops take a pair's nearest image: not at all (open), by
+// coordinates that are 32-bit integers of box / 2^32, whose difference wraps
+// by itself, or in float from nm.  The integers cost 18 issue cycles a pair,
+// the float image 30, but their quantum grows with the box, where the float
+// difference of two near beads is exact: a tube of 312 beads at the origin
+// moves in one step with an error (FP64, of the largest move) of 3-5e-7 by
+// either in boxes up to 4096 nm (2^-20 nm, a quarter of the rounding of a
+// coordinate there), by the integers with 5e-6 at 1e5 and 4e-5 at 1e6 nm.
+enum PairBox { OPEN_BOX, INT_BOX, FLOAT_BOX };
+constexpr float INT_BOX_MAX = 4096.f;
+// A batch's kernels are made for one of them: open batches, those whose boxes
+// are all within INT_BOX_MAX (an open trajectory among them is taken as such),
+// and the rest (there a float image with a box of 0 changes nothing).
+constexpr PairBox unboxed(PairBox b) { return b == FLOAT_BOX ? FLOAT_BOX : OPEN_BOX; }
+static PairBox batch_box(const mte_engine *e) {
+    return !e->periodic ? OPEN_BOX : e->box_max <= INT_BOX_MAX ? INT_BOX : FLOAT_BOX;
+}
+
+// One coordinate of the pair loops: x itself, or (INT_BOX) its place in the
 // periodic box as a 32-bit integer (bit pattern), taken modulo the box in FP64.
-template <bool INT>
+template <PairBox BOX>
 __device__ __forceinline__ float pair_coord(float x, double ibox) {
-    if (!INT) return x;
+    if (BOX != INT_BOX) return x;
     double v = (double)x * ibox;
     v -= rint(v);
     // 1.5 2^52 leaves the rounded integer in the low mantissa word
@@ -62,9 +80,12 @@ __host__ __device__ constexpr int wrap_diff(uint32_t a, uint32_t b) { return (in
 static_assert(wrap_diff(0x7fffffffu, 0x80000000u) == -1 && wrap_diff(0x80000000u, 0x7fffffffu) == 1 &&
                   wrap_diff(0u, 0x80000000u) == INT32_MIN && wrap_diff(5u, 7u) == -2,
               "differences across the faces of the box wrap");
-template <bool INT>
-__device__ __forceinline__ float pair_diff(float a, float b) {
-    return INT ? (float)wrap_diff(__float_as_uint(a), __float_as_uint(b)) : a - b;
+// side, iside: the box and its inverse (FLOAT_BOX; both 0 on open boundaries).
+template <PairBox BOX>
+__device__ __forceinline__ float pair_diff(float a, float b, float side, float iside) {
+    if (BOX == INT_BOX) return (float)wrap_diff(__float_as_uint(a), __float_as_uint(b));
+    const float d = a - b;
+    return BOX == FLOAT_BOX ? d - side * rintf(d * iside) : d;
 }
 
 // Epsilon partials and ci of bead i over all j of its trajectory
@@ -179,6 +200,7 @@ struct EpsCoef {
     float s2, c1, c2, c3, c4;   // a^2 and its multiples 2/3, -2, -2/3, 2
     float near2, ia, r2min;     // (2a)^2 with its margin, 1 / a, the floor of r^2
     float i0, i4;               // 1 / (9/16 a^2), 1 / (3/4 a)
+    float side, iside;          // FLOAT_BOX: the box
 };
 
 // One pair's five terms: added to the sums t and, unless ONE_SIDE, to t2,
@@ -186,10 +208,10 @@ struct EpsCoef {
 // rotation, done with the first of the lane's beads to meet this j).  WT: the
 // pair's weight ww is formed.
 enum EpsSides { ONE_SIDE, BOTH_SIDES, ROTATE };
-template <bool INT, bool WT, EpsSides SIDES>
+template <PairBox BOX, bool WT, EpsSides SIDES>
 __device__ __forceinline__ void eps_pair(const EpsCoef &K, float3 xa, float wa, float4 xj, float (&t)[5],
                                          float (&t2)[5]) {
-    const float dx = pair_diff<INT>(xj.x, xa.x), dy = pair_diff<INT>(xj.y, xa.y), dz = pair_diff<INT>(xj.z, xa.z);
+    const float dx = pair_diff<BOX>(xj.x, xa.x, K.side, K.iside), dy = pair_diff<BOX>(xj.y, xa.y, K.side, K.iside), dz = pair_diff<BOX>(xj.z, xa.z, K.side, K.iside);
     // r2min (1e-12 nm^2) keeps coincident beads finite and is below the
     // rounding of any other r^2
     const float qx = dx * dx, qy = dy * dy, qz = fmaf(dz, dz, K.r2min);
@@ -230,19 +252,19 @@ __device__ __forceinline__ void eps_pair(const EpsCoef &K, float3 xa, float wa, 
 }
 
 // The lane's N beads against every j of the staged chunk, both sides.
-template <bool INT, bool WT, int N>
+template <PairBox BOX, bool WT, int N>
 __device__ __forceinline__ void eps_sweep(const EpsCoef &K, const float4 *jl, const float3 *xi, const float *wi,
                                           float (*ai)[5], float (&gj)[5]) {
 #pragma unroll 1
     for (int s = 0; s < 64; s++) {
         const float4 xj = jl[s];
-        eps_pair<INT, WT, ROTATE>(K, xi[0], wi[0], xj, ai[0], gj);
+        eps_pair<BOX, WT, ROTATE>(K, xi[0], wi[0], xj, ai[0], gj);
 #pragma unroll
-        for (int h = 1; h < N; h++) eps_pair<INT, WT, BOTH_SIDES>(K, xi[h], wi[h], xj, ai[h], gj);
+        for (int h = 1; h < N; h++) eps_pair<BOX, WT, BOTH_SIDES>(K, xi[h], wi[h], xj, ai[h], gj);
     }
 }
 
-template <bool INT, bool WEIGHTED, int PER>
+template <PairBox BOX, bool WEIGHTED, int PER>
 __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, const DevState &S, int4 u, int ngrp,
                                          float *part, float4 *jx, float (*jred)[5][64]) {
     constexpr int WAVES = eps_waves(PER), CHUNKS = WAVES * PER;
@@ -250,8 +272,8 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
     const int base = T.tbase[u.x], n = T.tsize[u.x], nb = T.nb;
     const int nch = (n + 63) / 64;
     const float box = T.tbox[u.x];
-    const double ibox = INT ? 1.0 / (double)box : 0.0;
-    const float sc = INT ? box * 0x1p-32f : 1.f;   // nm per loop unit
+    const double ibox = BOX == INT_BOX ? 1.0 / (double)box : 0.0;
+    const float sc = BOX == INT_BOX ? box * 0x1p-32f : 1.f;   // nm per loop unit
     const float a = P.tea_a / sc, s2 = a * a, lim = 2.002f * a;
     EpsCoef K;
     K.s2 = s2;
@@ -264,6 +286,8 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
     K.r2min = in_vgpr(1e-12f / (sc * sc));
     K.i0 = 1.f / (0.5625f * s2);
     K.i4 = 1.f / (0.75f * a);
+    K.side = in_vgpr(box);
+    K.iside = in_vgpr(inv_side(box));
     // the lane's bead in each of the wave's chunks
     int cI[PER];
     bool vi[PER];
@@ -275,9 +299,9 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
         const float3 x = f3(S.xyz[base + li]);
         // a lost position (inf, NaN), which an integer cannot hold, spreads
         // through the bead's weight as it would through r
-        const float lost = INT ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
+        const float lost = BOX == INT_BOX ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
         wt = (T.extra[base + li] ? 0.f : 1.f) + lost;
-        return make_float3(pair_coord<INT>(x.x, ibox), pair_coord<INT>(x.y, ibox), pair_coord<INT>(x.z, ibox));
+        return make_float3(pair_coord<BOX>(x.x, ibox), pair_coord<BOX>(x.y, ibox), pair_coord<BOX>(x.z, ibox));
     };
     bool odd = false;   // a lost bead among the lane's own
 #pragma unroll
@@ -310,12 +334,12 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
 #pragma unroll
         for (int h = 0; h < PER; h++) low += cI[h] < nch && cJ > cI[h] ? 1 : 0;
         if (low == PER) {
-            if (wtj) eps_sweep<INT, true, PER>(K, jl, xi, wi, ai, gj);
-            else eps_sweep<INT, false, PER>(K, jl, xi, wi, ai, gj);
+            if (wtj) eps_sweep<BOX, true, PER>(K, jl, xi, wi, ai, gj);
+            else eps_sweep<BOX, false, PER>(K, jl, xi, wi, ai, gj);
         } else if (PER > 1) {
 #pragma unroll
             for (int h = 0; h < PER; h++)
-                if (h < low) eps_sweep<INT, true, 1>(K, jl, xi + h, wi + h, ai + h, gj);
+                if (h < low) eps_sweep<BOX, true, 1>(K, jl, xi + h, wi + h, ai + h, gj);
         }
 #pragma unroll
         for (int h = 0; h < PER; h++)
@@ -326,7 +350,7 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
                 const int jn = min(64, n - cJ * 64);
 #pragma unroll 1
                 for (int q = 0; q < jn; q++)
-                    eps_pair<INT, true, ONE_SIDE>(K, xi[h], q == l ? 0.f : wi[h], jx[q], ai[h], gj);
+                    eps_pair<BOX, true, ONE_SIDE>(K, xi[h], q == l ? 0.f : wi[h], jx[q], ai[h], gj);
             }
         // after a multiple of 64 rotations lane l holds the sums of j =
         // (l + 63) mod 64; with none, gj is zero
@@ -354,14 +378,14 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
         }
 }
 
-template <bool PERIODIC, bool WEIGHTED, int PER>
+template <PairBox BOX, bool WEIGHTED, int PER>
 __global__ void __launch_bounds__(64 * eps_waves(PER))
     k_tea_eps_sym(mte_params P, DevTopo T, DevState S, const int4 *units, int ngrp, float *part) {
     __shared__ float4 jx[2 * 64];              // chunk c_J: x, weight; twice, no wrap
     __shared__ float jred[eps_waves(PER)][5][64];   // j-side sums of each wave
     const int4 u = units[blockIdx.x];
-    if (PERIODIC && T.tbox[u.x] > 0.f) eps_unit<true, WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
-    else eps_unit<false, WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
+    if (BOX == INT_BOX && T.tbox[u.x] > 0.f) eps_unit<INT_BOX, WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
+    else eps_unit<unboxed(BOX), WEIGHTED, PER>(P, T, S, u, ngrp, part, jx, jred);
 }
 
 // Per bead: the group sums of k_tea_eps_sym added in fixed order into ci and
@@ -473,11 +497,11 @@ __global__ void __launch_bounds__(256)
 // in slot order).  Beads past the trajectory's end and extra beads carry
 // zero F and R, so their terms vanish.
 //
-// Lengths in the loop are nm on open boundaries.  In a periodic box they are
-// units of box / 2^32 and positions 32-bit integers, so a difference wraps
-// to the minimum image by itself: 3 subtractions and 3 conversions (18 issue
-// cycles) instead of subtract, scale, round, fused subtract (30).  A float
-// position far from the origin is the coarser of the two.
+// Lengths in the loop are nm on open boundaries and in large boxes (PairBox).
+// In other periodic boxes they are units of box / 2^32 and positions 32-bit
+// integers, so a difference wraps to the minimum image by itself: 3
+// subtractions and 3 conversions (18 issue cycles) instead of subtract, scale,
+// round, fused subtract (30).
 // The coefficients are those beyond 2a; a wave with a pair inside 2a (margin
 // over the rounding of r / a) selects the near ones in a branch.
 //
@@ -498,12 +522,14 @@ constexpr int SYM_CHUNK = 64;
 struct PairCoef {
     float k1, k3, k5;       // cii = k1 w + k3 w^3, crr / r^2 = w^3 (k1 + k5 w^2), w = 1 / r in loop units
     float near2, ia, r2min; // (2a)^2 with its margin, 1 / a, the clamp of coincident beads
+    float side, iside;      // FLOAT_BOX: the box
 };
 struct PairBead {
     float3 x, F, R, C;      // position (loop units), force, random force, beta C
 };
-// sc: nm per loop unit.
-__device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float sc) {
+template <PairBox BOX>
+__device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float box) {
+    const float sc = BOX == INT_BOX ? box * 0x1p-32f : 1.f;   // nm per loop unit
     const float a = P.tea_a / sc, a1 = fmaxf(P.tea_a, 1e-15f);
     // Coincident beads are taken apart to 1e-6 nm, or to a where that is less:
     // they are near ones (r <= 2a) for every radius, 0 among them, where the
@@ -516,21 +542,23 @@ __device__ __forceinline__ PairCoef pair_coef(const mte_params &P, float sc) {
     K.near2 = in_vgpr(lim * lim);
     K.ia = sc * rcp_fast(a1);
     K.r2min = fminf(1e-12f / (sc * sc), am * am);
+    K.side = in_vgpr(box);
+    K.iside = in_vgpr(inv_side(box));
     return K;
 }
 
 // Bead b (zeros where it is not valid); extra beads have zero F and R.
-template <bool INT>
+template <PairBox BOX>
 __device__ __forceinline__ PairBead pair_bead(const float4 *xyz, const float4 *fxyz, const float4 *R, const float4 *bc,
                                               int b, bool valid, double ibox) {
     PairBead v;
     v.x = v.F = v.R = v.C = make_float3(0.f, 0.f, 0.f);
     if (valid) {
         const float3 x = f3(xyz[b]), F = f3(fxyz[b]);
-        v.x = make_float3(pair_coord<INT>(x.x, ibox), pair_coord<INT>(x.y, ibox), pair_coord<INT>(x.z, ibox));
+        v.x = make_float3(pair_coord<BOX>(x.x, ibox), pair_coord<BOX>(x.y, ibox), pair_coord<BOX>(x.z, ibox));
         // zero for a finite position; a lost one (inf, NaN), which an
         // integer cannot hold, spreads through F as it would through r
-        const float lost = INT ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
+        const float lost = BOX == INT_BOX ? (x.x - x.x) + (x.y - x.y) + (x.z - x.z) : 0.f;
         v.F = make_float3(F.x + lost, F.y + lost, F.z + lost);
         v.R = f3(R[b]);
         v.C = f3(bc[b]);
@@ -540,10 +568,10 @@ __device__ __forceinline__ PairBead pair_bead(const float4 *xyz, const float4 *f
 
 // Bead I against the j of (A, B, Cq): i-side into acc, and j-side into g
 // (BOTH).
-template <bool INT, bool BOTH>
+template <PairBox BOX, bool BOTH>
 __device__ __forceinline__ void pair_block(const PairCoef &K, const PairBead &I, float4 A, float4 B, float4 Cq,
                                            float3 &acc, float3 &g) {
-    const float dx = pair_diff<INT>(A.x, I.x.x), dy = pair_diff<INT>(A.y, I.x.y), dz = pair_diff<INT>(A.z, I.x.z);
+    const float dx = pair_diff<BOX>(A.x, I.x.x, K.side, K.iside), dy = pair_diff<BOX>(A.y, I.x.y, K.side, K.iside), dz = pair_diff<BOX>(A.z, I.x.z, K.side, K.iside);
     const float r2 = dx * dx + dy * dy + dz * dz;
     const float w = rsq_fast(r2);
     const float w2 = w * w;
@@ -579,26 +607,26 @@ __device__ __forceinline__ void rotate(float3 &g) {
     g.z = wave_rol1(g.z);
 }
 
-template <bool INT, int SPLIT>
+template <PairBox BOX, int SPLIT>
 __device__ __forceinline__ void pair_unit(const mte_params &P, const PairUnit &U, int nb, const float4 *xyz,
                                           const float4 *fxyz, const float4 *R, const float4 *bc, int jrun, int ioff,
                                           float *partial, float4 (*jd)[2 * SYM_CHUNK],
                                           float (*red)[9][SPLIT == 1 ? 1 : SYM_CHUNK]) {
     const int l = threadIdx.x % SYM_CHUNK, k = threadIdx.x / SYM_CHUNK;
     const int base = U.base, n = U.n, pair = U.pair, J0 = U.J0, J1 = U.J0 + U.nJ;
-    const double ibox = INT ? 1.0 / (double)U.box : 0.0;
-    const PairCoef K = pair_coef(P, INT ? U.box * 0x1p-32f : 1.f);
+    const double ibox = BOX == INT_BOX ? 1.0 / (double)U.box : 0.0;
+    const PairCoef K = pair_coef<BOX>(P, U.box);
     const int c0 = 2 * pair, i0 = c0 * SYM_CHUNK + l;
     PairBead I[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const int li = i0 + h * SYM_CHUNK;
-        I[h] = pair_bead<INT>(xyz, fxyz, R, bc, base + li, li < n, ibox);
+        I[h] = pair_bead<BOX>(xyz, fxyz, R, bc, base + li, li < n, ibox);
     }
     float3 acc[2] = {make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f)};
     auto load_j = [&](int J) {
         const int lj = J * SYM_CHUNK + l;
-        return pair_bead<INT>(xyz, fxyz, R, bc, base + lj, lj < n, ibox);
+        return pair_bead<BOX>(xyz, fxyz, R, bc, base + lj, lj < n, ibox);
     };
     PairBead next{};
     if (SPLIT == 1) next = load_j(J0);
@@ -628,15 +656,15 @@ __device__ __forceinline__ void pair_unit(const mte_params &P, const PairUnit &U
 #pragma unroll 1
             for (int s = s0; s < s1; s++) {
                 const float4 A = j0[s], B = j1[s], Cq = j2[s];
-                pair_block<INT, true>(K, I[0], A, B, Cq, acc[0], g);
-                pair_block<INT, true>(K, I[1], A, B, Cq, acc[1], g);
+                pair_block<BOX, true>(K, I[0], A, B, Cq, acc[0], g);
+                pair_block<BOX, true>(K, I[1], A, B, Cq, acc[1], g);
                 rotate(g);
             }
         } else {
             if (J > c0)
 #pragma unroll 1
                 for (int s = s0; s < s1; s++) {
-                    pair_block<INT, true>(K, I[0], j0[s], j1[s], j2[s], acc[0], g);
+                    pair_block<BOX, true>(K, I[0], j0[s], j1[s], j2[s], acc[0], g);
                     rotate(g);
                 }
             const int h = J - c0;
@@ -645,10 +673,10 @@ __device__ __forceinline__ void pair_unit(const mte_params &P, const PairUnit &U
             const int t0 = 1 + k * D, t1 = t0 + D, t2 = min(t1, SYM_CHUNK / 2);
 #pragma unroll 1
             for (int s = t0; s < t2; s++) {
-                pair_block<INT, true>(K, D0, j0[s], j1[s], j2[s], own, gd);
+                pair_block<BOX, true>(K, D0, j0[s], j1[s], j2[s], own, gd);
                 rotate(gd);
             }
-            if (t2 < t1) pair_block<INT, false>(K, D0, j0[t2], j1[t2], j2[t2], own, gd);
+            if (t2 < t1) pair_block<BOX, false>(K, D0, j0[t2], j1[t2], j2[t2], own, gd);
             // lane l holds the j-side sums of bead l + t2 of the chunk
             const int src = (l - t2) & (SYM_CHUNK - 1);
             own.x += __shfl(gd.x, src);
@@ -714,7 +742,7 @@ __device__ __forceinline__ void pair_unit(const mte_params &P, const PairUnit &U
     }
 }
 
-template <bool PERIODIC, int SPLIT>
+template <PairBox BOX, int SPLIT>
 __global__ void __launch_bounds__(SYM_CHUNK *SPLIT, 5)
     k_tea_pairs_sym(mte_params P, int nb, const float4 *xyz, const float4 *fxyz, const float4 *R, const float4 *bc,
                     const PairUnit *units, int jrun, int ioff, float *partial) {
@@ -722,10 +750,10 @@ __global__ void __launch_bounds__(SYM_CHUNK *SPLIT, 5)
     __shared__ float4 jd[3][2 * SYM_CHUNK];
     __shared__ float red[SPLIT][9][SPLIT == 1 ? 1 : SYM_CHUNK];
     const PairUnit U = units[blockIdx.x];
-    if (PERIODIC && U.box > 0.f)
-        pair_unit<true, SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
+    if (BOX == INT_BOX && U.box > 0.f)
+        pair_unit<INT_BOX, SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
     else
-        pair_unit<false, SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
+        pair_unit<unboxed(BOX), SPLIT>(P, U, nb, xyz, fxyz, R, bc, jrun, ioff, partial, jd, red);
 }
 
 // Pair sums of one (trajectory, 256-bead i group, j chunk) work unit:
@@ -736,17 +764,17 @@ __global__ void __launch_bounds__(SYM_CHUNK *SPLIT, 5)
 // image of a pair half a box apart.
 // Splitting j into chunks gives ~10 work units per SIMD at 64 x 1040 beads,
 // against ~1 per SIMD for one thread per bead over the whole trajectory.
-template <bool INT, int CHUNK>
+template <PairBox BOX, int CHUNK>
 __device__ __forceinline__ void pair_chunk(const mte_params &P, const DevTopo &T, const DevState &S, const float4 *fxyz,
                                            const float4 *R, const float4 *bc, int4 u, float4 *partial,
                                            float4 (*jd)[CHUNK]) {
     const int base = T.tbase[u.x], n = T.tsize[u.x];
     const float box = T.tbox[u.x];
-    const double ibox = INT ? 1.0 / (double)box : 0.0;
-    const PairCoef K = pair_coef(P, INT ? box * 0x1p-32f : 1.f);
+    const double ibox = BOX == INT_BOX ? 1.0 / (double)box : 0.0;
+    const PairCoef K = pair_coef<BOX>(P, box);
     const int jn = min(CHUNK, n - u.z);
     for (int q = threadIdx.x; q < jn; q += TEA_TILE) {
-        const PairBead v = pair_bead<INT>(S.xyz, fxyz, R, bc, base + u.z + q, true, ibox);
+        const PairBead v = pair_bead<BOX>(S.xyz, fxyz, R, bc, base + u.z + q, true, ibox);
         jd[0][q] = make_float4(v.x.x, v.x.y, v.x.z, v.F.x);
         jd[1][q] = make_float4(v.F.y, v.F.z, v.R.x, v.R.y);
         jd[2][q] = make_float4(v.R.z, v.C.x, v.C.y, v.C.z);
@@ -757,9 +785,9 @@ __device__ __forceinline__ void pair_chunk(const mte_params &P, const DevTopo &T
     const int b = base + li;
     float3 acc = make_float3(0.f, 0.f, 0.f);
     if (!T.extra[b]) {
-        const PairBead I = pair_bead<INT>(S.xyz, fxyz, R, bc, b, true, ibox);
+        const PairBead I = pair_bead<BOX>(S.xyz, fxyz, R, bc, b, true, ibox);
         float3 none = acc;
-        for (int q = 0; q < jn; q++) pair_block<INT, false>(K, I, jd[0][q], jd[1][q], jd[2][q], acc, none);
+        for (int q = 0; q < jn; q++) pair_block<BOX, false>(K, I, jd[0][q], jd[1][q], jd[2][q], acc, none);
         const int self = li - u.z;   // position of i in this chunk, if any
         if (self >= 0 && self < jn) {
             // The loop took the j == i slot as a coincident bead: d = 0 leaves
@@ -774,16 +802,16 @@ __device__ __forceinline__ void pair_chunk(const mte_params &P, const DevTopo &T
     partial[(size_t)u.w * T.nb + b] = make_float4(acc.x, acc.y, acc.z, 0.f);
 }
 
-template <int CHUNK, bool PERIODIC>
+template <int CHUNK, PairBox BOX>
 __global__ void __launch_bounds__(TEA_TILE)
     k_tea_pairs(mte_params P, DevTopo T, DevState S, const float4 *fxyz, const float4 *R, const float4 *bc,
                 const int4 *units, float4 *partial) {
     __shared__ float4 jd[3][CHUNK];
     const int4 u = units[blockIdx.x];   // traj, i0, j0, chunk index
-    if (PERIODIC && T.tbox[u.x] > 0.f)
-        pair_chunk<true, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
+    if (BOX == INT_BOX && T.tbox[u.x] > 0.f)
+        pair_chunk<INT_BOX, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
     else
-        pair_chunk<false, CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
+        pair_chunk<unboxed(BOX), CHUNK>(P, T, S, fxyz, R, bc, u, partial, jd);
 }
 
 // What the update of a bead adds up and moves, k_tea_finish and k_tea_turn.
@@ -1387,12 +1415,19 @@ __global__ void __launch_bounds__(256)
     partial[(size_t)slot * chunk_stride + bi] = make_float4(f.x, f.y, f.z, 0.f);
 }
 
-template <int PER>
-static void launch_eps_per(mte_engine *e) {
-    auto kern = e->periodic ? (e->any_extra ? k_tea_eps_sym<true, true, PER> : k_tea_eps_sym<true, false, PER>)
-                            : (e->any_extra ? k_tea_eps_sym<false, true, PER> : k_tea_eps_sym<false, false, PER>);
+template <PairBox BOX, int PER>
+static void launch_eps_box(mte_engine *e) {
+    auto kern = e->any_extra ? k_tea_eps_sym<BOX, true, PER> : k_tea_eps_sym<BOX, false, PER>;
     hipLaunchKernelGGL(kern, dim3(e->tea.eps_nunits), dim3(64 * eps_waves(PER)), 0, e->stream, e->P, e->T, e->S[e->cur],
                        e->tea.eps_units, e->tea.eps_ngrp, e->tea.eps_part);
+}
+template <int PER>
+static void launch_eps_per(mte_engine *e) {
+    switch (batch_box(e)) {
+    case OPEN_BOX: launch_eps_box<OPEN_BOX, PER>(e); break;
+    case INT_BOX: launch_eps_box<INT_BOX, PER>(e); break;
+    case FLOAT_BOX: launch_eps_box<FLOAT_BOX, PER>(e); break;
+    }
 }
 static void launch_eps_units(mte_engine *e) {
     if (e->tea.eps_group == EPS_GROUP_MIN) launch_eps_per<1>(e);
@@ -1418,20 +1453,31 @@ hipError_t launch_tea_eps(mte_engine *e) {
 
 template <int CHUNK>
 static void launch_pairs_chunk(mte_engine *e) {
-    auto kern = e->periodic ? k_tea_pairs<CHUNK, true> : k_tea_pairs<CHUNK, false>;
+    const PairBox box = batch_box(e);
+    auto kern = box == OPEN_BOX ? k_tea_pairs<CHUNK, OPEN_BOX>
+                : box == INT_BOX ? k_tea_pairs<CHUNK, INT_BOX> : k_tea_pairs<CHUNK, FLOAT_BOX>;
     hipLaunchKernelGGL(kern, dim3(e->tea.nunits), dim3(TEA_TILE), 0, e->stream, e->P, e->T, e->S[e->cur], e->fxyz,
                        e->tea.R, e->tea.bc, e->tea.units, e->tea.partial);
+}
+
+template <int SPLIT>
+static void launch_pairs_sym(mte_engine *e) {
+    const PairBox box = batch_box(e);
+    auto kern = box == OPEN_BOX ? k_tea_pairs_sym<OPEN_BOX, SPLIT>
+                : box == INT_BOX ? k_tea_pairs_sym<INT_BOX, SPLIT> : k_tea_pairs_sym<FLOAT_BOX, SPLIT>;
+    hipLaunchKernelGGL(kern, dim3(e->tea.nunits), dim3(SYM_CHUNK * SPLIT), 0, e->stream, e->P, e->nb,
+                       e->S[e->cur].xyz, e->fxyz, e->tea.R, e->tea.bc, e->tea.pair_units, e->tea.jrun,
+                       e->tea.ioff, reinterpret_cast<float *>(e->tea.partial));
 }
 
 hipError_t launch_tea_pairs(mte_engine *e) {
     // the kernel's chunk must be the one the work units were built for
     if (e->tea.unit_chunk == MTE_TEA_SYMMETRIC) {
-        auto kern = e->tea.split == 8   ? (e->periodic ? k_tea_pairs_sym<true, 8> : k_tea_pairs_sym<false, 8>)
-                    : e->tea.split == 4 ? (e->periodic ? k_tea_pairs_sym<true, 4> : k_tea_pairs_sym<false, 4>)
-                                        : (e->periodic ? k_tea_pairs_sym<true, 1> : k_tea_pairs_sym<false, 1>);
-        hipLaunchKernelGGL(kern, dim3(e->tea.nunits), dim3(SYM_CHUNK * e->tea.split), 0, e->stream, e->P, e->nb,
-                           e->S[e->cur].xyz, e->fxyz, e->tea.R, e->tea.bc, e->tea.pair_units, e->tea.jrun,
-                           e->tea.ioff, reinterpret_cast<float *>(e->tea.partial));
+        switch (e->tea.split) {
+        case 8: launch_pairs_sym<8>(e); break;
+        case 4: launch_pairs_sym<4>(e); break;
+        default: launch_pairs_sym<1>(e); break;
+        }
         return hipGetLastError();
     }
     if (e->tea.unit_chunk == MTE_TEA_MFMA) {

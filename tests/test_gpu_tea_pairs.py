@@ -208,3 +208,58 @@ def test_pair_sums_of_any_radius(a, box, chunk):
     # the sums' FP32 rounding (1e-5 of the largest move) and the state's own
     tol = 1e-5 * np.abs(want[ok]).max() + 2 * 2.0 ** -24 * np.abs(b.coords[:, :3]).max()
     assert np.abs(moved - want)[ok].max() <= tol
+
+
+# the largest box of the integer coordinates, the next float, and boxes whose
+# 2^-32 is no longer below the rounding of a pair's distance
+@pytest.mark.parametrize("box", [1000.0, 4096.0, float(np.nextafter(np.float32(4096), np.float32(1e9))), 1e6, 1e7])
+@pytest.mark.parametrize("chunk", [128, TEA_SYMMETRIC])
+def test_tube_at_the_origin_of_a_large_box(box, chunk):
+    """Beads that are near one another and near the origin keep the precision
+    of their float differences however large the box."""
+    print(f"case TEA tube in a box of {box}, chunk={chunk}", flush=True)
+    p = P.derive(dict(P.TEA, tea_epsilon_freq=1, dt=1000.0))
+    at = lattice.microtubule(12)
+    b = topology.make_batch([at, at], [lattice.coords7(at, 0.2, np.random.default_rng(k)) for k in (3, 4)],
+                            box=[box, 0.0])
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    eng.set_tuning(tea_chunk=chunk)
+    F = eng.forces()[:, :3].astype(np.float64)
+    eng.set_noise(np.zeros((1, b.nb, 6), np.float32))
+    eng.run(1)
+    moved = eng.get_state()[:, :3].astype(np.float64) - b.coords[:, :3].astype(np.float64)
+    eps, _ = eng.tea_stats()
+    ci = eng.tea_ci().astype(np.float64)
+    eng.close()
+    want = p.dt / p.gammaR * _drift(p, b, F)
+    want_eps, want_ci = _eps_ci(p, b)
+    free = b.fixed == 0
+    # the sums' FP32 rounding (1e-5 of the largest move) and the state's own
+    tol = 1e-5 * np.abs(want).max() + 2 * 2.0 ** -24 * np.abs(b.coords[:, :3]).max()
+    assert np.abs(moved - want)[free].max() <= tol
+    np.testing.assert_allclose(eps, want_eps, rtol=1e-5)
+    np.testing.assert_allclose(ci, want_ci, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("chunk", [128, TEA_SYMMETRIC])
+def test_cluster_across_the_faces_of_a_large_box(chunk):
+    """Neighbours on both sides of every face of the largest box of the
+    integer coordinates."""
+    print(f"case TEA cluster across the faces, chunk={chunk}", flush=True)
+    box = 4096.0
+    p = P.derive(dict(P.TEA, tea_epsilon_freq=1, dt=1000.0, LJPairsCutoff=8.0))
+    rng = np.random.default_rng(11)
+    at = lattice.free_dimers(150, 80.0, rng, min_sep=8.0, chain="Y")
+    b = topology.make_batch([at], [lattice.coords7(at, 0.2, rng)], box=[box])
+    x = b.coords[:, :3].astype(np.float64) - 40.0
+    b.coords[:, :3] = np.where(x < 0, x + box, x).astype(np.float32)
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    eng.set_tuning(tea_chunk=chunk)
+    F = eng.forces()[:, :3].astype(np.float64)
+    eng.set_noise(np.zeros((1, b.nb, 6), np.float32))
+    eng.run(1)
+    moved = eng.get_state()[:, :3].astype(np.float64) - b.coords[:, :3].astype(np.float64)
+    eng.close()
+    want = p.dt / p.gammaR * _drift(p, b, F)
+    tol = 1e-5 * np.abs(want).max() + 2 * 2.0 ** -24 * box
+    assert np.abs(moved - want).max() <= tol
