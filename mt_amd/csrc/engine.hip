@@ -1308,24 +1308,59 @@ static int need_mlp(mte_engine *e) {
     return MTE_OK;
 }
 
-// Device rows for the samples of a call.
-static int mlp_reserve(mte_engine *e, int64_t n) {
+static void mlp_free(float *&p) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+}
+
+// Device rows for the samples of a call, and for the outputs of `outputs`.
+static int mlp_reserve(mte_engine *e, int64_t n, int64_t outputs) {
     MlpBuffers &M = e->mlp;
-    if (n <= M.cap) return MTE_OK;
-    (void)hipStreamSynchronize(e->stream);
-    for (float **p : {&M.x, &M.t, &M.y}) {
-        if (*p) (void)hipFree(*p);
-        *p = nullptr;
+    if (n > M.cap) {
+        (void)hipStreamSynchronize(e->stream);
+        mlp_free(M.x);
+        mlp_free(M.t);
+        M.cap = 0;
+        if (hipMalloc(&M.x, sizeof(float) * (size_t)n * MLP_IN) != hipSuccess ||
+            hipMalloc(&M.t, sizeof(float) * (size_t)n * MLP_OUT) != hipSuccess) {
+            mlp_free(M.x);
+            return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
+        }
+        M.cap = n;
     }
-    M.cap = 0;
-    const size_t nn = (size_t)n;
-    if (hipMalloc(&M.x, sizeof(float) * nn * MLP_IN) != hipSuccess ||
-        hipMalloc(&M.t, sizeof(float) * nn * MLP_OUT) != hipSuccess ||
-        hipMalloc(&M.y, sizeof(float) * nn * MLP_OUT) != hipSuccess)
-        return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
-    M.cap = n;
+    if (outputs > M.ycap) {
+        (void)hipStreamSynchronize(e->stream);
+        mlp_free(M.y);
+        M.ycap = 0;
+        if (hipMalloc(&M.y, sizeof(float) * (size_t)outputs * MLP_OUT) != hipSuccess)
+            return fail(e, MTE_ERR_HIP, "MLP work space allocation failed");
+        M.ycap = outputs;
+    }
     return MTE_OK;
 }
+
+// A training call's hold on the rows and losses: on every way out it gives
+// back what the call added beyond MLP_KEEP_ROWS and MLP_KEEP_LOSSES.
+struct TrainSet {
+    mte_engine *e;
+    const int64_t cap = e->mlp.cap;
+    const int loss_cap = e->mlp.loss_cap;
+    ~TrainSet() {
+        MlpBuffers &M = e->mlp;
+        if (M.cap <= std::max(cap, MLP_KEEP_ROWS) && M.loss_cap <= std::max(loss_cap, MLP_KEEP_LOSSES)) return;
+        (void)hipStreamSynchronize(e->stream);   // an error path: the call's kernels may still run
+        if (M.cap > std::max(cap, MLP_KEEP_ROWS)) {
+            mlp_free(M.x);
+            mlp_free(M.t);
+            M.cap = 0;
+        }
+        if (M.loss_cap > std::max(loss_cap, MLP_KEEP_LOSSES)) {
+            (void)hipFree(M.loss);
+            M.loss = nullptr;
+            M.loss_cap = 0;
+        }
+    }
+};
 
 // Partial gradients of as many workgroups as training launches at most, and
 // the losses of `iters` iterations.
@@ -1390,7 +1425,7 @@ int mte_mlp_forward(mte_engine *e, const float *features, int64_t n, float *out)
     if (rc) return rc;
     if (!features || !out || n <= 0) return fail(e, MTE_ERR_ARG, "mte_mlp_forward: bad arguments");
     HIPCHK(hipSetDevice(e->device));
-    rc = mlp_reserve(e, n);
+    rc = mlp_reserve(e, n, n);
     if (rc) return rc;
     Stage st(e->device, e->stream);
     HIPCHK(st.to_device(e->mlp.x, features, sizeof(float) * MLP_IN * n));
@@ -1423,7 +1458,7 @@ int mte_mlp_loss_grad(mte_engine *e, const float *features, const float *labels,
     if (rc) return rc;
     if (!features || !labels || n <= 0) return fail(e, MTE_ERR_ARG, "mte_mlp_loss_grad: bad arguments");
     HIPCHK(hipSetDevice(e->device));
-    if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, 1))) return rc;
+    if ((rc = mlp_reserve(e, n, 0)) || (rc = mlp_reserve_train(e, 1))) return rc;
     double l = 0.0;
     Stage st(e->device, e->stream);
     HIPCHK(st.to_device(e->mlp.x, features, sizeof(float) * MLP_IN * n));
@@ -1446,7 +1481,8 @@ int mte_mlp_train(mte_engine *e, const float *features, const float *labels, int
     HIPCHK(hipSetDevice(e->device));
     // the whole training set goes to the device; batches are consecutive
     // slices, and the losses come back together at the end
-    if ((rc = mlp_reserve(e, n)) || (rc = mlp_reserve_train(e, iters))) return rc;
+    TrainSet held{e};
+    if ((rc = mlp_reserve(e, n, 0)) || (rc = mlp_reserve_train(e, iters))) return rc;
     float *X = e->mlp.x, *Y = e->mlp.t;
     Stage st(e->device, e->stream);
     HIPCHK(st.to_device(X, features, sizeof(float) * MLP_IN * n));

@@ -99,6 +99,10 @@ constexpr int CELL_TABLE_MIN = 64;   // buckets of the smallest table
 constexpr int CELL_CURSOR_STRIDE = 32;   // words between cursors: a cache line each
 
 // MLP-HI network and work buffers (mlp.hip).
+// Rows of a training set and losses that stay allocated after a training call
+// (27 MB and 0.5 MB); what a larger call took beyond them is given back.
+constexpr int64_t MLP_KEEP_ROWS = 65536;
+constexpr int MLP_KEEP_LOSSES = 65536;
 constexpr int MLP_NN = 32, MLP_IN = 96, MLP_H = 128, MLP_OUT = 9;
 constexpr int MLP_SEARCH_BLOCK = 64;   // beads per workgroup of the neighbour search
 constexpr int MLP_ERR_PARTS = 16;      // workgroups per trajectory of the judge's error sums
@@ -118,8 +122,9 @@ struct MlpBuffers {
     double *err = nullptr;                    // per trajectory: squared error, squared label norm
     double *err_part = nullptr;               // their partial sums, MLP_ERR_PARTS per trajectory
     int *nbad = nullptr;                      // beads whose prediction failed the Cholesky check
-    // samples of a call (features, labels, outputs) for up to `cap` rows
-    int64_t cap = 0;
+    // samples of a call: features and labels for up to `cap` rows, outputs
+    // for up to `ycap`
+    int64_t cap = 0, ycap = 0;
     float *x = nullptr, *t = nullptr, *y = nullptr;
     // training: partial gradients and squared errors of the workgroups, and
     // the losses of up to `loss_cap` iterations

@@ -3,6 +3,7 @@ oracle at the edges of their 32-sample tiles and of one tile per compute
 unit, and Adam training repeating itself bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 from mt_amd import params as P
 from mt_amd.engine import Engine, MLP_IN, MLP_OUT, MODE_STREAMED
@@ -60,3 +61,22 @@ def test_training_repeats_and_follows_adam():
     # each step moves a weight by at most ~lr; rounding can turn a step only
     # where the gradient is near zero
     assert np.abs(out[0][1] - w).max() < 2e-3 and np.linalg.norm(out[0][1] - w) < 1e-4 * np.linalg.norm(w)
+
+
+def test_training_gives_back_the_memory_of_a_large_set():
+    """A set of 168 MB and as many losses as fit no small buffer: after the
+    call only what small calls keep too is held."""
+    print("case MLP training memory", flush=True)
+    eng = Engine(P.derive(dict(P.TEA)), c1_batch(), mode=MODE_STREAMED)
+    eng.mlp_set_weights(M.init_weights(3))
+    x, t = np.zeros((400000, MLP_IN), np.float32), np.zeros((400000, MLP_OUT), np.float32)
+    eng.mlp_train(x[:65536], t[:65536], iters=2, batch=500, lr=1e-3)
+    before = torch.cuda.mem_get_info()[0]
+    for _ in range(2):
+        losses = eng.mlp_train(x, t, iters=3, batch=500, lr=1e-3)
+        assert np.isfinite(losses).all() and len(losses) == 3
+        assert before - torch.cuda.mem_get_info()[0] < 30e6
+    # and small calls go on
+    assert np.isfinite(eng.mlp_train(x[:1000], t[:1000], iters=2, batch=500, lr=1e-3)).all()
+    assert eng.mlp_forward(x[:100]).shape == (100, MLP_OUT)
+    eng.close()
