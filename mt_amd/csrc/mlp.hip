@@ -113,6 +113,14 @@ template <int XOR>
 __device__ __forceinline__ double quad_swap(double v) {
     return __hiloint2double(quad_swap<XOR>(__double2hiint(v)), quad_swap<XOR>(__double2loint(v)));
 }
+// Orders the LDS accesses of a wave's lanes before and after it, for values
+// that pass between lanes of one wave: the hardware keeps a wave's LDS accesses
+// in order, and this keeps the compiler from moving them.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // The value of lane L of the bead's four.
 template <int L>
 __device__ __forceinline__ int quad_lane(int v) {
@@ -335,10 +343,7 @@ __global__ void __launch_bounds__(MLP_BLOCK * MLP_LANES, 3)
         } else {
             srg[lb][part] = dup0 ? Range::none() : Range::pack(r0, base);
             srg[lb][part + 4] = dup1 ? Range::none() : Range::pack(r1, base);
-            // the four lanes are of one wave: its LDS accesses only must keep their order
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_order();   // the four lanes are of one wave
             int total = n0 + n1;
             total += quad_swap<1>(total);
             total += quad_swap<2>(total);
@@ -995,6 +1000,7 @@ __device__ __forceinline__ void tr_back(const float (&a)[MLP_H / 4], const float
         dw[mt] = tr_outer(col, b, dw[mt]);
         tr_fence();
     }
+    wave_order();   // other lanes' columns have been read: the gradients overwrite them
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     tr_rows<MLP_H>(a, gout, TR_PH, g, i, acc);
 #pragma unroll
@@ -1085,6 +1091,7 @@ __global__ void __launch_bounds__(TR_THREADS)
             tr_column(H3, TR_PH, wv, g, i, hc);
             tr_column(G, TR_PY, 0, g, i, gc);
             dw4 = tr_outer(hc, gc, dw4);
+            wave_order();   // other lanes' columns have been read: the gradients overwrite them
             f32x4 acc[2] = {zero, zero};
 #pragma unroll
             for (int sc = 0; sc < 2; sc++) {
@@ -1101,6 +1108,7 @@ __global__ void __launch_bounds__(TR_THREADS)
         tr_back(r3, H3, H2, wv, g, i, dw3, db2);
         __syncthreads();
         tr_back(r2, H2, H1, wv, g, i, dw2, db1);
+        wave_order();   // the wave's other lanes have written their gradients
         {   // layer 1: the wave's own gradient columns against every input
             float gc[8];
             tr_column(H1, TR_PH, wv, g, i, gc);
