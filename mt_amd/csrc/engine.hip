@@ -1735,14 +1735,17 @@ int mte_autotune(mte_engine *e, int32_t trial_steps, mte_tuning *chosen, char *r
         }
         if ((rc = restore()) || (rc = mte_set_tuning(e, &best))) return rc;
     } else {
-        if (e->forces_lds > 0 && (rc = family("forces", {MTE_FORCES_LDS, MTE_FORCES_GLOBAL}, &e->tune.forces)))
-            return rc;
-        if ((rc = family("stream_block", {64, 128, 256}, &e->tune.stream_block))) return rc;
+        // The pair kernel first: which force pass is the faster depends on it
+        // (MTE_FORCES_LDS with MTE_TEA_SYMMETRIC takes k_tea_turn in short
+        // trajectories); then the force pass, and the workgroup of the global one.
         if (e->periodic || e->nmax > REBUILD_ORDER_MAX) {
             if ((rc = family("tea_chunk", {64, 128, 256, MTE_TEA_SYMMETRIC}, &e->tune.tea_chunk))) return rc;
         } else if ((rc = family("tea_chunk", {64, 128, 256, MTE_TEA_SYMMETRIC, MTE_TEA_MFMA}, &e->tune.tea_chunk))) {
             return rc;
         }
+        if (e->forces_lds > 0 && (rc = family("forces", {MTE_FORCES_LDS, MTE_FORCES_GLOBAL}, &e->tune.forces)))
+            return rc;
+        if ((rc = family("stream_block", {64, 128, 256}, &e->tune.stream_block))) return rc;
     }
     if (e->mode == MTE_MODE_STREAMED && e->use_cells && need_lists &&
         (rc = family("cell_stencil", {1, 2}, &e->tune.cell_stencil)))

@@ -141,3 +141,17 @@ def test_set_tuning_rejects_unusable_shapes():
     e.set_tuning(resident_per_thread=3)
     assert e.tuning()["resident_per_thread"] == 3
     e.close()
+
+
+def test_autotune_times_the_force_passes_with_the_chosen_pair_kernel():
+    """Forces from LDS and the symmetric pair kernel together take the fused
+    end and forces of a step, so the pair kernel is chosen first; and where
+    the trials ran with LDS forces, every pair kernel was timed with them."""
+    print("case autotune order of the TEA shapes", flush=True)
+    e = Engine(P.derive(dict(P.TEA, tea_epsilon_freq=10)), c1_batch(ntraj=2), max_lj=48, mode=MODE_STREAMED)
+    assert e.tuning()["forces"] == FORCES_LDS
+    _, report = e.autotune(5)
+    e.close()
+    order = [line.split()[0] for line in report]
+    assert order == sorted(order, key=["tea_chunk", "forces", "stream_block", "cell_stencil"].index)
+    assert order.count("tea_chunk") == 5 and order.count("forces") == 2
