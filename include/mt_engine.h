@@ -97,7 +97,8 @@ typedef struct {
     const int32_t *lateral_count;       /* B */
     const int32_t *lateral;             /* B * 16 */
     const uint8_t *fixed, *extra;       /* B */
-    const int32_t *mon_type, *gtp, *on_tubule; /* B */
+    const int32_t *mon_type;            /* B: 0 (A) or 1 (B) */
+    const int32_t *gtp, *on_tubule;     /* B */
     const float *wall_z;                /* ntraj: Parameters.zs */
     const float *box;                   /* ntraj: periodic cubic box side, 0 = open (the
                                            reference has open boundaries only); may be NULL */

@@ -338,7 +338,6 @@ static void generate_seeds(int32_t seed, size_t nwords, uint32_t *out) {
 }
 
 namespace mte {
-// The list-capacity flags into the host's pinned, device-mapped words.
 // Position and angle arrays as mte_coord records (seven words: x, y, z, fi,
 // theta, psi, 0) in pinned host memory: four consecutive words per thread, so
 // that a wave's store is one run of 1 KB over the bus.
@@ -358,6 +357,8 @@ __global__ void __launch_bounds__(256) k_pack_coords(const float4 *xyz, const fl
     }
 }
 
+// The list-capacity flags and TEA's status (0 without TEA) into the host's
+// pinned, device-mapped words.
 __global__ void k_publish_flags(const int *overflow, const int *frozen, const int *tea, int *out) {
     out[0] = *(volatile const int *)overflow;
     out[1] = *(volatile const int *)frozen;

@@ -11,11 +11,17 @@
 // with D_hat_ij = D_ij/D_ii the Rotne-Prager-Yamakawa block, N the count of
 // non-extra beads of the trajectory.
 //
-// Work layout of the per-step product: work units of (trajectory, 256-bead i
-// group, j chunk of 64, 128 or 256 beads as tuned), the chunk's positions, forces and random forces in
-// LDS, FP32 partial sums per chunk reduced in fixed order by the finish kernel,
-// which adds the self term and integrates.  Each (i, j) block costs one rsqrt
-// and ~35 FP32 operations: the product is VALU-bound.
+// The per-step product has three forms (mte_tuning.tea_chunk), the first two
+// bound by VALU issue:
+//   one-sided  work units of (trajectory, 256-bead i group, j chunk of 64, 128
+//              or 256 beads), each block evaluated for i (pair_chunk);
+//   symmetric  each block evaluated once for both beads, units of a pair of
+//              64-bead chunks against a run of chunks (pair_unit);
+//   moments    products of tabulated moments on the matrix cores
+//              (k_tea_pairs_mfma).
+// Their FP32 partial sums are added in a fixed order by the kernel that ends
+// the step (k_tea_finish; k_tea_turn, which also forms the next forces), with
+// the self term, and integrated.
 #include "bead_physics.h"
 #include "engine_internal.h"
 #include <type_traits>
@@ -197,7 +203,7 @@ __global__ void __launch_bounds__(TEA_TILE)
 constexpr int eps_waves(int per) { return per == 1 ? 4 : EPS_GROUP_MAX / 64 / per; }
 // What a pair's terms need beside the beads, in loop units.
 struct EpsCoef {
-    float s2, c1, c2, c3, c4;   // a^2 and its multiples 2/3, -2, -2/3, 2
+    float c1, c2, c3, c4;       // a^2 times 2/3, -2, -2/3, 2
     float near2, ia, r2min;     // (2a)^2 with its margin, 1 / a, the floor of r^2
     float i0, i4;               // 1 / (9/16 a^2), 1 / (3/4 a)
     float side, iside;          // FLOAT_BOX: the box
@@ -276,7 +282,6 @@ __device__ __forceinline__ void eps_unit(const mte_params &P, const DevTopo &T, 
     const float sc = BOX == INT_BOX ? box * 0x1p-32f : 1.f;   // nm per loop unit
     const float a = P.tea_a / sc, s2 = a * a, lim = 2.002f * a;
     EpsCoef K;
-    K.s2 = s2;
     K.c1 = in_vgpr(0.66666666666666667f * s2);
     K.c2 = in_vgpr(-2.f * s2);
     K.c3 = in_vgpr(-0.66666666666666667f * s2);
