@@ -450,7 +450,10 @@ __global__ void __launch_bounds__(256)
     }
     if (threadIdx.x == 0) {
         const double nn = (double)cnt[0];
-        double e = red[0] / (3. * nn * (3. * nn - 3.));
+        // A trajectory of one bead (the rest extra) has no tensor to average or
+        // to check: epsilon 0 and its beta, 0.5, where 0 / 0 would lose the bead.
+        const bool alone = cnt[0] < 2;
+        double e = alone ? 0.0 : red[0] / (3. * nn * (3. * nn - 3.));
         int fail = 0;
         if (e > 1.0) {
             if (P.tea_capricious) fail = 1;
@@ -461,7 +464,7 @@ __global__ void __launch_bounds__(256)
         double bt;
         if (fabs(a) < 1e-7) {
             bt = 0.5;
-            if (P.tea_capricious && P.tea_a > 0.0f) fail = 1;
+            if (P.tea_capricious && P.tea_a > 0.0f && !alone) fail = 1;
         } else {
             bt = (1. - sqrt(1. - a)) / a;
         }

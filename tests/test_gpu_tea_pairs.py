@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from mt_amd import lattice, params as P, topology
-from mt_amd.engine import Engine, MODE_STREAMED, TEA_SYMMETRIC
+from mt_amd.engine import Engine, MODE_STREAMED, TEA_EPS_ONEPASS, TEA_EPS_TWOSIDED, TEA_SYMMETRIC
 from oracle.oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -263,3 +263,36 @@ def test_cluster_across_the_faces_of_a_large_box(chunk):
     want = p.dt / p.gammaR * _drift(p, b, F)
     tol = 1e-5 * np.abs(want).max() + 2 * 2.0 ** -24 * box
     assert np.abs(moved - want).max() <= tol
+
+
+@pytest.mark.parametrize("box", [0.0, 60.0])
+@pytest.mark.parametrize("eps", [TEA_EPS_ONEPASS, TEA_EPS_TWOSIDED])
+@pytest.mark.parametrize("capricious", [False, True])
+def test_a_bead_alone_in_its_trajectory_drains_freely(box, eps, capricious):
+    """Dimers of which one bead, or both, are extra, beside whole ones: a
+    bead with no other to meet has beta 0.5, ci 0 and moves by its own force
+    and noise."""
+    print(f"case TEA bead alone, box={box}, eps={eps}, capricious={capricious}", flush=True)
+    p = P.derive(dict(P.TEA, tea_epsilon_freq=1, tea_capricious=capricious))
+    b = _dimers((1,) * 40 + (20,), box, 9)
+    one, none = np.arange(1, 40, 4), np.arange(2, 40, 4)   # trajectories with one bead left, with none
+    b.extra[b.off[one]] = 1
+    for k in (0, 1):
+        b.extra[b.off[none] + k] = 1
+    eng = Engine(p, b.copy(), mode=MODE_STREAMED)
+    eng.set_tuning(tea_chunk=TEA_SYMMETRIC, tea_eps=eps)
+    F = eng.forces()[:, :3].astype(np.float64)
+    nz = np.random.default_rng(1).standard_normal((1, b.nb, 6)).astype(np.float32)
+    eng.set_noise(nz)
+    eng.run(1)
+    e, beta = eng.tea_stats()
+    got = eng.get_state()
+    assert np.isfinite(got).all() and np.isfinite(e).all() and np.isfinite(beta).all()
+    np.testing.assert_array_equal(e[np.r_[one, none]], 0.0)
+    np.testing.assert_array_equal(beta[np.r_[one, none]], 0.5)
+    i = b.off[one] + 1
+    np.testing.assert_allclose(eng.tea_ci()[i], 0.0, atol=1e-6)
+    moved = got[i, :3].astype(np.float64) - b.coords[i, :3]
+    want = p.dt / p.gammaR * F[i] + p.varR * nz[0, i, :3]
+    assert np.abs(moved - want).max() <= 1e-5 * np.abs(want).max() + 2 * 2.0 ** -24 * np.abs(b.coords[:, :3]).max()
+    eng.close()
