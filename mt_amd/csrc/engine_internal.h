@@ -99,10 +99,6 @@ constexpr int CELL_TABLE_MIN = 64;   // buckets of the smallest table
 constexpr int CELL_CURSOR_STRIDE = 32;   // words between cursors: a cache line each
 
 // MLP-HI network and work buffers (mlp.hip).
-// Rows of a training set and losses that stay allocated after a training call
-// (27 MB and 0.5 MB); what a larger call took beyond them is given back.
-constexpr int64_t MLP_KEEP_ROWS = 65536;
-constexpr int MLP_KEEP_LOSSES = 65536;
 constexpr int MLP_NN = 32, MLP_IN = 96, MLP_H = 128, MLP_OUT = 9;
 constexpr int MLP_SEARCH_BLOCK = 64;   // beads per workgroup of the neighbour search
 constexpr int MLP_ERR_PARTS = 16;      // workgroups per trajectory of the judge's error sums
@@ -111,6 +107,10 @@ constexpr int MLP_NPARAM = MLP_IN * MLP_H + MLP_H + 2 * (MLP_H * MLP_H + MLP_H) 
 // and the device ordinals whose array address is kept.
 constexpr int MLP_NOALLOC_ROWS = MTE_MLP_NOALLOC_ROWS;
 constexpr int MLP_NOALLOC_MAX_DEVICES = 64;
+// Rows of a training set and losses that stay allocated after a training call
+// (27 MB and 0.5 MB); what a larger call took beyond them is given back.
+constexpr int64_t MLP_KEEP_ROWS = 65536;
+constexpr int MLP_KEEP_LOSSES = 65536;
 struct MlpBuffers {
     float *w = nullptr, *wi = nullptr;        // FP32 master weights, bf16-rounded copy for inference
     uint4 *img = nullptr;                     // inference image: bf16 MFMA fragments + biases (mlp_image_bytes())
